@@ -110,6 +110,25 @@ struct rf_blend_plan {
 hipError_t rf_launch_blend_dev(const rf_blend_dev& b, void* d_group, int dtype, hipStream_t s);
 int rf_moments_parts(int64_t N);
 int rf_corr_parts(int64_t N);
+// Correlations of several axes of one field by one matrix-core launch
+// (k_corr_gram).  An axis qualifies with 2 .. kCorrGramMaxN points (beyond,
+// the partial sums of its tile pairs outgrow the field) and
+// kCorrGramMinLines lines or more (fewer leave the instruction's K empty).
+constexpr int kCorrGramMaxN = 2048;
+constexpr int64_t kCorrGramMinLines = 16;
+struct rf_corr_axis {
+    int n, nS, pairs, chunks;   // points, 64-point tiles, tile pairs, shares of the lines per pair
+    int block0, lag0, out0;     // first block, first lag of the final launch, first output element
+    int64_t stride, nLines;
+};
+struct rf_corr_gram {
+    int nAx, blocks, lags;
+    rf_corr_axis ax[3];
+};
+bool rf_corr_gram_add(rf_corr_gram* q, int n, int64_t stride, int64_t N, int out0);
+size_t rf_corr_gram_plan(rf_corr_gram* q);   // doubles of partial sums
+hipError_t rf_launch_corr_gram(const rf_corr_gram& q, const void* u, int dtype, int64_t N, double avg, double std,
+                               double* d_part, double* d_R, hipStream_t s);
 hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, const double* xMin,
                             const double* xStep, int Nmc, const void* grid, int gridDtype, const double* x,
                             int64_t nNodes, void* out, int outDtype, int* d_flag, hipStream_t s);

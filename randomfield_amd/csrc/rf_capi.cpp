@@ -125,6 +125,7 @@ int rf_context_destroy(rf_context* ctx) {
     }
     dfree(ctx->d_scratch);
     dfree(ctx->d_io);
+    if (ctx->h_res) (void)hipHostFree(ctx->h_res);
     delete ctx;
     return RF_OK;
 }
@@ -831,6 +832,28 @@ int ensure_scratch(rf_context* ctx, size_t bytes) {
     return RF_OK;
 }
 
+// Where a synchronous call's `count` doubles are formed: the context's pinned
+// buffer when they fit (the last kernel writes them to host memory, no copy
+// to pageable memory: 15 us less per call), else the device buffer d_own.
+double* result_target(rf_context* ctx, size_t count, double* d_own) {
+    if (count > kResDoubles) return d_own;
+    if (!ctx->h_res &&
+        hipHostMalloc((void**)&ctx->h_res, kResDoubles * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->h_res = nullptr;
+    }
+    return ctx->h_res ? ctx->h_res : d_own;
+}
+
+// Waits for the stream and brings the doubles formed at `target` to host[].
+int result_fetch(rf_context* ctx, const double* target, size_t count, double* host, hipStream_t s) {
+    if (target != ctx->h_res)
+        RF_HIP_TRY(ctx, hipMemcpyAsync(host, target, count * sizeof(double), hipMemcpyDeviceToHost, s));
+    RF_HIP_TRY(ctx, hipStreamSynchronize(s));
+    if (target == ctx->h_res) std::memcpy(host, target, count * sizeof(double));
+    return RF_OK;
+}
+
 // Sums of u and u^2 per realization into host sums[2*Nmc] (synchronous).
 int moments(rf_context* ctx, const void* d, int64_t N, int Nmc, int dtype, hipStream_t s,
             std::vector<double>* sums) {
@@ -839,12 +862,10 @@ int moments(rf_context* ctx, const void* d, int64_t N, int Nmc, int dtype, hipSt
     int rc = ensure_scratch(ctx, bytes);
     if (rc) return rc;
     double* part = static_cast<double*>(ctx->d_scratch);
-    double* dsum = part + (size_t)nPart * Nmc * 2;
+    double* dsum = result_target(ctx, (size_t)Nmc * 2, part + (size_t)nPart * Nmc * 2);
     RF_HIP_TRY(ctx, rf_launch_moments(d, N, Nmc, dtype, part, nPart, dsum, s));
     sums->resize((size_t)Nmc * 2);
-    RF_HIP_TRY(ctx, hipMemcpyAsync(sums->data(), dsum, sizeof(double) * Nmc * 2, hipMemcpyDeviceToHost, s));
-    RF_HIP_TRY(ctx, hipStreamSynchronize(s));
-    return RF_OK;
+    return result_fetch(ctx, dsum, (size_t)Nmc * 2, sums->data(), s);
 }
 
 }  // namespace
@@ -883,32 +904,48 @@ int rf_corr_device(rf_context* ctx, const void* d_field, int32_t dtype, int32_t 
     if (dtype != RF_DTYPE_F64 && dtype != RF_DTYPE_F32) return rf_set_error(ctx, RF_E_ARG, "unknown dtype");
     if (!(std > 0.0) || realization < 0) return rf_set_error(ctx, RF_E_ARG, "std must be > 0, realization >= 0");
     int64_t N = 1, stride[3] = {1, 1, 1};
-    int Mtot = 0, Mmax = 0;
+    int Mtot = 0;
     for (int a = 0; a < nDim; a++) {
         if (nstep[a] < 1) return rf_set_error(ctx, RF_E_ARG, "grid counts must be >= 1");
         if (a > 0) stride[a] = stride[a - 1] * nstep[a - 1];
         N *= nstep[a];
         Mtot += nstep[a] / 2;
-        Mmax = std::max(Mmax, nstep[a] / 2);
     }
     RF_HIP_TRY(ctx, hipSetDevice(ctx->device));
     const hipStream_t s = ctx->stream;
-    const int nPart = rf_corr_parts(N);
-    const size_t bytes = sizeof(double) * ((size_t)nPart * Mmax + (size_t)Mtot);
-    int rc = ensure_scratch(ctx, bytes);
-    if (rc) return rc;
-    double* part = static_cast<double*>(ctx->d_scratch);
-    double* dR = part + (size_t)nPart * Mmax;
-    const size_t esz = dtype == RF_DTYPE_F64 ? 8 : 4;
-    const void* u = static_cast<const char*>(d_field) + (size_t)realization * N * esz;
-    int off = 0;
+    // the matrix-core pass for the axes it takes, a sweep per lag for the rest
+    rf_corr_gram gram{};
+    bool sweep[3] = {false, false, false};
+    int off = 0, Msweep = 0;
     for (int a = 0; a < nDim; a++) {
         const int M = nstep[a] / 2;
-        RF_HIP_TRY(ctx, rf_launch_corr(u, dtype, N, stride[a], nstep[a], M, avg, std, part, nPart, dR + off, s));
+        if (M > 0 && !rf_corr_gram_add(&gram, nstep[a], stride[a], N, off)) {
+            sweep[a] = true;
+            Msweep = std::max(Msweep, M);
+        }
         off += M;
     }
-    RF_HIP_TRY(ctx, hipMemcpyAsync(R, dR, sizeof(double) * Mtot, hipMemcpyDeviceToHost, s));
-    RF_HIP_TRY(ctx, hipStreamSynchronize(s));
+    const int nPart = rf_corr_parts(N);
+    const size_t nGram = gram.nAx ? rf_corr_gram_plan(&gram) : 0, nSweep = (size_t)nPart * Msweep;
+    int rc = ensure_scratch(ctx, sizeof(double) * (nGram + nSweep + (size_t)Mtot + 1));
+    if (rc) return rc;
+    double* partG = static_cast<double*>(ctx->d_scratch);
+    double* partS = partG + nGram;
+    double* dR = result_target(ctx, (size_t)Mtot, partS + nSweep);
+    const size_t esz = dtype == RF_DTYPE_F64 ? 8 : 4;
+    const void* u = static_cast<const char*>(d_field) + (size_t)realization * N * esz;
+    RF_HIP_TRY(ctx, rf_launch_corr_gram(gram, u, dtype, N, avg, std, partG, dR, s));
+    off = 0;
+    for (int a = 0; a < nDim; a++) {
+        const int M = nstep[a] / 2;
+        if (sweep[a])
+            RF_HIP_TRY(ctx, rf_launch_corr(u, dtype, N, stride[a], nstep[a], M, avg, std, partS, nPart, dR + off, s));
+        off += M;
+    }
+    if (Mtot > 0) {
+        rc = result_fetch(ctx, dR, (size_t)Mtot, R, s);
+        if (rc) return rc;
+    }
     // rebuild_corrL (statistics_RF.f90:438-445): twice the trapezoid of R
     if (corrL) {
         const double* r = R;

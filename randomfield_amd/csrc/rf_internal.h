@@ -39,7 +39,9 @@ struct rf_context {
     uint64_t useClock = 0;
     void* d_io = nullptr;        // host-buffer entry points' points and outputs (grown on demand)
     size_t ioBytes = 0;
+    double* h_res = nullptr;     // pinned results of the synchronous statistics (kResDoubles)
 };
+constexpr size_t kResDoubles = 4096;
 constexpr size_t kPlanCache = 4;
 
 // Host-side spectrum: the wavevector table in coordinates normalised by corrL.

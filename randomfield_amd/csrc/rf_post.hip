@@ -58,21 +58,53 @@ __global__ __launch_bounds__(kBlock) void k_marginal_vec(int margi, double scale
 }
 
 // Per-realization partial sums of u and u^2 in FP64; grid (nPart, Nmc).
-template <typename T>
+// Sums of u and u^2 of each realization (grid y); grid (nPart, Nmc).  Bound by
+// the read: two independent 16-byte loads per thread and turn where every
+// realization starts on a 16-byte boundary (VEC), one element otherwise
+// (128^3 x 16 FP32: 27 -> 22 us, 6.0 TB/s).
+template <typename T, bool VEC>
 __global__ __launch_bounds__(kBlock) void k_moments_partial(const T* __restrict__ d, int64_t N,
                                                             double* __restrict__ part) {
+    constexpr int L = VEC ? 16 / sizeof(T) : 1;
+    typedef T vec __attribute__((ext_vector_type(L)));
     __shared__ double s1[kBlock], s2[kBlock];
     const int r = blockIdx.y;
     const T* col = d + (int64_t)r * N;
-    double a = 0.0, b = 0.0;
+    double a = 0.0, b = 0.0, a2 = 0.0, b2 = 0.0;
     const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < N; i += stride) {
+    const int64_t nV = N / L;
+    int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (VEC) {
+        const vec* cv = reinterpret_cast<const vec*>(col);
+        for (; i + stride < nV; i += 2 * stride) {
+            const vec v = cv[i], w = cv[i + stride];
+#pragma unroll
+            for (int l = 0; l < L; l++) {
+                const double x = (double)v[l], y = (double)w[l];
+                a += x;
+                b = fma(x, x, b);
+                a2 += y;
+                b2 = fma(y, y, b2);
+            }
+        }
+        if (i < nV) {
+            const vec v = cv[i];
+#pragma unroll
+            for (int l = 0; l < L; l++) {
+                const double x = (double)v[l];
+                a += x;
+                b = fma(x, x, b);
+            }
+        }
+        i = nV * L + (int64_t)blockIdx.x * kBlock + threadIdx.x;   // the last N % L elements
+    }
+    for (; i < N; i += stride) {
         const double v = (double)col[i];
         a += v;
         b = fma(v, v, b);
     }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
+    s1[threadIdx.x] = a + a2;
+    s2[threadIdx.x] = b + b2;
     __syncthreads();
     for (int w = kBlock / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) {
@@ -123,18 +155,30 @@ __global__ __launch_bounds__(kBlock) void k_window_moments_partial(const T* __re
     }
 }
 
-// Fixed-order final reduction of the partials: sums[r] = (sum u, sum u^2).
-__global__ void k_moments_final(const double* __restrict__ part, int nPart, int Nmc,
-                                double* __restrict__ sums) {
-    const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (r >= Nmc) return;
+// Sum over a wave, the same order on every run; the result is in every lane.
+__device__ inline double wave_sum(double v) {
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) v += __shfl_xor(v, w);
+    return v;
+}
+
+// Fixed-order final reduction of the partials: sums[r] = (sum u, sum u^2),
+// one wave per realization (a serial chain over the 256 partials of a large
+// field took 26 us; 3 us so).
+__global__ __launch_bounds__(64) void k_moments_final(const double* __restrict__ part, int nPart,
+                                                      double* __restrict__ sums) {
+    const int r = blockIdx.x;
     double a = 0.0, b = 0.0;
-    for (int p = 0; p < nPart; p++) {
+    for (int p = threadIdx.x; p < nPart; p += 64) {
         a += part[((int64_t)r * nPart + p) * 2 + 0];
         b += part[((int64_t)r * nPart + p) * 2 + 1];
     }
-    sums[2 * r + 0] = a;
-    sums[2 * r + 1] = b;
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (threadIdx.x == 0) {
+        sums[2 * r + 0] = a;
+        sums[2 * r + 1] = b;
+    }
 }
 
 // u <- (u - shift_r) * mul_r
@@ -180,13 +224,172 @@ __global__ __launch_bounds__(kBlock) void k_corr_partial(const T* __restrict__ u
     if (threadIdx.x == 0) part[(int64_t)m * gridDim.x + blockIdx.x] = sh[0];
 }
 
-__global__ void k_corr_final(const double* __restrict__ part, int nPart, int M, double invN,
-                             double* __restrict__ R) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M) return;
+// One wave per lag (grid x), partials in fixed order.
+__global__ __launch_bounds__(64) void k_corr_final(const double* __restrict__ part, int nPart, double invN,
+                                                   double* __restrict__ R) {
+    const int m = blockIdx.x;
     double s = 0.0;
-    for (int p = 0; p < nPart; p++) s += part[(int64_t)m * nPart + p];
-    R[m] = s * invN;
+    for (int p = threadIdx.x; p < nPart; p += 64) s += part[(int64_t)m * nPart + p];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) R[m] = s * invN;
+}
+
+// The same correlations through the FP64 matrix cores.  With v_l the
+// normalised values of line l along the axis, G = sum_l v_l v_l^T holds every
+// product of two points of a line; the lag m is the sum of G over j - i = m and
+// j - i = m - n.  One pass over the field gives all lags, where the lag
+// sweep above reads it twice per lag.  A block holds the tile pair (SI, SJ),
+// SI <= SJ, of 64 positions each, and a share of the lines: 16 accumulator
+// tiles of v_mfma_f64_16x16x4_f64 per wave, whose A and B operands have the
+// same lane layout (position l % 16, line l / 16), so the fragments come
+// straight from global memory and one load serves a row and a column of
+// tiles.  The four lines of lane group g and step t are 4 g + t: 16
+// neighbouring lines per turn, contiguous for every axis but the first.  Bound
+// by the matrix cores (16 MFMAs of 64 cycles per 8 fragments); all axes of a
+// field share one launch.  128^3 FP32: 3 x 307 us (the sweep) -> 56 us.
+typedef double d4v __attribute__((ext_vector_type(4)));
+constexpr int kCorrT = 64;                 // positions per side of a tile pair
+constexpr int kCorrDiag = 2 * kCorrT;      // partial sums per block: j - i + 63 in 0 .. 126
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_corr_gram(rf_corr_gram q, const T* __restrict__ u, double avg, double std, double* __restrict__ part) {
+    __shared__ double tile[4][7 * 256];
+    __shared__ double diag[4][kCorrDiag];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int c = lane & 15, g = lane >> 4;
+    int ax = 0;
+    while (ax + 1 < q.nAx && (int)blockIdx.x >= q.ax[ax + 1].block0) ax++;
+    const rf_corr_axis A = q.ax[ax];
+    const int local = (int)blockIdx.x - A.block0;
+    const int chunk = local % A.chunks;
+    // tile pair: distance-major, pair(D, SI) = sum_{k < D} (nS - k) + SI
+    int SI = local / A.chunks, D = 0;
+    while (SI >= A.nS - D) {
+        SI -= A.nS - D;
+        D++;
+    }
+    const int SJ = SI + D;
+    const int pi = SI * kCorrT + c, pj = SJ * kCorrT + c;
+
+    // the lane's four lines, as (offset of the line's first point, index along
+    // the faster axes); 64 * chunks lines further on every turn
+    const int64_t S = A.stride, hop = S * (A.n - 1);
+    const int64_t dq = (int64_t)64 * A.chunks;
+    const int64_t dO = dq / S, dX = dq - dO * S;
+    int64_t line = (int64_t)(chunk * 4 + wave) * 16 + 4 * g;
+    int64_t x[4], base[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int64_t o = (line + t) / S;
+        x[t] = (line + t) - o * S;
+        base[t] = o * S * A.n + x[t];
+    }
+    d4v acc[4][4];
+#pragma unroll
+    for (int I = 0; I < 4; I++)
+#pragma unroll
+        for (int J = 0; J < 4; J++) acc[I][J] = d4v{0.0, 0.0, 0.0, 0.0};
+
+    const int64_t turns = (A.nLines - (int64_t)(chunk * 4 + wave) * 16 + dq - 1) / dq;   // wave-uniform
+    for (int64_t it = 0; it < turns; it++) {
+        T a[4][4], b[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const bool in = line + t < A.nLines;
+            const T* p = u + (in ? base[t] : 0);
+#pragma unroll
+            for (int I = 0; I < 4; I++) {
+                const int i = pi + 16 * I, j = pj + 16 * I;
+                a[t][I] = p[in && i < A.n ? i * S : 0];
+                b[t][I] = D == 0 ? a[t][I] : p[in && j < A.n ? j * S : 0];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const bool in = line + t < A.nLines;
+            double va[4], vb[4];
+#pragma unroll
+            for (int I = 0; I < 4; I++) {
+                va[I] = in && pi + 16 * I < A.n ? ((double)a[t][I] - avg) / std : 0.0;
+                if (D == 0) vb[I] = va[I];
+                else vb[I] = in && pj + 16 * I < A.n ? ((double)b[t][I] - avg) / std : 0.0;
+            }
+#pragma unroll
+            for (int I = 0; I < 4; I++)
+#pragma unroll
+                for (int J = 0; J < 4; J++)
+                    if (I <= J || D != 0)
+                        acc[I][J] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[I], vb[J], acc[I][J], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            x[t] += dX;
+            base[t] += dO * S * A.n + dX;
+            if (x[t] >= S) {
+                x[t] -= S;
+                base[t] += hop;
+            }
+        }
+        line += dq;
+    }
+
+    // tiles of equal J - I added up, then each diagonal of the wave's sums.
+    // Positions past the axis end enter no diagonal (a product with a value
+    // that is not finite is not zero there).
+    for (int k = -3; k <= 3; k++) {
+        d4v s = {0.0, 0.0, 0.0, 0.0};
+        if (k >= 0 || D != 0) {
+#pragma unroll
+            for (int I = 0; I < 4; I++)
+#pragma unroll
+                for (int J = 0; J < 4; J++)
+                    if (J - I == k) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            if (pi - c + 16 * I + 4 * e + g < A.n && pj + 16 * J < A.n) s[e] += acc[I][J][e];
+                    }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) tile[wave][(k + 3) * 256 + (4 * e + g) * 16 + c] = s[e];   // row 4 e + g, column c
+    }
+    __syncthreads();
+    for (int t = lane; t < kCorrDiag - 1; t += 64) {
+        const int d = t - (kCorrT - 1);
+        const int k = (d + 64) / 16 - 4, rem = d - 16 * k;            // d = 16 k + rem, 0 <= rem < 16
+        double s = 0.0;
+        if (d >= 0 || D != 0) {
+            if (k >= -3)
+                for (int r = 0; r + rem < 16; r++) s += tile[wave][(k + 3) * 256 + r * 16 + r + rem];
+            if (rem > 0 && k + 1 <= 3)
+                for (int r = 16 - rem; r < 16; r++) s += tile[wave][(k + 4) * 256 + r * 16 + r + rem - 16];
+        }
+        diag[wave][t] = s;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kCorrDiag - 1; t += kBlock)
+        part[(int64_t)blockIdx.x * kCorrDiag + t] = ((diag[0][t] + diag[1][t]) + diag[2][t]) + diag[3][t];
+}
+
+// R[m] of every axis from the blocks' diagonals: one wave per lag, fixed order.
+__global__ __launch_bounds__(64) void k_corr_gram_final(rf_corr_gram q, const double* __restrict__ part,
+                                                        double invN, double* __restrict__ R) {
+    int ax = 0;
+    while (ax + 1 < q.nAx && (int)blockIdx.x >= q.ax[ax + 1].lag0) ax++;
+    const rf_corr_axis A = q.ax[ax];
+    const int m = (int)blockIdx.x - A.lag0;
+    double s = 0.0;
+    for (int h = 0; h < (m > 0 ? 2 : 1); h++) {
+        const int d = h ? A.n - m : m;                  // j - i = d, lag m or n - m
+        for (int D = d / kCorrT; D <= (d + kCorrT - 1) / kCorrT && D < A.nS; D++) {
+            const int64_t b0 = A.block0 + (int64_t)(D * A.nS - D * (D - 1) / 2) * A.chunks;
+            const int64_t nB = (int64_t)(A.nS - D) * A.chunks;
+            const int t = d - D * kCorrT + kCorrT - 1;
+            for (int64_t b = threadIdx.x; b < nB; b += 64) s += part[(b0 + b) * kCorrDiag + t];
+        }
+    }
+    s = wave_sum(s);
+    if (threadIdx.x == 0) R[A.out0 + m] = s * invN;
 }
 
 // ------------------------------------------------ interpolation to nodes
@@ -604,14 +807,17 @@ int rf_moments_parts(int64_t N) {
 hipError_t rf_launch_moments(const void* d, int64_t N, int Nmc, int dtype, double* d_part,
                              int nPart, double* d_sums, hipStream_t s) {
     dim3 grid((unsigned)nPart, (unsigned)Nmc);
-    if (dtype == RF_DTYPE_F64)
-        hipLaunchKernelGGL(k_moments_partial<double>, grid, dim3(kBlock), 0, s,
-                           static_cast<const double*>(d), N, d_part);
+    const size_t esz = dtype == RF_DTYPE_F64 ? 8 : 4;
+    const bool vec = (uintptr_t)d % 16 == 0 && (Nmc == 1 || (size_t)N * esz % 16 == 0);
+    if (dtype == RF_DTYPE_F64 && vec)
+        hipLaunchKernelGGL((k_moments_partial<double, true>), grid, dim3(kBlock), 0, s, static_cast<const double*>(d), N, d_part);
+    else if (dtype == RF_DTYPE_F64)
+        hipLaunchKernelGGL((k_moments_partial<double, false>), grid, dim3(kBlock), 0, s, static_cast<const double*>(d), N, d_part);
+    else if (vec)
+        hipLaunchKernelGGL((k_moments_partial<float, true>), grid, dim3(kBlock), 0, s, static_cast<const float*>(d), N, d_part);
     else
-        hipLaunchKernelGGL(k_moments_partial<float>, grid, dim3(kBlock), 0, s,
-                           static_cast<const float*>(d), N, d_part);
-    hipLaunchKernelGGL(k_moments_final, dim3((unsigned)((Nmc + 63) / 64)), dim3(64), 0, s, d_part,
-                       nPart, Nmc, d_sums);
+        hipLaunchKernelGGL((k_moments_partial<float, false>), grid, dim3(kBlock), 0, s, static_cast<const float*>(d), N, d_part);
+    hipLaunchKernelGGL(k_moments_final, dim3((unsigned)Nmc), dim3(64), 0, s, d_part, nPart, d_sums);
     return hipGetLastError();
 }
 
@@ -623,7 +829,7 @@ hipError_t rf_launch_window_moments(const void* d, int dtype, const rf_window& w
     else
         hipLaunchKernelGGL(k_window_moments_partial<float>, dim3((unsigned)nPart), dim3(kBlock), 0, s,
                            static_cast<const float*>(d), w, d_part);
-    hipLaunchKernelGGL(k_moments_final, dim3(1), dim3(64), 0, s, d_part, nPart, 1, d_sums);
+    hipLaunchKernelGGL(k_moments_final, dim3(1), dim3(64), 0, s, d_part, nPart, d_sums);
     return hipGetLastError();
 }
 
@@ -668,8 +874,52 @@ hipError_t rf_launch_corr(const void* u, int dtype, int64_t N, int64_t strideA, 
     else
         hipLaunchKernelGGL(k_corr_partial<float>, grid, dim3(kBlock), 0, s, static_cast<const float*>(u), N,
                            strideA, nA, avg, std, d_part);
-    hipLaunchKernelGGL(k_corr_final, dim3((unsigned)((M + 63) / 64)), dim3(64), 0, s, d_part, nPart, M,
-                       1.0 / (double)N, d_R);
+    hipLaunchKernelGGL(k_corr_final, dim3((unsigned)M), dim3(64), 0, s, d_part, nPart, 1.0 / (double)N, d_R);
+    return hipGetLastError();
+}
+
+bool rf_corr_gram_add(rf_corr_gram* q, int n, int64_t stride, int64_t N, int out0) {
+    const int64_t nLines = N / n;
+    const int nS = (n + kCorrT - 1) / kCorrT;
+    if (n < 2 || n > kCorrGramMaxN || nLines < kCorrGramMinLines) return false;
+    rf_corr_axis& A = q->ax[q->nAx++];
+    A.n = n;
+    A.stride = stride;
+    A.nLines = nLines;
+    A.nS = nS;
+    A.pairs = nS * (nS + 1) / 2;
+    A.out0 = out0;
+    return true;
+}
+
+// Shares of the lines per tile pair: about 512 blocks in all (two 4-wave
+// blocks per CU), at least four turns of 64 lines per block.
+size_t rf_corr_gram_plan(rf_corr_gram* q) {
+    int pairs = 0;
+    for (int a = 0; a < q->nAx; a++) pairs += q->ax[a].pairs;
+    q->blocks = q->lags = 0;
+    for (int a = 0; a < q->nAx; a++) {
+        rf_corr_axis& A = q->ax[a];
+        const int64_t most = (A.nLines + 255) / 256, even = 512 / pairs > 1 ? 512 / pairs : 1;
+        A.chunks = (int)(most < even ? most : even);
+        A.block0 = q->blocks;
+        A.lag0 = q->lags;
+        q->blocks += A.pairs * A.chunks;
+        q->lags += A.n / 2;
+    }
+    return (size_t)q->blocks * kCorrDiag;
+}
+
+hipError_t rf_launch_corr_gram(const rf_corr_gram& q, const void* u, int dtype, int64_t N, double avg, double std,
+                               double* d_part, double* d_R, hipStream_t s) {
+    if (q.blocks <= 0) return hipSuccess;
+    if (dtype == RF_DTYPE_F64)
+        hipLaunchKernelGGL(k_corr_gram<double>, dim3((unsigned)q.blocks), dim3(kBlock), 0, s, q,
+                           static_cast<const double*>(u), avg, std, d_part);
+    else
+        hipLaunchKernelGGL(k_corr_gram<float>, dim3((unsigned)q.blocks), dim3(kBlock), 0, s, q,
+                           static_cast<const float*>(u), avg, std, d_part);
+    hipLaunchKernelGGL(k_corr_gram_final, dim3((unsigned)q.lags), dim3(64), 0, s, q, d_part, 1.0 / (double)N, d_R);
     return hipGetLastError();
 }
 
