@@ -42,7 +42,9 @@ int build_form_operands(rf_field_plan* P, hipStream_t s) {
     const int64_t kN = P->spec.info.kNTotal;
     const int Nmc = P->p.Nmc;
     const double ampMult = P->spec.info.ampMult;
-    if (P->p.form == RF_FORM_FP32) {
+    if (P->p.form == RF_FORM_FP64) {
+        RF_HIP_TRY(ctx, rf_launch_prep_fp64(kN, Nmc, P->Rpad, is_iso_direct(P->p), P->d_phase, P->d_amp, P->d_CS, s));
+    } else if (P->p.form == RF_FORM_FP32) {
         if (is_iso_direct(P->p)) {
             if (!P->d_kIsoT) RF_HIP_TRY(ctx, dmalloc(&P->d_kIsoT, (size_t)(kN * P->Rpad * P->p.nDim)));
             RF_HIP_TRY(ctx, rf_launch_prep_fp32_iso(P->p.nDim, kN, Nmc, P->Rpad, P->d_kIso, P->d_phase,
@@ -166,7 +168,7 @@ int rf_plan_destroy(rf_field_plan* P) {
     }
     dfree(P->d_k); dfree(P->d_kRad); dfree(P->d_kRev); dfree(P->d_kIso); dfree(P->d_kIsoT);
     dfree(P->d_phase); dfree(P->d_amp); dfree(P->d_uni); dfree(P->d_phT);
-    dfree(P->d_aT); dfree(P->d_B); dfree(P->d_Sk); dfree(P->d_calc); dfree(P->d_gridScratch);
+    dfree(P->d_aT); dfree(P->d_B); dfree(P->d_CS); dfree(P->d_Sk); dfree(P->d_calc); dfree(P->d_gridScratch);
     if (P->d_gridCoef) (void)hipFree(P->d_gridCoef);
     delete P;
     return RF_OK;
@@ -229,7 +231,8 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
     RF_HIP_TRY(ctx, hipMemcpyAsync(P->d_calc, P->calc.data(), (size_t)Nmc, hipMemcpyHostToDevice, s));
 
     const bool mfma = (p->form == RF_FORM_MFMA_F16 || p->form == RF_FORM_MFMA_BF16);
-    P->Rpad = mfma ? rf_mfma_npad(Nmc) : round_up(Nmc, rf_fp32_rchunk());
+    P->Rpad = mfma ? rf_mfma_npad(Nmc)
+                   : p->form == RF_FORM_FP64 ? rf_fp64_rpad(Nmc, is_iso_direct(*p)) : round_up(Nmc, rf_fp32_rchunk());
     P->kNpad = mfma ? (kN + rf_mfma_kpad(p->form) - 1) / rf_mfma_kpad(p->form) * rf_mfma_kpad(p->form) : kN;
 
     double maxAmp = 0.0;
@@ -295,6 +298,11 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
     }
 
     // operand buffers of the chosen form
+    if (p->form == RF_FORM_FP64) {
+        // isotropic: the components are bounded by the radii
+        for (double v : P->spec.k) P->kAbsMax = std::max(P->kAbsMax, std::fabs(v));
+        RF_HIP_TRY(ctx, dmalloc(&P->d_CS, (size_t)(kN * P->Rpad)));
+    }
     if (p->form == RF_FORM_FP32) {
         RF_HIP_TRY(ctx, dmalloc(&P->d_phT, (size_t)(kN * P->Rpad)));
         RF_HIP_TRY(ctx, dmalloc(&P->d_aT, (size_t)(kN * P->Rpad)));
@@ -362,8 +370,8 @@ int rf_plan_execute(rf_field_plan* P, const double* d_x, int64_t N, void* d_out,
         hipError_t e = hipSuccess;
         switch (p.form) {
             case RF_FORM_FP64:
-                if (is_iso_direct(p)) e = rf_launch_sum_fp64(a, P->d_kIso, kN * p.nDim, P->d_amp, P->d_phase, s);
-                else e = rf_launch_sum_fp64(a, P->d_k, 0, P->d_amp, P->d_phase, s);
+                e = rf_launch_sum_fp64(a, is_iso_direct(p) ? P->d_kIso : P->d_k, is_iso_direct(p), P->kAbsMax, P->d_calc,
+                                       P->d_CS, P->Rpad, s);
                 break;
             case RF_FORM_FP32:
                 if (is_iso_direct(p)) e = rf_launch_sum_fp32_iso_t(a, P->d_kIsoT, P->d_phT, P->d_aT, P->Rpad, s);

@@ -78,6 +78,8 @@ struct rf_field_plan {
     float* d_phT = nullptr;      // kN x Rpad   FP32 phase in revolutions
     float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult
     void* d_B = nullptr;         // MFMA coefficient panels (hi, lo)
+    double2* d_CS = nullptr;     // FP64 form: (amp cos phase, -amp sin phase)
+    double kAbsMax = 0.0;        // bound of the wavevector components (normalised units)
     int Rpad = 0;
     int64_t kNpad = 0;
     double bScale = 1.0;         // power-of-two scale folded into B
@@ -136,8 +138,15 @@ struct rf_sum_args {
     void* out;
     int outDtype;
 };
-hipError_t rf_launch_sum_fp64(const rf_sum_args& a, const double* d_k, int64_t kStrideR,
-                              const double* d_amp, const double* d_phase, hipStream_t s);
+// FP64 form: coefficients (a cos phi, -a sin phi) [kN][Rpad], or [Nmc][kN]
+// with per-realization wavevectors (iso); bound = max |k component|; masked
+// realizations (d_calc 0) are zero
+int rf_fp64_rchunk(int Nmc);
+int rf_fp64_rpad(int Nmc, int iso);
+hipError_t rf_launch_prep_fp64(int64_t kN, int Nmc, int Rpad, int iso, const double* d_phase, const double* d_amp,
+                               double2* d_CS, hipStream_t s);
+hipError_t rf_launch_sum_fp64(const rf_sum_args& a, const double* d_k, int iso, double bound, const uint8_t* d_calc,
+                              const double2* d_CS, int Rpad, hipStream_t s);
 hipError_t rf_launch_sum_fp32(const rf_sum_args& a, const double* d_kRev, const float* d_phT,
                               const float* d_aT, int Rpad, hipStream_t s);
 hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kT, const float* d_pT,

@@ -2,8 +2,9 @@
 // (randomFieldND.f90:184-337 methods 2/3, :368-514 method 1).
 //
 // Two precision forms:
-//  * FP64: one thread per (point, realization), sequential sum over j in the
-//    reference's order with FMA contraction off -- the on-GPU oracle form.
+//  * FP64: one sine and cosine per (point, wavevector), shared by all
+//    realizations of a chunk, cos(t + phi) = cos t cos phi - sin t sin phi; the
+//    wavevectors of a point are split over its block.
 //  * FP32: one thread per point holding R realization accumulators.  The
 //    argument k.x is formed in FP64, reduced to revolutions in [-1/2, 1/2)
 //    once per (point, k) and reused for all R realizations; each term is then
@@ -36,33 +37,154 @@ __device__ inline float epilogue32(float u, const rf_epilogue& e) {
 }
 
 // ---------------------------------------------------------------- FP64 form
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_sum_fp64(rf_sum_args a, const double* __restrict__ k,
-                                                     int64_t kStrideR,
-                                                     const double* __restrict__ amp,
-                                                     const double* __restrict__ phase) {
-#pragma clang fp contract(off)
-    const int64_t i = a.i0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int r = blockIdx.y;
-    if (i >= a.i1) return;
-    double xn[D];
+// sin t and cos t for |t| < 2^30: t = n pi/2 + r with pi/2 in two doubles (the
+// FMAs keep n P1 exact, so r is good to half an ulp and n 2^-107), then the
+// minimax polynomials of sin r / r and cos r on |r| <= pi/4 (errors 2^-58 and
+// 2^-64, from a Remez exchange in 50-digit arithmetic).  Branch-free: ~28
+// FP64 instructions against the library call's ~100 with its range tests.
+__device__ __forceinline__ void sincos_fast(double t, double* sn, double* cs) {
+    // n = rint(2 t / pi) by the rounding of an addition: the low word of the
+    // sum holds n (two's complement)
+    const double m = fma(t, 0.6366197723675814, 6755399441055744.0);   // 1.5 2^52
+    const unsigned q = (unsigned)__builtin_bit_cast(uint64_t, m);
+    const double n = m - 6755399441055744.0;
+    double r = fma(-n, 0x1.921fb54442d18p+0, t);
+    r = fma(-n, 0x1.1a62633145c07p-54, r);
+    const double z = r * r;
+    double ps = 1.5896795644221148e-10, pc = -1.1359647777745982e-11;
+    ps = fma(ps, z, -2.5050758115096302e-08);
+    pc = fma(pc, z, 2.087572327278296e-09);
+    ps = fma(ps, z, 2.7557313691916818e-06);
+    pc = fma(pc, z, -2.755731435233002e-07);
+    ps = fma(ps, z, -0.00019841269829807805);
+    pc = fma(pc, z, 2.4801587289482178e-05);
+    ps = fma(ps, z, 0.008333333333322413);
+    pc = fma(pc, z, -0.0013888888888874125);
+    ps = fma(ps, z, -0.16666666666666632);
+    pc = fma(pc, z, 0.0416666666666666);
+    const double s = fma(r * z, ps, r);
+    const double c = fma(z, fma(z, pc, -0.5), 1.0);
+    const double ss = (q & 1) ? c : s, cc = (q & 1) ? s : c;
+    const uint64_t fs = (uint64_t)((q << 30) & 0x80000000u) << 32;
+    const uint64_t fc = (uint64_t)(((q << 30) + 0x40000000u) & 0x80000000u) << 32;
+    *sn = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, ss) ^ fs);
+    *cs = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, cc) ^ fc);
+}
+
+constexpr int kF64Waves = 8;     // waves of a block
+constexpr int kF64Q = 4;         // points of a lane
+constexpr int kF64Points = 16;   // points of a block: 4 lanes' worth
+constexpr int kF64Shares = kF64Waves * 16;
+
+// One block: 16 points, R realizations, all wavevectors.  The wavevectors are
+// dealt to 128 shares (16 per wave, j = share mod 128), a lane takes one share
+// and four points.  CS holds (a cos phi, -a sin phi): [j][Rpad] for a shared
+// wavevector table, [r][j] with per-realization directions (ISO, R = 1).  A
+// term costs the FP64 VALU 3 FMAs for k.x, ~28 instructions of sine and cosine
+// and 2 FMAs per realization; that rate bounds it.  Why this split: with one
+// point per lane the operands (24 + 16 R bytes per term) bound it instead, by
+// latency as scalar loads (523 us) or by the vector memory path (575 us); four
+// points per load leave the VALU busy, and small blocks spread 20,000 points
+// evenly over the CUs.  20,000 points x 10,976 wavevectors x 4 realizations:
+// 366 us (before: one thread per point and realization, a library cosine
+// per term: 4159 us).  The shares are added in a fixed order.
+// bound: max |k component|, for the block-uniform choice of the sine.
+template <int D, int R, bool ISO>
+__global__ __launch_bounds__(64 * kF64Waves) void k_sum_fp64(rf_sum_args a, const double* __restrict__ k,
+                                                             double bound, const uint8_t* __restrict__ calc,
+                                                             const double2* __restrict__ CS, int Rpad) {
+    constexpr int Q = kF64Q, P = kF64Points;
+    __shared__ double red[kF64Waves][R][P];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, pl = lane & 3;
+    const int64_t p0 = a.i0 + (int64_t)blockIdx.x * P;
+    const int r0 = blockIdx.y * R;
+    double xn[Q][D];
+    bool slow = false;
 #pragma unroll
-    for (int d = 0; d < D; d++) xn[d] = a.x[i * D + d] / a.corrL[d];   // :59
-    const double* kr = k + (int64_t)r * kStrideR;
-    const double* am = amp + (int64_t)r * a.kN;
-    const double* ph = phase + (int64_t)r * a.kN;
-    double acc = 0.0;
-    for (int64_t j = 0; j < a.kN; j++) {
-        // dgemm.f90:246-253 (k.x then + phi), :310 cos, dgemm.f90:226-234
-        double t = 0.0;
+    for (int q = 0; q < Q; q++) {
+        const int64_t i = p0 + pl * Q + q, ic = i < a.i1 ? i : a.i1 - 1;
+        double reach = 0.0;
 #pragma unroll
-        for (int d = 0; d < D; d++) t = t + xn[d] * kr[j * D + d];
-        const double c = cos(t + ph[j]);
-        const double aj = am[j];
-        if (aj != 0.0) acc = acc + aj * c;
+        for (int d = 0; d < D; d++) {
+            xn[q][d] = a.x[ic * D + d] / a.corrL[d];   // :59
+            reach += fabs(xn[q][d]);
+        }
+        // arguments past the fast sine's range, infinities, NaN: library sine
+        slow |= !(reach * bound < 1073741824.0);
     }
-    const double u = epilogue64(a.ampMult * acc, a.epi);               // :330
-    store_out(a.out, (int64_t)r * a.N + i, u, a.outDtype);
+    const bool fast = !__syncthreads_or(slow);
+    double acc[Q][R];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[q][r] = 0.0;
+    const double* kr = k + (ISO ? (int64_t)r0 * a.kN * D : 0);
+    const double2* C = CS + (ISO ? (int64_t)r0 * a.kN : (int64_t)r0);
+    const int64_t cStep = ISO ? 1 : Rpad;
+    auto sweep = [&](auto sc) {
+        for (int64_t j = w * 16 + (lane >> 2); j < a.kN; j += kF64Shares) {
+            double kj[D];
+#pragma unroll
+            for (int d = 0; d < D; d++) kj[d] = kr[j * D + d];
+            double sn[Q], cs[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                double t = kj[0] * xn[q][0];
+#pragma unroll
+                for (int d = 1; d < D; d++) t = fma(kj[d], xn[q][d], t);
+                sc(t, &sn[q], &cs[q]);
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const double2 c = C[j * cStep + r];
+#pragma unroll
+                for (int q = 0; q < Q; q++) acc[q][r] = fma(c.x, cs[q], fma(c.y, sn[q], acc[q][r]));
+            }
+        }
+    };
+    if (fast) sweep([](double t, double* s, double* c) { sincos_fast(t, s, c); });
+    else sweep([](double t, double* s, double* c) { sincos(t, s, c); });
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            double v = acc[q][r];
+#pragma unroll
+            for (int o = 4; o < 64; o <<= 1) v += __shfl_xor(v, o);
+            if (lane < 4) red[w][r][pl * Q + q] = v;
+        }
+    __syncthreads();
+    for (int e = threadIdx.x; e < R * P; e += 64 * kF64Waves) {
+        const int r = e / P, p = e % P;
+        const int64_t ip = p0 + p;
+        if (ip >= a.i1 || r0 + r >= a.Nmc) continue;
+        double s = red[0][r][p];
+#pragma unroll
+        for (int v = 1; v < kF64Waves; v++) s += red[v][r][p];
+        // a realization the caller masks is zero at every point
+        const double u = epilogue64(calc[r0 + r] ? a.ampMult * s : 0.0, a.epi);   // :330
+        store_out(a.out, (int64_t)(r0 + r) * a.N + ip, u, a.outDtype);
+    }
+}
+
+// (a cos phi, -a sin phi) of the FP64 form from phases and amplitudes [r][j]:
+// [j][Rpad], zero for padded realizations, or [r][j] (ISO).
+__global__ __launch_bounds__(kBlock) void k_prep_fp64(int64_t kN, int Nmc, int Rpad, int iso,
+                                                      const double* __restrict__ phase,
+                                                      const double* __restrict__ amp, double2* __restrict__ CS) {
+    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= kN * Rpad) return;
+    const int64_t j = iso ? e % kN : e / Rpad;
+    const int r = (int)(iso ? e / kN : e - j * Rpad);
+    double2 v = {0.0, 0.0};
+    if (r < Nmc) {
+        const double A = amp[(int64_t)r * kN + j];
+        double sn, cs;
+        sincos(phase[(int64_t)r * kN + j], &sn, &cs);
+        v.x = A * cs;
+        v.y = -A * sn;
+    }
+    CS[e] = v;
 }
 
 // ---------------------------------------------------------------- FP32 form
@@ -175,13 +297,27 @@ __global__ __launch_bounds__(kBlock) void k_group_iso(const rf_group_req* __rest
                                       (int)(local % nChunk) * kGroupIsoR);
 }
 
-template <int D>
-hipError_t launch_fp64(const rf_sum_args& a, const double* k, int64_t ks, const double* amp,
-                       const double* ph, hipStream_t s) {
-    const int64_t n = a.i1 - a.i0;
-    dim3 grid((unsigned)((n + kBlock - 1) / kBlock), (unsigned)a.Nmc);
-    hipLaunchKernelGGL(k_sum_fp64<D>, grid, dim3(kBlock), 0, s, a, k, ks, amp, ph);
+template <int D, int R, bool ISO>
+hipError_t launch_fp64_r(const rf_sum_args& a, const double* k, double bound, const uint8_t* calc,
+                         const double2* CS, int Rpad, hipStream_t s) {
+    const int64_t blocks = (a.i1 - a.i0 + kF64Points - 1) / kF64Points;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_sum_fp64<D, R, ISO>), dim3((unsigned)blocks, (unsigned)(Rpad / R)), dim3(64 * kF64Waves), 0, s,
+                       a, k, bound, calc, CS, Rpad);
     return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_fp64(const rf_sum_args& a, const double* k, int iso, double bound, const uint8_t* calc,
+                       const double2* CS, int Rpad, hipStream_t s) {
+    if (iso) return launch_fp64_r<D, 1, true>(a, k, bound, calc, CS, Rpad, s);
+    switch (rf_fp64_rchunk(a.Nmc)) {
+        case 1: return launch_fp64_r<D, 1, false>(a, k, bound, calc, CS, Rpad, s);
+        case 2: return launch_fp64_r<D, 2, false>(a, k, bound, calc, CS, Rpad, s);
+        case 4: return launch_fp64_r<D, 4, false>(a, k, bound, calc, CS, Rpad, s);
+        case 8: return launch_fp64_r<D, 8, false>(a, k, bound, calc, CS, Rpad, s);
+        default: return launch_fp64_r<D, 16, false>(a, k, bound, calc, CS, Rpad, s);
+    }
 }
 
 }  // namespace
@@ -189,13 +325,35 @@ hipError_t launch_fp64(const rf_sum_args& a, const double* k, int64_t ks, const 
 // Realization chunk of the FP32 kernels (accumulators per thread).
 constexpr int kRChunk = 16;
 
-hipError_t rf_launch_sum_fp64(const rf_sum_args& a, const double* d_k, int64_t kStrideR,
-                              const double* d_amp, const double* d_phase, hipStream_t s) {
+// Realizations per block of the FP64 kernel: the power of two that holds Nmc,
+// at most 16 (the sine of a term is then shared by all of them).
+int rf_fp64_rchunk(int Nmc) {
+    int r = 1;
+    while (r < Nmc && r < 16) r <<= 1;
+    return r;
+}
+
+int rf_fp64_rpad(int Nmc, int iso) {
+    const int c = rf_fp64_rchunk(Nmc);
+    return iso ? Nmc : (Nmc + c - 1) / c * c;
+}
+
+hipError_t rf_launch_prep_fp64(int64_t kN, int Nmc, int Rpad, int iso, const double* d_phase, const double* d_amp,
+                               double2* d_CS, hipStream_t s) {
+    const int64_t n = kN * Rpad;
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_prep_fp64, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, kN, Nmc, Rpad,
+                       iso, d_phase, d_amp, d_CS);
+    return hipGetLastError();
+}
+
+hipError_t rf_launch_sum_fp64(const rf_sum_args& a, const double* d_k, int iso, double bound, const uint8_t* d_calc,
+                              const double2* d_CS, int Rpad, hipStream_t s) {
     if (a.i1 <= a.i0) return hipSuccess;
     switch (a.nDim) {
-        case 1: return launch_fp64<1>(a, d_k, kStrideR, d_amp, d_phase, s);
-        case 2: return launch_fp64<2>(a, d_k, kStrideR, d_amp, d_phase, s);
-        default: return launch_fp64<3>(a, d_k, kStrideR, d_amp, d_phase, s);
+        case 1: return launch_fp64<1>(a, d_k, iso, bound, d_calc, d_CS, Rpad, s);
+        case 2: return launch_fp64<2>(a, d_k, iso, bound, d_calc, d_CS, Rpad, s);
+        default: return launch_fp64<3>(a, d_k, iso, bound, d_calc, d_CS, Rpad, s);
     }
 }
 
