@@ -53,6 +53,9 @@ int build_form_operands(rf_field_plan* P, hipStream_t s) {
             RF_HIP_TRY(ctx, rf_launch_prep_fp32(kN, Nmc, P->Rpad, P->d_phase, P->d_amp, ampMult,
                                                 P->d_phT, P->d_aT, s));
         }
+    } else if (P->lat) {
+        RF_HIP_TRY(ctx, rf_launch_lat_prep(P->p.form, P->p.nDim, P->latD, Nmc, P->Rpad, P->d_phase, 0, P->d_amp, kN,
+                                           ampMult * P->bScale, P->d_B, s));
     } else if (P->p.form == RF_FORM_MFMA_F16 || P->p.form == RF_FORM_MFMA_BF16) {
         RF_HIP_TRY(ctx, rf_launch_mfma_prep(P->p.form, P->p.nDim, kN, P->kNpad, Nmc, P->Rpad,
                                             P->d_kRev, P->d_phase, P->d_amp, kN, ampMult * P->bScale,
@@ -307,7 +310,11 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
         RF_HIP_TRY(ctx, dmalloc(&P->d_phT, (size_t)(kN * P->Rpad)));
         RF_HIP_TRY(ctx, dmalloc(&P->d_aT, (size_t)(kN * P->Rpad)));
     }
-    if (p->form != RF_FORM_FP64 && !is_iso_direct(*p)) {
+    // the product form needs the intended lattice (REF_COMPAT reads its first
+    // sign block as zero wavevectors)
+    P->lat = mfma && p->method == RF_SHINOZUKA && p->mode == RF_FIXED &&
+             rf_lat_describe(d, info.kNStep, info.kDelta, &P->latD);
+    if (p->form != RF_FORM_FP64 && !is_iso_direct(*p) && !P->lat) {
         // the MFMA form reads whole K-steps: zero wavevectors pad the tail
         RF_HIP_TRY(ctx, dmalloc(&P->d_kRev, (size_t)(P->kNpad * d)));
         if (P->kNpad > kN)
@@ -316,8 +323,10 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
     }
     P->ampMax = maxAmp;
     if (mfma) {
-        P->bScale = rf_mfma_bscale(P->spec.info.ampMult, maxAmp);
-        RF_HIP_TRY(ctx, hipMalloc(&P->d_B, rf_mfma_bbytes(p->form, P->kNpad, P->Rpad)));
+        // product form: a coefficient sums up to four sign blocks
+        P->bScale = rf_mfma_bscale(P->spec.info.ampMult, P->lat ? 4.0 * maxAmp : maxAmp);
+        RF_HIP_TRY(ctx, hipMalloc(&P->d_B, P->lat ? rf_lat_bbytes(P->latD, P->Rpad)
+                                                  : rf_mfma_bbytes(p->form, P->kNpad, P->Rpad)));
     }
     const bool perSlab = (p->mode == RF_REF_COMPAT && p->method != RF_ISOTROPIC);
     if (!perSlab) {
@@ -378,7 +387,8 @@ int rf_plan_execute(rf_field_plan* P, const double* d_x, int64_t N, void* d_out,
                 else e = rf_launch_sum_fp32(a, P->d_kRev, P->d_phT, P->d_aT, P->Rpad, s);
                 break;
             default:
-                e = rf_launch_sum_mfma(p.form, P->mfmaVariant, a, P->kNpad, P->Rpad, P->d_B, 1.0 / P->bScale, s);
+                if (P->lat) e = rf_launch_sum_lat(p.form, a, P->latD, P->Rpad, P->d_B, 1.0 / P->bScale, s);
+                else e = rf_launch_sum_mfma(p.form, P->mfmaVariant, a, P->kNpad, P->Rpad, P->d_B, 1.0 / P->bScale, s);
                 break;
         }
         if (e != hipSuccess) return rf_set_error(ctx, RF_E_HIP, std::string("sum kernel launch: ") + hipGetErrorString(e));
@@ -568,6 +578,13 @@ int rf_plan_autotune(rf_field_plan* P, const double* d_x, int64_t N, void* d_out
     }
     RF_HIP_TRY(ctx, hipSetDevice(ctx->device));
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
+    if (P->lat) {                               // one launch shape; the field is formed as ever
+        const int rc = rf_plan_execute(P, d_x, N, d_out, outDtype, s);
+        if (rc) return rc;
+        RF_HIP_TRY(ctx, hipStreamSynchronize(s));
+        if (chosen) *chosen = P->mfmaVariant;
+        return RF_OK;
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     RF_HIP_TRY(ctx, hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {

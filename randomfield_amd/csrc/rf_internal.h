@@ -58,43 +58,6 @@ struct rf_epilogue {
     double shift;   // normalAvg
 };
 
-struct rf_field_plan {
-    rf_context* ctx = nullptr;
-    rf_params p{};
-    rf_spectrum spec;
-    std::vector<uint8_t> calc;        // Nmc flags
-    int nCalc = 0;
-    // device buffers (owned)
-    double* d_k = nullptr;       // shared k: kN x nDim (normalised units)
-    double* d_kRad = nullptr;    // isotropic: radii kN
-    double* d_kRev = nullptr;    // shared k / (2 pi)
-    double* d_kIso = nullptr;    // per-realization k: Nmc x kN x nDim
-    double* d_kIsoT = nullptr;   // FP32 isotropic form: kN x Rpad x nDim, revolutions
-    double* d_Sk = nullptr;      // isotropic spectral density
-    uint8_t* d_calc = nullptr;   // Nmc flags
-    double* d_phase = nullptr;   // Nmc x kN radians (2*pi_ref*U or psi)
-    double* d_amp = nullptr;     // Nmc x kN amplitudes (before ampMult)
-    double* d_uni = nullptr;     // device copy of the phase uniforms
-    float* d_phT = nullptr;      // kN x Rpad   FP32 phase in revolutions
-    float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult
-    void* d_B = nullptr;         // MFMA coefficient panels (hi, lo)
-    double2* d_CS = nullptr;     // FP64 form: (amp cos phase, -amp sin phase)
-    double kAbsMax = 0.0;        // bound of the wavevector components (normalised units)
-    int Rpad = 0;
-    int64_t kNpad = 0;
-    double bScale = 1.0;         // power-of-two scale folded into B
-    double ampMax = 1.0;         // bound of |amp| over all realizations
-    // REF_COMPAT: sqrt chain of Sk, row c = Sk^(2^-(c+1)), until it saturates
-    std::vector<std::vector<double>> sqrtChain;
-    bool coeffsReady = false;    // FIXED: coefficients independent of N
-    rf_epilogue epi{};
-    void* d_gridScratch = nullptr;   // structured-grid form (grown on demand)
-    size_t gridScratchBytes = 0;
-    float2* d_gridCoef = nullptr;    // folded grid coefficients (first grid execution)
-    double gridCoefKey = NAN;
-    int mfmaVariant = 0;         // MFMA launch shape (rf_plan_set_variant / rf_plan_autotune)
-};
-
 // ---- host spectrum (rf_spectrum.cpp)
 int rf_spectrum_build_info(const rf_params* p, rf_spectrum_info* info, std::string* err);
 int rf_spectrum_build_tables(const rf_params* p, const rf_spectrum_info& info,
@@ -176,6 +139,69 @@ inline double rf_mfma_bscale(double ampMult, double maxAmp) {
 }
 size_t rf_mfma_bbytes(int form, int64_t kNpad, int Npad);
 
+// Product form of the Shinozuka sum on points (rf_lat.hip): the lattice, its
+// K-steps and the per-axis table rows.
+struct rf_lat_dev {
+    int n1, n2, n3;        // lattice points per axis
+    int TS, P1;            // K-steps per (j2, j3), axis-1 table rows (n1 padded to whole steps)
+    int64_t nSteps;        // padded to a multiple of 16
+    double kd[3];          // wavenumber step per axis, revolutions per correlation length
+};
+constexpr int kLatMT = 2;                     // M-tiles per block (more: the MFMAs bound either way)
+constexpr int64_t kLatSmallN = 32768;         // up to here blocks of 128 points and split K-steps
+constexpr int kLatTableMax = 96 * 1024;       // LDS bytes of the per-point tables (beside 64 KB of panels)
+// false: no product form (1-D, or axes whose tables pass the LDS for 128
+// points: axis 1 + axis 2 above 96 lattice points)
+bool rf_lat_describe(int nDim, const int32_t* kNStep, const double* kDelta, rf_lat_dev* L);
+bool rf_lat_small(const rf_lat_dev& L, int64_t N);
+inline int rf_lat_waves(const rf_lat_dev& L, int64_t N) { return rf_lat_small(L, N) ? 4 : 8; }   // 32 points each
+size_t rf_lat_bbytes(const rf_lat_dev& L, int Npad);
+// phases d_phase, or, NULL, the device stream (seed, 2) from element 0
+hipError_t rf_launch_lat_prep(int form, int nDim, const rf_lat_dev& L, int Nmc, int Npad, const double* d_phase,
+                              uint64_t seed, const double* d_amp, int64_t ampStrideR, double scale, void* d_B,
+                              hipStream_t s);
+hipError_t rf_launch_sum_lat(int form, const rf_sum_args& a, const rf_lat_dev& L, int Npad, const void* d_B,
+                             double outScale, hipStream_t s);
+
+struct rf_field_plan {
+    rf_context* ctx = nullptr;
+    rf_params p{};
+    rf_spectrum spec;
+    std::vector<uint8_t> calc;        // Nmc flags
+    int nCalc = 0;
+    // device buffers (owned)
+    double* d_k = nullptr;       // shared k: kN x nDim (normalised units)
+    double* d_kRad = nullptr;    // isotropic: radii kN
+    double* d_kRev = nullptr;    // shared k / (2 pi)
+    double* d_kIso = nullptr;    // per-realization k: Nmc x kN x nDim
+    double* d_kIsoT = nullptr;   // FP32 isotropic form: kN x Rpad x nDim, revolutions
+    double* d_Sk = nullptr;      // isotropic spectral density
+    uint8_t* d_calc = nullptr;   // Nmc flags
+    double* d_phase = nullptr;   // Nmc x kN radians (2*pi_ref*U or psi)
+    double* d_amp = nullptr;     // Nmc x kN amplitudes (before ampMult)
+    double* d_uni = nullptr;     // device copy of the phase uniforms
+    float* d_phT = nullptr;      // kN x Rpad   FP32 phase in revolutions
+    float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult
+    void* d_B = nullptr;         // MFMA coefficient panels (hi, lo)
+    bool lat = false;            // MFMA forms: product form of the lattice (rf_lat.hip)
+    rf_lat_dev latD{};
+    double2* d_CS = nullptr;     // FP64 form: (amp cos phase, -amp sin phase)
+    double kAbsMax = 0.0;        // bound of the wavevector components (normalised units)
+    int Rpad = 0;
+    int64_t kNpad = 0;
+    double bScale = 1.0;         // power-of-two scale folded into B
+    double ampMax = 1.0;         // bound of |amp| over all realizations
+    // REF_COMPAT: sqrt chain of Sk, row c = Sk^(2^-(c+1)), until it saturates
+    std::vector<std::vector<double>> sqrtChain;
+    bool coeffsReady = false;    // FIXED: coefficients independent of N
+    rf_epilogue epi{};
+    void* d_gridScratch = nullptr;   // structured-grid form (grown on demand)
+    size_t gridScratchBytes = 0;
+    float2* d_gridCoef = nullptr;    // folded grid coefficients (first grid execution)
+    double gridCoefKey = NAN;
+    int mfmaVariant = 0;         // MFMA launch shape (rf_plan_set_variant / rf_plan_autotune)
+};
+
 // grouped launches: a batch of independent fields (serving requests) in one
 // launch.  Field q owns tiles tile0 .. tile0 + nTiles(q) - 1 (ascending in q);
 // block b finds its field by binary search over tile0.
@@ -196,14 +222,16 @@ constexpr int kGroupW = 8;        // waves per block, grouped MFMA kernel (256 p
 constexpr int kGroupIsoPts = 256; // points per tile, grouped direct isotropic kernel
 constexpr int kGroupIsoR = 16;    // realizations per tile, grouped direct isotropic kernel
 // tiles of one field
-inline int64_t rf_group_tiles_mfma(int64_t N, int mtTotal) {
-    return (N + 32 * kGroupW - 1) / (32 * kGroupW) * ((mtTotal + kGroupMT - 1) / kGroupMT);
+inline int64_t rf_group_tiles_mfma(int64_t N, int mtTotal, int waves, int mtBlock) {
+    return (N + 32 * waves - 1) / (32 * waves) * ((mtTotal + mtBlock - 1) / mtBlock);
 }
 inline int64_t rf_group_tiles_iso(int64_t N, int Rpad) {
     return (N + kGroupIsoPts - 1) / kGroupIsoPts * (Rpad / kGroupIsoR);
 }
 hipError_t rf_launch_group_mfma(int form, const rf_group_req* d_reqs, int nReq, int64_t nTiles,
                                 hipStream_t s);
+hipError_t rf_launch_group_lat(int form, int small, const rf_lat_dev& L, const rf_group_req* d_reqs, int nReq,
+                               int64_t nTiles, hipStream_t s);
 hipError_t rf_launch_group_iso(const rf_group_req* d_reqs, int nReq, int64_t nTiles, hipStream_t s);
 
 // epilogue constants of multiVariateTransformation (randomFieldND.f90:154-169)

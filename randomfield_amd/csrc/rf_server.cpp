@@ -45,6 +45,8 @@ struct Lattice {
     double* d_amp = nullptr;  // method 2: sqrt(Sk) [kN] (one row for every realization)
     int64_t kNpad = 0;
     double bScale = 1.0;      // method 2: panel scale
+    bool lat = false;         // method 2: product form of the lattice
+    rf_lat_dev latD{};
 };
 
 struct Req {
@@ -64,7 +66,7 @@ struct Slot {
     bool busy = false;
     int64_t batch = -1;
     std::vector<int64_t> ids;
-    rf_group_req* d_table = nullptr;   // [2 * maxBatch]: method 2 then method 1
+    rf_group_req* d_table = nullptr;   // [3 * maxBatch]: method 2, method 1, method 2 in the small shape
     rf_group_req* h_table = nullptr;   // pinned staging of the same
 };
 
@@ -93,6 +95,13 @@ struct rf_server {
 
     Lattice& L(int method) { return lat[method == RF_SHINOZUKA ? 1 : 0]; }
 
+    // method 2 tiles of a request (waves of 32 points, M-tiles per block)
+    int64_t tilesOf(int64_t N, int mtTotal) const {
+        const Lattice& l = lat[1];
+        return l.lat ? rf_group_tiles_mfma(N, mtTotal, rf_lat_waves(l.latD, N), kLatMT)
+                     : rf_group_tiles_mfma(N, mtTotal, kGroupW, kGroupMT);
+    }
+
     // device bytes of one request: output, point copy, scratch
     void sizes(Req& q) {
         const Lattice& l = L(q.r.method);
@@ -102,8 +111,9 @@ struct rf_server {
         q.bytesX = q.r.xOnDevice ? 0 : align256((size_t)N * 3 * sizeof(double));
         if (q.r.method == RF_SHINOZUKA) {
             q.Rpad = (Nmc + 31) / 32 * 32;       // whole 32-row tiles (any count)
-            q.bytesScr = 2 * align256((size_t)Nmc * kN * sizeof(double)) +   // uniforms, phases
-                         align256(rf_mfma_bbytes(cfg.form, l.kNpad, q.Rpad));
+            q.bytesScr = l.lat ? align256(rf_lat_bbytes(l.latD, q.Rpad))
+                               : 2 * align256((size_t)Nmc * kN * sizeof(double)) +   // uniforms, phases
+                                     align256(rf_mfma_bbytes(cfg.form, l.kNpad, q.Rpad));
         } else {
             q.Rpad = (Nmc + kGroupIsoR - 1) / kGroupIsoR * kGroupIsoR;
             q.bytesScr = align256((size_t)Nmc * 4 * kN * 8)        // uniforms
@@ -163,8 +173,8 @@ struct rf_server {
 int rf_server::launch(Slot& sl, const std::vector<Req*>& batch, std::string& err) {
     const hipStream_t s = sl.stream;
     const int maxB = cfg.maxBatch;
-    int nM = 0, nI = 0;
-    int64_t tilesM = 0, tilesI = 0;
+    int nM[2] = {0, 0}, nI = 0;                  // method 2: [1] the product form's small shape
+    int64_t tilesM[2] = {0, 0}, tilesI = 0;
     for (Req* q : batch) {
         const rf_request& r = q->r;
         const Lattice& l = L(r.method);
@@ -192,23 +202,31 @@ int rf_server::launch(Slot& sl, const std::vector<Req*>& batch, std::string& err
         g.a.outDtype = RF_DTYPE_F32;
         const int64_t nU = (int64_t)r.Nmc * kN;
         if (r.method == RF_SHINOZUKA) {
-            // phases 2 pi U from the (seed, 2) stream, then the panels
-            double* d_u = reinterpret_cast<double*>(scr);
-            double* d_ph = reinterpret_cast<double*>(scr + align256((size_t)nU * sizeof(double)));
-            char* d_B = scr + 2 * align256((size_t)nU * sizeof(double));
-            SRV_TRY(rf_launch_uniforms(r.seed, 2u, nU, d_u, s));
-            SRV_TRY(rf_launch_phase_from_uniform(d_u, nU, d_ph, s));
-            SRV_TRY(rf_launch_mfma_prep(cfg.form, 3, kN, l.kNpad, r.Nmc, q->Rpad, l.d_k, d_ph, l.d_amp, 0,
-                                        l.info.ampMult * l.bScale, d_B, s));
             const int mtTotal = q->Rpad / 32;
-            g.ops0 = d_B;
-            g.ops1 = d_B + (size_t)(l.kNpad / 8) * mtTotal * 128 * 16;
-            g.nSteps = l.kNpad / 8;
+            if (l.lat) {
+                // panels from phases 2 pi U drawn in place from the (seed, 2) stream
+                SRV_TRY(rf_launch_lat_prep(cfg.form, 3, l.latD, r.Nmc, q->Rpad, nullptr, r.seed, l.d_amp, 0,
+                                           l.info.ampMult * l.bScale, scr, s));
+                g.ops0 = scr;
+            } else {
+                // phases 2 pi U from the (seed, 2) stream, then the panels
+                double* d_u = reinterpret_cast<double*>(scr);
+                double* d_ph = reinterpret_cast<double*>(scr + align256((size_t)nU * sizeof(double)));
+                char* d_B = scr + 2 * align256((size_t)nU * sizeof(double));
+                SRV_TRY(rf_launch_uniforms(r.seed, 2u, nU, d_u, s));
+                SRV_TRY(rf_launch_phase_from_uniform(d_u, nU, d_ph, s));
+                SRV_TRY(rf_launch_mfma_prep(cfg.form, 3, kN, l.kNpad, r.Nmc, q->Rpad, l.d_k, d_ph, l.d_amp, 0,
+                                            l.info.ampMult * l.bScale, d_B, s));
+                g.ops0 = d_B;
+                g.ops1 = d_B + (size_t)(l.kNpad / 8) * mtTotal * 128 * 16;
+                g.nSteps = l.kNpad / 8;
+            }
             g.mtTotal = mtTotal;
             g.outScale = (float)(1.0 / l.bScale);
-            g.tile0 = tilesM;
-            tilesM += rf_group_tiles_mfma(r.N, mtTotal);
-            sl.h_table[nM++] = g;
+            const int small = l.lat && rf_lat_small(l.latD, r.N);
+            g.tile0 = tilesM[small];
+            tilesM[small] += tilesOf(r.N, mtTotal);
+            sl.h_table[(small ? 2 * maxB : 0) + nM[small]++] = g;
         } else {
             char* p = scr;
             double* d_u = reinterpret_cast<double*>(p);
@@ -238,8 +256,13 @@ int rf_server::launch(Slot& sl, const std::vector<Req*>& batch, std::string& err
             sl.h_table[maxB + nI++] = g;
         }
     }
-    SRV_TRY(hipMemcpyAsync(sl.d_table, sl.h_table, sizeof(rf_group_req) * 2 * maxB, hipMemcpyHostToDevice, s));
-    SRV_TRY(rf_launch_group_mfma(cfg.form, sl.d_table, nM, tilesM, s));
+    SRV_TRY(hipMemcpyAsync(sl.d_table, sl.h_table, sizeof(rf_group_req) * 3 * maxB, hipMemcpyHostToDevice, s));
+    if (lat[1].lat) {
+        SRV_TRY(rf_launch_group_lat(cfg.form, 0, lat[1].latD, sl.d_table, nM[0], tilesM[0], s));
+        SRV_TRY(rf_launch_group_lat(cfg.form, 1, lat[1].latD, sl.d_table + 2 * maxB, nM[1], tilesM[1], s));
+    } else {
+        SRV_TRY(rf_launch_group_mfma(cfg.form, sl.d_table, nM[0], tilesM[0], s));
+    }
     SRV_TRY(rf_launch_group_iso(sl.d_table + maxB, nI, tilesI, s));
     SRV_TRY(hipEventRecord(sl.done, s));
     return RF_OK;
@@ -390,7 +413,8 @@ int build_lattice(rf_server* S, int method, Lattice& l) {
             amp[(size_t)j] = std::sqrt(spec.Sk[(size_t)j]);
             maxAmp = std::max(maxAmp, amp[(size_t)j]);
         }
-        l.bScale = rf_mfma_bscale(l.info.ampMult, maxAmp);
+        l.lat = rf_lat_describe(3, l.info.kNStep, l.info.kDelta, &l.latD);
+        l.bScale = rf_mfma_bscale(l.info.ampMult, l.lat ? 4.0 * maxAmp : maxAmp);
         RF_HIP_TRY(ctx, hipMalloc((void**)&l.d_k, kRev.size() * sizeof(double)));
         RF_HIP_TRY(ctx, hipMalloc((void**)&l.d_amp, amp.size() * sizeof(double)));
         RF_HIP_TRY(ctx, hipMemcpyAsync(l.d_k, kRev.data(), kRev.size() * sizeof(double), hipMemcpyHostToDevice, s));
@@ -478,7 +502,7 @@ int rf_server_create(rf_context* ctx, const rf_server_config* cfg, rf_server** o
     }
     S->slots.resize((size_t)c.maxInflight);
     for (Slot& sl : S->slots) {
-        const size_t tb = sizeof(rf_group_req) * 2 * (size_t)c.maxBatch;
+        const size_t tb = sizeof(rf_group_req) * 3 * (size_t)c.maxBatch;
         if (hipStreamCreate(&sl.stream) != hipSuccess ||
             hipEventCreateWithFlags(&sl.done, hipEventDisableTiming) != hipSuccess ||
             hipMalloc((void**)&sl.d_table, tb) != hipSuccess ||
@@ -531,7 +555,7 @@ int rf_server_submit(rf_server* S, const rf_request* r, int64_t* id) {
     S->sizes(q);
     if (q.bytesOut + q.bytesX + q.bytesScr > S->arena.capacity())
         return rf_set_error(S->ctx, RF_E_NOMEM, "request exceeds the server's memory budget");
-    if (rf_group_tiles_mfma(r->N, q.Rpad / 32) > 0x7fffffffLL || rf_group_tiles_iso(r->N, q.Rpad) > 0x7fffffffLL)
+    if (S->tilesOf(r->N, q.Rpad / 32) > 0x7fffffffLL || rf_group_tiles_iso(r->N, q.Rpad) > 0x7fffffffLL)
         return rf_set_error(S->ctx, RF_E_ARG, "request too large for one grouped launch");
     q.tSubmit = now_s();
     {
