@@ -1004,10 +1004,11 @@ int interpolate_common(rf_context* ctx, int32_t nDim, const int32_t* nstep, cons
     RF_HIP_TRY(ctx, rf_launch_interp(nDim, nstep, lo, xMin, xStep, Nmc, d_grid, gridDtype, d_nodes, nNodes, d_out,
                                      outDtype, flag, s));
     if (outside) {
-        int h = 0;
-        RF_HIP_TRY(ctx, hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+        double* pin = result_target(ctx, 1, nullptr);
+        int h = 0, *dst = pin ? reinterpret_cast<int*>(pin) : &h;
+        RF_HIP_TRY(ctx, hipMemcpyAsync(dst, flag, sizeof(int), hipMemcpyDeviceToHost, s));
         RF_HIP_TRY(ctx, hipStreamSynchronize(s));
-        *outside = h;
+        *outside = *dst;
     } else {
         RF_HIP_TRY(ctx, hipStreamSynchronize(s));   // the flag word is context scratch
     }
