@@ -556,6 +556,17 @@ int rf_plan_redraw(rf_field_plan* P, int64_t drawIndex, void* stream) {
         P->gridCoefKey = NAN;
         return RF_OK;
     }
+    if (p.method != RF_ISOTROPIC) {
+        const bool ops = P->coeffsReady && p.form == RF_FORM_FP32;
+        RF_HIP_TRY(ctx, rf_launch_draw_prep(kN, p.Nmc, P->Rpad, p.seed, first, P->d_amp, P->spec.info.ampMult, P->d_uni,
+                                            P->d_phase, ops ? P->d_phT : nullptr, ops ? P->d_aT : nullptr, s));
+        if (P->coeffsReady && !ops) {
+            const int rc = build_form_operands(P, s);
+            if (rc) return rc;
+        }
+        P->gridCoefKey = NAN;
+        return RF_OK;
+    }
     RF_HIP_TRY(ctx, rf_launch_uniforms_at(p.seed, 2u, first, nPU, P->d_uni, s));
     return plan_reform(P, s);
 }

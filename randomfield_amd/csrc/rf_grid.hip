@@ -1516,32 +1516,43 @@ __global__ void k_iso_tables(int nDim, int64_t kN, int64_t kP, int Nmc, int n0, 
     T[dst] = make_float2((float)(m * cs), (float)(m * sn));
 }
 
-// E[v][j][x] = exp(i s_v k_j x), k_j = j dk, x = (o + i step) / L, in FP64;
-// variant v = 0 plain, v = 1 conjugate (negative sign).
-__global__ void k_phase_table(int nk, int nx, double dk, double o, double step, double invL,
-                              int variants, float2* __restrict__ E) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)nk * nx) return;
+// The tables of all axes of one execution (one launch: a grid of 129 x 129
+// points spent three launches of 5-9 us on what this does in one).  Axis a's
+// blocks start at block0[a].
+//   Shinozuka: E[v][j][x] = exp(i s_v k_j x), k_j = j dk, x = (o + i step) / L,
+//     in FP64; variant v = 0 plain, v = 1 conjugate (negative sign).
+//   Method 4: E[v][j][i] = (w_j cos(pi j (2i+1) / (2n)), 0), w_0 = 1, w_j = 2: the
+//     REDFT01 (DCT-III) of FFTW that gen_Std_Gauss_FFT applies along each axis
+//     (randomFieldND.f90:694-735), as a matrix; both variants equal.
+struct rf_table_args {
+    int dct, nAx;
+    int nk[3], nx[3];
+    unsigned block0[3];
+    double dk[3], o[3], step[3], invL[3];
+    float2* E[3];
+};
+__global__ __launch_bounds__(256) void k_axis_tables(rf_table_args t) {
+    int a = 0;
+    while (a + 1 < t.nAx && blockIdx.x >= t.block0[a + 1]) a++;
+    const int64_t e = (int64_t)(blockIdx.x - t.block0[a]) * 256 + threadIdx.x;
+    const int nx = t.nx[a];
+    const int64_t cnt = (int64_t)t.nk[a] * nx;
+    if (e >= cnt) return;
     const int j = (int)(e / nx), i = (int)(e % nx);
-    const double x = (o + step * (double)i) * invL;
-    const double t = (dk * (double)j) * x;
+    float2* E = t.E[a];
+    if (t.dct) {
+        const double w = j == 0 ? 1.0 : 2.0;
+        const double c = w * cos(3.14159265358979323846 * (double)j * (2.0 * i + 1.0) / (2.0 * nx));
+        E[e] = make_float2((float)c, 0.0f);
+        E[cnt + e] = make_float2((float)c, 0.0f);
+        return;
+    }
+    const double x = (t.o[a] + t.step[a] * (double)i) * t.invL[a];
+    const double th = (t.dk[a] * (double)j) * x;
     double s, c;
-    sincos(t, &s, &c);
+    sincos(th, &s, &c);
     E[e] = make_float2((float)c, (float)s);
-    if (variants > 1) E[(int64_t)nk * nx + e] = make_float2((float)c, (float)-s);
-}
-
-// Method 4: E[v][j][i] = (w_j cos(pi j (2i+1) / (2n)), 0), w_0 = 1, w_j = 2:
-// the REDFT01 (DCT-III) of FFTW that gen_Std_Gauss_FFT applies along each
-// axis (randomFieldND.f90:694-735), as a matrix; both variants equal.
-__global__ void k_dct_table(int n, float2* __restrict__ E) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)n * n) return;
-    const int j = (int)(e / n), i = (int)(e % n);
-    const double w = j == 0 ? 1.0 : 2.0;
-    const double c = w * cos(3.14159265358979323846 * (double)j * (2.0 * i + 1.0) / (2.0 * n));
-    E[e] = make_float2((float)c, 0.0f);
-    E[(int64_t)n * n + e] = make_float2((float)c, 0.0f);
+    E[cnt + e] = make_float2((float)c, (float)-s);
 }
 
 // Sign-block folding.  The field is Re of the sum, and the tables of a
@@ -1762,15 +1773,20 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
 
     float2* p = scratch;
     float2* E[3];
+    rf_table_args ta{};
+    ta.dct = kind == 1;
+    ta.nAx = nDim;
+    unsigned tabBlocks = 0;
     for (int a = 0; a < nDim; a++) {
         E[a] = p; p += 2LL * kNStep[a] * n[a];
-        const int64_t cnt = (int64_t)kNStep[a] * n[a];
-        if (kind == 1)
-            hipLaunchKernelGGL(k_dct_table, dim3(blocks_for(cnt)), dim3(256), 0, s, n[a], E[a]);
-        else
-            hipLaunchKernelGGL(k_phase_table, dim3(blocks_for(cnt)), dim3(256), 0, s, kNStep[a], n[a],
-                               kDelta[a], origin[a], step[a], 1.0 / corrL[a], 2, E[a]);
+        ta.nk[a] = kNStep[a];
+        ta.nx[a] = n[a];
+        ta.block0[a] = tabBlocks;
+        tabBlocks += blocks_for((int64_t)kNStep[a] * n[a]);
+        ta.dk[a] = kDelta[a]; ta.o[a] = origin[a]; ta.step[a] = step[a]; ta.invL[a] = 1.0 / corrL[a];
+        ta.E[a] = E[a];
     }
+    hipLaunchKernelGGL(k_axis_tables, dim3(tabBlocks), dim3(256), 0, s, ta);
     int64_t kNu = 1;
     for (int a = 0; a < nDim; a++) kNu *= kNStep[a];
     const int64_t nC = (int64_t)Nmc * nb * kNu;          // = Nmc x nk3 x Q x nk2 x H x nk1

@@ -79,6 +79,11 @@ hipError_t rf_launch_iso_prep(int nDim, int mode, int shared, int64_t kN, int Nm
 hipError_t rf_launch_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* d_phase,
                                const double* d_amp, double ampMult, float* d_phT, float* d_aT,
                                hipStream_t s);
+// uniforms first + r kN + j of stream (seed, 2), their phases and, d_phT given,
+// rf_launch_prep_fp32's operands, in one launch
+hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, const double* d_amp,
+                               double ampMult, double* d_uni, double* d_phase, float* d_phT, float* d_aT,
+                               hipStream_t s);
 hipError_t rf_launch_krev(int64_t count, const double* d_k, double* d_kRev, hipStream_t s);
 hipError_t rf_launch_fft_coeffs(int64_t kN, int Nmc, const double* d_Sk, const double* d_u,
                                 const uint8_t* d_calc, double* d_amp, double* d_phase, hipStream_t s);

@@ -101,6 +101,43 @@ __global__ void k_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* __restr
     }
 }
 
+// A plan's new realizations in one launch (methods 2 and 3): uniforms
+// first + r kN + j of stream (seed, tag 2) to uni[r][j], phases 2 pi U to
+// phase[r][j] and, phT given, the FP32 direct-sum operands of k_prep_fp32.  One
+// thread per wavevector: the uniforms and phases of a realization are written
+// along j, the Rpad operands of a wavevector as whole 64-byte pieces (bound by
+// those writes; three launches that read the phases back transposed took 27 us
+// for 332,928 wavevectors x 4 realizations, this one 21 us, 75 MB).
+__global__ __launch_bounds__(kBlock) void k_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first,
+                                                      const double* __restrict__ amp, double ampMult,
+                                                      double* __restrict__ uni, double* __restrict__ phase,
+                                                      float* __restrict__ phT, float* __restrict__ aT) {
+#pragma clang fp contract(off)
+    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= kN) return;
+    for (int r0 = blockIdx.y * 16; r0 < Rpad && r0 < (int)(blockIdx.y + 1) * 16; r0 += 4) {
+        float4 p = make_float4(0.f, 0.f, 0.f, 0.f), a = p;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int r = r0 + u;
+            if (r >= Nmc) break;
+            const int64_t s = (int64_t)r * kN + j;
+            const double U = rf_uniform(seed, 2u, first + (uint64_t)s);
+            const double ph = 2.0 * RF_PI_REF * U;
+            uni[s] = U;
+            phase[s] = ph;
+            if (phT) {
+                (&p.x)[u] = (float)to_rev(ph);
+                (&a.x)[u] = (float)(amp[s] * ampMult);
+            }
+        }
+        if (phT) {
+            *reinterpret_cast<float4*>(phT + j * Rpad + r0) = p;
+            *reinterpret_cast<float4*>(aT + j * Rpad + r0) = a;
+        }
+    }
+}
+
 // Isotropic FP32 operands: kT[j][r][D] = k_rj / (2 pi), pT[j][r] = psi_rj in
 // revolutions, aT[j][r] = amp_rj * ampMult; padded realizations are zero.
 __global__ void k_prep_fp32_iso(int nDim, int64_t kN, int Nmc, int Rpad,
@@ -219,6 +256,17 @@ hipError_t rf_launch_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* d_ph
     const int64_t n = kN * Rpad;
     hipLaunchKernelGGL(k_prep_fp32, dim3(grid_for(n)), dim3(kBlock), 0, s, kN, Nmc, Rpad, d_phase,
                        d_amp, ampMult, d_phT, d_aT);
+    return hipGetLastError();
+}
+
+hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, const double* d_amp,
+                               double ampMult, double* d_uni, double* d_phase, float* d_phT, float* d_aT,
+                               hipStream_t s) {
+    const int R = d_phT ? Rpad : (Nmc + 3) / 4 * 4;        // whole float4 pieces (Rpad is a multiple of 16)
+    const unsigned gy = (unsigned)((R + 15) / 16);
+    if (gy > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_draw_prep, dim3(grid_for(kN), gy), dim3(kBlock), 0, s, kN, Nmc, R, seed, first, d_amp, ampMult,
+                       d_uni, d_phase, d_phT, d_aT);
     return hipGetLastError();
 }
 
