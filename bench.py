@@ -222,7 +222,7 @@ def run_cfg4(args):
     batch = R.GridBatch(ctx, plans, [x[0] for x in geo], [step] * len(geo), [x[1] for x in geo], fields,
                         R.DTYPE_F32)
     bplan = R.BlendPlan(ctx, groupN, Nmc, origins, sizes, [nOvl] * 3, masks, R.FIXED, fields, R.DTYPE_F32)
-    # tile kinds per contraction (the autotuner) before any capture: the
+    # table tiles per wave of each contraction (the autotuner) before any capture: the
     # graphs keep the launch shapes of the time they were captured
     kinds = batch.autotune(sptr)
     fresh = R.Graph(ctx, sptr)
@@ -319,7 +319,7 @@ def run_cfg4(args):
         traffic["source"] = "profiles/traffic_cfg4_step.json (rocprofv3 --pmc of bench.py --config 4)"
     best_fused = wall_ff <= wall_f
     step_wall = wall_ff if best_fused else wall_f
-    # every first contraction on 64x160 tiles: those form the fresh
+    # the whole ~131-point first axis (5 tiles) in a wave: the strips form the fresh
     # coefficients themselves and the redraw only advances the draw state
     formed = int(kinds[0]) == 5
     return _line("points x realizations / s (cfg4 localization: fresh realizations, generation + blend)",

@@ -351,13 +351,11 @@ int rf_grid_batch_execute(rf_grid_batch* batch, void* stream);
  * draw per createRandomField call, randomFieldND.f90:276-279).  Allocation-
  * free, capturable; method 4 batches: RF_E_UNSUPPORTED. */
 #define RF_DRAW_NEXT (-1)
-/* Times each contraction stage of the batch with the wide tile kinds the
- * set-up chose, with 128 x 64 tiles where it chose a 64 x 160 tile spanning a
- * whole 129..160-point axis, and with 64 x 64 tiles on every GEMM of the
- * stage, keeps the fastest (chosen[3]: the kind now used per stage, 1 =
- * 64 x 64, 2 128x64, 3 64x128 real part, 4 64x128, 5 64x160) and
+/* Times each contraction stage of the batch with its phase-table axis held
+ * whole by a wave (up to five 32-entry tiles) or split over several, keeps the
+ * fastest (chosen[3]: tiles per wave now used per stage, 1..5) and
  * leaves one execute's result in the outputs.  The field values do not depend
- * on the tile kind (the same K order per element).  Synchronous; no
+ * on the split (the same K order per element).  Synchronous; no
  * counterpart in the reference.  This and rf_grid_batch_fuse_blend rewrite
  * the batch's device tables: a graph captured before either keeps its old
  * launch shapes and must be captured again. */

@@ -372,8 +372,9 @@ class GridBatch:
         check(lib().rf_grid_batch_execute(self._h, _ptr(stream)), self.ctx.handle)
 
     def autotune(self, stream=None):
-        """Times each stage with its wide tile kinds and with 64 x 64 tiles,
-        keeps the faster; returns the widest kind used per stage."""
+        """Times each stage with its phase-table axis held whole by a wave and
+        split over several, keeps the fastest; returns the 32-entry tiles per
+        wave of each stage."""
         chosen = (C.c_int32 * 3)()
         check(lib().rf_grid_batch_autotune(self._h, _ptr(stream), chosen), self.ctx.handle)
         return list(chosen)

@@ -9,6 +9,7 @@
 // geometry and the phases (phase tables, coefficients, GEMM descriptors);
 // rf_grid_batch_execute then enqueues three grouped GEMM launches and nothing
 // else, so it can be captured into a graph and replayed.
+#include <algorithm>
 #include <cstring>
 #include <cmath>
 #include <memory>
@@ -23,9 +24,11 @@ struct rf_grid_batch {
     char* d_mem = nullptr;              // scratch of every field, then descriptors
     rf_gemm_desc* d_desc[3] = {nullptr, nullptr, nullptr};
     int nDesc[3] = {0, 0, 0};
-    int64_t tiles[3] = {0, 0, 0};
-    int realOut[3] = {0, 0, 1};
-    int rwMax[3] = {1, 1, 1};           // wide tile kind used by a stage's GEMMs (1: none)
+    // a stage's strip GEMMs come first and run in one launch of mt[] tiles per
+    // wave, its FP32-operand GEMMs (normally none) in another
+    int nStrip[3] = {0, 0, 0};
+    int64_t stripTiles[3] = {0, 0, 0}, fp32Tiles[3] = {0, 0, 0};
+    int mt[3] = {1, 1, 1};
     // fresh realizations: every field's coefficient fold, its seed and Nmc,
     // and the device draw counter (realizations counter * Nmc .. of each
     // field's device stream)
@@ -37,10 +40,8 @@ struct rf_grid_batch {
     bool genActive = false;             // the last redraw left the first contraction forming the coefficients
     rf_fold_item* d_items = nullptr;    // the folds as one grouped launch
     int64_t foldBlocks = 0;
-    // host copies of the stage descriptors and the tile kinds the set-up
-    // chose (the autotuner switches a stage between those and 64 x 64)
+    // host copies of the stage descriptors
     std::vector<rf_gemm_desc> stage[3];
-    std::vector<int> kind0[3];
     int outDtype = RF_DTYPE_F32;
 };
 
@@ -53,25 +54,42 @@ struct rf_graph {
 namespace {
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
-// tile offsets, tile counts and widest kind of every stage, uploaded
+// tile offsets and tile counts of every stage for its mt, uploaded
 hipError_t upload_stages(rf_grid_batch* B, hipStream_t s) {
     std::vector<rf_gemm_desc> all;
     for (int k = 0; k < 3; k++) {
-        int64_t t = 0;
-        B->rwMax[k] = 1;
+        int64_t t[2] = {0, 0};                      // strips, FP32 tiles
+        B->nStrip[k] = 0;
         for (auto& g : B->stage[k]) {
-            g.tile0 = t;
-            t += rf_gemm_tiles(g);
-            if (g.rw > B->rwMax[k]) B->rwMax[k] = g.rw;
+            const int fp32 = g.mt == 0;
+            g.tile0 = t[fp32];
+            t[fp32] += rf_gemm_tiles(g, fp32 ? 0 : B->mt[k]);
+            if (!fp32) B->nStrip[k]++;
         }
-        B->tiles[k] = t;
+        B->stripTiles[k] = t[0];
+        B->fp32Tiles[k] = t[1];
         all.insert(all.end(), B->stage[k].begin(), B->stage[k].end());
     }
     for (int k = 0; k < 3; k++)
-        if (B->tiles[k] > 0x7fffffffLL) return hipErrorInvalidValue;
+        if (B->stripTiles[k] > 0x7fffffffLL || B->fp32Tiles[k] > 0x7fffffffLL) return hipErrorInvalidValue;
     hipError_t e = hipMemcpyAsync(B->d_desc[0], all.data(), all.size() * sizeof(rf_gemm_desc), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     return e;
+}
+
+hipError_t run_stage(const rf_grid_batch* B, int k, hipStream_t s) {
+    const int n = B->nStrip[k];
+    const hipError_t e = rf_launch_gemm_group(k, B->mt[k], B->d_desc[k], n, B->stripTiles[k], s);
+    if (e != hipSuccess) return e;
+    return rf_launch_gemm_group(k, 0, B->d_desc[k] + n, B->nDesc[k] - n, B->fp32Tiles[k], s);
+}
+
+// every field's coefficients are formed by the first contraction itself:
+// strips that hold the whole first axis (each coefficient formed once)
+bool first_forms_coefficients(const rf_grid_batch* B) {
+    bool gen = !B->stage[0].empty();
+    for (const auto& g : B->stage[0]) gen = gen && g.mt > 0 && g.genState && (g.M + 31) / 32 <= B->mt[0];
+    return gen;
 }
 }  // namespace
 
@@ -179,7 +197,10 @@ int rf_grid_batch_create(rf_context* ctx, int32_t n, rf_field_plan* const* plans
     size_t dOff = 0;
     for (int k = 0; k < 3; k++) {
         B->stage[k] = stage[k];
-        for (const auto& g : stage[k]) B->kind0[k].push_back(g.rw);
+        std::stable_partition(B->stage[k].begin(), B->stage[k].end(), [](const rf_gemm_desc& g) { return g.mt > 0; });
+        // the whole table axis in one wave: a batch fills the chip
+        for (const auto& g : stage[k])
+            if (g.mt > 0) B->mt[k] = std::max(B->mt[k], std::min((g.M + 31) / 32, kStripMaxMT));
         B->nDesc[k] = (int)stage[k].size();
         B->d_desc[k] = reinterpret_cast<rf_gemm_desc*>(B->d_mem + descOff) + dOff;
         dOff += stage[k].size();
@@ -215,8 +236,7 @@ int rf_grid_batch_execute(rf_grid_batch* B, void* stream) {
     if (!B) return rf_set_error(nullptr, RF_E_ARG, "batch is NULL");
     rf_context* ctx = B->ctx;
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    for (int k = 0; k < 3; k++)
-        RF_HIP_TRY(ctx, rf_launch_gemm_group(B->realOut[k], B->d_desc[k], B->nDesc[k], B->tiles[k], B->rwMax[k], s));
+    for (int k = 0; k < 3; k++) RF_HIP_TRY(ctx, run_stage(B, k, s));
     return RF_OK;
 }
 
@@ -226,8 +246,8 @@ int rf_grid_batch_autotune(rf_grid_batch* B, void* stream, int32_t* chosen) {
     RF_HIP_TRY(ctx, hipSetDevice(ctx->device));
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
     if (B->genActive) {
-        // the current realizations' coefficients stored, as every tile kind
-        // reads them, and the first contraction back to reading them
+        // the current realizations' coefficients stored, as every split
+        // of the table axis reads them, and the first contraction back to reading them
         RF_HIP_TRY(ctx, rf_launch_refold_draw(B->d_items, (int)B->folds.size(), B->foldBlocks, B->d_draw + 1, s));
         RF_HIP_TRY(ctx, rf_launch_draw_counter(B->d_draw, -3, 0, s));
         B->genActive = false;
@@ -242,10 +262,9 @@ int rf_grid_batch_autotune(rf_grid_batch* B, void* stream, int32_t* chosen) {
         return rf_set_error(ctx, RF_E_HIP, hipGetErrorString(he));
     }
     auto time_stage = [&](int k, float* ms) -> hipError_t {
-        hipError_t e = rf_launch_gemm_group(B->realOut[k], B->d_desc[k], B->nDesc[k], B->tiles[k], B->rwMax[k], s);
+        hipError_t e = run_stage(B, k, s);
         if (e == hipSuccess) e = hipEventRecord(e0, s);
-        for (int i = 0; i < 3 && e == hipSuccess; i++)
-            e = rf_launch_gemm_group(B->realOut[k], B->d_desc[k], B->nDesc[k], B->tiles[k], B->rwMax[k], s);
+        for (int i = 0; i < 3 && e == hipSuccess; i++) e = run_stage(B, k, s);
         if (e == hipSuccess) e = hipEventRecord(e1, s);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
         if (e == hipSuccess) e = hipEventElapsedTime(ms, e0, e1);
@@ -253,38 +272,31 @@ int rf_grid_batch_autotune(rf_grid_batch* B, void* stream, int32_t* chosen) {
     };
     hipError_t e = hipSuccess;
     for (int k = 0; k < 3 && e == hipSuccess; k++) {
-        bool wide = false;
-        for (int r : B->kind0[k]) wide |= r > 1;
-        if (!wide) continue;
-        // candidates: the set-up's wide kinds, 128x64 tiles where it chose
-        // the 64x160 whole-axis tile, and 64 x 64 tiles everywhere
-        auto kind_of = [&](int opt, int i) {
-            const int r = B->kind0[k][i];
-            return opt == 0 ? r : opt == 1 ? (r == 5 ? 2 : r) : 1;
-        };
-        bool narrower = false;
-        for (int r : B->kind0[k]) narrower |= r == 5;
+        if (!B->nStrip[k]) continue;
+        // candidates: the longest table axis in 1, 2, 3, .. groups
+        int mtTot = 1;
+        for (const auto& g : B->stage[k])
+            if (g.mt > 0) mtTot = std::max(mtTot, (g.M + 31) / 32);
         float best = 0.0f;
-        int bestOpt = 0;
-        for (int opt = 0; opt < 3 && e == hipSuccess; opt++) {
-            if (opt == 1 && !narrower) continue;
-            for (size_t i = 0; i < B->stage[k].size(); i++) B->stage[k][i].rw = kind_of(opt, (int)i);
+        int bestMt = B->mt[k];
+        for (int mt = std::min(mtTot, kStripMaxMT); mt >= 1 && e == hipSuccess; mt--) {
+            B->mt[k] = mt;
             e = upload_stages(B, s);
             float ms = 0.0f;
             if (e == hipSuccess) e = time_stage(k, &ms);
-            if (e == hipSuccess && (opt == 0 || ms < best)) {
+            if (e == hipSuccess && (best == 0.0f || ms < best)) {
                 best = ms;
-                bestOpt = opt;
+                bestMt = mt;
             }
         }
-        for (size_t i = 0; i < B->stage[k].size(); i++) B->stage[k][i].rw = kind_of(bestOpt, (int)i);
+        B->mt[k] = bestMt;
     }
     if (e == hipSuccess) e = upload_stages(B, s);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (e != hipSuccess) return rf_set_error(ctx, RF_E_HIP, std::string("batch autotune: ") + hipGetErrorString(e));
     if (chosen)
-        for (int k = 0; k < 3; k++) chosen[k] = B->rwMax[k];
+        for (int k = 0; k < 3; k++) chosen[k] = B->mt[k];
     return RF_OK;
 }
 
@@ -294,12 +306,10 @@ int rf_grid_batch_redraw(rf_grid_batch* B, int64_t drawIndex, void* stream) {
     if (!B->redrawable)
         return rf_set_error(ctx, RF_E_UNSUPPORTED, "rf_grid_batch_redraw: method 4 fields have no phases to redraw");
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    // when every field's first contraction runs on 64x160 tiles, those form
-    // the coefficients of the current draw themselves (no fold, no
-    // coefficient round trip through HBM); otherwise the grouped fold
-    // stores them
-    bool gen = !B->stage[0].empty();
-    for (const auto& g : B->stage[0]) gen = gen && g.rw == 5 && g.genState;
+    // when the first contraction's strips hold the whole first axis, they form
+    // the coefficients of the current draw themselves (no fold, no coefficient
+    // round trip through HBM); otherwise the grouped fold stores them
+    const bool gen = first_forms_coefficients(B);
     RF_HIP_TRY(ctx, rf_launch_draw_counter(B->d_draw, drawIndex >= 0 ? drawIndex : -1, gen ? 1 : 0, s));
     if (!gen)
         RF_HIP_TRY(ctx, rf_launch_refold_draw(B->d_items, (int)B->folds.size(), B->foldBlocks, B->d_draw + 1, s));
@@ -359,7 +369,7 @@ int rf_grid_batch_fuse_blend(rf_grid_batch* B, rf_blend_plan* P, void* d_group) 
     };
     std::vector<rf_gemm_desc> fused = last;
     for (auto& g : fused) {
-        if (!g.split16) return rf_set_error(ctx, RF_E_UNSUPPORTED, "fused blend: FP32-operand last stage");
+        if (g.mt == 0) return rf_set_error(ctx, RF_E_UNSUPPORTED, "fused blend: FP32-operand last stage");
         int s0 = -1;
         for (size_t k = 0; k < P->fields.size(); k++)
             if (P->fields[k] == g.D) { s0 = (int)k; break; }

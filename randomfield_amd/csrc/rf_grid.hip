@@ -14,9 +14,9 @@
 // Every stage is one tiled complex GEMM on the matrix cores,
 // D[m][n] = sum_k A[m][k] B[k][n] with per-stage strides: operands split
 // into FP16 hi + lo halves (power-of-two scaled into range), three
-// v_mfma_f32_32x32x16_f16 products with FP32 accumulation, on 64x64 tiles or
-// the wide kinds along each stage's long axis; an FP32-operand MFMA tile
-// (v_mfma_f32_32x32x2_f32) serves shapes whose K would leave the FP16 range.
+// v_mfma_f32_32x32x16_f16 products with FP32 accumulation (strip GEMMs, below);
+// an FP32-operand MFMA tile (v_mfma_f32_32x32x2_f32) serves shapes whose K would
+// leave the FP16 range or whose strides a strip's 32-bit offsets.
 // The negative sign blocks are folded into the first contraction
 // (conjugated tables and coefficients).  The phase tables are formed in FP64
 // and rounded to FP32; accumulation is FP32 over <= 4*N_k^(1/3) terms.
@@ -167,15 +167,6 @@ __device__ __forceinline__ void gemm_tile(const rf_gemm_desc& g, int m0, int n0,
     }
 }
 
-// The same tile on the FP16 matrix cores (v_mfma_f32_32x32x16_f16), operands
-// split into FP16 hi + lo and D += A_hi B_hi + A_hi B_lo + A_lo B_hi (FP32
-// accumulate): ~22 significant bits per operand, 3x the instructions of one
-// product at 10x the FP32 MFMA rate.  A chunk of 16 complex k is converted
-// once while staged: A into planes Re, Im, -Im (hi and lo each) as [row][k],
-// B into Re, Im (hi, lo) as [column][k], so every MFMA operand is one 16-byte
-// LDS read.  In the complex product a 32-row MFMA tile holds 16 complex rows,
-// Re D in rows 0-15 ([Re A | -Im A] against [Re B ; Im B]) and Im D in rows
-// 16-31 ([Im A | Re A]); K' = 16 covers 8 complex k, lanes 0-31 the Re half.
 typedef float f2v __attribute__((ext_vector_type(2)));
 typedef const f2v __attribute__((address_space(1))) gf2;      // global-memory views
 typedef f2v __attribute__((address_space(1))) gf2o;
@@ -224,24 +215,11 @@ __device__ __forceinline__ int64_t band_col(const rf_gemm_desc& g, int n, int ba
     return lo ? offLo : hi ? offHi : (int64_t)-1;
 }
 
-// Tile kinds (rf_gemm_desc::rw): 1 64x64; 2 128x64 complex product (two
-// 16-row groups per wave share each B fragment read); 3 64x128 real part
-// (two 32-column tiles per wave share each A fragment read; A holds only the
-// Re and -Im planes); 4 64x128 complex product (four 32-column tiles per
-// wave share each A fragment read); 5 64x160 complex product (a column axis
-// of 129..160 in one tile: each row slab of A is staged once, not once per
-// 64 columns with the last tile nearly empty; five 32-column tiles per wave
-// share each A fragment read)
-constexpr int kTN5 = 160;
-template <int RW>
+// Operand planes of a 64x128 real-part tile (the isotropic GEMM).
 struct HStage {
-    _Float16 a[RW == 3 ? 4 : 6][kTM * (RW == 2 ? 2 : 1)][kHP];   // Re hi, Re lo, Im hi, Im lo, -Im hi, -Im lo
-    _Float16 b[4][RW == 5 ? kTN5 : kTN * (RW >= 3 ? 2 : 1)][kHP];  // Re hi, Re lo, Im hi, Im lo
+    _Float16 a[4][kTM][kHP];          // Re hi, Re lo, -Im hi, -Im lo
+    _Float16 b[4][2 * kTN][kHP];      // Re hi, Re lo, Im hi, Im lo
 };
-__host__ __device__ inline int tile_m(const rf_gemm_desc& g) { return g.rw == 2 ? 2 * kTM : kTM; }
-__host__ __device__ inline int tile_n(const rf_gemm_desc& g) {
-    return g.rw == 5 ? kTN5 : (g.rw == 3 || g.rw == 4) ? 2 * kTN : kTN;
-}
 
 // v -> FP16 hi (round to nearest) and lo = v - hi: packed conversions for
 // hi and lo, the residuals by mixed-precision FMAs reading the f16 halves in
@@ -262,327 +240,10 @@ __device__ inline void split4(const float* v, hv4* hi, hv4* lo) {
     }
 }
 
-// split4 for two values
-typedef _Float16 hv2 __attribute__((ext_vector_type(2)));
-__device__ inline void split2(const float* v, hv2* hi, hv2* lo) {
-    const hv2 h = {(_Float16)v[0], (_Float16)v[1]};
-    const unsigned hb = __builtin_bit_cast(unsigned, h);
-    float l0, l1;
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(hb), "v"(v[0]));
-    asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(l1) : "v"(hb), "v"(v[1]));
-    *hi = h;
-    *lo = hv2{(_Float16)l0, (_Float16)l1};
-}
-
 // -x of FP16 values: the sign bits flipped
 __device__ inline hv4 neg4(hv4 x) {
     typedef unsigned u2 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(hv4, __builtin_bit_cast(u2, x) ^ 0x80008000u);
-}
-
-template <bool RealOnly>
-__device__ __forceinline__ void gemm_tile_h(const rf_gemm_desc& g, int m0, int n0, int batch, HStage<1>* st) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    // tile base pointers in 64-bit, offsets inside the tile in 32-bit (the
-    // launcher keeps K * stride and 64 * stride below 2^31)
-    // global address space: the descriptor of a grouped launch is read from
-    // memory, and generic (flat) loads would also count against the LDS
-    // wait counter, so every LDS read of the K-step would wait for the
-    // prefetch of the next one
-    const gf2* A = (const gf2*)(g.A + (int64_t)((batch / g.aDiv) % g.aMod) * g.aStrideB + (int64_t)m0 * g.aSm);
-    const int64_t bCol0 = col_b(g, n0);
-    const gf2* B = (const gf2*)(g.B + (int64_t)batch * g.bStrideB + bCol0);
-    const int aSm = (int)g.aSm, aSk = (int)g.aSk, bSk = (int)g.bSk;
-    f32x16 acc0, acc1;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        acc0[i] = 0.0f;
-        acc1[i] = 0.0f;
-    }
-    const int rt = wave >> 1, ct = wave & 1;
-    // staging: A row t/4, k 4(t%4)..+3; B column t%64, k 4(t/64)..+3
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 63, bK = (tid >> 6) * 4;
-    const bool aIn = m0 + aRow < g.M, bIn = n0 + bCol < g.N;
-    // rows / columns / k outside the operand stage zeros; the prefetch
-    // loads are waited for only when staged (a clamped, branch-free form
-    // with the zeroing at staging time measured 5 % slower: more VALU)
-    const int aOff = aRow * aSm, bOff = bIn ? (int)(col_b(g, n0 + bCol) - bCol0) : 0;
-    const int kLast = g.K - 1;
-    f2v ra[4], rb[4];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int ka = k0 + aK + i, kb = k0 + bK + i;
-            ra[i] = (aIn && ka <= kLast) ? A[aOff + ka * aSk] : f2v{0.f, 0.f};
-            rb[i] = (bIn && kb <= kLast) ? B[kb * bSk + bOff] : f2v{0.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = ra[i].x;
-            im[i] = ra[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[0][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[1][aRow][aK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[2][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[3][aRow][aK]) = lo;
-        *reinterpret_cast<hv4*>(&st->a[4][aRow][aK]) = neg4(hi);   // split(-x) = -split(x)
-        *reinterpret_cast<hv4*>(&st->a[5][aRow][aK]) = neg4(lo);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = rb[i].x;
-            im[i] = rb[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->b[0][bCol][bK]) = hi;
-        *reinterpret_cast<hv4*>(&st->b[1][bCol][bK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->b[2][bCol][bK]) = hi;
-        *reinterpret_cast<hv4*>(&st->b[3][bCol][bK]) = lo;
-    };
-    // this lane's operand planes: complex product, tile row l32 = Re (< 16)
-    // or Im row of complex row (l32 & 15); K' half 0 reads Re B, 1 reads Im B
-    const int isIm = l32 >> 4;
-    const int aPlane = RealOnly ? (half ? 4 : 0) : (isIm ? (half ? 0 : 2) : (half ? 4 : 0));
-    const int aRowL = RealOnly ? rt * 32 + l32 : wave * 16 + (l32 & 15);
-    const int bPlane = half ? 2 : 0;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-#pragma unroll
-        for (int kk = 0; kk < kTK; kk += 8) {
-            if (!RealOnly) {
-                if (m0 + wave * 16 < g.M) {
-                    const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                    const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-                    const hv8 bh0 = *reinterpret_cast<const hv8*>(&st->b[bPlane][l32][kk]);
-                    const hv8 bl0 = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][l32][kk]);
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh0, acc0, 0, 0, 0);
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl0, acc0, 0, 0, 0);
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh0, acc0, 0, 0, 0);
-                    if (n0 + 32 < g.N) {
-                        const hv8 bh1 = *reinterpret_cast<const hv8*>(&st->b[bPlane][32 + l32][kk]);
-                        const hv8 bl1 = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][32 + l32][kk]);
-                        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh1, acc1, 0, 0, 0);
-                        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl1, acc1, 0, 0, 0);
-                        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh1, acc1, 0, 0, 0);
-                    }
-                }
-            } else if (m0 + rt * 32 < g.M && n0 + ct * 32 < g.N) {
-                const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-                const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][ct * 32 + l32][kk]);
-                const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][ct * 32 + l32][kk]);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc0, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc0, 0, 0, 0);
-                acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc0, 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dCol0 = col_d(g, n0);
-    const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)m0 * g.dSm + dCol0;
-    const int dSm = (int)g.dSm;
-    // this lane's column offsets (32-bit inside the tile)
-    auto dcol = [&](int nn) { return n0 + nn < g.N ? (int)(col_d(g, n0 + nn) - dCol0) : 0; };
-    if (!RealOnly) {
-        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + dBase);
-        const int oc[2] = {dcol(l32), dcol(32 + l32)};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = wave * 16 + 8 * (i >> 2) + 4 * half + (i & 3);   // Re row r, Im row r + 16
-            if (m0 + r >= g.M) continue;
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int nn = c * 32 + l32;
-                if (n0 + nn >= g.N) continue;
-                D[r * dSm + oc[c]] = c ? f2v{acc1[i] * os, acc1[i + 8] * os}
-                                          : f2v{acc0[i] * os, acc0[i + 8] * os};
-            }
-        }
-    } else {
-        const int nn = ct * 32 + l32;
-        const bool nIn = n0 + nn < g.N;
-        const int oc = dcol(nn);
-        // fused blend: this lane's column offset in the group grid, or -1,
-        // and in a first-axis band array, or -1
-        const int64_t gc = (g.grp && nIn) ? grp_col(g, n0 + nn) : -1;
-        int bside = 0, bst = 0;
-        const int64_t bo = (g.grp && nIn && gc < 0) ? band_col(g, n0 + nn, batch, &bside, &bst) : -1;
-        auto store = [&](auto map, auto* D, auto* G, auto* BL, auto* BH) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int r = rt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (m0 + r < g.M && nIn) {
-                    const auto v = map(acc0[i] * os);
-                    const int64_t gr = gc >= 0 ? grp_row(g, m0 + r) : -1;
-                    if (gr >= 0) G[gr + gc] = v;
-                    else if (bo >= 0) (bside ? BH : BL)[bo + (int64_t)(m0 + r) * bst] = v;
-                    else D[r * dSm + oc] = v;
-                }
-            }
-        };
-        const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
-        gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
-        gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
-        gfo* G32 = (gfo*)(static_cast<float*>(g.grp) + (int64_t)batch * g.grpStrideB);
-        gdo* G64 = (gdo*)(static_cast<double*>(g.grp) + (int64_t)batch * g.grpStrideB);
-        gfo* L32 = (gfo*)static_cast<float*>(g.bandLo);
-        gfo* H32 = (gfo*)static_cast<float*>(g.bandHi);
-        gdo* L64 = (gdo*)static_cast<double*>(g.bandLo);
-        gdo* H64 = (gdo*)static_cast<double*>(g.bandHi);
-        if (g.outDtype == RF_DTYPE_F64) {
-            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64, G64, L64, H64);
-            else if (g.epi.margi == RF_FOM_LOGNORMAL)
-                store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64, G64, L64, H64);
-            else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64, G64, L64, H64);
-        } else {
-            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32, G32, L32, H32);
-            else if (g.epi.margi == RF_FOM_LOGNORMAL)
-                store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32, G32, L32, H32);
-            else store([=](float u) { return fmaf(u, sc, sh); }, D32, G32, L32, H32);
-        }
-    }
-}
-
-// 128-row tiles of the complex product (used where the row axis is long,
-// the first contraction): each wave owns two 16-complex-row groups and reads
-// each B fragment once for both (8 fragment reads per 12 MFMAs instead of 6
-// per 6); staging, operand split and epilogue as gemm_tile_h.
-__device__ __forceinline__ void gemm_tile_c128(const rf_gemm_desc& g, int m0, int n0, int batch, HStage<2>* st) {
-    constexpr int RW = 2;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)((batch / g.aDiv) % g.aMod) * g.aStrideB + (int64_t)m0 * g.aSm);
-    const int64_t bCol0 = col_b(g, n0);
-    const gf2* B = (const gf2*)(g.B + (int64_t)batch * g.bStrideB + bCol0);
-    const int aSm = (int)g.aSm, aSk = (int)g.aSk, bSk = (int)g.bSk;
-    f32x16 acc[RW][2];
-#pragma unroll
-    for (int rr = 0; rr < RW; rr++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            acc[rr][0][i] = 0.0f;
-            acc[rr][1][i] = 0.0f;
-        }
-    // staging: A rows t/4 and t/4 + 64, k 4(t%4)..+3; B column t%64, k 4(t/64)..+3
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 63, bK = (tid >> 6) * 4;
-    bool aIn[RW];
-#pragma unroll
-    for (int rr = 0; rr < RW; rr++) aIn[rr] = m0 + aRow + 64 * rr < g.M;
-    const bool bIn = n0 + bCol < g.N;
-    const int aOff = aRow * aSm, bOff = bIn ? (int)(col_b(g, n0 + bCol) - bCol0) : 0;
-    const int kLast = g.K - 1;
-    f2v ra[RW][4], rb[4];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int ka = k0 + aK + i, kb = k0 + bK + i;
-#pragma unroll
-            for (int rr = 0; rr < RW; rr++)
-                ra[rr][i] = (aIn[rr] && ka <= kLast) ? A[aOff + 64 * rr * aSm + ka * aSk] : f2v{0.f, 0.f};
-            rb[i] = (bIn && kb <= kLast) ? B[kb * bSk + bOff] : f2v{0.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int rr = 0; rr < RW; rr++) {
-            const int row = aRow + 64 * rr;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = ra[rr][i].x;
-                im[i] = ra[rr][i].y;
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->a[0][row][aK]) = hi;
-            *reinterpret_cast<hv4*>(&st->a[1][row][aK]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->a[2][row][aK]) = hi;
-            *reinterpret_cast<hv4*>(&st->a[3][row][aK]) = lo;
-            *reinterpret_cast<hv4*>(&st->a[4][row][aK]) = neg4(hi);   // split(-x) = -split(x)
-            *reinterpret_cast<hv4*>(&st->a[5][row][aK]) = neg4(lo);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = rb[i].x;
-            im[i] = rb[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->b[0][bCol][bK]) = hi;
-        *reinterpret_cast<hv4*>(&st->b[1][bCol][bK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->b[2][bCol][bK]) = hi;
-        *reinterpret_cast<hv4*>(&st->b[3][bCol][bK]) = lo;
-    };
-    // operand planes as in gemm_tile_h's complex product; row group rr of
-    // this wave starts at row (2 wave + rr) 16
-    const int isIm = l32 >> 4;
-    const int aPlane = isIm ? (half ? 0 : 2) : (half ? 4 : 0);
-    const int aRowL = wave * 16 * RW + (l32 & 15);
-    const int bPlane = half ? 2 : 0;
-    const bool c1 = n0 + 32 < g.N;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + wave * 16 * RW < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    if (c == 1 && !c1) break;                                      // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][32 * c + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][32 * c + l32][kk]);
-#pragma unroll
-                    for (int rr = 0; rr < RW; rr++) {
-                        if (rr > 0 && m0 + (wave * RW + rr) * 16 >= g.M) break;   // uniform
-                        const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL + 16 * rr][kk]);
-                        const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL + 16 * rr][kk]);
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[rr][c], 0, 0, 0);
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[rr][c], 0, 0, 0);
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[rr][c], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dCol0 = col_d(g, n0);
-    const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)m0 * g.dSm + dCol0;
-    const int dSm = (int)g.dSm;
-    auto dcol = [&](int nn) { return n0 + nn < g.N ? (int)(col_d(g, n0 + nn) - dCol0) : 0; };
-    gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + dBase);
-    const int oc[2] = {dcol(l32), dcol(32 + l32)};
-#pragma unroll
-    for (int rr = 0; rr < RW; rr++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = (wave * RW + rr) * 16 + 8 * (i >> 2) + 4 * half + (i & 3);   // Re row r, Im row r + 16
-            if (m0 + r >= g.M) continue;
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                const int nn = c * 32 + l32;
-                if (n0 + nn >= g.N) continue;
-                D[r * dSm + oc[c]] = f2v{acc[rr][c][i] * os, acc[rr][c][i + 8] * os};
-            }
-        }
 }
 
 // cos and sin of 2 pi U for U in [0, 1): FP32 sincospi of the FP32 part Uh
@@ -616,320 +277,310 @@ __device__ __forceinline__ float2 fold_coef_draw(const rf_fold_desc& f, unsigned
     return make_float2((float)(a * (double)cs), (float)(h ? -(a * (double)sn) : a * (double)sn));
 }
 
-// 64x160 tiles of the complex product (the first contraction when its
-// column axis, the first grid axis, has 129..160 points): wave w owns complex
-// rows 16 w.. and the five 32-column tiles, reading each A fragment once for
-// all five; B (the phase table, small) is staged for all 160 columns.
-// Staging, operand split and epilogue as gemm_tile_c128.
-__device__ __forceinline__ void gemm_tile_c160(const rf_gemm_desc& g, int m0, int n0, int batch, HStage<5>* st) {
-    constexpr int NC = kTN5 / 32;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)((batch / g.aDiv) % g.aMod) * g.aStrideB + (int64_t)m0 * g.aSm);
-    const int64_t bCol0 = col_b(g, n0);
-    const gf2* B = (const gf2*)(g.B + (int64_t)batch * g.bStrideB + bCol0);
-    const int aSm = (int)g.aSm, aSk = (int)g.aSk, bSk = (int)g.bSk;
-    f32x16 acc[NC];
+// The strip GEMM: every contraction of the grid form with FP16 operands.
+//
+// One operand of each contraction is a small phase table shared by the whole
+// launch (M entries of an axis x K), the other -- the coefficients or the
+// previous contraction's output -- is streamed, N lines of K complex values.
+// A wave owns 32 lines and MT 32-entry tiles of the table axis (with MT * 32 >=
+// M every streamed value is read from memory and converted once in the whole
+// launch).  Operands are split into FP16 hi + lo halves; three
+// v_mfma_f32_32x32x16_f16 products (hi hi, hi lo, lo hi) with FP32 accumulation.
+//
+// A K-step is 8 complex k = 16 MFMA K entries: the re parts in lane half 0, the
+// im parts in half 1.  A lane loads k = 8 s + 4 h + (0..3) of its own line straight
+// to registers (no LDS), splits them and trades with the other half
+// (v_permlane32_swap).  Re D pairs table (re, im) with streamed (re, -im); Im D pairs
+// (im, re) with (re, im) -- the lane reads the other half's slot -- or, in the
+// first contraction, (re, im) with (im, re).  The table is stored in HBM pre-split
+// in fragment order [step][tile][hi, lo][lane][8] (k_axis_tables) and goes to LDS by
+// direct loads, kStripCS steps ahead in a double buffer, shared by the block's
+// waves; one barrier per kStripCS steps.
+//
+// Replaces 64..160-wide block tiles that staged and split both operands in LDS
+// per 16 k, re-reading and re-splitting the streamed one per table tile, two
+// barriers per 16 k.  32 fields of ~131^3 x 16 realizations: first contraction
+// (with its draws) 1.48 -> 1.44 ms, middle 1.93 -> 1.27, last 3.1 -> 2.44; 128^3
+// x 8 of method 4: 104 / 88 / 73 -> 68 / 63 / 64 us.  Same bits.
+//
+// D orientation: the table is the A operand (lanes run along lines) where D
+// is stored with lines contiguous, the B operand (lanes run along the table
+// axis) in the first contraction, whose D has the table axis contiguous.
+constexpr int kStripW = 4;              // waves per block
+constexpr int kStripCS = 2;             // K-steps per LDS chunk
+constexpr int kStripL = 32 * kStripW;   // lines per block
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr int strip_units(int MT) { return kStripCS * MT * 128; }   // 16-byte units of a chunk
+
+__host__ __device__ inline int strip_groups(const rf_gemm_desc& g, int MT) {
+    return ((g.M + 31) / 32 + MT - 1) / MT;
+}
+
+// x and y hold k = 4 h + (0..3) in lane half h: half 0's x for all eight k in
+// half 0, half 1's y for all eight in half 1.
+__device__ __forceinline__ u32x4 half_swap(const hv4& x, const hv4& y) {
+    const u32x2 a = __builtin_bit_cast(u32x2, x), b = __builtin_bit_cast(u32x2, y);
+    const u32x2 p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a.x, b.x, false, false));
+    const u32x2 q = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a.y, b.y, false, false));
+    return u32x4{p.x, q.x, p.y, q.y};
+}
+
+template <int MT, int KIND>
+__device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local, u32x4* ldsA, u32x4* ldsB) {
+    constexpr bool kReal = KIND == RF_GEMM_LAST, kFirst = KIND == RF_GEMM_FIRST;
+    constexpr int NA = kReal ? 1 : 2;                 // accumulators per tile: Re, Im
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // table groups fastest: they share the streamed lines
+    const int mtTot = (g.M + 31) / 32, nGr = strip_groups(g, MT);
+    const int grp = (int)(local % nGr);
+    const int64_t rest = local / nGr;
+    const int nSB = (int)(((int64_t)g.N + kStripL - 1) / kStripL);
+    const int sb = (int)(rest % nSB), batch = (int)(rest / nSB);
+    const int t0 = grp * MT;
+    const int nSteps = (g.K + 7) / 8;
+    const int n0 = sb * kStripL + wave * 32;          // < 2^31: checked by the launcher
+    const bool active = n0 < g.N;                     // uniform
+    const int n0c = active ? n0 : 0;
+    const int n = n0c + l32, nc = n < g.N ? n : g.N - 1;
+    const bool nIn = active && n < g.N;
+
+    f32x16 acc[MT][NA];
 #pragma unroll
-    for (int c = 0; c < NC; c++)
+    for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[c][i] = 0.0f;
-    // staging: A row t/4, k 4(t%4)..+3; B columns t%128 (k 8(t/128)..+7) and
-    // 128 + t%32 (k 2(t/32)..+1)
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 127, bK = (tid >> 7) * 8;
-    const int bCol2 = 128 + (tid & 31), bK2 = (tid >> 5) * 2;
-    const bool aIn = m0 + aRow < g.M, bIn = n0 + bCol < g.N, bIn2 = n0 + bCol2 < g.N;
-    const int aOff = aRow * aSm;
-    const int bOff = bIn ? (int)(col_b(g, n0 + bCol) - bCol0) : 0;
-    const int bOff2 = bIn2 ? (int)(col_b(g, n0 + bCol2) - bCol0) : 0;
-    const int kLast = g.K - 1;
+        for (int a = 0; a < NA; a++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[t][a][i] = 0.0f;
+
+    // streamed operand: wave-uniform base, 32-bit lane offset (the launcher
+    // keeps a strip's span below 2^28 elements).  Global address space: the
+    // descriptor of a grouped launch is read from memory, and generic (flat)
+    // loads would also count against the LDS wait counter.
+    const int64_t col0 = col_b(g, n0c);
+    typedef const char __attribute__((address_space(1))) gch;
+    gch* S = (gch*)(g.B + (int64_t)batch * g.bStrideB + col0);
+    const unsigned kb = (unsigned)g.bSk * 8u;         // bytes per k
+    const unsigned lo0 = (unsigned)(col_b(g, nc) - col0) * 8u;
     // a batch's fresh realizations: the coefficients of the current draw are
-    // formed here (fold_coef_draw, as the fold would store them) instead of
-    // read; the row's digits (j2, q, j3, r) once per tile
-    const bool gen = g.genState != nullptr && g.genState[2] != 0;
+    // formed here (fold_coef_draw, as the fold would store them) instead of read
+    const bool gen = kFirst && g.genState != nullptr && g.genState[2] != 0;
     int64_t drawBase = 0;
     unsigned gr = 0, gj3 = 0, gq = 0, gj2 = 0;
-    if (gen) {
+    if (kFirst && gen) {
         drawBase = g.genState[1] * (int64_t)g.genNmc * g.gen.kNr;
         const unsigned Q = (g.gen.fold && g.gen.nDim == 3) ? 2u : 1u;
-        unsigned rem = (unsigned)(m0 + aRow);
+        unsigned rem = (unsigned)nc;
         gj2 = rem % (unsigned)g.gen.nk2; rem /= (unsigned)g.gen.nk2;
         gq = rem % Q; rem /= Q;
         gj3 = g.gen.nDim == 3 ? rem % (unsigned)g.gen.nk3 : 0u;
         gr = g.gen.nDim == 3 ? rem / (unsigned)g.gen.nk3 : rem;
     }
-    f2v ra[4], rb[8], rb2[2];
-    auto fetch = [&](int k0) {
-        if (gen) {
+    f2v r[kStripCS][4];
+    // a step's values of this lane; past K the table is zero and the last
+    // valid value is read again
+    auto fetch = [&](int s, f2v* v) {
+        if (kFirst && gen) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int ka = k0 + aK + i;
-                if (aIn && ka <= kLast) {
-                    const float2 c = fold_coef_draw(g.gen, gr, gj3, gq, gj2, (unsigned)ka % (unsigned)g.gen.nk1,
-                                                    (unsigned)ka / (unsigned)g.gen.nk1, g.genSeed, drawBase);
-                    ra[i] = f2v{c.x, c.y};
+                const int k = 8 * s + 4 * half + i;
+                if (k < g.K) {
+                    const unsigned h = k >= g.gen.nk1 ? 1u : 0u;
+                    const float2 c = fold_coef_draw(g.gen, gr, gj3, gq, gj2, (unsigned)k - (h ? g.gen.nk1 : 0), h, g.genSeed,
+                                                    drawBase);
+                    v[i] = f2v{c.x, c.y};
                 } else {
-                    ra[i] = f2v{0.f, 0.f};
+                    v[i] = f2v{0.f, 0.f};
                 }
             }
         } else {
+            gch* b = S + (int64_t)(8 * s) * kb;
+            const int left = g.K - 1 - 8 * s;         // >= 0
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int ka = k0 + aK + i;
-                ra[i] = (aIn && ka <= kLast) ? A[aOff + ka * aSk] : f2v{0.f, 0.f};
+                int k = 4 * half + i;
+                if (left < 7) k = k < left ? k : left;                            // uniform: the last step
+                v[i] = *(gf2*)(b + (lo0 + (unsigned)k * kb));
+            }
+        }
+    };
+    // chunk c of the table (steps kStripCS c ..): 1 KB pieces over the waves;
+    // tiles and steps past the table re-read its last ones, whose products are
+    // never stored, resp. never formed
+    const u32x4* T = static_cast<const u32x4*>(g.T);
+    auto dma = [&](int c, u32x4* dst) {
+        constexpr int kPieces = kStripCS * MT * 2;
+#pragma unroll
+        for (int i = 0; i < (kPieces + kStripW - 1) / kStripW; i++) {
+            const int p = wave + i * kStripW;
+            if (kPieces % kStripW == 0 || p < kPieces) {
+                const int st = p / (2 * MT), q = p % (2 * MT);
+                const int s = kStripCS * c + st < nSteps ? kStripCS * c + st : nSteps - 1;
+                const int t = t0 + (q >> 1) < mtTot ? t0 + (q >> 1) : mtTot - 1;
+                __builtin_amdgcn_global_load_lds((const void*)(T + (((int64_t)s * mtTot + t) * 2 + (q & 1)) * 64 + lane),
+                                                 (lds_void*)&dst[p * 64], 16, 0, 0);
+            }
+        }
+    };
+    const int nChunks = (nSteps + kStripCS - 1) / kStripCS;
+    const unsigned sgn = half ? 0x80008000u : 0u;
+    auto chunk = [&](int c, const u32x4* cur, u32x4* nxt) {
+        // fragments of this chunk's streamed values, then the loads of the next
+        u32x4 fh[kStripCS][NA], fl[kStripCS][NA];
+#pragma unroll
+        for (int st = 0; st < kStripCS; st++) {
+            float re[4], im[4];
+            hv4 rh, rl, ih, il;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                re[i] = r[st][i].x;
+                im[i] = r[st][i].y;
+            }
+            split4(re, &rh, &rl);
+            split4(im, &ih, &il);
+            const u32x4 h = half_swap(rh, ih), l = half_swap(rl, il);             // (Re, Im)
+            fh[st][0] = h ^ sgn;
+            fl[st][0] = l ^ sgn;
+            if (kFirst) {
+                fh[st][NA - 1] = half_swap(ih, rh);                               // (Im, Re)
+                fl[st][NA - 1] = half_swap(il, rl);
+            } else if (!kReal) {
+                fh[st][NA - 1] = h;
+                fl[st][NA - 1] = l;
+            }
+        }
+        if (c + 1 < nChunks) {                         // in flight during the MFMAs
+            dma(c + 1, nxt);
+#pragma unroll
+            for (int st = 0; st < kStripCS; st++) {
+                const int s = kStripCS * (c + 1) + st;
+                fetch(s < nSteps ? s : nSteps - 1, r[st]);
             }
         }
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int kb = k0 + bK + i;
-            rb[i] = (bIn && kb <= kLast) ? B[kb * bSk + bOff] : f2v{0.f, 0.f};
-        }
+        for (int st = 0; st < kStripCS; st++) {
+            if (!active || kStripCS * c + st >= nSteps) break;                    // uniform
+            const u32x4* p = cur + st * MT * 128;
+            auto mm = [](const u32x4& x, const u32x4& y, const f32x16& d) {
+                return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(hv8, x), __builtin_bit_cast(hv8, y), d, 0,
+                                                              0, 0);
+            };
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int kb = k0 + bK2 + i;
-            rb2[i] = (bIn2 && kb <= kLast) ? B[kb * bSk + bOff2] : f2v{0.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = ra[i].x;
-            im[i] = ra[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[0][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[1][aRow][aK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[2][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[3][aRow][aK]) = lo;
-        *reinterpret_cast<hv4*>(&st->a[4][aRow][aK]) = neg4(hi);   // split(-x) = -split(x)
-        *reinterpret_cast<hv4*>(&st->a[5][aRow][aK]) = neg4(lo);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = rb[4 * h + i].x;
-                im[i] = rb[4 * h + i].y;
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[0][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[1][bCol][bK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[2][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[3][bCol][bK + 4 * h]) = lo;
-        }
-        float re2[2] = {rb2[0].x, rb2[1].x}, im2[2] = {rb2[0].y, rb2[1].y};
-        hv2 hi2, lo2;
-        split2(re2, &hi2, &lo2);
-        *reinterpret_cast<hv2*>(&st->b[0][bCol2][bK2]) = hi2;
-        *reinterpret_cast<hv2*>(&st->b[1][bCol2][bK2]) = lo2;
-        split2(im2, &hi2, &lo2);
-        *reinterpret_cast<hv2*>(&st->b[2][bCol2][bK2]) = hi2;
-        *reinterpret_cast<hv2*>(&st->b[3][bCol2][bK2]) = lo2;
-    };
-    const int isIm = l32 >> 4;
-    const int aPlane = isIm ? (half ? 0 : 2) : (half ? 4 : 0);
-    const int aRowL = wave * 16 + (l32 & 15);
-    const int bPlane = half ? 2 : 0;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + wave * 16 < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-                const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-#pragma unroll
-                for (int c = 0; c < NC; c++) {
-                    if (n0 + 32 * c >= g.N) break;                                 // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][32 * c + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][32 * c + l32][kk]);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[c], 0, 0, 0);
+            for (int t = 0; t < MT; t++) {
+                u32x4 th[NA], tl[NA];
+                th[0] = p[(2 * t) * 64 + lane];
+                tl[0] = p[(2 * t + 1) * 64 + lane];
+                if (!kReal && !kFirst) {
+                    th[NA - 1] = p[(2 * t) * 64 + (lane ^ 32)];
+                    tl[NA - 1] = p[(2 * t + 1) * 64 + (lane ^ 32)];
+                } else {
+                    th[NA - 1] = th[0];
+                    tl[NA - 1] = tl[0];
                 }
+                // A hi B hi, A hi B lo, A lo B hi
+#pragma unroll
+                for (int a = 0; a < NA; a++)
+                    acc[t][a] = kFirst ? mm(fh[st][a], th[a], acc[t][a]) : mm(th[a], fh[st][a], acc[t][a]);
+#pragma unroll
+                for (int a = 0; a < NA; a++)
+                    acc[t][a] = kFirst ? mm(fh[st][a], tl[a], acc[t][a]) : mm(th[a], fl[st][a], acc[t][a]);
+#pragma unroll
+                for (int a = 0; a < NA; a++)
+                    acc[t][a] = kFirst ? mm(fl[st][a], th[a], acc[t][a]) : mm(tl[a], fh[st][a], acc[t][a]);
             }
         }
+        // this wave's direct loads are complete (vmcnt(0)) before the barrier
+        // publishes them
+        __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
+    };
+    dma(0, ldsA);
+#pragma unroll
+    for (int st = 0; st < kStripCS; st++) fetch(st < nSteps ? st : nSteps - 1, r[st]);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    for (int c = 0; c < nChunks; c += 2) {
+        chunk(c, ldsA, ldsB);
+        if (c + 1 < nChunks) chunk(c + 1, ldsB, ldsA);
     }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
+    if (!active) return;
+    // D layout of a 32x32 tile: lane column l32 (B operand), rows 8*(i/4) +
+    // 4*half + i%4 (A operand)
     const float os = g.outScale;
-    const int64_t dCol0 = col_d(g, n0);
-    const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)m0 * g.dSm + dCol0;
-    const int dSm = (int)g.dSm;
-    gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + dBase);
-    int oc[NC];
+    if constexpr (kFirst) {
+        // lane: table entry 32 (t0 + t) + l32; rows: lines
+        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)batch * g.dStrideB + (int64_t)n0 * g.dSn);
+        const int dSn = (int)g.dSn;
 #pragma unroll
-    for (int c = 0; c < NC; c++) oc[c] = n0 + 32 * c + l32 < g.N ? (int)(col_d(g, n0 + 32 * c + l32) - dCol0) : 0;
+        for (int t = 0; t < MT; t++) {
+            const int m = 32 * (t0 + t) + l32;
+            if (m >= g.M) continue;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int r = wave * 16 + 8 * (i >> 2) + 4 * half + (i & 3);   // Re row r, Im row r + 16
-        if (m0 + r >= g.M) continue;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            if (n0 + 32 * c + l32 >= g.N) continue;
-            D[r * dSm + oc[c]] = f2v{acc[c][i] * os, acc[c][i + 8] * os};
-        }
-    }
-}
-
-// 64x128 tiles of the real part (the last contraction, whose column axis is
-// the long (x2, x1) plane): wave w owns rows 32 (w / 2).. and the two 32-column
-// tiles from 64 (w % 2), reading each A fragment once for both (6 fragment
-// reads per 6 MFMAs instead of 4 per 3); half as many blocks, each with twice
-// the MFMAs per 16-k chunk.  Staging, operand split and epilogue as gemm_tile_h.
-__device__ __forceinline__ void gemm_tile_r128(const rf_gemm_desc& g, int m0, int n0, int batch, HStage<3>* st) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)((batch / g.aDiv) % g.aMod) * g.aStrideB + (int64_t)m0 * g.aSm);
-    const int64_t bCol0 = col_b(g, n0);
-    const gf2* B = (const gf2*)(g.B + (int64_t)batch * g.bStrideB + bCol0);
-    const int aSm = (int)g.aSm, aSk = (int)g.aSk, bSk = (int)g.bSk;
-    f32x16 acc[2];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        acc[0][i] = 0.0f;
-        acc[1][i] = 0.0f;
-    }
-    const int rt = wave >> 1, ct = wave & 1;
-    // staging: A row t/4, k 4(t%4)..+3; B column t%128, k 8(t/128)..+7
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 127, bK = (tid >> 7) * 8;
-    const bool aIn = m0 + aRow < g.M, bIn = n0 + bCol < g.N;
-    const int aOff = aRow * aSm, bOff = bIn ? (int)(col_b(g, n0 + bCol) - bCol0) : 0;
-    const int kLast = g.K - 1;
-    f2v ra[4], rb[8];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int ka = k0 + aK + i;
-            ra[i] = (aIn && ka <= kLast) ? A[aOff + ka * aSk] : f2v{0.f, 0.f};
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int kb = k0 + bK + i;
-            rb[i] = (bIn && kb <= kLast) ? B[kb * bSk + bOff] : f2v{0.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = ra[i].x;
-            im[i] = ra[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[0][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[1][aRow][aK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[2][aRow][aK]) = neg4(hi);   // split(-x) = -split(x)
-        *reinterpret_cast<hv4*>(&st->a[3][aRow][aK]) = neg4(lo);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = rb[4 * h + i].x;
-                im[i] = rb[4 * h + i].y;
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[0][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[1][bCol][bK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[2][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[3][bCol][bK + 4 * h]) = lo;
-        }
-    };
-    // K' half 0 pairs Re A with Re B, half 1 -Im A with Im B
-    const int aPlane = half ? 2 : 0, bPlane = half ? 2 : 0;
-    const int aRowL = rt * 32 + l32;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + rt * 32 < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-                const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const int col = 64 * ct + 32 * c;
-                    if (n0 + col >= g.N) break;                                    // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][col + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][col + l32][kk]);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[c], 0, 0, 0);
-                }
+            for (int i = 0; i < 16; i++) {
+                const int line = 8 * (i >> 2) + 4 * half + (i & 3);
+                if (n0 + line < g.N) D[line * dSn + m] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
             }
         }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dCol0 = col_d(g, n0);
-    const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)m0 * g.dSm + dCol0;
-    const int dSm = (int)g.dSm;
-    auto dcol = [&](int nn) { return n0 + nn < g.N ? (int)(col_d(g, n0 + nn) - dCol0) : 0; };
-    const int oc[2] = {dcol(64 * ct + l32), dcol(64 * ct + 32 + l32)};
-    const bool nIn[2] = {n0 + 64 * ct + l32 < g.N, n0 + 64 * ct + 32 + l32 < g.N};
-    // fused blend: the lane's column offsets in the group grid, or -1, and
-    // in a first-axis band array, or -1
-    int64_t gc[2], bo[2];
-    int bside[2], bst[2];
+    } else if constexpr (!kReal) {
+        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)batch * g.dStrideB + col_d(g, n0) +
+                          (int64_t)(32 * t0) * g.dSm);
+        const int dSm = (int)g.dSm, oc = (int)(col_d(g, nc) - col_d(g, n0));
+        if (!nIn) return;
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-        const int nn = n0 + 64 * ct + 32 * c + l32;
-        gc[c] = (g.grp && nIn[c]) ? grp_col(g, nn) : -1;
-        bside[c] = 0;
-        bst[c] = 0;
-        bo[c] = (g.grp && nIn[c] && gc[c] < 0) ? band_col(g, nn, batch, &bside[c], &bst[c]) : -1;
-    }
-    auto store = [&](auto map, auto* D, auto* G, auto* BL, auto* BH) {
+        for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = rt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-            if (m0 + r >= g.M) continue;
-            const int64_t gr = (gc[0] >= 0 || gc[1] >= 0) ? grp_row(g, m0 + r) : -1;
-#pragma unroll
-            for (int c = 0; c < 2; c++) {
-                if (!nIn[c]) continue;
-                const auto v = map(acc[c][i] * os);
-                if (gr >= 0 && gc[c] >= 0) G[gr + gc[c]] = v;
-                else if (bo[c] >= 0) (bside[c] ? BH : BL)[bo[c] + (int64_t)(m0 + r) * bst[c]] = v;
-                else D[r * dSm + oc[c]] = v;
+            for (int i = 0; i < 16; i++) {
+                const int m = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
+                if (32 * t0 + m < g.M) D[m * dSm + oc] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
             }
-        }
-    };
-    const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
-    gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
-    gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
-    gfo* G32 = (gfo*)(static_cast<float*>(g.grp) + (int64_t)batch * g.grpStrideB);
-    gdo* G64 = (gdo*)(static_cast<double*>(g.grp) + (int64_t)batch * g.grpStrideB);
-    gfo* L32 = (gfo*)static_cast<float*>(g.bandLo);
-    gfo* H32 = (gfo*)static_cast<float*>(g.bandHi);
-    gdo* L64 = (gdo*)static_cast<double*>(g.bandLo);
-    gdo* H64 = (gdo*)static_cast<double*>(g.bandHi);
-    if (g.outDtype == RF_DTYPE_F64) {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64, G64, L64, H64);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL)
-            store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64, G64, L64, H64);
-        else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64, G64, L64, H64);
     } else {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32, G32, L32, H32);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL)
-            store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32, G32, L32, H32);
-        else store([=](float u) { return fmaf(u, sc, sh); }, D32, G32, L32, H32);
+        if (!nIn) return;
+        const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)(32 * t0) * g.dSm + (int64_t)n0 * g.dSn;
+        const int dSm = (int)g.dSm;
+        // fused blend: this lane's column offset in the group grid, or -1,
+        // and in a first-axis band array, or -1
+        const int64_t gc = g.grp ? grp_col(g, n) : -1;
+        int bside = 0, bst = 0;
+        const int64_t bo = (g.grp && gc < 0) ? band_col(g, n, batch, &bside, &bst) : -1;
+        auto store = [&](auto map, auto* D, auto* G, auto* BL, auto* BH) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int m = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3), M = 32 * t0 + m;
+                    if (M < g.M) {
+                        const auto v = map(acc[t][0][i] * os);
+                        const int64_t go = gc >= 0 ? grp_row(g, M) : -1;
+                        if (go >= 0) G[go + gc] = v;
+                        else if (bo >= 0) (bside ? BH : BL)[bo + (int64_t)M * bst] = v;
+                        else D[m * dSm + l32] = v;
+                    }
+                }
+        };
+        const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
+        gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
+        gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
+        gfo* G32 = (gfo*)(static_cast<float*>(g.grp) + (int64_t)batch * g.grpStrideB);
+        gdo* G64 = (gdo*)(static_cast<double*>(g.grp) + (int64_t)batch * g.grpStrideB);
+        gfo* L32 = (gfo*)static_cast<float*>(g.bandLo);
+        gfo* H32 = (gfo*)static_cast<float*>(g.bandHi);
+        gdo* L64 = (gdo*)static_cast<double*>(g.bandLo);
+        gdo* H64 = (gdo*)static_cast<double*>(g.bandHi);
+        if (g.outDtype == RF_DTYPE_F64) {
+            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64, G64, L64, H64);
+            else if (g.epi.margi == RF_FOM_LOGNORMAL)
+                store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64, G64, L64, H64);
+            else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64, G64, L64, H64);
+        } else {
+            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32, G32, L32, H32);
+            else if (g.epi.margi == RF_FOM_LOGNORMAL)
+                store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32, G32, L32, H32);
+            else store([=](float u) { return fmaf(u, sc, sh); }, D32, G32, L32, H32);
+        }
     }
 }
-
 // Isotropic sum on a structured grid, per-realization directions.  With
 // x = o + i step per axis, e^{i(k.x + phi)} factorises over the axes, so per
 // realization r
@@ -942,7 +593,7 @@ __device__ __forceinline__ void gemm_tile_r128(const rf_gemm_desc& g, int m0, in
 // a thread's k run of a chunk is one 16-byte-aligned piece of a row, read
 // by 16-byte loads from one address, with no masks; rows and columns past a
 // tile's edge read the last row / column (finite values in accumulators
-// that are never stored).  A 64x128 tile of the real part as gemm_tile_r128.
+// that are never stored).  Tiles of 64x128.
 struct rf_iso_gemm {
     const float2* A;              // last-axis table [r][k][m]
     const float2* W;              // first-axis table with the coefficients [r][k][i]
@@ -954,7 +605,7 @@ struct rf_iso_gemm {
     rf_epilogue epi;
     float outScale;
 };
-__device__ __forceinline__ void gemm_tile_iso(const rf_iso_gemm& g, int m0, int n0, int batch, HStage<3>* st) {
+__device__ __forceinline__ void gemm_tile_iso(const rf_iso_gemm& g, int m0, int n0, int batch, HStage* st) {
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const gf2* A = (const gf2*)(g.A + (int64_t)batch * g.aStrideB + (int64_t)m0 * g.K);
@@ -1211,260 +862,94 @@ __device__ __forceinline__ void gemm_tile_iso128(const rf_iso_gemm& g, int m0, i
     }
 }
 
-// 64x128 tiles of the complex product (the middle contraction, whose
-// columns (j3, x1) are long): wave w owns complex rows 16 w.. and four
-// 32-column tiles, reading each A fragment once for all four (10 fragment
-// reads per 12 MFMAs instead of 6 per 6).  Staging, operand split and
-// epilogue as gemm_tile_h.
-__device__ __forceinline__ void gemm_tile_cw(const rf_gemm_desc& g, int m0, int n0, int batch, HStage<4>* st) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)((batch / g.aDiv) % g.aMod) * g.aStrideB + (int64_t)m0 * g.aSm);
-    const int64_t bCol0 = col_b(g, n0);
-    const gf2* B = (const gf2*)(g.B + (int64_t)batch * g.bStrideB + bCol0);
-    const int aSm = (int)g.aSm, aSk = (int)g.aSk, bSk = (int)g.bSk;
-    f32x16 acc[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) acc[c][i] = 0.0f;
-    // staging: A row t/4, k 4(t%4)..+3; B column t%128, k 8(t/128)..+7
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 127, bK = (tid >> 7) * 8;
-    const bool aIn = m0 + aRow < g.M, bIn = n0 + bCol < g.N;
-    const int aOff = aRow * aSm, bOff = bIn ? (int)(col_b(g, n0 + bCol) - bCol0) : 0;
-    const int kLast = g.K - 1;
-    f2v ra[4], rb[8];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int ka = k0 + aK + i;
-            ra[i] = (aIn && ka <= kLast) ? A[aOff + ka * aSk] : f2v{0.f, 0.f};
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int kb = k0 + bK + i;
-            rb[i] = (bIn && kb <= kLast) ? B[kb * bSk + bOff] : f2v{0.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = ra[i].x;
-            im[i] = ra[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[0][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[1][aRow][aK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[2][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[3][aRow][aK]) = lo;
-        *reinterpret_cast<hv4*>(&st->a[4][aRow][aK]) = neg4(hi);   // split(-x) = -split(x)
-        *reinterpret_cast<hv4*>(&st->a[5][aRow][aK]) = neg4(lo);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = rb[4 * h + i].x;
-                im[i] = rb[4 * h + i].y;
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[0][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[1][bCol][bK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[2][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[3][bCol][bK + 4 * h]) = lo;
-        }
-    };
-    // operand planes as in gemm_tile_h's complex product
-    const int isIm = l32 >> 4;
-    const int aPlane = isIm ? (half ? 0 : 2) : (half ? 4 : 0);
-    const int aRowL = wave * 16 + (l32 & 15);
-    const int bPlane = half ? 2 : 0;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + wave * 16 < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-                const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    if (n0 + 32 * c >= g.N) break;                                 // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][32 * c + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][32 * c + l32][kk]);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[c], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dCol0 = col_d(g, n0);
-    const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)m0 * g.dSm + dCol0;
-    const int dSm = (int)g.dSm;
-    auto dcol = [&](int nn) { return n0 + nn < g.N ? (int)(col_d(g, n0 + nn) - dCol0) : 0; };
-    gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + dBase);
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int nn = 32 * c + l32;
-        if (n0 + nn >= g.N) continue;
-        const int oc = dcol(nn);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int r = wave * 16 + 8 * (i >> 2) + 4 * half + (i & 3);   // Re row r, Im row r + 16
-            if (m0 + r < g.M) D[r * dSm + oc] = f2v{acc[c][i] * os, acc[c][i + 8] * os};
-        }
-    }
-}
-
 struct FStage {
     float2 a[kTK][kTM + 1];
     float2 b[kTK][kTN + 1];
 };
-template <int RW>
-constexpr size_t kStageBytes = sizeof(HStage<RW>) > sizeof(FStage) ? sizeof(HStage<RW>) : sizeof(FStage);
 
-// Tile kind RW (rf_gemm_desc::rw) > 1 only with FP16 operands: the host sets
-// rw = 1 wherever it falls back to the FP32-operand tile.
-template <bool RealOnly, int RW = 1>
-__device__ __forceinline__ void run_tile(const rf_gemm_desc& g, int m0, int n0, int batch, char* smem) {
-    if constexpr (RW == 2) {
-        static_assert(!RealOnly, "kind 2 is the complex product");
-        gemm_tile_c128(g, m0, n0, batch, reinterpret_cast<HStage<2>*>(smem));
-    } else if constexpr (RW == 3) {
-        static_assert(RealOnly, "kind 3 is the real part");
-        gemm_tile_r128(g, m0, n0, batch, reinterpret_cast<HStage<3>*>(smem));
-    } else if constexpr (RW == 4) {
-        static_assert(!RealOnly, "kind 4 is the complex product");
-        gemm_tile_cw(g, m0, n0, batch, reinterpret_cast<HStage<4>*>(smem));
-    } else if constexpr (RW == 5) {
-        static_assert(!RealOnly, "kind 5 is the complex product");
-        gemm_tile_c160(g, m0, n0, batch, reinterpret_cast<HStage<5>*>(smem));
-    } else if (g.split16) {
-        gemm_tile_h<RealOnly>(g, m0, n0, batch, reinterpret_cast<HStage<1>*>(smem));
-    } else {
-        FStage* f = reinterpret_cast<FStage*>(smem);
-        gemm_tile<RealOnly>(g, m0, n0, batch, f->a, f->b);
-    }
-}
-
-// Tile order and placement.  A GEMM's tiles are numbered so that the tiles
-// sharing the larger operand are consecutive: row tiles fastest when there
-// are no more of them than column tiles (they share a column slab of B, the
-// previous stage's output), column tiles fastest otherwise (they share a row
-// slab of A, the coefficients).  Workgroups go round-robin to the 8 XCDs, each
-// with its own L2; block b runs logical tile (b % 8) * P + b / 8, so every XCD
-// walks a contiguous range of P tiles and a shared slab is re-read from its
-// L2, not from HBM.
+// Placement.  Workgroups go round-robin to the 8 XCDs, each with its own L2;
+// block b runs logical tile (b % 8) * P + b / 8, so every XCD walks a contiguous
+// range of P tiles and what neighbours share (streamed lines between table
+// groups, amplitudes, cache lines at strip edges) is re-read from its L2.
 constexpr int kXcd = 8;
-
-__device__ inline void tile_coords(const rf_gemm_desc& g, int64_t local, int* mI, int* nI, int* batch) {
-    const int tm = tile_m(g), tn = tile_n(g);
-    const int ntN = (g.N + tn - 1) / tn, ntM = (g.M + tm - 1) / tm;
-    if (ntM <= ntN) {
-        *mI = (int)(local % ntM);
-        const int64_t r = local / ntM;
-        *nI = (int)(r % ntN);
-        *batch = (int)(r / ntN);
-    } else {
-        *nI = (int)(local % ntN);
-        const int64_t r = local / ntN;
-        *mI = (int)(r % ntM);
-        *batch = (int)(r / ntM);
-    }
-}
 
 __device__ inline int64_t xcd_tile(int64_t b, int64_t nTiles) {
     const int64_t per = (nTiles + kXcd - 1) / kXcd;
     return (b % kXcd) * per + b / kXcd;
 }
 
-template <bool RealOnly, int RW>
-__device__ __forceinline__ void cgemm_body(const rf_gemm_desc& g, int64_t nTiles, char* smem) {
-    const int64_t L = xcd_tile(blockIdx.x, nTiles);
-    if (L >= nTiles) return;
-    int mI, nI, batch;
-    tile_coords(g, L, &mI, &nI, &batch);
-    run_tile<RealOnly, RW>(g, mI * tile_m(g), nI * tile_n(g), batch, smem);
+// An FP32-operand tile: row tiles fastest (they share a column slab of B).
+template <bool RealOnly>
+__device__ __forceinline__ void run_tile(const rf_gemm_desc& g, int64_t local, char* smem) {
+    const int ntN = (g.N + kTN - 1) / kTN, ntM = (g.M + kTM - 1) / kTM;
+    const int mI = (int)(local % ntM);
+    const int64_t r = local / ntM;
+    FStage* f = reinterpret_cast<FStage*>(smem);
+    gemm_tile<RealOnly>(g, mI * kTM, (int)(r % ntN) * kTN, (int)(r / ntN), f->a, f->b);
 }
 
-template <bool RealOnly, int RW>
-__global__ __launch_bounds__(256) void k_cgemm(rf_gemm_desc g, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<RW>];
-    cgemm_body<RealOnly, RW>(g, nTiles, smem);
+// Registers: 16 MT accumulators per lane (32 MT complex) decide the waves per
+// SIMD; the compiler then keeps them in VGPRs without spills.
+constexpr int strip_waves(int MT, int KIND) {
+    return KIND == RF_GEMM_LAST ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4);
+}
+
+template <int MT, int KIND>
+__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, KIND))))
+void k_strip(rf_gemm_desc g, int64_t nTiles) {
+    __shared__ u32x4 ldsA[strip_units(MT)];
+    __shared__ u32x4 ldsB[strip_units(MT)];
+    const int64_t L = xcd_tile(blockIdx.x, nTiles);
+    if (L >= nTiles) return;
+    strip_tile<MT, KIND>(g, L, ldsA, ldsB);
 }
 
 // Grouped form: the GEMMs of several fields in one launch; GEMM q owns
 // logical tiles tile0 .. tile0 + tiles(q) - 1.
-// RWMAX > 1: the GEMMs of the group with rw = RWMAX use that tile kind
-template <bool RealOnly, int RWMAX>
-__device__ __forceinline__ void cgemm_group_body(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles,
-                                                 char* smem) {
-    const int64_t b = xcd_tile(blockIdx.x, nTiles);
-    if (b >= nTiles) return;
+__device__ inline int gemm_find(const rf_gemm_desc* __restrict__ gs, int nG, int64_t b) {
     int lo = 0, hi = nG - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (gs[mid].tile0 <= b) lo = mid;
         else hi = mid - 1;
     }
-    const rf_gemm_desc g = gs[lo];                 // uniform: scalar registers
-    int mI, nI, batch;
-    tile_coords(g, b - g.tile0, &mI, &nI, &batch);
-    if (RWMAX > 1 && g.rw == RWMAX) run_tile<RealOnly, RWMAX>(g, mI * tile_m(g), nI * tile_n(g), batch, smem);
-    else run_tile<RealOnly, 1>(g, mI * kTM, nI * kTN, batch, smem);
+    return lo;
 }
 
-template <bool RealOnly, int RWMAX>
+template <int MT, int KIND>
+__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, KIND))))
+void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
+    __shared__ u32x4 ldsA[strip_units(MT)];
+    __shared__ u32x4 ldsB[strip_units(MT)];
+    const int64_t L = xcd_tile(blockIdx.x, nTiles);
+    if (L >= nTiles) return;
+    const rf_gemm_desc g = gs[gemm_find(gs, nG, L)];   // uniform: scalar registers
+    strip_tile<MT, KIND>(g, L - g.tile0, ldsA, ldsB);
+}
+
+// The FP32-operand tile (a first contraction whose K would leave the FP16
+// range).
+template <bool RealOnly>
+__global__ __launch_bounds__(256) void k_cgemm(rf_gemm_desc g, int64_t nTiles) {
+    __shared__ __attribute__((aligned(16))) char smem[sizeof(FStage)];
+    const int64_t L = xcd_tile(blockIdx.x, nTiles);
+    if (L >= nTiles) return;
+    run_tile<RealOnly>(g, L, smem);
+}
+template <bool RealOnly>
 __global__ __launch_bounds__(256) void k_cgemm_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<RWMAX>];
-    cgemm_group_body<RealOnly, RWMAX>(gs, nG, nTiles, smem);
-}
-
-// Kind 5 holds 80 accumulators per lane: asked for three waves per SIMD (its
-// LDS allows three blocks per CU) the compiler keeps them in the VGPRs
-// (160 registers, no spill) instead of 94 VGPRs + 80 AGPRs, which would
-// allow two.  The other kinds keep their own allocation.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_cgemm_c160(rf_gemm_desc g,
-                                                                                         int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<5>];
-    cgemm_body<false, 5>(g, nTiles, smem);
-}
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_cgemm_group_c160(
-    const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<5>];
-    cgemm_group_body<false, 5>(gs, nG, nTiles, smem);
-}
-
-// Kind 3 asked for four waves per SIMD (its LDS allows four blocks per CU):
-// the 32 accumulators live in the VGPRs (114 registers, no spill) instead of
-// 86 VGPRs + 32 AGPRs; the localization step's last contraction ran ~1 %
-// faster so.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_cgemm_r128(rf_gemm_desc g,
-                                                                                         int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<3>];
-    cgemm_body<true, 3>(g, nTiles, smem);
-}
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_cgemm_group_r128(
-    const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes<3>];
-    cgemm_group_body<true, 3>(gs, nG, nTiles, smem);
+    __shared__ __attribute__((aligned(16))) char smem[sizeof(FStage)];
+    const int64_t L = xcd_tile(blockIdx.x, nTiles);
+    if (L >= nTiles) return;
+    const rf_gemm_desc g = gs[gemm_find(gs, nG, L)];
+    run_tile<RealOnly>(g, L - g.tile0, smem);
 }
 
 // One 64x128 tile of one realization's isotropic grid GEMM per block; tiles
 // numbered row tiles fastest (they share a column slab of B), placed per XCD.
 template <int TM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_iso_gemm(rf_iso_gemm g, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[TM == 128 ? sizeof(IsoStage128) : sizeof(HStage<3>)];
+    __shared__ __attribute__((aligned(16))) char smem[TM == 128 ? sizeof(IsoStage128) : sizeof(HStage)];
     const int64_t L = xcd_tile(blockIdx.x, nTiles);
     if (L >= nTiles) return;
     const int ntM = (g.M + TM - 1) / TM, ntN = (g.N + 2 * kTN - 1) / (2 * kTN);
@@ -1475,7 +960,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     if constexpr (TM == 128)
         gemm_tile_iso128(g, mI * TM, nI * 2 * kTN, batch, reinterpret_cast<IsoStage128*>(smem));
     else
-        gemm_tile_iso(g, mI * TM, nI * 2 * kTN, batch, reinterpret_cast<HStage<3>*>(smem));
+        gemm_tile_iso(g, mI * TM, nI * 2 * kTN, batch, reinterpret_cast<HStage*>(smem));
 }
 
 // Isotropic phase tables [r][index][k] for the axes of the grid, in FP64
@@ -1524,22 +1009,51 @@ __global__ void k_iso_tables(int nDim, int64_t kN, int64_t kP, int Nmc, int n0, 
 //   Method 4: E[v][j][i] = (w_j cos(pi j (2i+1) / (2n)), 0), w_0 = 1, w_j = 2: the
 //     REDFT01 (DCT-III) of FFTW that gen_Std_Gauss_FFT applies along each axis
 //     (randomFieldND.f90:694-735), as a matrix; both variants equal.
+//   frag: in the strip GEMM's fragment order instead, split into FP16 hi + lo:
+//     K entry k is entry k % nk of variant k / nk, [step k / 8][tile x / 32][hi,
+//     lo][re, im][x % 32][k % 8], zero past K and past nx.
 struct rf_table_args {
-    int dct, nAx;
-    int nk[3], nx[3];
+    int dct, nAx, frag;
+    int nk[3], nx[3], K[3];
     unsigned block0[3];
     double dk[3], o[3], step[3], invL[3];
-    float2* E[3];
+    void* E[3];
 };
 __global__ __launch_bounds__(256) void k_axis_tables(rf_table_args t) {
     int a = 0;
     while (a + 1 < t.nAx && blockIdx.x >= t.block0[a + 1]) a++;
     const int64_t e = (int64_t)(blockIdx.x - t.block0[a]) * 256 + threadIdx.x;
     const int nx = t.nx[a];
+    if (t.frag) {
+        const int nT = (nx + 31) / 32;
+        const int64_t st = e >> 8;                       // step * nT + tile
+        const int64_t s = st / nT;
+        if (s >= (t.K[a] + 7) / 8) return;
+        const int row = (int)(e >> 3) & 31, q = (int)e & 7;
+        const int k = (int)(8 * s) + q, i = (int)(st - s * nT) * 32 + row;
+        const int v = k / t.nk[a], j = k - v * t.nk[a];
+        double c = 0.0, sn = 0.0;
+        if (k < t.K[a] && i < nx) {
+            if (t.dct) {
+                c = (j == 0 ? 1.0 : 2.0) * cos(3.14159265358979323846 * (double)j * (2.0 * i + 1.0) / (2.0 * nx));
+            } else {
+                sincos((t.dk[a] * (double)j) * ((t.o[a] + t.step[a] * (double)i) * t.invL[a]), &sn, &c);
+                if (v) sn = -sn;
+            }
+        }
+        const float cf = (float)c, sf = (float)sn;
+        const _Float16 ch = (_Float16)cf, sh = (_Float16)sf;
+        _Float16* F = static_cast<_Float16*>(t.E[a]) + st * 1024 + row * 8 + q;
+        F[0] = ch;
+        F[256] = sh;
+        F[512] = (_Float16)(cf - (float)ch);
+        F[768] = (_Float16)(sf - (float)sh);
+        return;
+    }
     const int64_t cnt = (int64_t)t.nk[a] * nx;
     if (e >= cnt) return;
     const int j = (int)(e / nx), i = (int)(e % nx);
-    float2* E = t.E[a];
+    float2* E = static_cast<float2*>(t.E[a]);
     if (t.dct) {
         const double w = j == 0 ? 1.0 : 2.0;
         const double c = w * cos(3.14159265358979323846 * (double)j * (2.0 * i + 1.0) / (2.0 * nx));
@@ -1686,56 +1200,86 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-int64_t rf_gemm_tiles(const rf_gemm_desc& g) {
-    const int tm = tile_m(g), tn = tile_n(g);
-    return (int64_t)((g.N + tn - 1) / tn) * ((g.M + tm - 1) / tm) * g.batches;
+int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt) {
+    if (mt > 0) return (int64_t)strip_groups(g, mt) * (((int64_t)g.N + kStripL - 1) / kStripL) * g.batches;
+    return (int64_t)((g.N + kTN - 1) / kTN) * ((g.M + kTM - 1) / kTM) * g.batches;
 }
 
 // blocks of a launch over nTiles logical tiles (a multiple of the XCD count)
 inline int64_t xcd_blocks(int64_t nTiles) { return (nTiles + kXcd - 1) / kXcd * kXcd; }
 
-hipError_t rf_launch_gemm(const rf_gemm_desc& g, hipStream_t s) {
-    const int64_t nTiles = rf_gemm_tiles(g);
+namespace {
+template <int MT, int KIND>
+void strip_launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, unsigned blocks, hipStream_t s) {
+    const dim3 b(64 * kStripW);
+    if (g) hipLaunchKernelGGL((k_strip<MT, KIND>), dim3(blocks), b, 0, s, *g, nTiles);
+    else hipLaunchKernelGGL((k_strip_group<MT, KIND>), dim3(blocks), b, 0, s, d_gs, nG, nTiles);
+}
+template <int KIND>
+void strip_launch_mt(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, unsigned blocks,
+                     hipStream_t s) {
+    switch (mt) {
+        case 1: return strip_launch<1, KIND>(g, d_gs, nG, nTiles, blocks, s);
+        case 2: return strip_launch<2, KIND>(g, d_gs, nG, nTiles, blocks, s);
+        case 3: return strip_launch<3, KIND>(g, d_gs, nG, nTiles, blocks, s);
+        case 4: return strip_launch<4, KIND>(g, d_gs, nG, nTiles, blocks, s);
+        default: return strip_launch<kStripMaxMT, KIND>(g, d_gs, nG, nTiles, blocks, s);
+    }
+}
+// One GEMM (g) or a group of them (d_gs, nG), all of one kind, on strips of
+// mt tiles or, mt 0, FP32-operand tiles.
+hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles,
+                      hipStream_t s) {
     if (nTiles <= 0) return hipSuccess;
-    const int64_t blocks = xcd_blocks(nTiles);
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (g.realOut && g.rw == 3) hipLaunchKernelGGL(k_cgemm_r128, dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else if (g.realOut) hipLaunchKernelGGL((k_cgemm<true, 1>), dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else if (g.rw == 2) hipLaunchKernelGGL((k_cgemm<false, 2>), dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else if (g.rw == 4) hipLaunchKernelGGL((k_cgemm<false, 4>), dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else if (g.rw == 5) hipLaunchKernelGGL(k_cgemm_c160, dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else hipLaunchKernelGGL((k_cgemm<false, 1>), dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
+    const int64_t nb = xcd_blocks(nTiles);
+    if (nb > 0x7fffffffLL || mt < 0 || mt > kStripMaxMT) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)nb;
+    if (mt > 0) {
+        if (kind == RF_GEMM_FIRST) strip_launch_mt<RF_GEMM_FIRST>(mt, g, d_gs, nG, nTiles, blocks, s);
+        else if (kind == RF_GEMM_MIDDLE) strip_launch_mt<RF_GEMM_MIDDLE>(mt, g, d_gs, nG, nTiles, blocks, s);
+        else strip_launch_mt<RF_GEMM_LAST>(mt, g, d_gs, nG, nTiles, blocks, s);
+    } else if (kind == RF_GEMM_LAST) {
+        if (g) hipLaunchKernelGGL(k_cgemm<true>, dim3(blocks), dim3(256), 0, s, *g, nTiles);
+        else hipLaunchKernelGGL(k_cgemm_group<true>, dim3(blocks), dim3(256), 0, s, d_gs, nG, nTiles);
+    } else {
+        if (g) hipLaunchKernelGGL(k_cgemm<false>, dim3(blocks), dim3(256), 0, s, *g, nTiles);
+        else hipLaunchKernelGGL(k_cgemm_group<false>, dim3(blocks), dim3(256), 0, s, d_gs, nG, nTiles);
+    }
     return hipGetLastError();
 }
 
-hipError_t rf_launch_gemm_group(int realOut, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, int rwMax,
-                                hipStream_t s) {
-    if (nG <= 0 || nTiles <= 0) return hipSuccess;
-    const int64_t blocks = xcd_blocks(nTiles);
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (realOut && rwMax == 3)
-        hipLaunchKernelGGL(k_cgemm_group_r128, dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    else if (realOut)
-        hipLaunchKernelGGL((k_cgemm_group<true, 1>), dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    else if (rwMax == 2)
-        hipLaunchKernelGGL((k_cgemm_group<false, 2>), dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    else if (rwMax == 4)
-        hipLaunchKernelGGL((k_cgemm_group<false, 4>), dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    else if (rwMax == 5)
-        hipLaunchKernelGGL(k_cgemm_group_c160, dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    else
-        hipLaunchKernelGGL((k_cgemm_group<false, 1>), dim3((unsigned)blocks), dim3(256), 0, s, d_gs, nG, nTiles);
-    return hipGetLastError();
+// MT of a strip GEMM: all of the table axis in one wave (up to kStripMaxMT
+// tiles) so that every streamed value is read and converted once, unless the
+// launch would then leave SIMDs without a wave.
+int strip_choose(const rf_gemm_desc& g) {
+    const int mt = (g.M + 31) / 32;
+    const int64_t strips = (((int64_t)g.N + 31) / 32) * g.batches;
+    int gr = (mt + kStripMaxMT - 1) / kStripMaxMT;
+    while (gr < mt && strips * gr < kStripFill) gr++;
+    return (mt + gr - 1) / gr;
+}
+}  // namespace
+
+hipError_t rf_launch_gemm_group(int kind, int mt, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, hipStream_t s) {
+    if (nG <= 0) return hipSuccess;
+    return launch_any(kind, mt, nullptr, d_gs, nG, nTiles, s);
+}
+
+// Room for an axis' table in either layout (float2 elements; fragment order:
+// K entries to whole steps, 32-entry tiles; 256-byte aligned).
+static int64_t table_elems(int nk, int n) {
+    const int64_t frag = (2LL * nk + 7) / 8 * 8 * (((int64_t)n + 31) / 32 * 32), plain = 2LL * nk * n;
+    return ((frag > plain ? frag : plain) + 31) / 32 * 32;
 }
 
 // Scratch for one grid execution (float2 elements): tables (both sign
 // variants per axis), folded coefficients, V and (3-D) W.
 size_t rf_grid_scratch_elems(int nDim, const int32_t* kNStep, int nb, int Nmc, const int32_t* n) {
+    const int fold = nb > 1, Q = (fold && nDim == 3) ? 2 : 1;
     int64_t tables = 0;
-    for (int a = 0; a < nDim; a++) tables += 2LL * kNStep[a] * n[a];
+    for (int a = 0; a < nDim; a++) tables += table_elems(kNStep[a], n[a]);
     int64_t coeff = (int64_t)nb * Nmc;
     for (int a = 0; a < nDim; a++) coeff *= kNStep[a];
-    const int fold = nb > 1, Q = (fold && nDim == 3) ? 2 : 1;
     int64_t v = (int64_t)Nmc * Q * n[0];
     for (int a = 1; a < nDim; a++) v *= kNStep[a];
     const int64_t w = nDim == 3 ? (int64_t)Nmc * kNStep[2] * n[1] * n[0] : 0;
@@ -1771,18 +1315,38 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
     while (nDim == 3 && std::ldexp(bound2, -m2) > 16384.0) m2++;
     int split = bound1 <= 16384.0 ? 1 : 0;
 
+    // the strip GEMM addresses inside a strip with 32-bit offsets: one k of the
+    // streamed operand, one row or line of D (elements)
+    {
+        const int64_t lim = (int64_t)1 << 27;
+        int64_t rows1 = (int64_t)Nmc * Q, plane = n[0];
+        for (int a = 1; a < nDim; a++) rows1 *= kNStep[a];
+        if (nDim == 3) plane *= n[1];
+        int64_t span = 8 * rows1;                                       // first: K-major coefficients
+        if (32LL * n[0] > span) span = 32LL * n[0];                     // first: D
+        if (8 * plane > span) span = 8 * plane;                         // last: streamed
+        if (32LL * kStripMaxMT * plane > span) span = 32LL * kStripMaxMT * plane;   // last: D
+        if (nDim == 3 && ((int64_t)K2 + 160) * n[0] + plane > span)     // middle: streamed and D
+            span = ((int64_t)K2 + 160) * n[0] + plane;
+        if (span >= lim) split = 0;
+    }
+
     float2* p = scratch;
-    float2* E[3];
+    void* E[3];
     rf_table_args ta{};
     ta.dct = kind == 1;
     ta.nAx = nDim;
+    ta.frag = split;
     unsigned tabBlocks = 0;
     for (int a = 0; a < nDim; a++) {
-        E[a] = p; p += 2LL * kNStep[a] * n[a];
+        E[a] = p; p += table_elems(kNStep[a], n[a]);
         ta.nk[a] = kNStep[a];
         ta.nx[a] = n[a];
+        // the last axis has no sign variants left (folded)
+        ta.K[a] = a == nDim - 1 ? kNStep[a] : a == 0 ? K1 : K2;
         ta.block0[a] = tabBlocks;
-        tabBlocks += blocks_for((int64_t)kNStep[a] * n[a]);
+        tabBlocks += split ? (unsigned)((ta.K[a] + 7) / 8) * (unsigned)((n[a] + 31) / 32)
+                           : blocks_for((int64_t)kNStep[a] * n[a]);
         ta.dk[a] = kDelta[a]; ta.o[a] = origin[a]; ta.step[a] = step[a]; ta.invL[a] = 1.0 / corrL[a];
         ta.E[a] = E[a];
     }
@@ -1812,18 +1376,35 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
         hipLaunchKernelGGL(k_coeffs_fold,
                            dim3((unsigned)((fd.rows + kFoldM - 1) / kFoldM), (unsigned)((K1 + kFoldK - 1) / kFoldK)),
                            dim3(256), 0, s, fd);
-    // stage 1: rows (r, j3, q, j2) x K (h, j1) -> V[r][j3][q][j2][x1]
+    // stage 1: rows (r, j3, q, j2) x K (h, j1) -> V[r][j3][q][j2][x1].  FP32
+    // tiles: A = the coefficients, B = the table; strips: the table x1 x K
+    // against the lines (r, j3, q, j2) of the K-major coefficients
     const int64_t rows1 = nC / K1;
     float2* V = p; p += rows1 * n[0];
+    auto table = [&](rf_gemm_desc& q, int a) {       // the table operand of axis a, rows x
+        if (split) q.T = E[a];
+        else {
+            q.A = static_cast<const float2*>(E[a]);
+            q.aSm = 1; q.aSk = n[a];
+        }
+        q.aDiv = 1; q.aMod = 1;
+        q.M = n[a]; q.dSm = 1;
+    };
     rf_gemm_desc& g = st->g[st->n++];
-    g.A = Cf; g.aSm = 1; g.aSk = rows1; g.aStrideB = 0; g.aDiv = 1; g.aMod = 1;   // K-major
-    g.B = E[0]; g.bSk = n[0]; g.bSn = 1; g.bStrideB = 0;     // K (h, j1): variant h of E1
-    g.D = V; g.dSm = n[0]; g.dSn = 1; g.dStrideB = 0;
-    g.M = (int)rows1; g.N = n[0]; g.K = K1; g.batches = 1; g.realOut = 0;
-    // 128-row tiles over the long row axis; a first axis of 129..160 points
-    // in one 160-column tile
-    g.rw = n[0] > 2 * kTN && n[0] <= kTN5 ? 5 : rows1 >= 128 ? 2 : 1;
-    g.outScale = 1.0f; g.split16 = split;
+    g.kind = RF_GEMM_FIRST;
+    if (split) {
+        table(g, 0);
+        g.B = Cf; g.bSk = rows1; g.bSn = 1;          // K-major
+        g.D = V; g.dSn = n[0];
+        g.N = (int)rows1;
+    } else {
+        g.A = Cf; g.aSm = 1; g.aSk = rows1; g.aDiv = 1; g.aMod = 1;
+        g.B = static_cast<const float2*>(E[0]); g.bSk = n[0]; g.bSn = 1;     // K (h, j1): variant h of E1
+        g.D = V; g.dSm = n[0]; g.dSn = 1;
+        g.M = (int)rows1; g.N = n[0];
+    }
+    g.K = K1; g.batches = 1;
+    g.outScale = 1.0f;
     const float2* last = V;
     int64_t plane = n[0];                      // points already resolved
     int64_t lastStrideB = (int64_t)kNStep[1] * n[0];
@@ -1832,13 +1413,13 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
         // W[j3][x2][x1] = sum_{q,j2} E2^q[j2][x2] V[j3][q][j2][x1]
         float2* W = p; p += (int64_t)Nmc * kNStep[2] * n[1] * n[0];
         rf_gemm_desc& h = st->g[st->n++];
-        h.A = E[1]; h.aSm = 1; h.aSk = n[1]; h.aStrideB = 0; h.aDiv = 1; h.aMod = 1;
+        h.kind = RF_GEMM_MIDDLE;
+        table(h, 1);
         h.B = V; h.bSk = n[0]; h.bSn = 1; h.bStrideB = (int64_t)kNStep[2] * K2 * n[0];
         h.D = W; h.dSm = n[0]; h.dSn = 1; h.dStrideB = (int64_t)kNStep[2] * n[1] * n[0];
         h.nLo = n[0]; h.bSnHi = (int64_t)K2 * n[0]; h.dSnHi = (int64_t)n[1] * n[0];
-        h.M = n[1]; h.N = kNStep[2] * n[0]; h.K = K2; h.batches = Nmc; h.realOut = 0;
-        h.rw = h.N >= 128 ? 4 : 1;            // 128-column tiles over the long (j3, x1) axis
-        h.outScale = (float)std::ldexp(1.0, -m2); h.split16 = split;
+        h.N = kNStep[2] * n[0]; h.K = K2; h.batches = Nmc;
+        h.outScale = (float)std::ldexp(1.0, -m2);
         last = W;
         plane = (int64_t)n[0] * n[1];
         lastStrideB = (int64_t)kNStep[2] * plane;
@@ -1846,29 +1427,14 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
     // last stage per realization: u[x_d][plane] = Re sum_j E_d^+[j][x_d] last[j][plane]
     const int ad = nDim - 1;
     rf_gemm_desc& f = st->g[st->n++];
-    f.A = E[ad]; f.aSm = 1; f.aSk = n[ad]; f.aStrideB = 0; f.aDiv = 1; f.aMod = 1;
+    f.kind = RF_GEMM_LAST;
+    table(f, ad);
     f.B = last; f.bSk = plane; f.bSn = 1; f.bStrideB = lastStrideB;
     f.D = d_out; f.dSm = plane; f.dSn = 1; f.dStrideB = plane * n[ad];
-    f.M = n[ad]; f.N = (int)plane; f.K = kNStep[ad]; f.batches = Nmc; f.realOut = 1;
+    f.N = (int)plane; f.K = kNStep[ad]; f.batches = Nmc;
     f.outDtype = outDtype; f.epi = epi;
-    f.outScale = (float)(1.0 / (sc * std::ldexp(1.0, -m2))); f.split16 = split;
-    f.rw = plane >= 128 ? 3 : 1;              // 128-column tiles over the long plane axis
-    // the wide tiles (kinds 2..4) exist with FP16 operands only: a K beyond
-    // the FP16 range of the first contraction runs every stage on the FP32 tile
-    if (!split)
-        for (int j = 0; j < st->n; j++) st->g[j].rw = 1;
-    // the split-precision tile addresses inside a tile with 32-bit offsets
-    for (int i = 0; i < st->n; i++) {
-        rf_gemm_desc& q = st->g[i];
-        const int64_t lim = (int64_t)1 << 30;
-        const int64_t tm = tile_m(q), tn = tile_n(q);
-        if ((int64_t)q.K * q.aSk + tm * q.aSm >= lim || (int64_t)q.K * q.bSk + tn * q.bSn + q.bSnHi >= lim ||
-            tm * q.dSm + tn * q.dSn + q.dSnHi >= lim)
-            for (int j = 0; j < st->n; j++) {
-                st->g[j].split16 = 0;
-                st->g[j].rw = 1;                  // the FP32 tile is 64 x 64
-            }
-    }
+    f.outScale = (float)(1.0 / (sc * std::ldexp(1.0, -m2)));
+    for (int i = 0; i < st->n; i++) st->g[i].mt = split ? strip_choose(st->g[i]) : 0;
     return hipGetLastError();
 }
 
@@ -1917,7 +1483,8 @@ hipError_t rf_launch_draw_counter(int64_t* d_state, int64_t value, int gen, hipS
 
 hipError_t rf_grid_run(const rf_grid_stages& st, hipStream_t s) {
     for (int i = 0; i < st.n; i++) {
-        const hipError_t e = rf_launch_gemm(st.g[i], s);
+        const rf_gemm_desc& g = st.g[i];
+        const hipError_t e = launch_any(g.kind, g.mt, &g, nullptr, 0, rf_gemm_tiles(g, g.mt), s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

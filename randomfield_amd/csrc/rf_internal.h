@@ -257,7 +257,13 @@ inline rf_epilogue rf_make_epilogue(int margi, double avg, double var) {
 }
 
 // structured-grid form (rf_grid.hip), nDim 2 or 3, Shinozuka lattice:
-// batched complex FP32 GEMMs D[b] = A[(b / aDiv) % aMod] B[b]
+// batched complex GEMMs D[b] = A[(b / aDiv) % aMod] B[b] on FP32-operand tiles
+// (mt 0) or, FP16 hi/lo operands, as strip GEMMs (mt 1 .. kStripMaxMT tiles of 32
+// table entries per wave): D over M table entries (T, fragment order) and N
+// streamed lines (B)
+constexpr int kStripMaxMT = 5;
+constexpr int64_t kStripFill = 1024;  // waves below which a strip GEMM splits its table axis
+enum rf_gemm_kind { RF_GEMM_FIRST, RF_GEMM_MIDDLE, RF_GEMM_LAST };   // LAST: Re(D), epilogue, outDtype
 // The coefficient fold of one grid execution: Cf[k][m] for rows m (r, j3, q,
 // j2) and K index k (h, j1) from amp / phase [r][b][j] (rf_grid.hip).
 struct rf_fold_desc {
@@ -273,20 +279,19 @@ struct rf_gemm_desc {
     const float2* B; int64_t bSk, bSn, bStrideB;
     void* D; int64_t dSm, dSn, dStrideB;
     int M, N, K, batches;
-    int realOut;          // 0: complex D, 1: Re(D) with the epilogue, outDtype
+    int kind;             // rf_gemm_kind
+    int mt;               // strip tiles per wave; 0: FP32-operand tiles (operand A instead of T)
+    const void* T;        // strips: the table
     int outDtype;
     rf_epilogue epi;
     int64_t tile0;        // grouped launches: first tile of this GEMM
     float outScale;       // D = outScale * (A B) (power of two)
-    int split16;          // 1: FP16 hi/lo operands (3 products), 0: FP32 operands
     // two-level columns (nLo > 0): column n = (n / nLo, n % nLo) sits at
     // (n / nLo) * xSnHi + (n % nLo) * xSn in B and in D, so one GEMM spans
     // several batch blocks along N (a short axis is then padded once, not
     // once per block)
     int nLo;
     int64_t bSnHi, dSnHi;
-    int rw;               // tile kind, FP16 operands only: 2 128x64 (complex), 3 64x128 (real),
-                          // 4 64x128 (complex); 0, 1: 64x64
     // blend fused into a real last stage (grp != NULL): output row m (the
     // last axis) and column n = x + grpNx y (the plane) whose indices all lie
     // in the part of the field no other field covers (grpZlo <= m < grpZhi,
@@ -380,10 +385,8 @@ struct rf_iso_grid_args {
 };
 size_t rf_iso_grid_scratch_elems(int nDim, int64_t kN, int Nmc, const int32_t* n);
 hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s);
-int64_t rf_gemm_tiles(const rf_gemm_desc& g);
-hipError_t rf_launch_gemm(const rf_gemm_desc& g, hipStream_t s);
-hipError_t rf_launch_gemm_group(int realOut, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, int rwMax,
-                                hipStream_t s);
+int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt);
+hipError_t rf_launch_gemm_group(int kind, int mt, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, hipStream_t s);
 
 // post-processing (rf_post.hip)
 hipError_t rf_launch_marginal(int margi, double scale, double shift, void* d, int64_t count,
