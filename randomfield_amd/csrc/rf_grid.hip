@@ -14,7 +14,8 @@
 // Every stage is one tiled complex GEMM on the matrix cores,
 // D[m][n] = sum_k A[m][k] B[k][n] with per-stage strides: operands split
 // into FP16 hi + lo halves (power-of-two scaled into range), three
-// v_mfma_f32_32x32x16_f16 products with FP32 accumulation (strip GEMMs, below);
+// v_mfma_f32_32x32x16_f16 products with FP32 accumulation (strip GEMMs,
+// rf_strip.hip);
 // an FP32-operand MFMA tile (v_mfma_f32_32x32x2_f32) serves shapes whose K would
 // leave the FP16 range or whose strides a strip's 32-bit offsets.
 // The negative sign blocks are folded into the first contraction
@@ -25,28 +26,17 @@
 // grid each of its terms still factorises over the axes: per realization one
 // real-part GEMM over the shells whose operands are per-axis phase tables
 // (k_iso_tables, k_iso_gemm).
-#include "rf_internal.h"
-#include "rf_philox.h"
+#include "rf_grid_dev.h"
 
 namespace {
 
 constexpr int kTM = 64, kTN = 64, kTK = 16;   // block tile; 256 threads, 4x4 each
-
-// element offsets of column n in B and in D (two-level when nLo > 0)
-__device__ __forceinline__ int64_t col_b(const rf_gemm_desc& g, int n) {
-    return g.nLo ? (int64_t)(n / g.nLo) * g.bSnHi + (int64_t)(n % g.nLo) * g.bSn : (int64_t)n * g.bSn;
-}
-__device__ __forceinline__ int64_t col_d(const rf_gemm_desc& g, int n) {
-    return g.nLo ? (int64_t)(n / g.nLo) * g.dSnHi + (int64_t)(n % g.nLo) * g.dSn : (int64_t)n * g.dSn;
-}
 
 __device__ inline float epi32(float u, const rf_epilogue& e) {
     if (e.margi == RF_FOM_NONE) return u;
     const float y = fmaf(u, (float)e.scale, (float)e.shift);
     return (e.margi == RF_FOM_LOGNORMAL) ? expf(y) : y;
 }
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // One 64 x 64 output tile (complex rows m0.., columns n0.., batch) of
 // D = A B on the matrix cores in FP32 (v_mfma_f32_32x32x2_f32): the complex
@@ -167,11 +157,6 @@ __device__ __forceinline__ void gemm_tile(const rf_gemm_desc& g, int m0, int n0,
     }
 }
 
-typedef float f2v __attribute__((ext_vector_type(2)));
-typedef const f2v __attribute__((address_space(1))) gf2;      // global-memory views
-typedef f2v __attribute__((address_space(1))) gf2o;
-typedef float __attribute__((address_space(1))) gfo;
-typedef double __attribute__((address_space(1))) gdo;
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef const f4v __attribute__((address_space(1))) gf4;
 // n consecutive float2 (n even, 16-byte aligned) by 16-byte loads
@@ -185,60 +170,12 @@ __device__ __forceinline__ void ld_run(const gf2* p, f2v* v) {
         v[2 * i + 1] = f2v{t.z, t.w};
     }
 }
-typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
-typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
 constexpr int kHP = 24;                       // LDS row pitch (halves): 16 k + pad
-// Fused blend: the group-grid column offset of plane column n, or -1 where
-// another field also covers it; the group row offset of row m, or -1.
-__device__ __forceinline__ int64_t grp_col(const rf_gemm_desc& g, int n) {
-    const int x = n % g.grpNx, y = n / g.grpNx;
-    return (x >= g.grpXlo && x < g.grpXhi && y >= g.grpYlo && y < g.grpYhi)
-               ? g.grpCol0 + x + g.grpG0 * (int64_t)y : (int64_t)-1;
-}
-__device__ __forceinline__ int64_t grp_row(const rf_gemm_desc& g, int m) {
-    return (m >= g.grpZlo && m < g.grpZhi) ? g.grpRow0 + g.grpPlaneG * (int64_t)m : (int64_t)-1;
-}
-// Fused blend: plane column n inside a first-axis overlap band sits in the
-// band array of its side (*side 0 low, 1 high) at element offset (return) +
-// m * (*rowStride) for row m; -1 outside the bands.
-// (selects, not early returns: the blend's lookup of the same bands was
-// miscompiled in an if-return form)
-__device__ __forceinline__ int64_t band_col(const rf_gemm_desc& g, int n, int batch, int* side, int* rowStride) {
-    const int x = n % g.grpNx, y = n / g.grpNx;
-    const int wLo = g.grpXlo, wHi = g.grpNx - g.grpXhi;
-    const bool lo = g.bandLo != nullptr && x < g.grpXlo;
-    const bool hi = !lo && g.bandHi != nullptr && x >= g.grpXhi;
-    const int64_t offLo = (int64_t)batch * g.bandLoStrideB + (int64_t)y * wLo + x;
-    const int64_t offHi = (int64_t)batch * g.bandHiStrideB + (int64_t)y * wHi + (x - g.grpXhi);
-    *side = hi ? 1 : 0;
-    *rowStride = lo ? g.grpNy * wLo : hi ? g.grpNy * wHi : 0;
-    return lo ? offLo : hi ? offHi : (int64_t)-1;
-}
-
 // Operand planes of a 64x128 real-part tile (the isotropic GEMM).
 struct HStage {
     _Float16 a[4][kTM][kHP];          // Re hi, Re lo, -Im hi, -Im lo
     _Float16 b[4][2 * kTN][kHP];      // Re hi, Re lo, Im hi, Im lo
 };
-
-// v -> FP16 hi (round to nearest) and lo = v - hi: packed conversions for
-// hi and lo, the residuals by mixed-precision FMAs reading the f16 halves in
-// place (v_fma_mix_f32), two instructions per value.
-__device__ inline void split4(const float* v, hv4* hi, hv4* lo) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-        const h2 h = {(_Float16)v[i], (_Float16)v[i + 1]};       // v_cvt_pk_f16_f32
-        const unsigned hb = __builtin_bit_cast(unsigned, h);
-        float l0, l1;
-        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(hb), "v"(v[i]));
-        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(l1) : "v"(hb), "v"(v[i + 1]));
-        (*hi)[i] = h.x;
-        (*hi)[i + 1] = h.y;
-        (*lo)[i] = (_Float16)l0;
-        (*lo)[i + 1] = (_Float16)l1;
-    }
-}
 
 // -x of FP16 values: the sign bits flipped
 __device__ inline hv4 neg4(hv4 x) {
@@ -246,341 +183,6 @@ __device__ inline hv4 neg4(hv4 x) {
     return __builtin_bit_cast(hv4, __builtin_bit_cast(u2, x) ^ 0x80008000u);
 }
 
-// cos and sin of 2 pi U for U in [0, 1): FP32 sincospi of the FP32 part Uh
-// and the first-order term of the remainder U - Uh (|U - Uh| <= 2^-25), a few
-// FP32 ulps from the FP64 values -- the coefficients are FP32.
-__device__ __forceinline__ void cis_rev(double U, float* c, float* s) {
-    const float uh = (float)U;
-    const float ul = (float)(U - (double)uh);
-    float sh, ch;
-    sincospif(2.0f * uh, &sh, &ch);
-    const float d = 6.28318530717958648f * ul;
-    *s = fmaf(d, ch, sh);
-    *c = fmaf(-d, sh, ch);
-}
-
-// The folded coefficient of row (r, j3, q, j2) and column (h, j1) with its
-// phase drawn from element drawBase + src of the stream (seed, tag 2): the
-// one formula of the coefficient fold and of the first contraction that forms
-// its coefficients itself.
-__device__ __forceinline__ float2 fold_coef_draw(const rf_fold_desc& f, unsigned r, unsigned j3, unsigned q,
-                                                 unsigned j2, unsigned j1, unsigned h, uint64_t seed,
-                                                 int64_t drawBase) {
-#pragma clang fp contract(off)
-    unsigned b = 0;
-    if (f.fold) b = f.nDim == 3 ? (q == 0 ? (h ? 3u : 0u) : (h ? 1u : 2u)) : h;
-    const int64_t jb = (int64_t)b * f.kNu + ((int64_t)j3 * f.nk2 + j2) * f.nk1 + j1;   // b kNu + j
-    const int64_t src = (int64_t)r * f.kNr + jb;
-    const double a = f.amp[(int64_t)r * f.ampStrideR + jb] * f.ampMult;
-    float cs, sn;
-    cis_rev(rf_uniform(seed, 2u, (uint64_t)(drawBase + src)), &cs, &sn);
-    return make_float2((float)(a * (double)cs), (float)(h ? -(a * (double)sn) : a * (double)sn));
-}
-
-// The strip GEMM: every contraction of the grid form with FP16 operands.
-//
-// One operand of each contraction is a small phase table shared by the whole
-// launch (M entries of an axis x K), the other -- the coefficients or the
-// previous contraction's output -- is streamed, N lines of K complex values.
-// A wave owns 32 lines and MT 32-entry tiles of the table axis (with MT * 32 >=
-// M every streamed value is read from memory and converted once in the whole
-// launch).  Operands are split into FP16 hi + lo halves; three
-// v_mfma_f32_32x32x16_f16 products (hi hi, hi lo, lo hi) with FP32 accumulation.
-//
-// A K-step is 8 complex k = 16 MFMA K entries: the re parts in lane half 0, the
-// im parts in half 1.  A lane loads k = 8 s + 4 h + (0..3) of its own line straight
-// to registers (no LDS), splits them and trades with the other half
-// (v_permlane32_swap).  Re D pairs table (re, im) with streamed (re, -im); Im D pairs
-// (im, re) with (re, im) -- the lane reads the other half's slot -- or, in the
-// first contraction, (re, im) with (im, re).  The table is stored in HBM pre-split
-// in fragment order [step][tile][hi, lo][lane][8] (k_axis_tables) and goes to LDS by
-// direct loads, kStripCS steps ahead in a double buffer, shared by the block's
-// waves; one barrier per kStripCS steps.
-//
-// Replaces 64..160-wide block tiles that staged and split both operands in LDS
-// per 16 k, re-reading and re-splitting the streamed one per table tile, two
-// barriers per 16 k.  32 fields of ~131^3 x 16 realizations: first contraction
-// (with its draws) 1.48 -> 1.44 ms, middle 1.93 -> 1.27, last 3.1 -> 2.44; 128^3
-// x 8 of method 4: 104 / 88 / 73 -> 68 / 63 / 64 us.  Same bits.
-//
-// D orientation: the table is the A operand (lanes run along lines) where D
-// is stored with lines contiguous, the B operand (lanes run along the table
-// axis) in the first contraction, whose D has the table axis contiguous.
-constexpr int kStripW = 4;              // waves per block
-constexpr int kStripCS = 2;             // K-steps per LDS chunk
-constexpr int kStripL = 32 * kStripW;   // lines per block
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void;
-constexpr int strip_units(int MT) { return kStripCS * MT * 128; }   // 16-byte units of a chunk
-
-__host__ __device__ inline int strip_groups(const rf_gemm_desc& g, int MT) {
-    return ((g.M + 31) / 32 + MT - 1) / MT;
-}
-
-// x and y hold k = 4 h + (0..3) in lane half h: half 0's x for all eight k in
-// half 0, half 1's y for all eight in half 1.
-__device__ __forceinline__ u32x4 half_swap(const hv4& x, const hv4& y) {
-    const u32x2 a = __builtin_bit_cast(u32x2, x), b = __builtin_bit_cast(u32x2, y);
-    const u32x2 p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a.x, b.x, false, false));
-    const u32x2 q = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a.y, b.y, false, false));
-    return u32x4{p.x, q.x, p.y, q.y};
-}
-
-template <int MT, int KIND>
-__device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local, u32x4* ldsA, u32x4* ldsB) {
-    constexpr bool kReal = KIND == RF_GEMM_LAST, kFirst = KIND == RF_GEMM_FIRST;
-    constexpr int NA = kReal ? 1 : 2;                 // accumulators per tile: Re, Im
-    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // table groups fastest: they share the streamed lines
-    const int mtTot = (g.M + 31) / 32, nGr = strip_groups(g, MT);
-    const int grp = (int)(local % nGr);
-    const int64_t rest = local / nGr;
-    const int nSB = (int)(((int64_t)g.N + kStripL - 1) / kStripL);
-    const int sb = (int)(rest % nSB), batch = (int)(rest / nSB);
-    const int t0 = grp * MT;
-    const int nSteps = (g.K + 7) / 8;
-    const int n0 = sb * kStripL + wave * 32;          // < 2^31: checked by the launcher
-    const bool active = n0 < g.N;                     // uniform
-    const int n0c = active ? n0 : 0;
-    const int n = n0c + l32, nc = n < g.N ? n : g.N - 1;
-    const bool nIn = active && n < g.N;
-
-    f32x16 acc[MT][NA];
-#pragma unroll
-    for (int t = 0; t < MT; t++)
-#pragma unroll
-        for (int a = 0; a < NA; a++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[t][a][i] = 0.0f;
-
-    // streamed operand: wave-uniform base, 32-bit lane offset (the launcher
-    // keeps a strip's span below 2^28 elements).  Global address space: the
-    // descriptor of a grouped launch is read from memory, and generic (flat)
-    // loads would also count against the LDS wait counter.
-    const int64_t col0 = col_b(g, n0c);
-    typedef const char __attribute__((address_space(1))) gch;
-    gch* S = (gch*)(g.B + (int64_t)batch * g.bStrideB + col0);
-    const unsigned kb = (unsigned)g.bSk * 8u;         // bytes per k
-    const unsigned lo0 = (unsigned)(col_b(g, nc) - col0) * 8u;
-    // a batch's fresh realizations: the coefficients of the current draw are
-    // formed here (fold_coef_draw, as the fold would store them) instead of read
-    const bool gen = kFirst && g.genState != nullptr && g.genState[2] != 0;
-    int64_t drawBase = 0;
-    unsigned gr = 0, gj3 = 0, gq = 0, gj2 = 0;
-    if (kFirst && gen) {
-        drawBase = g.genState[1] * (int64_t)g.genNmc * g.gen.kNr;
-        const unsigned Q = (g.gen.fold && g.gen.nDim == 3) ? 2u : 1u;
-        unsigned rem = (unsigned)nc;
-        gj2 = rem % (unsigned)g.gen.nk2; rem /= (unsigned)g.gen.nk2;
-        gq = rem % Q; rem /= Q;
-        gj3 = g.gen.nDim == 3 ? rem % (unsigned)g.gen.nk3 : 0u;
-        gr = g.gen.nDim == 3 ? rem / (unsigned)g.gen.nk3 : rem;
-    }
-    f2v r[kStripCS][4];
-    // a step's values of this lane; past K the table is zero and the last
-    // valid value is read again
-    auto fetch = [&](int s, f2v* v) {
-        if (kFirst && gen) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int k = 8 * s + 4 * half + i;
-                if (k < g.K) {
-                    const unsigned h = k >= g.gen.nk1 ? 1u : 0u;
-                    const float2 c = fold_coef_draw(g.gen, gr, gj3, gq, gj2, (unsigned)k - (h ? g.gen.nk1 : 0), h, g.genSeed,
-                                                    drawBase);
-                    v[i] = f2v{c.x, c.y};
-                } else {
-                    v[i] = f2v{0.f, 0.f};
-                }
-            }
-        } else {
-            gch* b = S + (int64_t)(8 * s) * kb;
-            const int left = g.K - 1 - 8 * s;         // >= 0
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                int k = 4 * half + i;
-                if (left < 7) k = k < left ? k : left;                            // uniform: the last step
-                v[i] = *(gf2*)(b + (lo0 + (unsigned)k * kb));
-            }
-        }
-    };
-    // chunk c of the table (steps kStripCS c ..): 1 KB pieces over the waves;
-    // tiles and steps past the table re-read its last ones, whose products are
-    // never stored, resp. never formed
-    const u32x4* T = static_cast<const u32x4*>(g.T);
-    auto dma = [&](int c, u32x4* dst) {
-        constexpr int kPieces = kStripCS * MT * 2;
-#pragma unroll
-        for (int i = 0; i < (kPieces + kStripW - 1) / kStripW; i++) {
-            const int p = wave + i * kStripW;
-            if (kPieces % kStripW == 0 || p < kPieces) {
-                const int st = p / (2 * MT), q = p % (2 * MT);
-                const int s = kStripCS * c + st < nSteps ? kStripCS * c + st : nSteps - 1;
-                const int t = t0 + (q >> 1) < mtTot ? t0 + (q >> 1) : mtTot - 1;
-                __builtin_amdgcn_global_load_lds((const void*)(T + (((int64_t)s * mtTot + t) * 2 + (q & 1)) * 64 + lane),
-                                                 (lds_void*)&dst[p * 64], 16, 0, 0);
-            }
-        }
-    };
-    const int nChunks = (nSteps + kStripCS - 1) / kStripCS;
-    const unsigned sgn = half ? 0x80008000u : 0u;
-    auto chunk = [&](int c, const u32x4* cur, u32x4* nxt) {
-        // fragments of this chunk's streamed values, then the loads of the next
-        u32x4 fh[kStripCS][NA], fl[kStripCS][NA];
-#pragma unroll
-        for (int st = 0; st < kStripCS; st++) {
-            float re[4], im[4];
-            hv4 rh, rl, ih, il;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = r[st][i].x;
-                im[i] = r[st][i].y;
-            }
-            split4(re, &rh, &rl);
-            split4(im, &ih, &il);
-            const u32x4 h = half_swap(rh, ih), l = half_swap(rl, il);             // (Re, Im)
-            fh[st][0] = h ^ sgn;
-            fl[st][0] = l ^ sgn;
-            if (kFirst) {
-                fh[st][NA - 1] = half_swap(ih, rh);                               // (Im, Re)
-                fl[st][NA - 1] = half_swap(il, rl);
-            } else if (!kReal) {
-                fh[st][NA - 1] = h;
-                fl[st][NA - 1] = l;
-            }
-        }
-        if (c + 1 < nChunks) {                         // in flight during the MFMAs
-            dma(c + 1, nxt);
-#pragma unroll
-            for (int st = 0; st < kStripCS; st++) {
-                const int s = kStripCS * (c + 1) + st;
-                fetch(s < nSteps ? s : nSteps - 1, r[st]);
-            }
-        }
-#pragma unroll
-        for (int st = 0; st < kStripCS; st++) {
-            if (!active || kStripCS * c + st >= nSteps) break;                    // uniform
-            const u32x4* p = cur + st * MT * 128;
-            auto mm = [](const u32x4& x, const u32x4& y, const f32x16& d) {
-                return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(hv8, x), __builtin_bit_cast(hv8, y), d, 0,
-                                                              0, 0);
-            };
-#pragma unroll
-            for (int t = 0; t < MT; t++) {
-                u32x4 th[NA], tl[NA];
-                th[0] = p[(2 * t) * 64 + lane];
-                tl[0] = p[(2 * t + 1) * 64 + lane];
-                if (!kReal && !kFirst) {
-                    th[NA - 1] = p[(2 * t) * 64 + (lane ^ 32)];
-                    tl[NA - 1] = p[(2 * t + 1) * 64 + (lane ^ 32)];
-                } else {
-                    th[NA - 1] = th[0];
-                    tl[NA - 1] = tl[0];
-                }
-                // A hi B hi, A hi B lo, A lo B hi
-#pragma unroll
-                for (int a = 0; a < NA; a++)
-                    acc[t][a] = kFirst ? mm(fh[st][a], th[a], acc[t][a]) : mm(th[a], fh[st][a], acc[t][a]);
-#pragma unroll
-                for (int a = 0; a < NA; a++)
-                    acc[t][a] = kFirst ? mm(fh[st][a], tl[a], acc[t][a]) : mm(th[a], fl[st][a], acc[t][a]);
-#pragma unroll
-                for (int a = 0; a < NA; a++)
-                    acc[t][a] = kFirst ? mm(fl[st][a], th[a], acc[t][a]) : mm(tl[a], fh[st][a], acc[t][a]);
-            }
-        }
-        // this wave's direct loads are complete (vmcnt(0)) before the barrier
-        // publishes them
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-    };
-    dma(0, ldsA);
-#pragma unroll
-    for (int st = 0; st < kStripCS; st++) fetch(st < nSteps ? st : nSteps - 1, r[st]);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    for (int c = 0; c < nChunks; c += 2) {
-        chunk(c, ldsA, ldsB);
-        if (c + 1 < nChunks) chunk(c + 1, ldsB, ldsA);
-    }
-    if (!active) return;
-    // D layout of a 32x32 tile: lane column l32 (B operand), rows 8*(i/4) +
-    // 4*half + i%4 (A operand)
-    const float os = g.outScale;
-    if constexpr (kFirst) {
-        // lane: table entry 32 (t0 + t) + l32; rows: lines
-        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)batch * g.dStrideB + (int64_t)n0 * g.dSn);
-        const int dSn = (int)g.dSn;
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-            const int m = 32 * (t0 + t) + l32;
-            if (m >= g.M) continue;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int line = 8 * (i >> 2) + 4 * half + (i & 3);
-                if (n0 + line < g.N) D[line * dSn + m] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
-            }
-        }
-    } else if constexpr (!kReal) {
-        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)batch * g.dStrideB + col_d(g, n0) +
-                          (int64_t)(32 * t0) * g.dSm);
-        const int dSm = (int)g.dSm, oc = (int)(col_d(g, nc) - col_d(g, n0));
-        if (!nIn) return;
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int m = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (32 * t0 + m < g.M) D[m * dSm + oc] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
-            }
-    } else {
-        if (!nIn) return;
-        const int64_t dBase = (int64_t)batch * g.dStrideB + (int64_t)(32 * t0) * g.dSm + (int64_t)n0 * g.dSn;
-        const int dSm = (int)g.dSm;
-        // fused blend: this lane's column offset in the group grid, or -1,
-        // and in a first-axis band array, or -1
-        const int64_t gc = g.grp ? grp_col(g, n) : -1;
-        int bside = 0, bst = 0;
-        const int64_t bo = (g.grp && gc < 0) ? band_col(g, n, batch, &bside, &bst) : -1;
-        auto store = [&](auto map, auto* D, auto* G, auto* BL, auto* BH) {
-#pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int m = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3), M = 32 * t0 + m;
-                    if (M < g.M) {
-                        const auto v = map(acc[t][0][i] * os);
-                        const int64_t go = gc >= 0 ? grp_row(g, M) : -1;
-                        if (go >= 0) G[go + gc] = v;
-                        else if (bo >= 0) (bside ? BH : BL)[bo + (int64_t)M * bst] = v;
-                        else D[m * dSm + l32] = v;
-                    }
-                }
-        };
-        const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
-        gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
-        gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
-        gfo* G32 = (gfo*)(static_cast<float*>(g.grp) + (int64_t)batch * g.grpStrideB);
-        gdo* G64 = (gdo*)(static_cast<double*>(g.grp) + (int64_t)batch * g.grpStrideB);
-        gfo* L32 = (gfo*)static_cast<float*>(g.bandLo);
-        gfo* H32 = (gfo*)static_cast<float*>(g.bandHi);
-        gdo* L64 = (gdo*)static_cast<double*>(g.bandLo);
-        gdo* H64 = (gdo*)static_cast<double*>(g.bandHi);
-        if (g.outDtype == RF_DTYPE_F64) {
-            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64, G64, L64, H64);
-            else if (g.epi.margi == RF_FOM_LOGNORMAL)
-                store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64, G64, L64, H64);
-            else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64, G64, L64, H64);
-        } else {
-            if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32, G32, L32, H32);
-            else if (g.epi.margi == RF_FOM_LOGNORMAL)
-                store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32, G32, L32, H32);
-            else store([=](float u) { return fmaf(u, sc, sh); }, D32, G32, L32, H32);
-        }
-    }
-}
 // Isotropic sum on a structured grid, per-realization directions.  With
 // x = o + i step per axis, e^{i(k.x + phi)} factorises over the axes, so per
 // realization r
@@ -867,17 +469,6 @@ struct FStage {
     float2 b[kTK][kTN + 1];
 };
 
-// Placement.  Workgroups go round-robin to the 8 XCDs, each with its own L2;
-// block b runs logical tile (b % 8) * P + b / 8, so every XCD walks a contiguous
-// range of P tiles and what neighbours share (streamed lines between table
-// groups, amplitudes, cache lines at strip edges) is re-read from its L2.
-constexpr int kXcd = 8;
-
-__device__ inline int64_t xcd_tile(int64_t b, int64_t nTiles) {
-    const int64_t per = (nTiles + kXcd - 1) / kXcd;
-    return (b % kXcd) * per + b / kXcd;
-}
-
 // An FP32-operand tile: row tiles fastest (they share a column slab of B).
 template <bool RealOnly>
 __device__ __forceinline__ void run_tile(const rf_gemm_desc& g, int64_t local, char* smem) {
@@ -886,45 +477,6 @@ __device__ __forceinline__ void run_tile(const rf_gemm_desc& g, int64_t local, c
     const int64_t r = local / ntM;
     FStage* f = reinterpret_cast<FStage*>(smem);
     gemm_tile<RealOnly>(g, mI * kTM, (int)(r % ntN) * kTN, (int)(r / ntN), f->a, f->b);
-}
-
-// Registers: 16 MT accumulators per lane (32 MT complex) decide the waves per
-// SIMD; the compiler then keeps them in VGPRs without spills.
-constexpr int strip_waves(int MT, int KIND) {
-    return KIND == RF_GEMM_LAST ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4);
-}
-
-template <int MT, int KIND>
-__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, KIND))))
-void k_strip(rf_gemm_desc g, int64_t nTiles) {
-    __shared__ u32x4 ldsA[strip_units(MT)];
-    __shared__ u32x4 ldsB[strip_units(MT)];
-    const int64_t L = xcd_tile(blockIdx.x, nTiles);
-    if (L >= nTiles) return;
-    strip_tile<MT, KIND>(g, L, ldsA, ldsB);
-}
-
-// Grouped form: the GEMMs of several fields in one launch; GEMM q owns
-// logical tiles tile0 .. tile0 + tiles(q) - 1.
-__device__ inline int gemm_find(const rf_gemm_desc* __restrict__ gs, int nG, int64_t b) {
-    int lo = 0, hi = nG - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (gs[mid].tile0 <= b) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-template <int MT, int KIND>
-__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, KIND))))
-void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
-    __shared__ u32x4 ldsA[strip_units(MT)];
-    __shared__ u32x4 ldsB[strip_units(MT)];
-    const int64_t L = xcd_tile(blockIdx.x, nTiles);
-    if (L >= nTiles) return;
-    const rf_gemm_desc g = gs[gemm_find(gs, nG, L)];   // uniform: scalar registers
-    strip_tile<MT, KIND>(g, L - g.tile0, ldsA, ldsB);
 }
 
 // The FP32-operand tile (a first contraction whose K would leave the FP16
@@ -1200,8 +752,10 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
+// Logical tiles of a GEMM: blocks of strips x table groups, or FP32 tiles.
 int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt) {
-    if (mt > 0) return (int64_t)strip_groups(g, mt) * (((int64_t)g.N + kStripL - 1) / kStripL) * g.batches;
+    if (mt > 0)
+        return (int64_t)(((g.M + 31) / 32 + mt - 1) / mt) * (((int64_t)g.N + kStripL - 1) / kStripL) * g.batches;
     return (int64_t)((g.N + kTN - 1) / kTN) * ((g.M + kTM - 1) / kTM) * g.batches;
 }
 
@@ -1209,24 +763,7 @@ int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt) {
 inline int64_t xcd_blocks(int64_t nTiles) { return (nTiles + kXcd - 1) / kXcd * kXcd; }
 
 namespace {
-template <int MT, int KIND>
-void strip_launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, unsigned blocks, hipStream_t s) {
-    const dim3 b(64 * kStripW);
-    if (g) hipLaunchKernelGGL((k_strip<MT, KIND>), dim3(blocks), b, 0, s, *g, nTiles);
-    else hipLaunchKernelGGL((k_strip_group<MT, KIND>), dim3(blocks), b, 0, s, d_gs, nG, nTiles);
-}
-template <int KIND>
-void strip_launch_mt(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, unsigned blocks,
-                     hipStream_t s) {
-    switch (mt) {
-        case 1: return strip_launch<1, KIND>(g, d_gs, nG, nTiles, blocks, s);
-        case 2: return strip_launch<2, KIND>(g, d_gs, nG, nTiles, blocks, s);
-        case 3: return strip_launch<3, KIND>(g, d_gs, nG, nTiles, blocks, s);
-        case 4: return strip_launch<4, KIND>(g, d_gs, nG, nTiles, blocks, s);
-        default: return strip_launch<kStripMaxMT, KIND>(g, d_gs, nG, nTiles, blocks, s);
-    }
-}
-// One GEMM (g) or a group of them (d_gs, nG), all of one kind, on strips of
+// One GEMM (g) or a group of them (d_gs, nG), all of one kind: strips of
 // mt tiles or, mt 0, FP32-operand tiles.
 hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t nTiles,
                       hipStream_t s) {
@@ -1235,10 +772,11 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
     if (nb > 0x7fffffffLL || mt < 0 || mt > kStripMaxMT) return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)nb;
     if (mt > 0) {
-        if (kind == RF_GEMM_FIRST) strip_launch_mt<RF_GEMM_FIRST>(mt, g, d_gs, nG, nTiles, blocks, s);
-        else if (kind == RF_GEMM_MIDDLE) strip_launch_mt<RF_GEMM_MIDDLE>(mt, g, d_gs, nG, nTiles, blocks, s);
-        else strip_launch_mt<RF_GEMM_LAST>(mt, g, d_gs, nG, nTiles, blocks, s);
-    } else if (kind == RF_GEMM_LAST) {
+        if (kind == RF_GEMM_FIRST) return rf_strip_launch_first(mt, g, d_gs, nG, nTiles, blocks, s);
+        if (kind == RF_GEMM_MIDDLE) return rf_strip_launch_middle(mt, g, d_gs, nG, nTiles, blocks, s);
+        return rf_strip_launch_last(mt, g, d_gs, nG, nTiles, blocks, s);
+    }
+    if (kind == RF_GEMM_LAST) {
         if (g) hipLaunchKernelGGL(k_cgemm<true>, dim3(blocks), dim3(256), 0, s, *g, nTiles);
         else hipLaunchKernelGGL(k_cgemm_group<true>, dim3(blocks), dim3(256), 0, s, d_gs, nG, nTiles);
     } else {
@@ -1250,11 +788,15 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
 
 // MT of a strip GEMM: all of the table axis in one wave (up to kStripMaxMT
 // tiles) so that every streamed value is read and converted once, unless the
-// launch would then leave SIMDs without a wave.
+// launch would then leave SIMDs without a wave.  The last contraction, whose
+// K is short and whose stores bound it, takes at most 3 tiles: 32 fields of
+// ~131^3 x 16 on 5 / 4 / 3 / 2 / 1 tiles: 2.62 / 2.31 / 2.29 / 2.29 / 2.66 ms;
+// 135 x 131 x 131 x 4 on 5 / 3: 24.8 / 20.6 us (128^3 x 8 on 4 / 2: 51 / 55).
 int strip_choose(const rf_gemm_desc& g) {
     const int mt = (g.M + 31) / 32;
     const int64_t strips = (((int64_t)g.N + 31) / 32) * g.batches;
-    int gr = (mt + kStripMaxMT - 1) / kStripMaxMT;
+    const int most = g.kind == RF_GEMM_LAST ? 3 : kStripMaxMT;
+    int gr = (mt + most - 1) / most;
     while (gr < mt && strips * gr < kStripFill) gr++;
     return (mt + gr - 1) / gr;
 }

@@ -262,6 +262,9 @@ inline rf_epilogue rf_make_epilogue(int margi, double avg, double var) {
 // table entries per wave): D over M table entries (T, fragment order) and N
 // streamed lines (B)
 constexpr int kStripMaxMT = 5;
+constexpr int kStripW = 4;            // waves per block
+constexpr int kStripCS = 2;           // K-steps per fetch and table chunk
+constexpr int kStripL = 32 * kStripW; // lines per block
 constexpr int64_t kStripFill = 1024;  // waves below which a strip GEMM splits its table axis
 enum rf_gemm_kind { RF_GEMM_FIRST, RF_GEMM_MIDDLE, RF_GEMM_LAST };   // LAST: Re(D), epilogue, outDtype
 // The coefficient fold of one grid execution: Cf[k][m] for rows m (r, j3, q,
@@ -387,6 +390,13 @@ size_t rf_iso_grid_scratch_elems(int nDim, int64_t kN, int Nmc, const int32_t* n
 hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s);
 int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt);
 hipError_t rf_launch_gemm_group(int kind, int mt, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, hipStream_t s);
+// strips of one kind (rf_strip.hip): one GEMM (g) or a group (d_gs, nG)
+hipError_t rf_strip_launch_first(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
+                                 unsigned blocks, hipStream_t s);
+hipError_t rf_strip_launch_middle(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
+                                  unsigned blocks, hipStream_t s);
+hipError_t rf_strip_launch_last(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
+                                unsigned blocks, hipStream_t s);
 
 // post-processing (rf_post.hip)
 hipError_t rf_launch_marginal(int margi, double scale, double shift, void* d, int64_t count,
