@@ -46,9 +46,8 @@ int build_form_operands(rf_field_plan* P, hipStream_t s) {
         RF_HIP_TRY(ctx, rf_launch_prep_fp64(kN, Nmc, P->Rpad, is_iso_direct(P->p), P->d_phase, P->d_amp, P->d_CS, s));
     } else if (P->p.form == RF_FORM_FP32) {
         if (is_iso_direct(P->p)) {
-            if (!P->d_kIsoT) RF_HIP_TRY(ctx, dmalloc(&P->d_kIsoT, (size_t)(kN * P->Rpad * P->p.nDim)));
-            RF_HIP_TRY(ctx, rf_launch_prep_fp32_iso(P->p.nDim, kN, Nmc, P->Rpad, P->d_kIso, P->d_phase,
-                                                    P->d_amp, ampMult, P->d_kIsoT, P->d_phT, P->d_aT, s));
+            RF_HIP_TRY(ctx, rf_launch_prep_fp32_iso(P->p.nDim, kN, Nmc, P->d_kIso, P->d_phase, P->d_amp, ampMult,
+                                                    P->d_kIsoT, P->d_aT, s));
         } else {
             RF_HIP_TRY(ctx, rf_launch_prep_fp32(kN, Nmc, P->Rpad, P->d_phase, P->d_amp, ampMult,
                                                 P->d_phT, P->d_aT, s));
@@ -301,12 +300,14 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
     }
 
     // operand buffers of the chosen form
-    if (p->form == RF_FORM_FP64) {
-        // isotropic: the components are bounded by the radii
-        for (double v : P->spec.k) P->kAbsMax = std::max(P->kAbsMax, std::fabs(v));
-        RF_HIP_TRY(ctx, dmalloc(&P->d_CS, (size_t)(kN * P->Rpad)));
-    }
-    if (p->form == RF_FORM_FP32) {
+    // isotropic: the components are bounded by the radii
+    for (double v : P->spec.k) P->kAbsMax = std::max(P->kAbsMax, std::fabs(v));
+    if (p->form == RF_FORM_FP64) RF_HIP_TRY(ctx, dmalloc(&P->d_CS, (size_t)(kN * P->Rpad)));
+    if (p->form == RF_FORM_FP32 && is_iso_direct(*p)) {
+        const int64_t nb = rf_iso_blocks(kN, Nmc);
+        RF_HIP_TRY(ctx, dmalloc(&P->d_kIsoT, (size_t)(nb * 64)));
+        RF_HIP_TRY(ctx, dmalloc(&P->d_aT, (size_t)(nb * 16)));
+    } else if (p->form == RF_FORM_FP32) {
         RF_HIP_TRY(ctx, dmalloc(&P->d_phT, (size_t)(kN * P->Rpad)));
         RF_HIP_TRY(ctx, dmalloc(&P->d_aT, (size_t)(kN * P->Rpad)));
     }
@@ -383,7 +384,7 @@ int rf_plan_execute(rf_field_plan* P, const double* d_x, int64_t N, void* d_out,
                                        P->d_CS, P->Rpad, s);
                 break;
             case RF_FORM_FP32:
-                if (is_iso_direct(p)) e = rf_launch_sum_fp32_iso_t(a, P->d_kIsoT, P->d_phT, P->d_aT, P->Rpad, s);
+                if (is_iso_direct(p)) e = rf_launch_sum_fp32_iso_t(a, P->d_kIsoT, P->d_aT, P->kAbsMax * RF_INV_TWO_PI, s);
                 else e = rf_launch_sum_fp32(a, P->d_kRev, P->d_phT, P->d_aT, P->Rpad, s);
                 break;
             default:

@@ -117,11 +117,29 @@ hipError_t rf_launch_sum_fp64(const rf_sum_args& a, const double* d_k, int iso, 
                               const double2* d_CS, int Rpad, hipStream_t s);
 hipError_t rf_launch_sum_fp32(const rf_sum_args& a, const double* d_kRev, const float* d_phT,
                               const float* d_aT, int Rpad, hipStream_t s);
-hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kT, const float* d_pT,
-                                    const float* d_aT, int Rpad, hipStream_t s);
-hipError_t rf_launch_prep_fp32_iso(int nDim, int64_t kN, int Nmc, int Rpad, const double* d_kIso,
-                                   const double* d_phase, const double* d_amp, double ampMult,
-                                   double* d_kT, float* d_pT, float* d_aT, hipStream_t s);
+// direct isotropic sum, per-realization directions: operand rows of 16 / Rp
+// wavevectors x Rp realizations (Rp the power of two, at most 16, that holds
+// Nmc), nJ wavevector blocks x nChunk chunks of 16 realizations
+struct rf_iso_shape { int64_t nJ; int nChunk, Rp; };
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline rf_iso_shape rf_iso_rows(int64_t kN, int Nmc) {
+    int Rp = 1;
+    while (Rp < Nmc && Rp < 16) Rp <<= 1;
+    const int J = 16 / Rp;
+    return rf_iso_shape{(kN + J - 1) / J, (Nmc + 15) / 16, Rp};
+}
+inline int64_t rf_iso_blocks(int64_t kN, int Nmc) {
+    const rf_iso_shape s = rf_iso_rows(kN, Nmc);
+    return s.nJ * s.nChunk;
+}
+// d_kA 64 doubles, d_aA 16 floats per block; kMax = max |k component| in
+// revolutions
+hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kA, const float* d_aA, double kMax,
+                                    hipStream_t s);
+hipError_t rf_launch_prep_fp32_iso(int nDim, int64_t kN, int Nmc, const double* d_kIso, const double* d_phase,
+                                   const double* d_amp, double ampMult, double* d_kA, float* d_aA, hipStream_t s);
 int rf_fp32_rchunk();
 
 // MFMA form (rf_mfma.hip)
@@ -212,26 +230,23 @@ struct rf_field_plan {
 // block b finds its field by binary search over tile0.
 struct rf_group_req {
     rf_sum_args a;        // points, output, epilogue of the field (i0 = 0, i1 = N)
-    const void* ops0;     // MFMA: coefficient panels; direct isotropic: kT
-    const void* ops1;     // MFMA: wavevector stream;  direct isotropic: pT
-    const void* ops2;     //                           direct isotropic: aT
+    const void* ops0;     // MFMA: coefficient panels; direct isotropic: kA
+    const void* ops1;     // MFMA: wavevector stream;  direct isotropic: aA
+    double kMax;          //                           direct isotropic: max |k component|, revolutions
     int64_t tile0;        // first tile of the field
     int64_t nSteps;       // MFMA K-steps (multiple of 4)
     int32_t mtTotal;      // MFMA M-tiles of the panels
-    int32_t Rpad;         // direct isotropic: padded realizations (multiple of 16)
     float outScale;       // MFMA: 1 / panel scale
-    int32_t pad;
 };
 constexpr int kGroupMT = 4;       // M-tiles per tile, grouped MFMA kernel
 constexpr int kGroupW = 8;        // waves per block, grouped MFMA kernel (256 points)
-constexpr int kGroupIsoPts = 256; // points per tile, grouped direct isotropic kernel
-constexpr int kGroupIsoR = 16;    // realizations per tile, grouped direct isotropic kernel
+constexpr int kGroupIsoPts = 128; // points per tile, direct isotropic kernels
 // tiles of one field
 inline int64_t rf_group_tiles_mfma(int64_t N, int mtTotal, int waves, int mtBlock) {
     return (N + 32 * waves - 1) / (32 * waves) * ((mtTotal + mtBlock - 1) / mtBlock);
 }
-inline int64_t rf_group_tiles_iso(int64_t N, int Rpad) {
-    return (N + kGroupIsoPts - 1) / kGroupIsoPts * (Rpad / kGroupIsoR);
+inline int64_t rf_group_tiles_iso(int64_t N, int Nmc) {
+    return (N + kGroupIsoPts - 1) / kGroupIsoPts * ((Nmc + 15) / 16);
 }
 hipError_t rf_launch_group_mfma(int form, const rf_group_req* d_reqs, int nReq, int64_t nTiles,
                                 hipStream_t s);

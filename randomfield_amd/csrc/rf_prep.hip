@@ -138,27 +138,26 @@ __global__ __launch_bounds__(kBlock) void k_draw_prep(int64_t kN, int Nmc, int R
     }
 }
 
-// Isotropic FP32 operands: kT[j][r][D] = k_rj / (2 pi), pT[j][r] = psi_rj in
-// revolutions, aT[j][r] = amp_rj * ampMult; padded realizations are zero.
-__global__ void k_prep_fp32_iso(int nDim, int64_t kN, int Nmc, int Rpad,
+// Isotropic FP32 operands (rf_iso_rows): block (wavevector block jb, chunk) holds
+// rows = 16 / Rp wavevectors x Rp realizations; kA[block][0..3][row] = k / (2 pi)
+// and phi in revolutions, aA[block][row % 4][row / 4] = amp * ampMult; zero in
+// padded rows.
+__global__ void k_prep_fp32_iso(int nDim, int64_t kN, int Nmc, rf_iso_shape sh,
                                 const double* __restrict__ kIso, const double* __restrict__ phase,
                                 const double* __restrict__ amp, double ampMult,
-                                double* __restrict__ kT, float* __restrict__ pT,
-                                float* __restrict__ aT) {
+                                double* __restrict__ kA, float* __restrict__ aA) {
     const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (e >= kN * Rpad) return;
-    const int64_t j = e / Rpad;
-    const int r = (int)(e - j * Rpad);
-    if (r < Nmc) {
-        const int64_t s = (int64_t)r * kN + j;
-        for (int d = 0; d < nDim; d++) kT[e * nDim + d] = kIso[s * nDim + d] * RF_INV_TWO_PI;
-        pT[e] = (float)to_rev(phase[s]);
-        aT[e] = (float)(amp[s] * ampMult);
-    } else {
-        for (int d = 0; d < nDim; d++) kT[e * nDim + d] = 0.0;
-        pT[e] = 0.0f;
-        aT[e] = 0.0f;
-    }
+    if (e >= sh.nJ * sh.nChunk * 16) return;
+    const int row = (int)(e & 15);
+    const int64_t blk = e >> 4;
+    const int64_t j = blk / sh.nChunk * (16 / sh.Rp) + row / sh.Rp;
+    const int r = (int)(blk % sh.nChunk) * 16 + row % sh.Rp;
+    const bool in = r < Nmc && j < kN;
+    const int64_t s = (int64_t)r * kN + j;
+    double* k = kA + blk * 64 + row;
+    for (int d = 0; d < 3; d++) k[16 * d] = in && d < nDim ? kIso[s * nDim + d] * RF_INV_TWO_PI : 0.0;
+    k[48] = in ? to_rev(phase[s]) : 0.0;
+    aA[blk * 16 + (row & 3) * 4 + (row >> 2)] = in ? (float)(amp[s] * ampMult) : 0.0f;
 }
 
 // cos(2 pi U) for U in [0, 1) in FP32: cospi of the FP32 part Uh with the
@@ -276,12 +275,12 @@ hipError_t rf_launch_krev(int64_t count, const double* d_k, double* d_kRev, hipS
     return hipGetLastError();
 }
 
-hipError_t rf_launch_prep_fp32_iso(int nDim, int64_t kN, int Nmc, int Rpad, const double* d_kIso,
-                                   const double* d_phase, const double* d_amp, double ampMult,
-                                   double* d_kT, float* d_pT, float* d_aT, hipStream_t s) {
-    const int64_t n = kN * Rpad;
-    hipLaunchKernelGGL(k_prep_fp32_iso, dim3(grid_for(n)), dim3(kBlock), 0, s, nDim, kN, Nmc, Rpad,
-                       d_kIso, d_phase, d_amp, ampMult, d_kT, d_pT, d_aT);
+hipError_t rf_launch_prep_fp32_iso(int nDim, int64_t kN, int Nmc, const double* d_kIso, const double* d_phase,
+                                   const double* d_amp, double ampMult, double* d_kA, float* d_aA, hipStream_t s) {
+    const rf_iso_shape sh = rf_iso_rows(kN, Nmc);
+    const int64_t n = sh.nJ * sh.nChunk * 16;
+    hipLaunchKernelGGL(k_prep_fp32_iso, dim3(grid_for(n)), dim3(kBlock), 0, s, nDim, kN, Nmc, sh, d_kIso, d_phase, d_amp,
+                       ampMult, d_kA, d_aA);
     return hipGetLastError();
 }
 

@@ -44,6 +44,7 @@ struct Lattice {
     double* d_Sk = nullptr;   // method 1: spectral density [kN]
     double* d_amp = nullptr;  // method 2: sqrt(Sk) [kN] (one row for every realization)
     int64_t kNpad = 0;
+    double kMax = 0.0;                // max |k component|, revolutions
     double bScale = 1.0;      // method 2: panel scale
     bool lat = false;         // method 2: product form of the lattice
     rf_lat_dev latD{};
@@ -115,12 +116,13 @@ struct rf_server {
                                : 2 * align256((size_t)Nmc * kN * sizeof(double)) +   // uniforms, phases
                                      align256(rf_mfma_bbytes(cfg.form, l.kNpad, q.Rpad));
         } else {
-            q.Rpad = (Nmc + kGroupIsoR - 1) / kGroupIsoR * kGroupIsoR;
+            q.Rpad = 0;
+            const int64_t nb = rf_iso_blocks(kN, Nmc);
             q.bytesScr = align256((size_t)Nmc * 4 * kN * 8)        // uniforms
                          + align256((size_t)Nmc * kN * 3 * 8)      // directions
                          + 2 * align256((size_t)Nmc * kN * 8)      // amp, phase
-                         + align256((size_t)kN * q.Rpad * 3 * 8)   // kT
-                         + 2 * align256((size_t)kN * q.Rpad * 4);  // pT, aT
+                         + align256((size_t)nb * 64 * 8)           // kA
+                         + align256((size_t)nb * 16 * 4);          // aA
         }
     }
 
@@ -237,22 +239,18 @@ int rf_server::launch(Slot& sl, const std::vector<Req*>& batch, std::string& err
             p += align256((size_t)nU * 8);
             double* d_phase = reinterpret_cast<double*>(p);
             p += align256((size_t)nU * 8);
-            double* d_kT = reinterpret_cast<double*>(p);
-            p += align256((size_t)kN * q->Rpad * 3 * 8);
-            float* d_pT = reinterpret_cast<float*>(p);
-            p += align256((size_t)kN * q->Rpad * 4);
-            float* d_aT = reinterpret_cast<float*>(p);
+            double* d_kA = reinterpret_cast<double*>(p);
+            p += align256((size_t)rf_iso_blocks(kN, r.Nmc) * 64 * 8);
+            float* d_aA = reinterpret_cast<float*>(p);
             SRV_TRY(rf_launch_uniforms(r.seed, 2u, (int64_t)r.Nmc * 4 * kN, d_u, s));
             SRV_TRY(rf_launch_iso_prep(3, RF_FIXED, 0, kN, r.Nmc, l.d_k, l.d_Sk, d_u, d_ones, d_kIso, d_amp,
                                        d_phase, s));
-            SRV_TRY(rf_launch_prep_fp32_iso(3, kN, r.Nmc, q->Rpad, d_kIso, d_phase, d_amp, l.info.ampMult, d_kT,
-                                            d_pT, d_aT, s));
-            g.ops0 = d_kT;
-            g.ops1 = d_pT;
-            g.ops2 = d_aT;
-            g.Rpad = q->Rpad;
+            SRV_TRY(rf_launch_prep_fp32_iso(3, kN, r.Nmc, d_kIso, d_phase, d_amp, l.info.ampMult, d_kA, d_aA, s));
+            g.ops0 = d_kA;
+            g.ops1 = d_aA;
+            g.kMax = l.kMax;
             g.tile0 = tilesI;
-            tilesI += rf_group_tiles_iso(r.N, q->Rpad);
+            tilesI += rf_group_tiles_iso(r.N, r.Nmc);
             sl.h_table[maxB + nI++] = g;
         }
     }
@@ -403,6 +401,7 @@ int build_lattice(rf_server* S, int method, Lattice& l) {
     rc = rf_spectrum_build_tables(&p, l.info, nullptr, &spec, &err);
     if (rc) return rf_set_error(ctx, rc, err);
     const int64_t kN = l.info.kNTotal;
+    for (double v : spec.k) l.kMax = std::max(l.kMax, std::fabs(v) * RF_INV_TWO_PI);
     const hipStream_t s = ctx->stream;
     if (method == RF_SHINOZUKA) {
         l.kNpad = (kN + rf_mfma_kpad(p.form) - 1) / rf_mfma_kpad(p.form) * rf_mfma_kpad(p.form);
@@ -555,7 +554,7 @@ int rf_server_submit(rf_server* S, const rf_request* r, int64_t* id) {
     S->sizes(q);
     if (q.bytesOut + q.bytesX + q.bytesScr > S->arena.capacity())
         return rf_set_error(S->ctx, RF_E_NOMEM, "request exceeds the server's memory budget");
-    if (S->tilesOf(r->N, q.Rpad / 32) > 0x7fffffffLL || rf_group_tiles_iso(r->N, q.Rpad) > 0x7fffffffLL)
+    if (S->tilesOf(r->N, q.Rpad / 32) > 0x7fffffffLL || rf_group_tiles_iso(r->N, r->Nmc) > 0x7fffffffLL)
         return rf_set_error(S->ctx, RF_E_ARG, "request too large for one grouped launch");
     q.tSubmit = now_s();
     {

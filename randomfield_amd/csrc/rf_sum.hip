@@ -11,6 +11,7 @@
 //    one FP32 add, one hardware cosine (v_cos_f32 takes revolutions) and one
 //    FMA.  Wavevector, phase and amplitude operands are wave-uniform and come
 //    through scalar loads, so the inner loop is pure VALU/transcendental work.
+//    With per-realization directions the arguments come from the FP64 matrix cores.
 #include "rf_internal.h"
 
 namespace {
@@ -223,64 +224,103 @@ __global__ __launch_bounds__(kBlock) void k_sum_fp32(rf_sum_args a, const double
     }
 }
 
-// FP32 form of the isotropic sum with per-realization directions: the
-// argument cannot be shared across realizations, so each term forms its own
-// FP64 k.x.  kT[j][r][D] in revolutions, aT/pT[j][r] as in k_sum_fp32.
-// Padded realizations of a chunk (zero amplitude) are computed and not stored:
-// a per-realization exit would serialize the chunk's scalar loads and
-// transcendentals (measured slower on the cfg 5 stream).
-// Global-address-space views of the direction / phase / amplitude streams:
-// their reads are uniform across a wave, and only through such pointers (as
-// kernel arguments are, but not pointers read from a request record) does
-// the compiler issue them as batched scalar loads rather than one flat
-// vector load and wait per realization.
+// FP32 form of the isotropic sum with per-realization directions: no argument
+// is shared between realizations, so every term forms its own FP64 k.x + phi --
+// on the FP64 matrix cores.  A row of v_mfma_f64_16x16x4_f64's A operand is one
+// (wavevector, realization): (kx, ky, kz, phi) in revolutions; a column of B is one
+// point: (x, y, z, 1).  The 16 rows are 16 / Rp wavevectors x Rp realizations, Rp
+// the power of two (at most 16) that holds Nmc; larger Nmc in chunks of 16.
+// The accumulator starts at 1.5 2^20 + 2^-24, whose last place is 2^-32: the
+// low word of D is then the argument modulo one revolution, and one v_alignbit
+// makes it the float 1 + argument (23 bits, rounded by the 2^-24) that v_cos_f32
+// takes.  A term costs three VALU instructions (alignbit, cosine, FMA), the
+// matrix cores run beside them.  Formerly eight, four of them FP64 (k.x by FMAs,
+// v_fract_f64): 200,000 points x 16 realizations ISOFIGS
+// Arguments that may reach 2^19 revolutions (or are not finite) take a zero
+// accumulator and v_fract_f64; the choice is per wave.
+// kA [block][4][16], aA [block][row % 4][row / 4], block = wavevector block x chunks
+// + chunk; padded rows have zero amplitude.  Two groups of 16 points per wave:
+// four waves of 32 points spread 20,000 points over the CUs more evenly than 64 would.
+typedef double d4v __attribute__((ext_vector_type(4)));
 typedef const double __attribute__((address_space(1))) gdbl;
-typedef const float __attribute__((address_space(1))) gflt;
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef const f4v __attribute__((address_space(1))) gf4;
+constexpr int kIsoQ = 2;                               // 16-point groups of a wave
+static_assert(kGroupIsoPts == kBlock / 64 * 16 * kIsoQ, "points of a block");
 
-template <int D, int R>
-__device__ __forceinline__ void sum_fp32_iso_point(const rf_sum_args& a, gdbl* __restrict__ kT,
-                                                   gflt* __restrict__ pT,
-                                                   gflt* __restrict__ aT, int Rpad, int64_t i,
-                                                   int r0) {
-    double xn[D];
+__device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict__ kA, gf4* __restrict__ aA, int64_t nJ,
+                                          int nChunk, int chunk, int Rp, double kMax, int64_t p0, float (*red)[16 * kIsoQ]) {
+    constexpr int Q = kIsoQ, P = 16 * Q;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+    const int64_t pw = p0 + wave * P;
+    double b[Q];
+    bool far = false;
 #pragma unroll
-    for (int d = 0; d < D; d++) xn[d] = a.x[i * D + d] / a.corrL[d];
-    float acc[R];
+    for (int q = 0; q < Q; q++) {
+        const int64_t i = pw + 16 * q + c, ic = i < a.i1 ? i : a.i1 - 1;
+        b[q] = g == 3 ? 1.0 : g < a.nDim ? a.x[ic * a.nDim + g] / a.corrL[g] : 0.0;
+        far |= !(3.0 * kMax * fabs(b[q]) + 1.0 < 524288.0);
+    }
+    float acc[Q][4];
 #pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = 0.0f;
-    for (int64_t j = 0; j < a.kN; j++) {
-        gdbl* kj = kT + (j * Rpad + r0) * D;
-        gflt* pj = pT + j * Rpad + r0;
-        gflt* aj = aT + j * Rpad + r0;
+    for (int q = 0; q < Q; q++)
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            double t = kj[r * D] * xn[0];
+        for (int e = 0; e < 4; e++) acc[q][e] = 0.0f;
+    auto sweep = [&](double c0, auto turn) {
+        const d4v C = {c0, c0, c0, c0};
+        gdbl* kp = kA + (int64_t)chunk * 64 + lane;
+        gf4* ap = aA + (int64_t)chunk * 4 + g;
+        double kn = *kp;
+        f4v an = *ap;
+        for (int64_t j = 0; j < nJ; j++) {
+            const double kj = kn;
+            const f4v aj = an;
+            if (j + 1 < nJ) {                          // one block ahead
+                kp += nChunk * 64;
+                ap += nChunk * 4;
+                kn = *kp;
+                an = *ap;
+            }
 #pragma unroll
-            for (int d = 1; d < D; d++) t = fma(kj[r * D + d], xn[d], t);
-            t = __builtin_amdgcn_fract(t);   // k.x mod 1 revolution: one v_fract_f64, exact
-            acc[r] = fmaf(aj[r], __builtin_amdgcn_cosf((float)t + pj[r]), acc[r]);
+            for (int q = 0; q < Q; q++) {
+                const d4v t = __builtin_amdgcn_mfma_f64_16x16x4f64(kj, b[q], C, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[q][e] = fmaf(aj[e], __builtin_amdgcn_cosf(turn(t[e])), acc[q][e]);
+            }
         }
-    }
+    };
+    if (!__any(far))
+        sweep(1572864.0 + 0x1p-24, [](double t) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_alignbit(0x7Fu, (unsigned)__builtin_bit_cast(uint64_t, t), 9));
+        });
+    else
+        sweep(0.0, [](double t) { return (float)__builtin_amdgcn_fract(t); });
+    // D: column c, rows 4 e + g; the wavevectors of a block added in row order
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        if (r0 + r < a.Nmc)
-            store_out(a.out, (int64_t)(r0 + r) * a.N + i, epilogue32(acc[r], a.epi), a.outDtype);
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) red[wave * 16 + 4 * e + g][16 * q + c] = acc[q][e];
+    __syncthreads();
+    for (int idx = lane; idx < Rp * P; idx += 64) {
+        const int r = idx / P, p = idx % P, R = chunk * 16 + r;
+        if (R >= a.Nmc || pw + p >= a.i1) continue;
+        float s = 0.0f;
+        for (int row = r; row < 16; row += Rp) s += red[wave * 16 + row][p];
+        store_out(a.out, (int64_t)R * a.N + pw + p, epilogue32(s, a.epi), a.outDtype);
     }
 }
 
-template <int D, int R>
-__global__ __launch_bounds__(kBlock) void k_sum_fp32_iso(rf_sum_args a, const double* __restrict__ kT,
-                                                         const float* __restrict__ pT,
-                                                         const float* __restrict__ aT, int Rpad) {
-    const int64_t i = a.i0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= a.i1) return;
-    sum_fp32_iso_point<D, R>(a, (gdbl*)kT, (gflt*)pT, (gflt*)aT, Rpad, i, blockIdx.y * R);
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_sum_fp32_iso(rf_sum_args a, const double* __restrict__ kA,
+                                                         const float* __restrict__ aA, int64_t nJ, int Rp, double kMax) {
+    __shared__ float red[kBlock / 64 * 16][16 * kIsoQ];
+    iso_block(a, (gdbl*)kA, (gf4*)aA, nJ, gridDim.y, blockIdx.y, Rp, kMax, a.i0 + (int64_t)blockIdx.x * kGroupIsoPts, red);
 }
 
-// Grouped form: block b runs one tile = (field, block of kGroupIsoPts points,
-// chunk of kGroupIsoR realizations), found by binary search over the fields'
-// first tiles; same per-point operation order as k_sum_fp32_iso.
-__global__ __launch_bounds__(kBlock) void k_group_iso(const rf_group_req* __restrict__ reqs, int nReq) {
+// Grouped form: block b runs one tile = (field, kGroupIsoPts points, chunk of
+// 16 realizations), found by binary search over the fields' first tiles; same
+// per-point operation order as k_sum_fp32_iso.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_group_iso(const rf_group_req* __restrict__ reqs, int nReq) {
+    __shared__ float red[kBlock / 64 * 16][16 * kIsoQ];
     const int64_t b = blockIdx.x;
     int lo = 0, hi = nReq - 1;
     while (lo < hi) {
@@ -289,12 +329,10 @@ __global__ __launch_bounds__(kBlock) void k_group_iso(const rf_group_req* __rest
         else hi = mid - 1;
     }
     const rf_group_req& q = reqs[lo];
-    const int nChunk = q.Rpad / kGroupIsoR;
+    const rf_iso_shape sh = rf_iso_rows(q.a.kN, q.a.Nmc);
     const int64_t local = b - q.tile0;
-    const int64_t i = (local / nChunk) * kGroupIsoPts + threadIdx.x;
-    if (i >= q.a.N) return;
-    sum_fp32_iso_point<3, kGroupIsoR>(q.a, (gdbl*)q.ops0, (gflt*)q.ops1, (gflt*)q.ops2, q.Rpad, i,
-                                      (int)(local % nChunk) * kGroupIsoR);
+    iso_block(q.a, (gdbl*)q.ops0, (gf4*)q.ops1, sh.nJ, sh.nChunk, (int)(local % sh.nChunk), sh.Rp, q.kMax,
+              (local / sh.nChunk) * kGroupIsoPts, red);
 }
 
 template <int D, int R, bool ISO>
@@ -376,22 +414,20 @@ hipError_t rf_launch_sum_fp32(const rf_sum_args& a, const double* d_kRev, const 
     return hipGetLastError();
 }
 
-hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kT, const float* d_pT,
-                                    const float* d_aT, int Rpad, hipStream_t s) {
+hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kA, const float* d_aA, double kMax,
+                                    hipStream_t s) {
     if (a.i1 <= a.i0) return hipSuccess;
-    const int64_t n = a.i1 - a.i0;
-    dim3 grid((unsigned)((n + kBlock - 1) / kBlock), (unsigned)(Rpad / kRChunk));
-    if (a.nDim == 2)
-        hipLaunchKernelGGL((k_sum_fp32_iso<2, kRChunk>), grid, dim3(kBlock), 0, s, a, d_kT, d_pT, d_aT, Rpad);
-    else
-        hipLaunchKernelGGL((k_sum_fp32_iso<3, kRChunk>), grid, dim3(kBlock), 0, s, a, d_kT, d_pT, d_aT, Rpad);
+    const rf_iso_shape sh = rf_iso_rows(a.kN, a.Nmc);
+    const int64_t blocks = (a.i1 - a.i0 + kGroupIsoPts - 1) / kGroupIsoPts;
+    if (blocks > 0x7fffffffLL || sh.nChunk > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_sum_fp32_iso, dim3((unsigned)blocks, (unsigned)sh.nChunk), dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ,
+                       sh.Rp, kMax);
     return hipGetLastError();
 }
 
 int rf_fp32_rchunk() { return kRChunk; }
 
 hipError_t rf_launch_group_iso(const rf_group_req* d_reqs, int nReq, int64_t nTiles, hipStream_t s) {
-    static_assert(kGroupIsoPts == kBlock, "one thread per point");
     if (nTiles <= 0 || nReq <= 0) return hipSuccess;
     if (nTiles > 0x7fffffffLL) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_group_iso, dim3((unsigned)nTiles), dim3(kBlock), 0, s, d_reqs, nReq);
