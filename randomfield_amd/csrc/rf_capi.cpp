@@ -36,6 +36,15 @@ bool is_iso_direct(const rf_params& p) { return p.method == RF_ISOTROPIC && !p.i
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
+// Whether a matrix-core execution of N points takes the product form of the
+// lattice.  It does but for large fields of many realizations, where up to eight
+// realization tiles share each basis value of the general form: 171,011 points x
+// 161 realizations BF16 4198 us against 3788 (x 128: 1495 against 1807; 200,000 x 40
+// F16: 1364 against 3190; 5,000 x 256: 225 against 991, its K-steps split over the
+// waves).  In 2-D, where the per-axis sines weigh against few wavevectors, from 65
+// realizations: 300,000 x 100 176 against 141, 500,000 x 64 151 against 165.
+bool use_lat(const rf_field_plan* P, int64_t N) { return P->lat && !(P->d_Bw && N > kLatSmallN); }
+
 // Form-specific operand build from d_phase / d_amp (Nmc x kN, FP64).
 int build_form_operands(rf_field_plan* P, hipStream_t s) {
     rf_context* ctx = P->ctx;
@@ -55,6 +64,9 @@ int build_form_operands(rf_field_plan* P, hipStream_t s) {
     } else if (P->lat) {
         RF_HIP_TRY(ctx, rf_launch_lat_prep(P->p.form, P->p.nDim, P->latD, Nmc, P->Rpad, P->d_phase, 0, P->d_amp, kN,
                                            ampMult * P->bScale, P->d_B, s));
+        if (P->d_Bw)
+            RF_HIP_TRY(ctx, rf_launch_mfma_prep(P->p.form, P->p.nDim, kN, P->kNpad, Nmc, P->Rpad, P->d_kRev, P->d_phase,
+                                                P->d_amp, kN, ampMult * P->bwScale, P->d_Bw, s));
     } else if (P->p.form == RF_FORM_MFMA_F16 || P->p.form == RF_FORM_MFMA_BF16) {
         RF_HIP_TRY(ctx, rf_launch_mfma_prep(P->p.form, P->p.nDim, kN, P->kNpad, Nmc, P->Rpad,
                                             P->d_kRev, P->d_phase, P->d_amp, kN, ampMult * P->bScale,
@@ -170,7 +182,7 @@ int rf_plan_destroy(rf_field_plan* P) {
     }
     dfree(P->d_k); dfree(P->d_kRad); dfree(P->d_kRev); dfree(P->d_kIso); dfree(P->d_kIsoT);
     dfree(P->d_phase); dfree(P->d_amp); dfree(P->d_uni); dfree(P->d_phT);
-    dfree(P->d_aT); dfree(P->d_B); dfree(P->d_CS); dfree(P->d_Sk); dfree(P->d_calc); dfree(P->d_gridScratch);
+    dfree(P->d_aT); dfree(P->d_B); dfree(P->d_Bw); dfree(P->d_CS); dfree(P->d_Sk); dfree(P->d_calc); dfree(P->d_gridScratch);
     if (P->d_gridCoef) (void)hipFree(P->d_gridCoef);
     delete P;
     return RF_OK;
@@ -315,7 +327,8 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
     // sign block as zero wavevectors)
     P->lat = mfma && p->method == RF_SHINOZUKA && p->mode == RF_FIXED &&
              rf_lat_describe(d, info.kNStep, info.kDelta, &P->latD);
-    if (p->form != RF_FORM_FP64 && !is_iso_direct(*p) && !P->lat) {
+    const bool both = P->lat && P->Rpad > (d == 3 ? 128 : 64);   // the general form's operands too (use_lat)
+    if (p->form != RF_FORM_FP64 && !is_iso_direct(*p) && (!P->lat || both)) {
         // the MFMA form reads whole K-steps: zero wavevectors pad the tail
         RF_HIP_TRY(ctx, dmalloc(&P->d_kRev, (size_t)(P->kNpad * d)));
         if (P->kNpad > kN)
@@ -328,6 +341,10 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
         P->bScale = rf_mfma_bscale(P->spec.info.ampMult, P->lat ? 4.0 * maxAmp : maxAmp);
         RF_HIP_TRY(ctx, hipMalloc(&P->d_B, P->lat ? rf_lat_bbytes(P->latD, P->Rpad)
                                                   : rf_mfma_bbytes(p->form, P->kNpad, P->Rpad)));
+        if (both) {
+            P->bwScale = rf_mfma_bscale(P->spec.info.ampMult, maxAmp);
+            RF_HIP_TRY(ctx, hipMalloc(&P->d_Bw, rf_mfma_bbytes(p->form, P->kNpad, P->Rpad)));
+        }
     }
     const bool perSlab = (p->mode == RF_REF_COMPAT && p->method != RF_ISOTROPIC);
     if (!perSlab) {
@@ -388,7 +405,9 @@ int rf_plan_execute(rf_field_plan* P, const double* d_x, int64_t N, void* d_out,
                 else e = rf_launch_sum_fp32(a, P->d_kRev, P->d_phT, P->d_aT, P->Rpad, s);
                 break;
             default:
-                if (P->lat) e = rf_launch_sum_lat(p.form, a, P->latD, P->Rpad, P->d_B, 1.0 / P->bScale, s);
+                if (use_lat(P, N)) e = rf_launch_sum_lat(p.form, a, P->latD, P->Rpad, P->d_B, 1.0 / P->bScale, s);
+                else if (P->lat)
+                    e = rf_launch_sum_mfma(p.form, P->mfmaVariant, a, P->kNpad, P->Rpad, P->d_Bw, 1.0 / P->bwScale, s);
                 else e = rf_launch_sum_mfma(p.form, P->mfmaVariant, a, P->kNpad, P->Rpad, P->d_B, 1.0 / P->bScale, s);
                 break;
         }
@@ -590,7 +609,7 @@ int rf_plan_autotune(rf_field_plan* P, const double* d_x, int64_t N, void* d_out
     }
     RF_HIP_TRY(ctx, hipSetDevice(ctx->device));
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    if (P->lat) {                               // one launch shape; the field is formed as ever
+    if (use_lat(P, N)) {                        // one launch shape; the field is formed as ever
         const int rc = rf_plan_execute(P, d_x, N, d_out, outDtype, s);
         if (rc) return rc;
         RF_HIP_TRY(ctx, hipStreamSynchronize(s));

@@ -206,6 +206,7 @@ struct rf_field_plan {
     float* d_phT = nullptr;      // kN x Rpad   FP32 phase in revolutions
     float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult
     void* d_B = nullptr;         // MFMA coefficient panels (hi, lo)
+    void* d_Bw = nullptr;        // the general form's panels beside the product form's (many realizations)
     bool lat = false;            // MFMA forms: product form of the lattice (rf_lat.hip)
     rf_lat_dev latD{};
     double2* d_CS = nullptr;     // FP64 form: (amp cos phase, -amp sin phase)
@@ -213,6 +214,7 @@ struct rf_field_plan {
     int Rpad = 0;
     int64_t kNpad = 0;
     double bScale = 1.0;         // power-of-two scale folded into B
+    double bwScale = 1.0;        // the same of d_Bw
     double ampMax = 1.0;         // bound of |amp| over all realizations
     // REF_COMPAT: sqrt chain of Sk, row c = Sk^(2^-(c+1)), until it saturates
     std::vector<std::vector<double>> sqrtChain;

@@ -437,7 +437,7 @@ typedef __attribute__((address_space(3))) void interp_lds;
 // 1.2 times).  Two blocks of 1024 per CU (64 VGPRs) share more of the planes
 // in their XCD's L2 than one: 500 us with the next realization held in
 // registers; chunks of realizations repeat the set-up: 8 +20 %, 4 +60 %.
-constexpr int interp_k(int NT) { return NT == 1024 ? 12 : 24; }
+constexpr int interp_k(int NT, int size) { return NT == 256 && size == 4 ? 24 : 12; }
 
 template <typename TG, typename TO, int D, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(TG) == 4 ? 8 : 4))) void k_interp(rf_interp_dev q, const TG* __restrict__ grid,
@@ -445,7 +445,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(TG) =
                                                int* __restrict__ flag, int64_t nBlocks, int RC) {
 #pragma clang fp contract(off)
     constexpr int kX = 8;                          // XCDs, blocks dealt round them
-    constexpr int K = interp_k(NT);
+    constexpr int K = interp_k(NT, sizeof(TG));
     __shared__ TG box[K * NT];
     __shared__ int lim[6];
     const int64_t per = (nBlocks + kX - 1) / kX;
@@ -1068,7 +1068,11 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
     // and weights formed once) where that still gives every CU two; else 256
     // nodes and 4 realizations
     const bool wide = nNodes >= 512 * 1024;
-    const int NT = wide ? 1024 : 256, RC = wide ? Nmc : 4;
+    // (FP64 grids: 512, whose box leaves room for two blocks per CU; 136 x 35 x 101,
+    // 3.6M nodes, 8 realizations: 253 us in blocks of 1024, 215 in 512)
+    const int RC = wide ? Nmc : 4;
+    const bool g64 = gridDtype == RF_DTYPE_F64, o64 = outDtype == RF_DTYPE_F64;
+    const int NT = !wide ? 256 : g64 ? 512 : 1024;
     const int64_t nBlocks = (nNodes + NT - 1) / NT;
     if (nBlocks > 0x7ffffff8LL) return hipErrorInvalidValue;
     const dim3 grid2((unsigned)((nBlocks + 7) / 8 * 8), (unsigned)((Nmc + RC - 1) / RC));
@@ -1076,8 +1080,8 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
     auto run = [&](auto dim, auto* g, auto* o) {
         typedef std::remove_const_t<std::remove_pointer_t<decltype(g)>> TG;
         typedef std::remove_pointer_t<decltype(o)> TO;
-        constexpr int D = decltype(dim)::value;
-        if (wide) hipLaunchKernelGGL((k_interp<TG, TO, D, 1024>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
+        constexpr int D = decltype(dim)::value, NW = sizeof(TG) == 8 ? 512 : 1024;
+        if (wide) hipLaunchKernelGGL((k_interp<TG, TO, D, NW>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
         else hipLaunchKernelGGL((k_interp<TG, TO, D, 256>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
     };
     auto go = [&](auto* g, auto* o) {
@@ -1085,7 +1089,6 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
         else if (nDim == 2) run(std::integral_constant<int, 2>(), g, o);
         else run(std::integral_constant<int, 1>(), g, o);
     };
-    const bool g64 = gridDtype == RF_DTYPE_F64, o64 = outDtype == RF_DTYPE_F64;
     if (g64 && o64) go(static_cast<const double*>(grid), static_cast<double*>(out));
     else if (g64) go(static_cast<const double*>(grid), static_cast<float*>(out));
     else if (o64) go(static_cast<const float*>(grid), static_cast<double*>(out));

@@ -68,3 +68,11 @@ def test_wide_lattices(ctx, xr, N):
 @pytest.mark.parametrize("margi", [R.FOM_GAUSSIAN, R.FOM_LOGNORMAL])
 def test_marginals(ctx, dtype, margi):
     assert _run(ctx, R.FORM_MFMA_F16, (3.1, 2.2, 3.9), 200, 6, dtype=dtype, margi=margi) <= TOL[R.FORM_MFMA_F16]
+
+
+@pytest.mark.parametrize("xr,Nmc", [((2.2, 1.5, 2.2), 129), ((3.1, 3.9), 65)])
+@pytest.mark.parametrize("N", [32768, 32769])
+def test_many_realizations(ctx, xr, N, Nmc):
+    """Small fields keep the product form, larger ones of many realizations take
+    the general form (its tolerance: hardware sines, one-level FP32 sums)."""
+    assert _run(ctx, R.FORM_MFMA_F16, xr, N, Nmc, sample=100) <= 1e-5
