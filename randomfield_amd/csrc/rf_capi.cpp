@@ -578,8 +578,8 @@ int rf_plan_redraw(rf_field_plan* P, int64_t drawIndex, void* stream) {
     }
     if (p.method != RF_ISOTROPIC) {
         const bool ops = P->coeffsReady && p.form == RF_FORM_FP32;
-        RF_HIP_TRY(ctx, rf_launch_draw_prep(kN, p.Nmc, P->Rpad, p.seed, first, P->d_amp, P->spec.info.ampMult, P->d_uni,
-                                            P->d_phase, ops ? P->d_phT : nullptr, ops ? P->d_aT : nullptr, s));
+        RF_HIP_TRY(ctx, rf_launch_draw_prep(kN, p.Nmc, P->Rpad, p.seed, first, P->d_uni, P->d_phase,
+                                            ops ? P->d_phT : nullptr, s));
         if (P->coeffsReady && !ops) {
             const int rc = build_form_operands(P, s);
             if (rc) return rc;
@@ -763,7 +763,7 @@ int rf_plan_execute_grid(rf_field_plan* P, const double* origin, const double* s
         ampMult = (p.nDim == 3 ? 2.0 : 1.0) * std::sqrt(v);
     }
     rf_grid_stages st;
-    if (!P->d_gridCoef) {
+    if (!P->d_gridCoef && !fft) {
         int64_t nC = (int64_t)in.nSignBlocks * p.Nmc;
         for (int a = 0; a < p.nDim; a++) nC *= in.kNStep[a];
         RF_HIP_TRY(ctx, hipMalloc((void**)&P->d_gridCoef, (size_t)nC * sizeof(float2)));

@@ -771,6 +771,11 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
     const int64_t nb = xcd_blocks(nTiles);
     if (nb > 0x7fffffffLL || mt < 0 || mt > kStripMaxMT) return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)nb;
+    if (mt > 0 && g && g->real) {
+        if (kind == RF_GEMM_FIRST) return rf_strip_launch_first_real(mt, g, d_gs, nG, nTiles, blocks, s);
+        if (kind == RF_GEMM_MIDDLE) return rf_strip_launch_middle_real(mt, g, d_gs, nG, nTiles, blocks, s);
+        return rf_strip_launch_last_real(mt, g, d_gs, nG, nTiles, blocks, s);
+    }
     if (mt > 0) {
         if (kind == RF_GEMM_FIRST) return rf_strip_launch_first(mt, g, d_gs, nG, nTiles, blocks, s);
         if (kind == RF_GEMM_MIDDLE) return rf_strip_launch_middle(mt, g, d_gs, nG, nTiles, blocks, s);
@@ -898,11 +903,14 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
     const int64_t nC = (int64_t)Nmc * nb * kNu;          // = Nmc x nk3 x Q x nk2 x H x nk1
     float2* Cf = p; p += nC;
     // a caller-owned coefficient buffer is reused while its scale matches
-    // (the coefficients depend only on the plan and the scale)
-    bool fresh = false;
-    if (coef) {
+    // (the coefficients depend only on the plan and the scale).  Method 4 of a
+    // plan: its real amplitudes go into the first contraction as they are (no
+    // fold, 50 us of 128^3 x 8), on real operands throughout
+    const bool real = coef && split && kind == 1;
+    bool fresh = real;
+    if (coef && coef->buf) {
         Cf = coef->buf;
-        fresh = coef->key == ampMult * sc;
+        fresh = fresh || coef->key == ampMult * sc;
         coef->key = ampMult * sc;
     }
     *st = rf_grid_stages{};
@@ -946,6 +954,12 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
         g.M = (int)rows1; g.N = n[0];
     }
     g.K = K1; g.batches = 1;
+    g.gen = fd;
+    if (real) {
+        // lines (r, j3, j2) of the amplitudes, k contiguous (no sign blocks)
+        g.B = reinterpret_cast<const float2*>(d_amp);
+        g.bSk = 1; g.bSn = kNStep[0];
+    }
     g.outScale = 1.0f;
     const float2* last = V;
     int64_t plane = n[0];                      // points already resolved
@@ -976,7 +990,10 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
     f.N = (int)plane; f.K = kNStep[ad]; f.batches = Nmc;
     f.outDtype = outDtype; f.epi = epi;
     f.outScale = (float)(1.0 / (sc * std::ldexp(1.0, -m2)));
-    for (int i = 0; i < st->n; i++) st->g[i].mt = split ? strip_choose(st->g[i]) : 0;
+    for (int i = 0; i < st->n; i++) {
+        st->g[i].mt = split ? strip_choose(st->g[i]) : 0;
+        st->g[i].real = real;
+    }
     return hipGetLastError();
 }
 

@@ -80,10 +80,9 @@ hipError_t rf_launch_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* d_ph
                                const double* d_amp, double ampMult, float* d_phT, float* d_aT,
                                hipStream_t s);
 // uniforms first + r kN + j of stream (seed, 2), their phases and, d_phT given,
-// rf_launch_prep_fp32's operands, in one launch
-hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, const double* d_amp,
-                               double ampMult, double* d_uni, double* d_phase, float* d_phT, float* d_aT,
-                               hipStream_t s);
+// rf_launch_prep_fp32's phases (not its amplitudes), in one launch
+hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, double* d_uni,
+                               double* d_phase, float* d_phT, hipStream_t s);
 hipError_t rf_launch_krev(int64_t count, const double* d_k, double* d_kRev, hipStream_t s);
 hipError_t rf_launch_fft_coeffs(int64_t kN, int Nmc, const double* d_Sk, const double* d_u,
                                 const uint8_t* d_calc, double* d_amp, double* d_phase, hipStream_t s);
@@ -337,6 +336,8 @@ struct rf_gemm_desc {
     uint64_t genSeed;
     int genNmc;
     const int64_t* genState;
+    int real;             // strips: real operands and intermediates (method 4; first contraction: B the FP64
+                          // amplitudes, scaled by gen.ampMult)
 };
 struct rf_grid_stages {
     rf_gemm_desc g[3];    // stage 1, stage 2 (3-D only), last stage (real)
@@ -408,12 +409,15 @@ hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s);
 int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt);
 hipError_t rf_launch_gemm_group(int kind, int mt, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, hipStream_t s);
 // strips of one kind (rf_strip.hip): one GEMM (g) or a group (d_gs, nG)
-hipError_t rf_strip_launch_first(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
-                                 unsigned blocks, hipStream_t s);
-hipError_t rf_strip_launch_middle(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
-                                  unsigned blocks, hipStream_t s);
-hipError_t rf_strip_launch_last(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n,
-                                unsigned blocks, hipStream_t s);
+#define RF_STRIP_DECL(NAME)                                                                              \
+    hipError_t NAME(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks, \
+                    hipStream_t s)
+RF_STRIP_DECL(rf_strip_launch_first);
+RF_STRIP_DECL(rf_strip_launch_middle);
+RF_STRIP_DECL(rf_strip_launch_last);
+RF_STRIP_DECL(rf_strip_launch_first_real);      // real operands, single GEMMs only
+RF_STRIP_DECL(rf_strip_launch_middle_real);
+RF_STRIP_DECL(rf_strip_launch_last_real);
 
 // post-processing (rf_post.hip)
 hipError_t rf_launch_marginal(int margi, double scale, double shift, void* d, int64_t count,

@@ -1,6 +1,8 @@
 // rf_prep.hip -- O(N_k * Nmc) coefficient preparation on the device: phases
 // from uniforms, the isotropic per-realization direction tables, and the
 // operand layouts of the FP32 direct-sum kernels.  All FP64.
+#include <algorithm>
+
 #include "rf_internal.h"
 #include "rf_philox.h"
 
@@ -103,20 +105,19 @@ __global__ void k_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* __restr
 
 // A plan's new realizations in one launch (methods 2 and 3): uniforms
 // first + r kN + j of stream (seed, tag 2) to uni[r][j], phases 2 pi U to
-// phase[r][j] and, phT given, the FP32 direct-sum operands of k_prep_fp32.  One
-// thread per wavevector: the uniforms and phases of a realization are written
-// along j, the Rpad operands of a wavevector as whole 64-byte pieces (bound by
-// those writes; three launches that read the phases back transposed took 27 us
-// for 332,928 wavevectors x 4 realizations, this one 21 us, 75 MB).
+// phase[r][j] and, phT given, the phases of the FP32 direct sum (k_prep_fp32; its
+// amplitudes and padding do not change between draws).  One thread per wavevector
+// and four realizations: the uniforms and phases of a realization are written
+// along j, the operands of a wavevector as 16-byte pieces.  332,928 wavevectors x 4
+// realizations: 10 us (with the amplitudes and padding rewritten 21, 75 MB).
 __global__ __launch_bounds__(kBlock) void k_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first,
-                                                      const double* __restrict__ amp, double ampMult,
                                                       double* __restrict__ uni, double* __restrict__ phase,
-                                                      float* __restrict__ phT, float* __restrict__ aT) {
+                                                      float* __restrict__ phT) {
 #pragma clang fp contract(off)
     const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (j >= kN) return;
-    for (int r0 = blockIdx.y * 16; r0 < Rpad && r0 < (int)(blockIdx.y + 1) * 16; r0 += 4) {
-        float4 p = make_float4(0.f, 0.f, 0.f, 0.f), a = p;
+    for (int r0 = blockIdx.y * 4; r0 < Nmc; r0 += gridDim.y * 4) {
+        float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int r = r0 + u;
@@ -126,15 +127,9 @@ __global__ __launch_bounds__(kBlock) void k_draw_prep(int64_t kN, int Nmc, int R
             const double ph = 2.0 * RF_PI_REF * U;
             uni[s] = U;
             phase[s] = ph;
-            if (phT) {
-                (&p.x)[u] = (float)to_rev(ph);
-                (&a.x)[u] = (float)(amp[s] * ampMult);
-            }
+            (&p.x)[u] = (float)to_rev(ph);
         }
-        if (phT) {
-            *reinterpret_cast<float4*>(phT + j * Rpad + r0) = p;
-            *reinterpret_cast<float4*>(aT + j * Rpad + r0) = a;
-        }
+        if (phT) *reinterpret_cast<float4*>(phT + j * Rpad + r0) = p;
     }
 }
 
@@ -193,23 +188,29 @@ __global__ void k_fft_coeffs(int64_t kN, int Nmc, const double* __restrict__ Sk,
 
 // The same coefficients with the uniforms drawn in place: element
 // first + r (3 kN - 1) + i of stream (seed, tag 2) is U[r][i] (the values
-// k_uniforms writes); the discarded third is never drawn.  Phase stays 0.
-__global__ void k_fft_coeffs_draw(int64_t kN, int Nmc, const double* __restrict__ Sk,
-                                  const uint8_t* __restrict__ calc, uint64_t seed, uint64_t first,
-                                  double* __restrict__ amp) {
+// k_uniforms writes); the discarded third is never drawn.  Phase stays 0.  Bound
+// by the two Philox evaluations per coefficient (VALU); a thread takes one
+// wavevector of up to kFftR realizations, whose square root they share.  128^3 x
+// 8 realizations 89 us (a thread per coefficient 110).
+constexpr int kFftR = 4;
+__global__ __launch_bounds__(kBlock) void k_fft_coeffs_draw(int64_t kN, int Nmc, const double* __restrict__ Sk,
+                                                            const uint8_t* __restrict__ calc, uint64_t seed,
+                                                            uint64_t first, double* __restrict__ amp) {
 #pragma clang fp contract(off)
-    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (e >= kN * Nmc) return;
-    const int r = (int)(e / kN);
-    const int64_t j = e - (int64_t)r * kN;
-    if (!calc[r]) {
-        amp[e] = 0.0;
-        return;
-    }
-    const uint64_t row = first + (uint64_t)r * (uint64_t)(3 * kN - 1);
-    const double g = rf_uniform(seed, 2u, row + (uint64_t)j) - 0.5;
-    const double ph = rf_uniform(seed, 2u, row + (uint64_t)(2 * kN - 1 + j));
-    amp[e] = g * sqrt(Sk[j]) * (double)cos_rev(ph);
+    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= kN) return;
+    const double root = sqrt(Sk[j]);
+    for (int r0 = blockIdx.y * kFftR; r0 < Nmc; r0 += gridDim.y * kFftR)
+        for (int r = r0; r < r0 + kFftR && r < Nmc; r++) {
+            double v = 0.0;
+            if (calc[r]) {
+                const uint64_t row = first + (uint64_t)r * (uint64_t)(3 * kN - 1);
+                const double g = rf_uniform(seed, 2u, row + (uint64_t)j) - 0.5;
+                const double ph = rf_uniform(seed, 2u, row + (uint64_t)(2 * kN - 1 + j));
+                v = g * root * (double)cos_rev(ph);
+            }
+            amp[(int64_t)r * kN + j] = v;
+        }
 }
 
 __global__ void k_scale(int64_t n, const double* __restrict__ a, double s, double* __restrict__ b) {
@@ -258,14 +259,11 @@ hipError_t rf_launch_prep_fp32(int64_t kN, int Nmc, int Rpad, const double* d_ph
     return hipGetLastError();
 }
 
-hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, const double* d_amp,
-                               double ampMult, double* d_uni, double* d_phase, float* d_phT, float* d_aT,
-                               hipStream_t s) {
-    const int R = d_phT ? Rpad : (Nmc + 3) / 4 * 4;        // whole float4 pieces (Rpad is a multiple of 16)
-    const unsigned gy = (unsigned)((R + 15) / 16);
-    if (gy > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_draw_prep, dim3(grid_for(kN), gy), dim3(kBlock), 0, s, kN, Nmc, R, seed, first, d_amp, ampMult,
-                       d_uni, d_phase, d_phT, d_aT);
+hipError_t rf_launch_draw_prep(int64_t kN, int Nmc, int Rpad, uint64_t seed, uint64_t first, double* d_uni,
+                               double* d_phase, float* d_phT, hipStream_t s) {
+    const unsigned gy = (unsigned)std::min((Nmc + 3) / 4, 65535);
+    hipLaunchKernelGGL(k_draw_prep, dim3(grid_for(kN), gy), dim3(kBlock), 0, s, kN, Nmc, Rpad, seed, first, d_uni, d_phase,
+                       d_phT);
     return hipGetLastError();
 }
 
@@ -286,10 +284,10 @@ hipError_t rf_launch_prep_fp32_iso(int nDim, int64_t kN, int Nmc, const double* 
 
 hipError_t rf_launch_fft_coeffs_draw(int64_t kN, int Nmc, const double* d_Sk, const uint8_t* d_calc,
                                      uint64_t seed, uint64_t first, double* d_amp, hipStream_t s) {
-    const int64_t n = kN * Nmc;
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fft_coeffs_draw, dim3(grid_for(n)), dim3(kBlock), 0, s, kN, Nmc, d_Sk, d_calc, seed,
-                       first, d_amp);
+    if (kN <= 0 || Nmc <= 0) return hipSuccess;
+    const unsigned gy = (unsigned)std::min((Nmc + kFftR - 1) / kFftR, 65535);
+    hipLaunchKernelGGL(k_fft_coeffs_draw, dim3(grid_for(kN), gy), dim3(kBlock), 0, s, kN, Nmc, d_Sk, d_calc, seed, first,
+                       d_amp);
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
 // rf_strip.hip -- the strip GEMM: every contraction of the grid form with FP16
-// operands.  Compiled once per kind (RF_STRIP_PART: rf_gemm_kind).
+// operands.  Compiled once per kind and operand type (RF_STRIP_PART: rf_gemm_kind, +3
+// real operands).
 //
 // One operand of each contraction is a small phase table shared by the whole
 // launch (M entries of an axis x K), the other -- the coefficients or the
@@ -22,7 +23,7 @@
 // per 16 k, re-reading and re-splitting the streamed one per table tile, two
 // barriers per 16 k.  32 fields of ~131^3 x 16 realizations: first contraction
 // (with its draws) 1.48 -> 1.44 ms, middle 1.93 -> 1.26, last 3.1 -> 2.3-2.4; 128^3
-// x 8 of method 4: 104 / 88 / 73 -> 68 / 63 / 55 us.  Same bits.  By counters the
+// x 8 of method 4: 104 / 88 / 73 -> 68 / 63 / 55 us, on real operands 63 / 35 / 42.  Same bits.  By counters the
 // first is bound by its draws (VALU 63 % of the cycles, matrix cores 21 %), the
 // middle moves 5.3 GB at 4.2 TB/s (matrix cores 38 %), the last 8.4 GB at 3.5.
 //
@@ -35,14 +36,18 @@
 #include "rf_grid_dev.h"
 
 #ifndef RF_STRIP_PART
-#error "rf_strip.hip is compiled once per RF_STRIP_PART (0..2)"
+#error "rf_strip.hip is compiled once per RF_STRIP_PART (0..5)"
 #endif
 
 namespace {
 
-constexpr int kKind = RF_STRIP_PART;
-constexpr bool kFirst = kKind == RF_GEMM_FIRST, kReal = kKind == RF_GEMM_LAST;
+constexpr int kKind = RF_STRIP_PART % 3;
+// real operands throughout (method 4): the im halves are zero, intermediates float
+constexpr bool kRealOps = RF_STRIP_PART >= 3;
+constexpr bool kFirst = kKind == RF_GEMM_FIRST, kLast = kKind == RF_GEMM_LAST;
+constexpr bool kReal = kLast || kRealOps;   // Re D only
 constexpr int NA = kReal ? 1 : 2;       // accumulators per tile: Re, Im
+constexpr unsigned kElem = kRealOps && !kFirst ? 4u : 8u;   // bytes of a streamed element (real first: FP64)
 constexpr int CS = kStripCS;            // K-steps per fetch (and per table chunk)
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -78,8 +83,8 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
     p.n0 = n0;
     const int nc = n0 + l32 < g.N ? n0 + l32 : g.N - 1;
     const int64_t col0 = col_b(g, n0);
-    p.S = (gch*)(g.B + (int64_t)batch * g.bStrideB + col0);
-    p.lo0 = (unsigned)(col_b(g, nc) - col0) * 8u;
+    p.S = (gch*)g.B + ((int64_t)batch * g.bStrideB + col0) * (int64_t)kElem;
+    p.lo0 = (unsigned)(col_b(g, nc) - col0) * kElem;
     p.gr = p.gj3 = p.gq = p.gj2 = 0;
     if (kFirst && gen) {
         const unsigned Q = (g.gen.fold && g.gen.nDim == 3) ? 2u : 1u;
@@ -95,14 +100,32 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
 // The values of steps CS c .. of this lane (a step past the last repeats it);
 // past K the table is zero and the last valid value is read again.  gen: a
 // batch's fresh realizations, the coefficients of the current draw formed here
-// (fold_coef_draw, as the fold would store them) instead of read.
+// (fold_coef_draw, as the fold would store them) instead of read.  Real first
+// contraction: the plan's FP64 amplitudes as they are (strip_split scales them),
+// k contiguous.
 __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& p, int c, int nSteps, bool gen,
                                             int64_t drawBase, int half, f2v (*v)[4]) {
-    const unsigned kb = (unsigned)g.bSk * 8u;         // bytes per k
+    const unsigned kb = (unsigned)g.bSk * kElem;      // bytes per k
 #pragma unroll
     for (int st = 0; st < CS; st++) {
         const int s = CS * c + st < nSteps ? CS * c + st : nSteps - 1;
-        if (kFirst && gen) {
+        if constexpr (kFirst && kRealOps) {
+            struct __attribute__((packed, aligned(8))) pair { f2v a, b; };
+            typedef const pair __attribute__((address_space(1))) gpair;
+            gch* b = p.S + (p.lo0 + 64u * (unsigned)s);
+            const int left = g.K - 1 - 8 * s;
+            if (left >= 7) {                                                      // uniform
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const gpair* e = (const gpair*)(b + 8 * (4 * half + i));
+                    v[st][i] = e->a;
+                    v[st][i + 1] = e->b;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[st][i] = *(gf2*)(b + 8 * (4 * half + i < left ? 4 * half + i : left));
+            }
+        } else if (kFirst && gen) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int k = 8 * s + 4 * half + i;
@@ -122,28 +145,33 @@ __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& 
             for (int i = 0; i < 4; i++) {
                 int k = 4 * half + i;
                 if (left < 7) k = k < left ? k : left;                            // uniform: the last step
-                v[st][i] = *(gf2*)(b + (p.lo0 + (unsigned)k * kb));
+                gch* e = b + (p.lo0 + (unsigned)k * kb);
+                if constexpr (kElem == 4) v[st][i] = f2v{*(const gfo*)e, 0.0f};
+                else v[st][i] = *(gf2*)e;
             }
         }
     }
 }
 
-__device__ __forceinline__ void strip_split(const f2v (*r)[4], unsigned sgn, u32x4 (*fh)[NA], u32x4 (*fl)[NA]) {
+__device__ __forceinline__ void strip_split(const f2v (*r)[4], double scale, unsigned sgn, u32x4 (*fh)[NA],
+                                            u32x4 (*fl)[NA]) {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int st = 0; st < CS; st++) {
         float re[4], im[4];
         hv4 rh, rl, ih, il;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            re[i] = r[st][i].x;
+            re[i] = kFirst && kRealOps ? (float)(__builtin_bit_cast(double, r[st][i]) * scale) : r[st][i].x;
             im[i] = r[st][i].y;
         }
         split4(re, &rh, &rl);
-        split4(im, &ih, &il);
+        if (kRealOps) ih = il = hv4{0, 0, 0, 0};
+        else split4(im, &ih, &il);
         const u32x4 h = half_swap(rh, ih), l = half_swap(rl, il);                 // (Re, Im)
         fh[st][0] = h ^ sgn;
         fl[st][0] = l ^ sgn;
-        if (kFirst) {
+        if (kFirst && !kReal) {
             fh[st][NA - 1] = half_swap(ih, rh);                                   // (Im, Re)
             fl[st][NA - 1] = half_swap(il, rl);
         } else if (!kReal) {
@@ -200,9 +228,18 @@ __device__ __forceinline__ void strip_store(const rf_gemm_desc& g, const strip& 
     const float os = g.outScale;
     const int n0 = p.n0, n = n0 + l32;
     const int dSm = (int)g.dSm, dSn = (int)g.dSn, rows = g.M;
+    // an intermediate's element type, address and value
+    auto at = [&](int64_t e) {
+        if constexpr (kRealOps) return (gfo*)(static_cast<float*>(g.D) + e);
+        else return (gf2o*)(static_cast<float2*>(g.D) + e);
+    };
+    auto val = [&](int t, int i) {
+        if constexpr (kRealOps) return acc[t][0][i] * os;
+        else return f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
+    };
     if constexpr (kFirst) {
         // lane: table entry 32 (t0 + t) + l32; rows: lines
-        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)p.batch * g.dStrideB + (int64_t)n0 * g.dSn);
+        auto* D = at((int64_t)p.batch * g.dStrideB + (int64_t)n0 * g.dSn);
 #pragma unroll
         for (int t = 0; t < MT; t++) {
             const int m = 32 * (t0 + t) + l32;
@@ -210,20 +247,20 @@ __device__ __forceinline__ void strip_store(const rf_gemm_desc& g, const strip& 
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int line = 8 * (i >> 2) + 4 * half + (i & 3);
-                if (n0 + line < g.N) D[line * dSn + m] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
+                if (n0 + line < g.N) D[line * dSn + m] = val(t, i);
             }
         }
-    } else if constexpr (!kReal) {
+    } else if constexpr (!kLast) {
         if (n >= g.N) return;
         const int64_t d0 = col_d(g, n0);
-        gf2o* D = (gf2o*)(static_cast<float2*>(g.D) + (int64_t)p.batch * g.dStrideB + d0 + (int64_t)(32 * t0) * g.dSm);
+        auto* D = at((int64_t)p.batch * g.dStrideB + d0 + (int64_t)(32 * t0) * g.dSm);
         const int oc = (int)(col_d(g, n) - d0);
 #pragma unroll
         for (int t = 0; t < MT; t++)
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int m = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (32 * t0 + m < rows) D[m * dSm + oc] = f2v{acc[t][0][i] * os, acc[t][NA - 1][i] * os};
+                if (32 * t0 + m < rows) D[m * dSm + oc] = val(t, i);
             }
     } else {
         // the epilogue's map, in place
@@ -315,7 +352,7 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
     const bool active = first < g.N;                  // uniform
     const int nSteps = (g.K + 7) / 8, nChunks = (nSteps + CS - 1) / CS;
     const unsigned sgn = half ? 0x80008000u : 0u;
-    const bool gen = kFirst && g.genState != nullptr && g.genState[2] != 0;
+    const bool gen = kFirst && !kRealOps && g.genState != nullptr && g.genState[2] != 0;
     const int64_t drawBase = gen ? g.genState[1] * (int64_t)g.genNmc * g.gen.kNr : 0;
     const strip p = strip_at(g, batch, active ? (int)first : 0, gen, l32);
 
@@ -343,7 +380,7 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
     auto chunk = [&](int c, const u32x4* cur, u32x4* nxt) {
         // fragments of this chunk's streamed values, then the loads of the next
         u32x4 fh[CS][NA], fl[CS][NA];
-        strip_split(r, sgn, fh, fl);
+        strip_split(r, kFirst ? g.gen.ampMult : 1.0, sgn, fh, fl);
         if (c + 1 < nChunks) {                        // in flight during the MFMAs
             dma(c + 1, nxt);
             strip_fetch(g, p, c + 1, nSteps, gen, drawBase, half, r);
@@ -371,9 +408,9 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
 
 // Registers: 16 MT accumulators per lane (32 MT complex) decide the waves per
 // SIMD; the compiler then keeps them in VGPRs without spills.
-constexpr int strip_waves(int MT) { return kReal ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4); }
+constexpr int strip_waves(int MT) { return NA == 1 ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4); }
 
-template <int MT, int KIND>
+template <int MT, int KIND, bool REAL>
 __global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT))))
 void k_strip(rf_gemm_desc g, int64_t nTiles) {
     __shared__ u32x4 ldsA[strip_units(MT)];
@@ -383,7 +420,7 @@ void k_strip(rf_gemm_desc g, int64_t nTiles) {
     strip_tile<MT>(g, L, ldsA, ldsB);
 }
 
-template <int MT, int KIND>
+template <int MT, int KIND, bool REAL>
 __global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT))))
 void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
     __shared__ u32x4 ldsA[strip_units(MT)];
@@ -396,8 +433,9 @@ void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) 
 
 template <int MT>
 hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks, hipStream_t s) {
-    if (g) hipLaunchKernelGGL((k_strip<MT, kKind>), dim3(blocks), dim3(64 * kStripW), 0, s, *g, n);
-    else hipLaunchKernelGGL((k_strip_group<MT, kKind>), dim3(blocks), dim3(64 * kStripW), 0, s, d_gs, nG, n);
+    if (g) hipLaunchKernelGGL((k_strip<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, *g, n);
+    else if constexpr (kRealOps) return hipErrorInvalidValue;
+    else hipLaunchKernelGGL((k_strip_group<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, d_gs, nG, n);
     return hipGetLastError();
 }
 
@@ -407,8 +445,14 @@ hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64
 #define RF_STRIP_LAUNCH rf_strip_launch_first
 #elif RF_STRIP_PART == 1
 #define RF_STRIP_LAUNCH rf_strip_launch_middle
-#else
+#elif RF_STRIP_PART == 2
 #define RF_STRIP_LAUNCH rf_strip_launch_last
+#elif RF_STRIP_PART == 3
+#define RF_STRIP_LAUNCH rf_strip_launch_first_real
+#elif RF_STRIP_PART == 4
+#define RF_STRIP_LAUNCH rf_strip_launch_middle_real
+#else
+#define RF_STRIP_LAUNCH rf_strip_launch_last_real
 #endif
 hipError_t RF_STRIP_LAUNCH(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks,
                            hipStream_t s) {

@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void k_sum_fp32(rf_sum_args a, const double
 // makes it the float 1 + argument (23 bits, rounded by the 2^-24) that v_cos_f32
 // takes.  A term costs three VALU instructions (alignbit, cosine, FMA), the
 // matrix cores run beside them.  Formerly eight, four of them FP64 (k.x by FMAs,
-// v_fract_f64): 200,000 points x 16 realizations ISOFIGS
+// v_fract_f64): 200,000 points x 16 realizations, ~480 shells 375 -> 254 us.
 // Arguments that may reach 2^19 revolutions (or are not finite) take a zero
 // accumulator and v_fract_f64; the choice is per wave.
 // kA [block][4][16], aA [block][row % 4][row / 4], block = wavevector block x chunks
