@@ -41,7 +41,7 @@ HIP_FLAGS = [
 
 
 # sources compiled as several translation units (one per value of a macro)
-SPLIT = {"rf_mfma.hip": 7, "rf_strip.hip": 6}
+SPLIT = {"rf_mfma.hip": 7, "rf_strip.hip": 7}
 SPLIT_MACRO = {"rf_mfma.hip": "RF_MFMA_PART", "rf_strip.hip": "RF_STRIP_PART"}
 
 

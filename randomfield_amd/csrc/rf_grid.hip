@@ -25,7 +25,7 @@
 // The isotropic method (randomFieldND.f90:368-514) has no lattice, but on a
 // grid each of its terms still factorises over the axes: per realization one
 // real-part GEMM over the shells whose operands are per-axis phase tables
-// (k_iso_tables, k_iso_gemm).
+// (k_iso_tables, the isotropic strip GEMM).
 #include "rf_grid_dev.h"
 
 namespace {
@@ -157,313 +157,6 @@ __device__ __forceinline__ void gemm_tile(const rf_gemm_desc& g, int m0, int n0,
     }
 }
 
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef const f4v __attribute__((address_space(1))) gf4;
-// n consecutive float2 (n even, 16-byte aligned) by 16-byte loads
-template <int n>
-__device__ __forceinline__ void ld_run(const gf2* p, f2v* v) {
-    const gf4* q = reinterpret_cast<const gf4*>(p);
-#pragma unroll
-    for (int i = 0; i < n / 2; i++) {
-        const f4v t = q[i];
-        v[2 * i] = f2v{t.x, t.y};
-        v[2 * i + 1] = f2v{t.z, t.w};
-    }
-}
-constexpr int kHP = 24;                       // LDS row pitch (halves): 16 k + pad
-// Operand planes of a 64x128 real-part tile (the isotropic GEMM).
-struct HStage {
-    _Float16 a[4][kTM][kHP];          // Re hi, Re lo, -Im hi, -Im lo
-    _Float16 b[4][2 * kTN][kHP];      // Re hi, Re lo, Im hi, Im lo
-};
-
-// -x of FP16 values: the sign bits flipped
-__device__ inline hv4 neg4(hv4 x) {
-    typedef unsigned u2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(hv4, __builtin_bit_cast(u2, x) ^ 0x80008000u);
-}
-
-// Isotropic sum on a structured grid, per-realization directions.  With
-// x = o + i step per axis, e^{i(k.x + phi)} factorises over the axes, so per
-// realization r
-//   u_r[l][(i, j)] = Re sum_k Z_k[l] B_k[(i, j)],   B_k[(i, j)] = W_k[i] Y_k[j],
-//   W_k[i] = a_k e^{i(k_x x_i + phi_k)},  Y_k[j] = e^{i k_y y_j},  Z_k[l] = e^{i k_z z_l}
-// (2-D: u_r[j][i] = Re sum_k Y_k[j] W_k[i]): one real-part GEMM with M the
-// last axis, N the plane and K the shells, whose B operand is formed while
-// staged -- one complex product per element -- instead of read.  Tables are
-// [r][index][k], k fastest and padded to whole kTK chunks by zero entries:
-// a thread's k run of a chunk is one 16-byte-aligned piece of a row, read
-// by 16-byte loads from one address, with no masks; rows and columns past a
-// tile's edge read the last row / column (finite values in accumulators
-// that are never stored).  Tiles of 64x128.
-struct rf_iso_gemm {
-    const float2* A;              // last-axis table [r][k][m]
-    const float2* W;              // first-axis table with the coefficients [r][k][i]
-    const float2* Y;              // second-axis table [r][k][j] (3-D; NULL in 2-D)
-    int M, N, K, nx, ny;
-    int64_t aStrideB, wStrideB, yStrideB;
-    void* D;                      // [r][m][n]
-    int outDtype;
-    rf_epilogue epi;
-    float outScale;
-};
-__device__ __forceinline__ void gemm_tile_iso(const rf_iso_gemm& g, int m0, int n0, int batch, HStage* st) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)batch * g.aStrideB + (int64_t)m0 * g.K);
-    const gf2* Wt = (const gf2*)(g.W + (int64_t)batch * g.wStrideB);
-    const gf2* Yt = (const gf2*)(g.Y ? g.Y + (int64_t)batch * g.yStrideB : nullptr);
-    f32x16 acc[2];
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        acc[0][i] = 0.0f;
-        acc[1][i] = 0.0f;
-    }
-    const int rt = wave >> 1, ct = wave & 1;
-    // staging: A row t/4, k 4(t%4)..+3; B column t%128, k 8(t/128)..+7
-    const int aRow = tid >> 2, aK = (tid & 3) * 4;
-    const int bCol = tid & 127, bK = (tid >> 7) * 8;
-    const int aRowC = m0 + aRow < g.M ? aRow : g.M - 1 - m0;
-    const int bColC = n0 + bCol < g.N ? n0 + bCol : g.N - 1;
-    const int bI = bColC % g.nx, bJ = bColC / g.nx;
-    const bool hasY = Yt != nullptr;
-    const gf2* aP = A + (int64_t)aRowC * g.K + aK;
-    const gf2* wP = Wt + (int64_t)bI * g.K + bK;
-    const gf2* yP = hasY ? Yt + (int64_t)bJ * g.K + bK : nullptr;
-    f2v ra[4], rw[8], ry[8];
-    auto fetch = [&](int k0) {
-        ld_run<4>(aP + k0, ra);
-        ld_run<8>(wP + k0, rw);
-        if (hasY) ld_run<8>(yP + k0, ry);
-        else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) ry[i] = f2v{1.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            re[i] = ra[i].x;
-            im[i] = ra[i].y;
-        }
-        split4(re, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[0][aRow][aK]) = hi;
-        *reinterpret_cast<hv4*>(&st->a[1][aRow][aK]) = lo;
-        split4(im, &hi, &lo);
-        *reinterpret_cast<hv4*>(&st->a[2][aRow][aK]) = neg4(hi);   // split(-x) = -split(x)
-        *reinterpret_cast<hv4*>(&st->a[3][aRow][aK]) = neg4(lo);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const f2v w = rw[4 * h + i], y = ry[4 * h + i];
-                re[i] = fmaf(w.x, y.x, -w.y * y.y);
-                im[i] = fmaf(w.x, y.y, w.y * y.x);
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[0][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[1][bCol][bK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[2][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[3][bCol][bK + 4 * h]) = lo;
-        }
-    };
-    // K' half 0 pairs Re A with Re B, half 1 -Im A with Im B
-    const int aPlane = half ? 2 : 0, bPlane = half ? 2 : 0;
-    const int aRowL = rt * 32 + l32;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + rt * 32 < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-                const hv8 ah = *reinterpret_cast<const hv8*>(&st->a[aPlane][aRowL][kk]);
-                const hv8 al = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][aRowL][kk]);
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const int col = 64 * ct + 32 * c;
-                    if (n0 + col >= g.N) break;                                    // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][col + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][col + l32][kk]);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc[c], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dBase = (int64_t)batch * g.M * g.N + (int64_t)m0 * g.N + n0;
-    const int nc[2] = {64 * ct + l32, 64 * ct + 32 + l32};
-    const bool nIn[2] = {n0 + nc[0] < g.N, n0 + nc[1] < g.N};
-    auto store = [&](auto map, auto* D) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = rt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-            if (m0 + r >= g.M) continue;
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-                if (nIn[c]) D[(int64_t)r * g.N + nc[c]] = map(acc[c][i] * os);
-        }
-    };
-    const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
-    gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
-    gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
-    if (g.outDtype == RF_DTYPE_F64) {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL) store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64);
-        else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64);
-    } else {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL) store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32);
-        else store([=](float u) { return fmaf(u, sc, sh); }, D32);
-    }
-}
-
-// The isotropic grid GEMM on 128x128 tiles (a last axis longer than 64):
-// each B element formed once per realization instead of once per 64 rows;
-// wave w owns rows 64 (w / 2).. and columns 64 (w % 2).., four 32x32 MFMA
-// tiles sharing two A and two B fragment reads per K-step.
-struct IsoStage128 {
-    _Float16 a[4][128][kHP];      // Re hi, Re lo, -Im hi, -Im lo
-    _Float16 b[4][128][kHP];      // Re hi, Re lo, Im hi, Im lo
-};
-__device__ __forceinline__ void gemm_tile_iso128(const rf_iso_gemm& g, int m0, int n0, int batch, IsoStage128* st) {
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
-    const gf2* A = (const gf2*)(g.A + (int64_t)batch * g.aStrideB + (int64_t)m0 * g.K);
-    const gf2* Wt = (const gf2*)(g.W + (int64_t)batch * g.wStrideB);
-    const gf2* Yt = (const gf2*)(g.Y ? g.Y + (int64_t)batch * g.yStrideB : nullptr);
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 16; i++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) acc[q >> 1][q & 1][i] = 0.0f;
-    const int rt = wave >> 1, ct = wave & 1;
-    // staging: A row t/2, k 8(t%2)..+7; B column t%128, k 8(t/128)..+7
-    const int aRow = tid >> 1, aK = (tid & 1) * 8;
-    const int bCol = tid & 127, bK = (tid >> 7) * 8;
-    const int aRowC = m0 + aRow < g.M ? aRow : g.M - 1 - m0;
-    const int bColC = n0 + bCol < g.N ? n0 + bCol : g.N - 1;
-    const int bI = bColC % g.nx, bJ = bColC / g.nx;
-    const bool hasY = Yt != nullptr;
-    const gf2* aP = A + (int64_t)aRowC * g.K + aK;
-    const gf2* wP = Wt + (int64_t)bI * g.K + bK;
-    const gf2* yP = hasY ? Yt + (int64_t)bJ * g.K + bK : nullptr;
-    f2v ra[8], rw[8], ry[8];
-    auto fetch = [&](int k0) {
-        ld_run<8>(aP + k0, ra);
-        ld_run<8>(wP + k0, rw);
-        if (hasY) ld_run<8>(yP + k0, ry);
-        else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) ry[i] = f2v{1.f, 0.f};
-        }
-    };
-    auto stash = [&]() {
-        float re[4], im[4];
-        hv4 hi, lo;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                re[i] = ra[4 * h + i].x;
-                im[i] = ra[4 * h + i].y;
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->a[0][aRow][aK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->a[1][aRow][aK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->a[2][aRow][aK + 4 * h]) = neg4(hi);   // split(-x) = -split(x)
-            *reinterpret_cast<hv4*>(&st->a[3][aRow][aK + 4 * h]) = neg4(lo);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const f2v w = rw[4 * h + i], y = ry[4 * h + i];
-                re[i] = fmaf(w.x, y.x, -w.y * y.y);
-                im[i] = fmaf(w.x, y.y, w.y * y.x);
-            }
-            split4(re, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[0][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[1][bCol][bK + 4 * h]) = lo;
-            split4(im, &hi, &lo);
-            *reinterpret_cast<hv4*>(&st->b[2][bCol][bK + 4 * h]) = hi;
-            *reinterpret_cast<hv4*>(&st->b[3][bCol][bK + 4 * h]) = lo;
-        }
-    };
-    // K' half 0 pairs Re A with Re B, half 1 -Im A with Im B
-    const int aPlane = half ? 2 : 0, bPlane = half ? 2 : 0;
-    fetch(0);
-    for (int k0 = 0; k0 < g.K; k0 += kTK) {
-        stash();
-        __syncthreads();
-        if (k0 + kTK < g.K) fetch(k0 + kTK);      // in flight during the MFMAs
-        if (m0 + rt * 64 < g.M) {
-#pragma unroll
-            for (int kk = 0; kk < kTK; kk += 8) {
-                hv8 ah[2], al[2];
-#pragma unroll
-                for (int rr = 0; rr < 2; rr++) {
-                    ah[rr] = *reinterpret_cast<const hv8*>(&st->a[aPlane][rt * 64 + 32 * rr + l32][kk]);
-                    al[rr] = *reinterpret_cast<const hv8*>(&st->a[aPlane + 1][rt * 64 + 32 * rr + l32][kk]);
-                }
-#pragma unroll
-                for (int c = 0; c < 2; c++) {
-                    const int col = 64 * ct + 32 * c;
-                    if (n0 + col >= g.N) break;                                    // uniform
-                    const hv8 bh = *reinterpret_cast<const hv8*>(&st->b[bPlane][col + l32][kk]);
-                    const hv8 bl = *reinterpret_cast<const hv8*>(&st->b[bPlane + 1][col + l32][kk]);
-#pragma unroll
-                    for (int rr = 0; rr < 2; rr++) {
-                        if (rr > 0 && m0 + rt * 64 + 32 >= g.M) break;            // uniform
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[rr], bh, acc[rr][c], 0, 0, 0);
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[rr], bl, acc[rr][c], 0, 0, 0);
-                        acc[rr][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[rr], bh, acc[rr][c], 0, 0, 0);
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    // D layout of a 32x32 tile: lane column l32, rows 8*(i/4) + 4*half + i%4
-    const float os = g.outScale;
-    const int64_t dBase = (int64_t)batch * g.M * g.N + (int64_t)m0 * g.N + n0;
-    const int nc[2] = {64 * ct + l32, 64 * ct + 32 + l32};
-    const bool nIn[2] = {n0 + nc[0] < g.N, n0 + nc[1] < g.N};
-    auto store = [&](auto map, auto* D) {
-#pragma unroll
-        for (int rr = 0; rr < 2; rr++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int r = rt * 64 + 32 * rr + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (m0 + r >= g.M) continue;
-#pragma unroll
-                for (int c = 0; c < 2; c++)
-                    if (nIn[c]) D[(int64_t)r * g.N + nc[c]] = map(acc[rr][c][i] * os);
-            }
-    };
-    const float sc = (float)g.epi.scale, sh = (float)g.epi.shift;
-    gfo* D32 = (gfo*)(static_cast<float*>(g.D) + dBase);
-    gdo* D64 = (gdo*)(static_cast<double*>(g.D) + dBase);
-    if (g.outDtype == RF_DTYPE_F64) {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return (double)u; }, D64);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL) store([=](float u) { return (double)expf(fmaf(u, sc, sh)); }, D64);
-        else store([=](float u) { return (double)fmaf(u, sc, sh); }, D64);
-    } else {
-        if (g.epi.margi == RF_FOM_NONE) store([](float u) { return u; }, D32);
-        else if (g.epi.margi == RF_FOM_LOGNORMAL) store([=](float u) { return expf(fmaf(u, sc, sh)); }, D32);
-        else store([=](float u) { return fmaf(u, sc, sh); }, D32);
-    }
-}
-
 struct FStage {
     float2 a[kTK][kTM + 1];
     float2 b[kTK][kTN + 1];
@@ -497,60 +190,63 @@ __global__ __launch_bounds__(256) void k_cgemm_group(const rf_gemm_desc* __restr
     run_tile<RealOnly>(g, L - g.tile0, smem);
 }
 
-// One 64x128 tile of one realization's isotropic grid GEMM per block; tiles
-// numbered row tiles fastest (they share a column slab of B), placed per XCD.
-template <int TM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_iso_gemm(rf_iso_gemm g, int64_t nTiles) {
-    __shared__ __attribute__((aligned(16))) char smem[TM == 128 ? sizeof(IsoStage128) : sizeof(HStage)];
-    const int64_t L = xcd_tile(blockIdx.x, nTiles);
-    if (L >= nTiles) return;
-    const int ntM = (g.M + TM - 1) / TM, ntN = (g.N + 2 * kTN - 1) / (2 * kTN);
-    const int mI = (int)(L % ntM);
-    const int64_t rest = L / ntM;
-    const int nI = (int)(rest % ntN);
-    const int batch = (int)(rest / ntN);
-    if constexpr (TM == 128)
-        gemm_tile_iso128(g, mI * TM, nI * 2 * kTN, batch, reinterpret_cast<IsoStage128*>(smem));
-    else
-        gemm_tile_iso(g, mI * TM, nI * 2 * kTN, batch, reinterpret_cast<HStage*>(smem));
-}
-
-// Isotropic phase tables [r][index][k] for the axes of the grid, in FP64
-// then rounded: axis 0 carries the coefficient, W = c a e^{i(k_x x + phi)}
-// (c: ampMult times a power of two), the others e^{i k_a x}; k runs to kP
-// (kN rounded up to whole chunks), zero past kN.
-__global__ void k_iso_tables(int nDim, int64_t kN, int64_t kP, int Nmc, int n0, int n1, int n2,
-                             const double* __restrict__ kIso,
-                             const double* __restrict__ amp, const double* __restrict__ phase, double coef,
-                             double o0, double o1, double o2, double s0, double s1, double s2, double i0, double i1,
-                             double i2, float2* __restrict__ T0, float2* __restrict__ T1, float2* __restrict__ T2) {
-    const int nT = n0 + n1 + (nDim == 3 ? n2 : 0);
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (int64_t)Nmc * kP * nT) return;
-    const int64_t k = e % kP;                        // k fastest, as stored
-    const int64_t rt = e / kP;                       // r * nT + t
-    const int t = (int)(rt % nT);
-    const int64_t r = rt / nT;
-    const int64_t rk = r * kN + k;
-    const int a = t < n0 ? 0 : (t < n0 + n1 ? 1 : 2);
-    const int idx = a == 0 ? t : (a == 1 ? t - n0 : t - n0 - n1);
-    const int na = a == 0 ? n0 : (a == 1 ? n1 : n2);
-    float2* T = a == 0 ? T0 : (a == 1 ? T1 : T2);
-    const int64_t dst = (r * na + idx) * kP + k;     // [r][idx][k]
-    if (k >= kN) {
-        T[dst] = make_float2(0.f, 0.f);
+// Isotropic phase tables of the grid's axes, in FP64 then rounded: axis 0
+// carries the coefficient, W = c a e^{i(k_x x + phi)} (c: ampMult times a power of
+// two), the others e^{i k_a x}; k runs to kP (kN rounded up to whole steps), zero
+// past kN.  The last axis goes to Z in the strip GEMM's fragment order, split into
+// FP16 hi + lo ([r][k / 8][x / 32][hi, lo][re, im][x % 32][k % 8]), the others to T0
+// and T1 as [r][k / 4][x][k % 4]; a thread's position runs along what it writes.
+struct rf_iso_tables {
+    int nDim, Nmc;
+    int64_t kN, kP;
+    int n[3], w[3];                // points; entries written (the last axis: whole tiles)
+    double o[3], st[3], inv[3], coef;
+    const double* kIso; const double* amp; const double* phase;
+    float2* T[2];
+    _Float16* Z;
+};
+__global__ __launch_bounds__(256) void k_iso_tables(rf_iso_tables t) {
+    const int64_t per = t.kP * (t.w[0] + t.w[1] + t.w[2]);       // of a realization
+    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= t.Nmc * per) return;
+    const int64_t r = e / per;
+    e -= r * per;
+    int a = 0;
+    while (a + 1 < t.nDim && e >= t.kP * t.w[a]) e -= t.kP * t.w[a++];
+    const bool last = a == t.nDim - 1;
+    int64_t k;
+    int idx;
+    if (last) {
+        const int nT = t.w[a] / 32;
+        const int64_t st = e >> 8;                               // step * nT + tile
+        k = st / nT * 8 + (e & 7);
+        idx = (int)(st % nT) * 32 + ((int)(e >> 3) & 31);
+    } else {
+        const int64_t c = e / (4 * t.w[a]);
+        k = 4 * c + (e & 3);
+        idx = (int)((e - c * 4 * t.w[a]) >> 2);
+    }
+    float2 v = make_float2(0.f, 0.f);
+    if (k < t.kN && idx < t.n[a]) {
+        const int64_t rk = r * t.kN + k;
+        const double x = (t.o[a] + t.st[a] * (double)idx) * t.inv[a];
+        double th = t.kIso[rk * t.nDim + a] * x;
+        if (a == 0) th += t.phase[rk];
+        double sn, cs;
+        sincos(th, &sn, &cs);
+        const double m = a == 0 ? t.amp[rk] * t.coef : 1.0;
+        v = make_float2((float)(m * cs), (float)(m * sn));
+    }
+    if (!last) {
+        t.T[a][r * t.kP * t.w[a] + e] = v;
         return;
     }
-    const double o = a == 0 ? o0 : (a == 1 ? o1 : o2);
-    const double st = a == 0 ? s0 : (a == 1 ? s1 : s2);
-    const double inv = a == 0 ? i0 : (a == 1 ? i1 : i2);
-    const double x = (o + st * (double)idx) * inv;
-    double th = kIso[rk * nDim + a] * x;
-    if (a == 0) th += phase[rk];
-    double sn, cs;
-    sincos(th, &sn, &cs);
-    const double m = a == 0 ? amp[rk] * coef : 1.0;
-    T[dst] = make_float2((float)(m * cs), (float)(m * sn));
+    _Float16* F = t.Z + (r * t.kP * t.w[a] + (e & ~(int64_t)255)) * 4 + (e & 255);
+    const _Float16 ch = (_Float16)v.x, sh = (_Float16)v.y;
+    F[0] = ch;
+    F[256] = sh;
+    F[512] = (_Float16)(v.x - (float)ch);
+    F[768] = (_Float16)(v.y - (float)sh);
 }
 
 // The tables of all axes of one execution (one launch: a grid of 129 x 129
@@ -771,6 +467,7 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
     const int64_t nb = xcd_blocks(nTiles);
     if (nb > 0x7fffffffLL || mt < 0 || mt > kStripMaxMT) return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)nb;
+    if (kind == RF_GEMM_ISO) return rf_strip_launch_iso(mt, g, d_gs, nG, nTiles, blocks, s);
     if (mt > 0 && g && g->real) {
         if (kind == RF_GEMM_FIRST) return rf_strip_launch_first_real(mt, g, d_gs, nG, nTiles, blocks, s);
         if (kind == RF_GEMM_MIDDLE) return rf_strip_launch_middle_real(mt, g, d_gs, nG, nTiles, blocks, s);
@@ -1049,11 +746,12 @@ hipError_t rf_grid_run(const rf_grid_stages& st, hipStream_t s) {
     return hipSuccess;
 }
 
-static int64_t iso_k_padded(int64_t kN) { return (kN + kTK - 1) / kTK * kTK; }
+static int64_t iso_k_padded(int64_t kN) { return (kN + 7) / 8 * 8; }
 
+// the last axis' table in whole 32-entry tiles
 size_t rf_iso_grid_scratch_elems(int nDim, int64_t kN, int Nmc, const int32_t* n) {
     int64_t t = 0;
-    for (int a = 0; a < nDim; a++) t += n[a];
+    for (int a = 0; a < nDim; a++) t += a == nDim - 1 ? ((int64_t)n[a] + 31) / 32 * 32 : n[a];
     return (size_t)(Nmc * iso_k_padded(kN) * t);
 }
 
@@ -1066,40 +764,37 @@ hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s) {
         std::frexp(a.coefMax, &e);
         sc = std::ldexp(1.0, -e);
     }
-    const int n0 = a.n[0], n1 = a.n[1], n2 = a.nDim == 3 ? a.n[2] : 1;
     const int64_t kP = iso_k_padded(a.kN);
-    float2* T0 = a.scratch;
-    float2* T1 = T0 + (int64_t)a.Nmc * kP * n0;
-    float2* T2 = T1 + (int64_t)a.Nmc * kP * n1;
-    const int64_t cnt = (int64_t)a.Nmc * kP * (n0 + n1 + (a.nDim == 3 ? n2 : 0));
-    hipLaunchKernelGGL(k_iso_tables, dim3(blocks_for(cnt)), dim3(256), 0, s, a.nDim, a.kN, kP, a.Nmc, n0, n1, n2, a.kIso,
-                       a.amp, a.phase, a.ampMult * sc, a.origin[0], a.origin[1], a.origin[2], a.step[0], a.step[1],
-                       a.step[2], a.invL[0], a.invL[1], a.invL[2], T0, T1, T2);
-    rf_iso_gemm g{};
-    g.K = (int)kP;
-    g.W = T0;
-    g.nx = n0;
-    g.wStrideB = kP * n0;
-    if (a.nDim == 3) {
-        g.A = T2; g.M = n2; g.aStrideB = kP * n2;
-        g.Y = T1; g.ny = n1; g.yStrideB = kP * n1;
-        g.N = n0 * n1;
-    } else {
-        g.A = T1; g.M = n1; g.aStrideB = kP * n1;
-        g.Y = nullptr; g.ny = 1; g.yStrideB = 0;
-        g.N = n0;
+    rf_iso_tables t{};
+    t.nDim = a.nDim; t.Nmc = a.Nmc; t.kN = a.kN; t.kP = kP;
+    t.kIso = a.kIso; t.amp = a.amp; t.phase = a.phase;
+    t.coef = a.ampMult * sc;
+    const int ad = a.nDim - 1;
+    float2* p = a.scratch;
+    for (int d = 0; d < a.nDim; d++) {
+        t.n[d] = a.n[d];
+        t.w[d] = d == ad ? (a.n[d] + 31) / 32 * 32 : a.n[d];
+        t.o[d] = a.origin[d]; t.st[d] = a.step[d]; t.inv[d] = a.invL[d];
+        if (d == ad) t.Z = reinterpret_cast<_Float16*>(p);
+        else t.T[d] = p;
+        p += a.Nmc * kP * t.w[d];
     }
-    g.D = a.d_out;
+    const int64_t cnt = a.Nmc * kP * ((int64_t)t.w[0] + t.w[1] + t.w[2]);
+    if ((cnt + 255) / 256 > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_iso_tables, dim3(blocks_for(cnt)), dim3(256), 0, s, t);
+    rf_gemm_desc g{};
+    g.kind = RF_GEMM_ISO;
+    g.T = t.Z; g.M = a.n[ad]; g.K = (int)kP; g.batches = a.Nmc;
+    g.B = t.T[0]; g.bStrideB = kP * a.n[0]; g.isoNx = a.n[0]; g.isoNy = 1;
+    g.N = a.n[0];
+    if (a.nDim == 3) {
+        g.isoY = t.T[1]; g.isoNy = a.n[1]; g.isoYStrideB = kP * a.n[1];
+        g.N = a.n[0] * a.n[1];
+    }
+    g.D = a.d_out; g.dSm = g.N; g.dSn = 1; g.dStrideB = (int64_t)g.M * g.N;
     g.outDtype = a.outDtype;
     g.epi = a.epi;
     g.outScale = (float)(1.0 / sc);
-    // a last axis longer than 64 on 128-row tiles (each B element formed once
-    // per 128 rows)
-    const int TM = g.M > kTM ? 128 : kTM;
-    const int64_t nTiles = (int64_t)((g.M + TM - 1) / TM) * ((g.N + 2 * kTN - 1) / (2 * kTN)) * a.Nmc;
-    const int64_t blocks = xcd_blocks(nTiles);
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (TM == 128) hipLaunchKernelGGL(k_iso_gemm<128>, dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    else hipLaunchKernelGGL(k_iso_gemm<kTM>, dim3((unsigned)blocks), dim3(256), 0, s, g, nTiles);
-    return hipGetLastError();
+    g.mt = strip_choose(g);
+    return launch_any(g.kind, g.mt, &g, nullptr, 0, rf_gemm_tiles(g, g.mt), s);
 }

@@ -22,6 +22,8 @@ typedef const f2v __attribute__((address_space(1))) gf2;      // global-memory v
 typedef f2v __attribute__((address_space(1))) gf2o;
 typedef float __attribute__((address_space(1))) gfo;
 typedef double __attribute__((address_space(1))) gdo;
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef const f4v __attribute__((address_space(1))) gf4;
 typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
 typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
 

@@ -282,7 +282,8 @@ constexpr int kStripW = 4;            // waves per block
 constexpr int kStripCS = 2;           // K-steps per fetch and table chunk
 constexpr int kStripL = 32 * kStripW; // lines per block
 constexpr int64_t kStripFill = 1024;  // waves below which a strip GEMM splits its table axis
-enum rf_gemm_kind { RF_GEMM_FIRST, RF_GEMM_MIDDLE, RF_GEMM_LAST };   // LAST: Re(D), epilogue, outDtype
+// LAST, ISO: Re(D), epilogue, outDtype; ISO: a table per batch, lines the products of two factors
+enum rf_gemm_kind { RF_GEMM_FIRST, RF_GEMM_MIDDLE, RF_GEMM_LAST, RF_GEMM_ISO };
 // The coefficient fold of one grid execution: Cf[k][m] for rows m (r, j3, q,
 // j2) and K index k (h, j1) from amp / phase [r][b][j] (rf_grid.hip).
 struct rf_fold_desc {
@@ -336,6 +337,9 @@ struct rf_gemm_desc {
     uint64_t genSeed;
     int genNmc;
     const int64_t* genState;
+    const float2* isoY;   // ISO: B[k / 4][x][k % 4] times isoY[k / 4][y][k % 4] (NULL: 1), line x + isoNx y
+    int isoNx, isoNy;
+    int64_t isoYStrideB;
     int real;             // strips: real operands and intermediates (method 4; first contraction: B the FP64
                           // amplitudes, scaled by gen.ampMult)
 };
@@ -418,6 +422,7 @@ RF_STRIP_DECL(rf_strip_launch_last);
 RF_STRIP_DECL(rf_strip_launch_first_real);      // real operands, single GEMMs only
 RF_STRIP_DECL(rf_strip_launch_middle_real);
 RF_STRIP_DECL(rf_strip_launch_last_real);
+RF_STRIP_DECL(rf_strip_launch_iso);             // single GEMMs only
 
 // post-processing (rf_post.hip)
 hipError_t rf_launch_marginal(int margi, double scale, double shift, void* d, int64_t count,

@@ -1,6 +1,6 @@
 // rf_strip.hip -- the strip GEMM: every contraction of the grid form with FP16
 // operands.  Compiled once per kind and operand type (RF_STRIP_PART: rf_gemm_kind, +3
-// real operands).
+// real operands; 6 isotropic).
 //
 // One operand of each contraction is a small phase table shared by the whole
 // launch (M entries of an axis x K), the other -- the coefficients or the
@@ -27,6 +27,16 @@
 // first is bound by its draws (VALU 63 % of the cycles, matrix cores 21 %), the
 // middle moves 5.3 GB at 4.2 TB/s (matrix cores 38 %), the last 8.4 GB at 3.5.
 //
+// Isotropic sum on a grid, per-realization directions.  With x = o + i step per
+// axis, e^{i(k.x + phi)} factorises over the axes, so per realization r
+//   u_r[l][(i, j)] = Re sum_k Z_k[l] B_k[(i, j)],   B_k[(i, j)] = W_k[i] Y_k[j],
+//   W_k[i] = a_k e^{i(k_x x_i + phi_k)},  Y_k[j] = e^{i k_y y_j},  Z_k[l] = e^{i k_z z_l}
+// (2-D: u_r[j][i] = Re sum_k Y_k[j] W_k[i]): the table is Z, one per realization,
+// the lines are the points of the plane and a streamed value is the product of
+// two table entries, formed as it is split.  128^3 x 64 lognormal, 286 shells: 570 us
+// of kernel (128 x 128 block tiles with both operands staged 620); the matrix
+// cores are busy 41 % of the cycles, the VALU 48 % (a third of it the exponentials).
+//
 // D orientation: the table is the A operand (lanes run along lines) where D
 // is stored with lines contiguous, the B operand (lanes run along the table
 // axis) in the first contraction, whose D has the table axis contiguous.
@@ -35,20 +45,24 @@
 // double buffer, one barrier per chunk.
 #include "rf_grid_dev.h"
 
+#include <type_traits>
+
 #ifndef RF_STRIP_PART
-#error "rf_strip.hip is compiled once per RF_STRIP_PART (0..5)"
+#error "rf_strip.hip is compiled once per RF_STRIP_PART (0..6)"
 #endif
 
 namespace {
 
-constexpr int kKind = RF_STRIP_PART % 3;
+constexpr bool kIso = RF_STRIP_PART == 6;
+constexpr int kKind = kIso ? RF_GEMM_ISO : RF_STRIP_PART % 3;
 // real operands throughout (method 4): the im halves are zero, intermediates float
-constexpr bool kRealOps = RF_STRIP_PART >= 3;
-constexpr bool kFirst = kKind == RF_GEMM_FIRST, kLast = kKind == RF_GEMM_LAST;
+constexpr bool kRealOps = RF_STRIP_PART >= 3 && !kIso;
+constexpr bool kFirst = kKind == RF_GEMM_FIRST, kLast = kKind == RF_GEMM_LAST || kIso;
 constexpr bool kReal = kLast || kRealOps;   // Re D only
 constexpr int NA = kReal ? 1 : 2;       // accumulators per tile: Re, Im
 constexpr unsigned kElem = kRealOps && !kFirst ? 4u : 8u;   // bytes of a streamed element (real first: FP64)
 constexpr int CS = kStripCS;            // K-steps per fetch (and per table chunk)
+constexpr int NV = kIso ? 8 : 4;        // values of a lane per step (isotropic: two factors)
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void;
@@ -72,7 +86,8 @@ struct strip {
     // descriptor of a grouped launch is read from memory, and generic (flat)
     // loads would also count against the LDS wait counter.
     gch* S;
-    unsigned lo0;
+    gch* Y;                               // isotropic: the second factor
+    unsigned lo0, lo1;
     int batch, n0;
     unsigned gr, gj3, gq, gj2;            // drawn coefficients: the line's digits
 };
@@ -82,10 +97,20 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
     p.batch = batch;
     p.n0 = n0;
     const int nc = n0 + l32 < g.N ? n0 + l32 : g.N - 1;
+    p.Y = nullptr;
+    p.lo1 = 0;
+    p.gr = p.gj3 = p.gq = p.gj2 = 0;
+    if constexpr (kIso) {
+        // tables [k / 4][index][k % 4]: a lane's four k are 32 bytes
+        p.S = (gch*)(g.B + (int64_t)batch * g.bStrideB);
+        p.Y = (gch*)(g.isoY + (int64_t)batch * g.isoYStrideB);
+        p.lo0 = 32u * (unsigned)(nc % g.isoNx);
+        p.lo1 = 32u * (unsigned)(nc / g.isoNx);
+        return p;
+    }
     const int64_t col0 = col_b(g, n0);
     p.S = (gch*)g.B + ((int64_t)batch * g.bStrideB + col0) * (int64_t)kElem;
     p.lo0 = (unsigned)(col_b(g, nc) - col0) * kElem;
-    p.gr = p.gj3 = p.gq = p.gj2 = 0;
     if (kFirst && gen) {
         const unsigned Q = (g.gen.fold && g.gen.nDim == 3) ? 2u : 1u;
         unsigned rem = (unsigned)nc;
@@ -104,12 +129,28 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
 // contraction: the plan's FP64 amplitudes as they are (strip_split scales them),
 // k contiguous.
 __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& p, int c, int nSteps, bool gen,
-                                            int64_t drawBase, int half, f2v (*v)[4]) {
+                                            int64_t drawBase, int half, f2v (*v)[NV]) {
     const unsigned kb = (unsigned)g.bSk * kElem;      // bytes per k
 #pragma unroll
     for (int st = 0; st < CS; st++) {
         const int s = CS * c + st < nSteps ? CS * c + st : nSteps - 1;
-        if constexpr (kFirst && kRealOps) {
+        if constexpr (kIso) {
+            auto run = [&](gch* t, unsigned lo, int n, f2v* o) {
+                const gf4* q = (const gf4*)(t + (int64_t)(2 * s) * n * 32 + (lo + (unsigned)(half * n) * 32u));
+                const f4v a = q[0], b = q[1];
+                o[0] = f2v{a.x, a.y};
+                o[1] = f2v{a.z, a.w};
+                o[2] = f2v{b.x, b.y};
+                o[3] = f2v{b.z, b.w};
+            };
+            run(p.S, p.lo0, g.isoNx, v[st]);
+            if (g.isoY) {
+                run(p.Y, p.lo1, g.isoNy, v[st] + 4);
+            } else {
+#pragma unroll
+                for (int i = 4; i < NV; i++) v[st][i] = f2v{1.f, 0.f};
+            }
+        } else if constexpr (kFirst && kRealOps) {
             struct __attribute__((packed, aligned(8))) pair { f2v a, b; };
             typedef const pair __attribute__((address_space(1))) gpair;
             gch* b = p.S + (p.lo0 + 64u * (unsigned)s);
@@ -153,7 +194,7 @@ __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& 
     }
 }
 
-__device__ __forceinline__ void strip_split(const f2v (*r)[4], double scale, unsigned sgn, u32x4 (*fh)[NA],
+__device__ __forceinline__ void strip_split(const f2v (*r)[NV], double scale, unsigned sgn, u32x4 (*fh)[NA],
                                             u32x4 (*fl)[NA]) {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -162,6 +203,12 @@ __device__ __forceinline__ void strip_split(const f2v (*r)[4], double scale, uns
         hv4 rh, rl, ih, il;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
+            if constexpr (kIso) {
+                const f2v w = r[st][i], y = r[st][4 + i];
+                re[i] = fmaf(w.x, y.x, -w.y * y.y);
+                im[i] = fmaf(w.x, y.y, w.y * y.x);
+                continue;
+            }
             re[i] = kFirst && kRealOps ? (float)(__builtin_bit_cast(double, r[st][i]) * scale) : r[st][i].x;
             im[i] = r[st][i].y;
         }
@@ -278,7 +325,8 @@ __device__ __forceinline__ void strip_store(const rf_gemm_desc& g, const strip& 
         const bool nIn = n < g.N;
         auto store = [&](auto* D, auto* G, auto* BL, auto* BH, auto one) {
             typedef decltype(one) T;
-            if (!g.grp) {
+            typedef std::conditional_t<kIso, int64_t, int> index;     // (isotropic planes of any size)
+            if (kIso || !g.grp) {
 #pragma unroll
                 for (int t = 0; t < MT; t++) {
                     const int R0 = 32 * (t0 + t);
@@ -288,7 +336,7 @@ __device__ __forceinline__ void strip_store(const rf_gemm_desc& g, const strip& 
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
                         const int m = 8 * (i >> 2) + 4 * half + (i & 3);
-                        if (nIn && (whole || R0 + m < rows)) d[m * dSm + l32] = (T)acc[t][0][i];
+                        if (nIn && (whole || R0 + m < rows)) d[(index)m * dSm + l32] = (T)acc[t][0][i];
                     }
                 }
                 return;
@@ -358,11 +406,11 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
 
     f32x16 acc[MT][NA];
     strip_zero<MT>(acc);
-    f2v r[CS][4];
+    f2v r[CS][NV];
     // chunk c of the table (steps CS c ..): 1 KB pieces over the waves; tiles
     // and steps past the table re-read its last ones, whose products are never
     // stored, resp. never formed
-    const u32x4* T = static_cast<const u32x4*>(g.T);
+    const u32x4* T = static_cast<const u32x4*>(g.T) + (kIso ? (int64_t)batch * nSteps * mtTot * 128 : 0);
     auto dma = [&](int c, u32x4* dst) {
         constexpr int kPieces = CS * MT * 2;
 #pragma unroll
@@ -434,7 +482,7 @@ void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) 
 template <int MT>
 hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks, hipStream_t s) {
     if (g) hipLaunchKernelGGL((k_strip<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, *g, n);
-    else if constexpr (kRealOps) return hipErrorInvalidValue;
+    else if constexpr (kRealOps || kIso) return hipErrorInvalidValue;
     else hipLaunchKernelGGL((k_strip_group<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, d_gs, nG, n);
     return hipGetLastError();
 }
@@ -451,8 +499,10 @@ hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64
 #define RF_STRIP_LAUNCH rf_strip_launch_first_real
 #elif RF_STRIP_PART == 4
 #define RF_STRIP_LAUNCH rf_strip_launch_middle_real
-#else
+#elif RF_STRIP_PART == 5
 #define RF_STRIP_LAUNCH rf_strip_launch_last_real
+#else
+#define RF_STRIP_LAUNCH rf_strip_launch_iso
 #endif
 hipError_t RF_STRIP_LAUNCH(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks,
                            hipStream_t s) {
