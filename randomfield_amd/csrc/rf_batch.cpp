@@ -29,6 +29,7 @@ struct rf_grid_batch {
     int nStrip[3] = {0, 0, 0};
     int64_t stripTiles[3] = {0, 0, 0}, fp32Tiles[3] = {0, 0, 0};
     int mt[3] = {1, 1, 1};
+    bool brief[3] = {false, false, false};   // every strip GEMM of the stage takes the short form
     // fresh realizations: every field's coefficient fold, its seed and Nmc,
     // and the device draw counter (realizations counter * Nmc .. of each
     // field's device stream)
@@ -60,11 +61,14 @@ hipError_t upload_stages(rf_grid_batch* B, hipStream_t s) {
     for (int k = 0; k < 3; k++) {
         int64_t t[2] = {0, 0};                      // strips, FP32 tiles
         B->nStrip[k] = 0;
+        B->brief[k] = true;
         for (auto& g : B->stage[k]) {
             const int fp32 = g.mt == 0;
             g.tile0 = t[fp32];
             t[fp32] += rf_gemm_tiles(g, fp32 ? 0 : B->mt[k]);
-            if (!fp32) B->nStrip[k]++;
+            if (fp32) continue;
+            B->nStrip[k]++;
+            B->brief[k] = B->brief[k] && rf_strip_short(g);
         }
         B->stripTiles[k] = t[0];
         B->fp32Tiles[k] = t[1];
@@ -79,7 +83,8 @@ hipError_t upload_stages(rf_grid_batch* B, hipStream_t s) {
 
 hipError_t run_stage(const rf_grid_batch* B, int k, hipStream_t s) {
     const int n = B->nStrip[k];
-    const hipError_t e = rf_launch_gemm_group(k, B->mt[k], B->d_desc[k], n, B->stripTiles[k], s);
+    const hipError_t e = rf_launch_gemm_group(k, B->mt[k] | (B->brief[k] ? kStripShort : 0), B->d_desc[k], n,
+                                              B->stripTiles[k], s);
     if (e != hipSuccess) return e;
     return rf_launch_gemm_group(k, 0, B->d_desc[k] + n, B->nDesc[k] - n, B->fp32Tiles[k], s);
 }

@@ -450,6 +450,7 @@ inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 // Logical tiles of a GEMM: blocks of strips x table groups, or FP32 tiles.
 int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt) {
+    mt &= ~kStripShort;
     if (mt > 0)
         return (int64_t)(((g.M + 31) / 32 + mt - 1) / mt) * (((int64_t)g.N + kStripL - 1) / kStripL) * g.batches;
     return (int64_t)((g.N + kTN - 1) / kTN) * ((g.M + kTM - 1) / kTM) * g.batches;
@@ -465,7 +466,7 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
                       hipStream_t s) {
     if (nTiles <= 0) return hipSuccess;
     const int64_t nb = xcd_blocks(nTiles);
-    if (nb > 0x7fffffffLL || mt < 0 || mt > kStripMaxMT) return hipErrorInvalidValue;
+    if (nb > 0x7fffffffLL || mt < 0 || (mt & ~kStripShort) > kStripMaxMT) return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)nb;
     if (kind == RF_GEMM_ISO) return rf_strip_launch_iso(mt, g, d_gs, nG, nTiles, blocks, s);
     if (mt > 0 && g && g->real) {
@@ -491,16 +492,16 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
 // MT of a strip GEMM: all of the table axis in one wave (up to kStripMaxMT
 // tiles) so that every streamed value is read and converted once, unless the
 // launch would then leave SIMDs without a wave.  The last contraction, whose
-// K is short and whose stores bound it, takes at most 3 tiles: 32 fields of
-// ~131^3 x 16 on 5 / 4 / 3 / 2 / 1 tiles: 2.62 / 2.31 / 2.29 / 2.29 / 2.66 ms;
-// 135 x 131 x 131 x 4 on 5 / 3: 24.8 / 20.6 us (128^3 x 8 on 4 / 2: 51 / 55).
+// stores bound it, takes at most 3 tiles: 32 fields of ~131^3 x 16 (K 44, short
+// form) on 4 / 3 / 2 / 1 tiles: 2.15 / 1.96 / 2.18 / 2.67 ms, in chunks 2.31 / 2.29 /
+// 2.29 / 2.66; 135 x 131 x 131 x 4 in chunks on 5 / 3: 24.8 / 20.6 us (a batch tunes it).
 int strip_choose(const rf_gemm_desc& g) {
     const int mt = (g.M + 31) / 32;
     const int64_t strips = (((int64_t)g.N + 31) / 32) * g.batches;
     const int most = g.kind == RF_GEMM_LAST ? 3 : kStripMaxMT;
     int gr = (mt + most - 1) / most;
     while (gr < mt && strips * gr < kStripFill) gr++;
-    return (mt + gr - 1) / gr;
+    return (mt + gr - 1) / gr | (rf_strip_short(g) ? kStripShort : 0);
 }
 }  // namespace
 

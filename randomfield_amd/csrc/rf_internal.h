@@ -279,6 +279,8 @@ inline rf_epilogue rf_make_epilogue(int margi, double avg, double var) {
 // streamed lines (B)
 constexpr int kStripMaxMT = 5;
 constexpr int kStripW = 4;            // waves per block
+constexpr int kStripShort = 8;        // flag of mt: all of K in one chunk (last contraction)
+constexpr int kStripShortCS = 6;      // its K-steps at most
 constexpr int kStripCS = 2;           // K-steps per fetch and table chunk
 constexpr int kStripL = 32 * kStripW; // lines per block
 constexpr int64_t kStripFill = 1024;  // waves below which a strip GEMM splits its table axis
@@ -411,6 +413,11 @@ struct rf_iso_grid_args {
 size_t rf_iso_grid_scratch_elems(int nDim, int64_t kN, int Nmc, const int32_t* n);
 hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s);
 int64_t rf_gemm_tiles(const rf_gemm_desc& g, int mt);
+// whether a strip GEMM may take the short form
+inline bool rf_strip_short(const rf_gemm_desc& g) {
+    const int steps = (g.K + 7) / 8;
+    return g.kind == RF_GEMM_LAST && steps > kStripCS && steps <= kStripShortCS;
+}
 hipError_t rf_launch_gemm_group(int kind, int mt, const rf_gemm_desc* d_gs, int nG, int64_t nTiles, hipStream_t s);
 // strips of one kind (rf_strip.hip): one GEMM (g) or a group (d_gs, nG)
 #define RF_STRIP_DECL(NAME)                                                                              \

@@ -42,7 +42,11 @@
 // axis) in the first contraction, whose D has the table axis contiguous.
 //
 // A block is kStripW waves; the table goes to LDS kStripCS steps at a time in a
-// double buffer, one barrier per chunk.
+// double buffer, one barrier per chunk.  A last contraction of at most
+// kStripShortCS steps (kStripShort) loads everything -- table and lines -- at once
+// instead: it is bound by its loads and stores, and every chunk exposed one more
+// memory latency.  The last contraction above 2.29 -> 1.96 ms to the fields, 2.45 ->
+// 2.40 into the group grid.
 #include "rf_grid_dev.h"
 
 #include <type_traits>
@@ -61,13 +65,12 @@ constexpr bool kFirst = kKind == RF_GEMM_FIRST, kLast = kKind == RF_GEMM_LAST ||
 constexpr bool kReal = kLast || kRealOps;   // Re D only
 constexpr int NA = kReal ? 1 : 2;       // accumulators per tile: Re, Im
 constexpr unsigned kElem = kRealOps && !kFirst ? 4u : 8u;   // bytes of a streamed element (real first: FP64)
-constexpr int CS = kStripCS;            // K-steps per fetch (and per table chunk)
 constexpr int NV = kIso ? 8 : 4;        // values of a lane per step (isotropic: two factors)
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const char __attribute__((address_space(1))) gch;
-constexpr int strip_units(int MT) { return CS * MT * 128; }   // 16-byte units of a chunk
+constexpr int strip_units(int MT, int CS) { return CS * MT * 128; }   // 16-byte units of a chunk
 
 // x and y hold k = 4 h + (0..3) in lane half h: half 0's x for all eight k in
 // half 0, half 1's y for all eight in half 1.
@@ -128,6 +131,7 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
 // (fold_coef_draw, as the fold would store them) instead of read.  Real first
 // contraction: the plan's FP64 amplitudes as they are (strip_split scales them),
 // k contiguous.
+template <int CS>
 __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& p, int c, int nSteps, bool gen,
                                             int64_t drawBase, int half, f2v (*v)[NV]) {
     const unsigned kb = (unsigned)g.bSk * kElem;      // bytes per k
@@ -194,6 +198,7 @@ __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& 
     }
 }
 
+template <int CS>
 __device__ __forceinline__ void strip_split(const f2v (*r)[NV], double scale, unsigned sgn, u32x4 (*fh)[NA],
                                             u32x4 (*fl)[NA]) {
 #pragma clang fp contract(off)
@@ -387,7 +392,7 @@ __device__ __forceinline__ void strip_store(const rf_gemm_desc& g, const strip& 
 
 // Logical tile `local` = (table group fastest -- the groups share
 // the streamed lines --, block of kStripW strips, batch).
-template <int MT>
+template <int MT, int CS>
 __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local, u32x4* ldsA, u32x4* ldsB) {
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -427,24 +432,29 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
     };
     auto chunk = [&](int c, const u32x4* cur, u32x4* nxt) {
         // fragments of this chunk's streamed values, then the loads of the next
-        u32x4 fh[CS][NA], fl[CS][NA];
-        strip_split(r, kFirst ? g.gen.ampMult : 1.0, sgn, fh, fl);
-        if (c + 1 < nChunks) {                        // in flight during the MFMAs
+        // (all of K in one chunk: step by step, for the registers)
+        constexpr bool kAll = CS == kStripCS;
+        const double scale = kFirst ? g.gen.ampMult : 1.0;
+        u32x4 fh[kAll ? CS : 1][NA], fl[kAll ? CS : 1][NA];
+        if constexpr (kAll) strip_split<CS>(r, scale, sgn, fh, fl);
+        if (CS == kStripCS && c + 1 < nChunks) {      // in flight during the MFMAs
             dma(c + 1, nxt);
-            strip_fetch(g, p, c + 1, nSteps, gen, drawBase, half, r);
+            strip_fetch<CS>(g, p, c + 1, nSteps, gen, drawBase, half, r);
         }
 #pragma unroll
         for (int st = 0; st < CS; st++) {
             if (!active || CS * c + st >= nSteps) break;                          // uniform
-            strip_step<MT>(cur + st * MT * 128, fh[st], fl[st], lane, acc);
+            if constexpr (!kAll) strip_split<1>(r + st, scale, sgn, fh, fl);
+            strip_step<MT>(cur + st * MT * 128, fh[kAll ? st : 0], fl[kAll ? st : 0], lane, acc);
         }
+        if (CS != kStripCS) return;                   // all of K in one chunk
         // this wave's direct loads are complete (vmcnt(0)) before the barrier
         // publishes them
         __builtin_amdgcn_s_waitcnt(0x0F70);
         __syncthreads();
     };
     dma(0, ldsA);
-    strip_fetch(g, p, 0, nSteps, gen, drawBase, half, r);
+    strip_fetch<CS>(g, p, 0, nSteps, gen, drawBase, half, r);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
     for (int c = 0; c < nChunks; c += 2) {
@@ -456,35 +466,47 @@ __device__ __forceinline__ void strip_tile(const rf_gemm_desc& g, int64_t local,
 
 // Registers: 16 MT accumulators per lane (32 MT complex) decide the waves per
 // SIMD; the compiler then keeps them in VGPRs without spills.
-constexpr int strip_waves(int MT) { return NA == 1 ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4); }
-
-template <int MT, int KIND, bool REAL>
-__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT))))
-void k_strip(rf_gemm_desc g, int64_t nTiles) {
-    __shared__ u32x4 ldsA[strip_units(MT)];
-    __shared__ u32x4 ldsB[strip_units(MT)];
-    const int64_t L = xcd_tile(blockIdx.x, nTiles);
-    if (L >= nTiles) return;
-    strip_tile<MT>(g, L, ldsA, ldsB);
+constexpr int strip_waves(int MT, int CS) {
+    if (CS != kStripCS) return MT >= 4 ? 2 : 3;
+    return NA == 1 ? (MT >= 3 ? 3 : 4) : (MT >= 3 ? 2 : MT == 2 ? 3 : 4);
 }
 
-template <int MT, int KIND, bool REAL>
-__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT))))
+template <int MT, int CS, int KIND, bool REAL>
+__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, CS))))
+void k_strip(rf_gemm_desc g, int64_t nTiles) {
+    __shared__ u32x4 ldsA[strip_units(MT, CS)];
+    __shared__ u32x4 ldsB[CS == kStripCS ? strip_units(MT, CS) : 1];
+    const int64_t L = xcd_tile(blockIdx.x, nTiles);
+    if (L >= nTiles) return;
+    strip_tile<MT, CS>(g, L, ldsA, ldsB);
+}
+
+template <int MT, int CS, int KIND, bool REAL>
+__global__ __launch_bounds__(64 * kStripW) __attribute__((amdgpu_waves_per_eu(strip_waves(MT, CS))))
 void k_strip_group(const rf_gemm_desc* __restrict__ gs, int nG, int64_t nTiles) {
-    __shared__ u32x4 ldsA[strip_units(MT)];
-    __shared__ u32x4 ldsB[strip_units(MT)];
+    __shared__ u32x4 ldsA[strip_units(MT, CS)];
+    __shared__ u32x4 ldsB[CS == kStripCS ? strip_units(MT, CS) : 1];
     const int64_t L = xcd_tile(blockIdx.x, nTiles);
     if (L >= nTiles) return;
     const rf_gemm_desc g = gs[gemm_find(gs, nG, L)];   // uniform: scalar registers
-    strip_tile<MT>(g, L - g.tile0, ldsA, ldsB);
+    strip_tile<MT, CS>(g, L - g.tile0, ldsA, ldsB);
+}
+
+template <int MT, int CS>
+hipError_t launch_cs(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks, hipStream_t s) {
+    if (g) hipLaunchKernelGGL((k_strip<MT, CS, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, *g, n);
+    else if constexpr (kRealOps || kIso) return hipErrorInvalidValue;
+    else hipLaunchKernelGGL((k_strip_group<MT, CS, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, d_gs, nG, n);
+    return hipGetLastError();
 }
 
 template <int MT>
-hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks, hipStream_t s) {
-    if (g) hipLaunchKernelGGL((k_strip<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, *g, n);
-    else if constexpr (kRealOps || kIso) return hipErrorInvalidValue;
-    else hipLaunchKernelGGL((k_strip_group<MT, kKind, kRealOps>), dim3(blocks), dim3(64 * kStripW), 0, s, d_gs, nG, n);
-    return hipGetLastError();
+hipError_t launch(bool brief, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks,
+                  hipStream_t s) {
+    if constexpr (kKind == RF_GEMM_LAST) {
+        if (brief) return launch_cs<MT, kStripShortCS>(g, d_gs, nG, n, blocks, s);
+    }
+    return launch_cs<MT, kStripCS>(g, d_gs, nG, n, blocks, s);
 }
 
 }  // namespace
@@ -506,11 +528,12 @@ hipError_t launch(const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64
 #endif
 hipError_t RF_STRIP_LAUNCH(int mt, const rf_gemm_desc* g, const rf_gemm_desc* d_gs, int nG, int64_t n, unsigned blocks,
                            hipStream_t s) {
-    switch (mt) {
-        case 1: return launch<1>(g, d_gs, nG, n, blocks, s);
-        case 2: return launch<2>(g, d_gs, nG, n, blocks, s);
-        case 3: return launch<3>(g, d_gs, nG, n, blocks, s);
-        case 4: return launch<4>(g, d_gs, nG, n, blocks, s);
-        default: return launch<kStripMaxMT>(g, d_gs, nG, n, blocks, s);
+    const bool brief = mt & kStripShort;
+    switch (mt & ~kStripShort) {
+        case 1: return launch<1>(brief, g, d_gs, nG, n, blocks, s);
+        case 2: return launch<2>(brief, g, d_gs, nG, n, blocks, s);
+        case 3: return launch<3>(brief, g, d_gs, nG, n, blocks, s);
+        case 4: return launch<4>(brief, g, d_gs, nG, n, blocks, s);
+        default: return launch<kStripMaxMT>(brief, g, d_gs, nG, n, blocks, s);
     }
 }
