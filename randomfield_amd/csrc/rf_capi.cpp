@@ -313,7 +313,8 @@ int rf_plan_create(rf_context* ctx, const rf_params* p, const double* kUniform,
 
     // operand buffers of the chosen form
     // isotropic: the components are bounded by the radii
-    for (double v : P->spec.k) P->kAbsMax = std::max(P->kAbsMax, std::fabs(v));
+    if (p->form == RF_FORM_FP64 || (p->form == RF_FORM_FP32 && is_iso_direct(*p)))
+        for (double v : P->spec.k) P->kAbsMax = std::max(P->kAbsMax, std::fabs(v));
     if (p->form == RF_FORM_FP64) RF_HIP_TRY(ctx, dmalloc(&P->d_CS, (size_t)(kN * P->Rpad)));
     if (p->form == RF_FORM_FP32 && is_iso_direct(*p)) {
         const int64_t nb = rf_iso_blocks(kN, Nmc);

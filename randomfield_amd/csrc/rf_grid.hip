@@ -242,6 +242,7 @@ __global__ __launch_bounds__(256) void k_iso_tables(rf_iso_tables t) {
         return;
     }
     _Float16* F = t.Z + (r * t.kP * t.w[a] + (e & ~(int64_t)255)) * 4 + (e & 255);
+    asm("" : "+v"(v.x), "+v"(v.y));
     const _Float16 ch = (_Float16)v.x, sh = (_Float16)v.y;
     F[0] = ch;
     F[256] = sh;
@@ -289,7 +290,10 @@ __global__ __launch_bounds__(256) void k_axis_tables(rf_table_args t) {
                 if (v) sn = -sn;
             }
         }
-        const float cf = (float)c, sf = (float)sn;
+        // rounded to FP32 first, then split (opaque: the two conversions would be
+        // folded into one)
+        float cf = (float)c, sf = (float)sn;
+        asm("" : "+v"(cf), "+v"(sf));
         const _Float16 ch = (_Float16)cf, sh = (_Float16)sf;
         _Float16* F = static_cast<_Float16*>(t.E[a]) + st * 1024 + row * 8 + q;
         F[0] = ch;
