@@ -284,7 +284,10 @@ int rf_grid_batch_autotune(rf_grid_batch* B, void* stream, int32_t* chosen) {
             if (g.mt > 0) mtTot = std::max(mtTot, (g.M + 31) / 32);
         float best = 0.0f;
         int bestMt = B->mt[k];
-        for (int mt = std::min(mtTot, kStripMaxMT); mt >= 1 && e == hipSuccess; mt--) {
+        const int top = std::min(mtTot, kStripMaxMT);
+        for (int mt = top; mt >= 1 && e == hipSuccess; mt--) {
+            // the smallest of each number of groups; single tiles only where there are few
+            if (mt == 1 ? mtTot > 3 : (mtTot + mt - 1) / mt == (mtTot + mt - 2) / (mt - 1)) continue;
             B->mt[k] = mt;
             e = upload_stages(B, s);
             float ms = 0.0f;

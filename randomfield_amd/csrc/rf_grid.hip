@@ -564,19 +564,18 @@ hipError_t rf_grid_prepare(int kind, int nDim, int Nmc, const int32_t* kNStep, c
     while (nDim == 3 && std::ldexp(bound2, -m2) > 16384.0) m2++;
     int split = bound1 <= 16384.0 ? 1 : 0;
 
-    // the strip GEMM addresses inside a strip with 32-bit offsets: one k of the
-    // streamed operand, one row or line of D (elements)
+    // the strip GEMM addresses eight k of a strip's lines in 32-bit bytes and a
+    // tile of D in 32-bit elements
     {
-        const int64_t lim = (int64_t)1 << 27;
+        const int64_t lim = (int64_t)1 << 29;
         int64_t rows1 = (int64_t)Nmc * Q, plane = n[0];
         for (int a = 1; a < nDim; a++) rows1 *= kNStep[a];
         if (nDim == 3) plane *= n[1];
         int64_t span = 8 * rows1;                                       // first: K-major coefficients
-        if (32LL * n[0] > span) span = 32LL * n[0];                     // first: D
-        if (8 * plane > span) span = 8 * plane;                         // last: streamed
-        if (32LL * kStripMaxMT * plane > span) span = 32LL * kStripMaxMT * plane;   // last: D
-        if (nDim == 3 && ((int64_t)K2 + 160) * n[0] + plane > span)     // middle: streamed and D
-            span = ((int64_t)K2 + 160) * n[0] + plane;
+        if (8LL * n[0] > span) span = 8LL * n[0];                       // first: D (32 lines), a quarter
+        if (8 * plane > span) span = 8 * plane;                         // last: streamed, D
+        if (nDim == 3 && ((int64_t)K2 + 8) * n[0] > span) span = ((int64_t)K2 + 8) * n[0];      // middle: streamed
+        if (nDim == 3 && 40LL * n[0] + plane > span) span = 40LL * n[0] + plane;                // middle: D
         if (span >= lim) split = 0;
     }
 

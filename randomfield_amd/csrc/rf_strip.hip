@@ -89,8 +89,8 @@ struct strip {
     // descriptor of a grouped launch is read from memory, and generic (flat)
     // loads would also count against the LDS wait counter.
     gch* S;
-    gch* Y;                               // isotropic: the second factor
-    unsigned lo0, lo1;
+    gch* Y;                               // isotropic: the lane's values of the second factor (S: of the first)
+    unsigned lo0;
     int batch, n0;
     unsigned gr, gj3, gq, gj2;            // drawn coefficients: the line's digits
 };
@@ -101,14 +101,13 @@ __device__ __forceinline__ strip strip_at(const rf_gemm_desc& g, int batch, int 
     p.n0 = n0;
     const int nc = n0 + l32 < g.N ? n0 + l32 : g.N - 1;
     p.Y = nullptr;
-    p.lo1 = 0;
     p.gr = p.gj3 = p.gq = p.gj2 = 0;
     if constexpr (kIso) {
         // tables [k / 4][index][k % 4]: a lane's four k are 32 bytes
-        p.S = (gch*)(g.B + (int64_t)batch * g.bStrideB);
-        p.Y = (gch*)(g.isoY + (int64_t)batch * g.isoYStrideB);
-        p.lo0 = 32u * (unsigned)(nc % g.isoNx);
-        p.lo1 = 32u * (unsigned)(nc / g.isoNx);
+        const int64_t half = (threadIdx.x >> 5) & 1;
+        p.S = (gch*)(g.B + (int64_t)batch * g.bStrideB) + 32 * (nc % g.isoNx + half * g.isoNx);
+        p.Y = (gch*)(g.isoY + (int64_t)batch * g.isoYStrideB) + 32 * (nc / g.isoNx + half * g.isoNy);
+        p.lo0 = 0;
         return p;
     }
     const int64_t col0 = col_b(g, n0);
@@ -139,17 +138,17 @@ __device__ __forceinline__ void strip_fetch(const rf_gemm_desc& g, const strip& 
     for (int st = 0; st < CS; st++) {
         const int s = CS * c + st < nSteps ? CS * c + st : nSteps - 1;
         if constexpr (kIso) {
-            auto run = [&](gch* t, unsigned lo, int n, f2v* o) {
-                const gf4* q = (const gf4*)(t + (int64_t)(2 * s) * n * 32 + (lo + (unsigned)(half * n) * 32u));
+            auto run = [&](gch* t, int n, f2v* o) {
+                const gf4* q = (const gf4*)(t + (int64_t)(2 * s) * n * 32);
                 const f4v a = q[0], b = q[1];
                 o[0] = f2v{a.x, a.y};
                 o[1] = f2v{a.z, a.w};
                 o[2] = f2v{b.x, b.y};
                 o[3] = f2v{b.z, b.w};
             };
-            run(p.S, p.lo0, g.isoNx, v[st]);
+            run(p.S, g.isoNx, v[st]);
             if (g.isoY) {
-                run(p.Y, p.lo1, g.isoNy, v[st] + 4);
+                run(p.Y, g.isoNy, v[st] + 4);
             } else {
 #pragma unroll
                 for (int i = 4; i < NV; i++) v[st][i] = f2v{1.f, 0.f};

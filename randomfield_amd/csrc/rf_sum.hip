@@ -235,12 +235,13 @@ __global__ __launch_bounds__(kBlock) void k_sum_fp32(rf_sum_args a, const double
 // makes it the float 1 + argument (23 bits, rounded by the 2^-24) that v_cos_f32
 // takes.  A term costs three VALU instructions (alignbit, cosine, FMA), the
 // matrix cores run beside them.  Formerly eight, four of them FP64 (k.x by FMAs,
-// v_fract_f64): 200,000 points x 16 realizations, ~480 shells 375 -> 254 us.
+// v_fract_f64): 200,000 points x 16 realizations, 286 shells 382 -> 254
+// us (128^3 x 64: 9.2 -> 8.7 ms).
 // Arguments that may reach 2^19 revolutions (or are not finite) take a zero
 // accumulator and v_fract_f64; the choice is per wave.
 // kA [block][4][16], aA [block][row % 4][row / 4], block = wavevector block x chunks
 // + chunk; padded rows have zero amplitude.  Two groups of 16 points per wave:
-// four waves of 32 points spread 20,000 points over the CUs more evenly than 64 would.
+// four waves of 32 points spread 200,000 points over the CUs more evenly than 64 would.
 typedef double d4v __attribute__((ext_vector_type(4)));
 typedef const double __attribute__((address_space(1))) gdbl;
 typedef float f4v __attribute__((ext_vector_type(4)));

@@ -101,3 +101,24 @@ def test_real_operands(ctx, gn):
     assert e <= 1e-5
     b.close()
     plan.close()
+
+
+def test_wide_planes(ctx):
+    """A plane of a million points stays on the strips (64 points against the oracle)."""
+    import torch
+    n, step = (1000, 1024, 2), (0.02, 0.02, 0.5)
+    ext = [(n[a] - 1) * step[a] for a in range(3)]
+    p = R.make_params(nDim=3, method=R.SHINOZUKA, mode=R.FIXED, form=R.FORM_FP32, Nmc=1, corrL=(1.0,) * 3, xRange=ext)
+    _, phU = R.reference_draws(p, R.reference_seed(3))
+    plan = R.FieldPlan(ctx, p, None, phU)
+    out = torch.empty((1, int(np.prod(n))), dtype=torch.float32, device="cuda")
+    plan.execute_grid((0.0,) * 3, step, n, out)
+    ctx.sync()
+    pick = np.unique(np.r_[0, np.prod(n) - 1, np.random.default_rng(1).integers(0, np.prod(n), 62)])
+    x = np.stack([pick % n[0] * step[0], pick // n[0] % n[1] * step[1], pick // (n[0] * n[1]) * step[2]], 1)
+    po = O.make_plan(3, O.SHINOZUKA, O.FIXED, ext)
+    k = O.kpoints(po)
+    ref = O.shinozuka(po, x, k, O.skvec(po, k), phU)
+    got = out.cpu().numpy()[:, pick]
+    assert float(np.sqrt(np.mean((got - ref) ** 2) / np.mean(ref ** 2))) <= 3e-6
+    plan.close()
