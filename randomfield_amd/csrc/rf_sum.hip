@@ -230,28 +230,32 @@ __global__ __launch_bounds__(kBlock) void k_sum_fp32(rf_sum_args a, const double
 // (wavevector, realization): (kx, ky, kz, phi) in revolutions; a column of B is one
 // point: (x, y, z, 1).  The 16 rows are 16 / Rp wavevectors x Rp realizations, Rp
 // the power of two (at most 16) that holds Nmc; larger Nmc in chunks of 16.
-// The accumulator starts at 1.5 2^20 + 2^-24, whose last place is 2^-32: the
-// low word of D is then the argument modulo one revolution, and one v_alignbit
-// makes it the float 1 + argument (23 bits, rounded by the 2^-24) that v_cos_f32
-// takes.  A term costs three VALU instructions (alignbit, cosine, FMA), the
-// matrix cores run beside them.  Formerly eight, four of them FP64 (k.x by FMAs,
-// v_fract_f64): 200,000 points x 16 realizations, 286 shells 382 -> 254
-// us (128^3 x 64: 9.2 -> 8.7 ms).
+// The accumulator starts at 1.5 2^20, whose last place is 2^-32: the low word of
+// D is then the argument modulo one revolution in 2^-32 (signed), converted and
+// scaled for v_cos_f32.  A term costs four VALU instructions and a sixteenth of
+// an MFMA of 64 cycles, which the VALU does not overlap; k.x by FMAs, v_fract_f64 and
+// the phase cost eight (36 cycles either way), so what is gained is the
+// packing of few realizations and waves of 32 points where a field is small:
+// 200,000 points x 16 realizations, 286 shells 375 -> 284 us (error 1.9e-7 -> 1.8e-7),
+// 128^3 x 64 9.25 -> 9.27 ms.  One instruction less -- v_alignbit of the word to a
+// float 1 + argument of 23 bits -- gave 254 us and 8.66 ms with an error of 2.1e-7.
 // Arguments that may reach 2^19 revolutions (or are not finite) take a zero
 // accumulator and v_fract_f64; the choice is per wave.
 // kA [block][4][16], aA [block][row % 4][row / 4], block = wavevector block x chunks
-// + chunk; padded rows have zero amplitude.  Two groups of 16 points per wave:
-// four waves of 32 points spread 200,000 points over the CUs more evenly than 64 would.
+// + chunk; padded rows have zero amplitude.  Q groups of 16 points per wave: 2
+// spread 200,000 points over the CUs more evenly than 4, whose operand loads and
+// loop weigh half (128^3 x 64: 9.70 ms on 2, 9.27 on 4).
 typedef double d4v __attribute__((ext_vector_type(4)));
 typedef const double __attribute__((address_space(1))) gdbl;
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef const f4v __attribute__((address_space(1))) gf4;
-constexpr int kIsoQ = 2;                               // 16-point groups of a wave
+constexpr int kIsoQ = 2;                               // 16-point groups of a wave, small fields and batches
 static_assert(kGroupIsoPts == kBlock / 64 * 16 * kIsoQ, "points of a block");
 
+template <int Q>
 __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict__ kA, gf4* __restrict__ aA, int64_t nJ,
-                                          int nChunk, int chunk, int Rp, double kMax, int64_t p0, float (*red)[16 * kIsoQ]) {
-    constexpr int Q = kIsoQ, P = 16 * Q;
+                                          int nChunk, int chunk, int Rp, double kMax, int64_t p0, float (*red)[16 * Q]) {
+    constexpr int P = 16 * Q;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
     const int64_t pw = p0 + wave * P;
     double b[Q];
@@ -271,6 +275,14 @@ __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict
         const d4v C = {c0, c0, c0, c0};
         gdbl* kp = kA + (int64_t)chunk * 64 + lane;
         gf4* ap = aA + (int64_t)chunk * 4 + g;
+        auto terms = [&](double kj, const f4v& aj) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                const d4v t = __builtin_amdgcn_mfma_f64_16x16x4f64(kj, b[q], C, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[q][e] = fmaf(aj[e], __builtin_amdgcn_cosf(turn(t[e])), acc[q][e]);
+            }
+        };
         double kn = *kp;
         f4v an = *ap;
         for (int64_t j = 0; j < nJ; j++) {
@@ -282,18 +294,11 @@ __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict
                 kn = *kp;
                 an = *ap;
             }
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const d4v t = __builtin_amdgcn_mfma_f64_16x16x4f64(kj, b[q], C, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[q][e] = fmaf(aj[e], __builtin_amdgcn_cosf(turn(t[e])), acc[q][e]);
-            }
+            terms(kj, aj);
         }
     };
     if (!__any(far))
-        sweep(1572864.0 + 0x1p-24, [](double t) {
-            return __builtin_bit_cast(float, __builtin_amdgcn_alignbit(0x7Fu, (unsigned)__builtin_bit_cast(uint64_t, t), 9));
-        });
+        sweep(1572864.0, [](double t) { return (float)(int)(unsigned)__builtin_bit_cast(uint64_t, t) * 0x1p-32f; });
     else
         sweep(0.0, [](double t) { return (float)__builtin_amdgcn_fract(t); });
     // D: column c, rows 4 e + g; the wavevectors of a block added in row order
@@ -311,10 +316,12 @@ __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict
     }
 }
 
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_sum_fp32_iso(rf_sum_args a, const double* __restrict__ kA,
-                                                         const float* __restrict__ aA, int64_t nJ, int Rp, double kMax) {
-    __shared__ float red[kBlock / 64 * 16][16 * kIsoQ];
-    iso_block(a, (gdbl*)kA, (gf4*)aA, nJ, gridDim.y, blockIdx.y, Rp, kMax, a.i0 + (int64_t)blockIdx.x * kGroupIsoPts, red);
+template <int Q>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(Q > 2 ? 6 : 8))) void k_sum_fp32_iso(
+    rf_sum_args a, const double* __restrict__ kA, const float* __restrict__ aA, int64_t nJ, int Rp, double kMax) {
+    __shared__ float red[kBlock / 64 * 16][16 * Q];
+    iso_block<Q>(a, (gdbl*)kA, (gf4*)aA, nJ, gridDim.y, blockIdx.y, Rp, kMax, a.i0 + (int64_t)blockIdx.x * (kBlock / 4 * Q),
+                 red);
 }
 
 // Grouped form: block b runs one tile = (field, kGroupIsoPts points, chunk of
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     const rf_group_req& q = reqs[lo];
     const rf_iso_shape sh = rf_iso_rows(q.a.kN, q.a.Nmc);
     const int64_t local = b - q.tile0;
-    iso_block(q.a, (gdbl*)q.ops0, (gf4*)q.ops1, sh.nJ, sh.nChunk, (int)(local % sh.nChunk), sh.Rp, q.kMax,
+    iso_block<kIsoQ>(q.a, (gdbl*)q.ops0, (gf4*)q.ops1, sh.nJ, sh.nChunk, (int)(local % sh.nChunk), sh.Rp, q.kMax,
               (local / sh.nChunk) * kGroupIsoPts, red);
 }
 
@@ -419,10 +426,15 @@ hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kA, co
                                     hipStream_t s) {
     if (a.i1 <= a.i0) return hipSuccess;
     const rf_iso_shape sh = rf_iso_rows(a.kN, a.Nmc);
-    const int64_t blocks = (a.i1 - a.i0 + kGroupIsoPts - 1) / kGroupIsoPts;
+    // 64 points per wave where that still gives every SIMD about sixteen waves
+    // (the operand loads and the loop weigh half), else 32
+    const bool wide = (a.i1 - a.i0) / 64 * sh.nChunk >= 16384;
+    const int pts = kBlock / 4 * (wide ? 4 : kIsoQ);
+    const int64_t blocks = (a.i1 - a.i0 + pts - 1) / pts;
     if (blocks > 0x7fffffffLL || sh.nChunk > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_sum_fp32_iso, dim3((unsigned)blocks, (unsigned)sh.nChunk), dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ,
-                       sh.Rp, kMax);
+    const dim3 grid((unsigned)blocks, (unsigned)sh.nChunk);
+    if (wide) hipLaunchKernelGGL(k_sum_fp32_iso<4>, grid, dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
+    else hipLaunchKernelGGL(k_sum_fp32_iso<kIsoQ>, grid, dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
     return hipGetLastError();
 }
 
