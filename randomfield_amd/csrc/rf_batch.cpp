@@ -75,7 +75,7 @@ hipError_t upload_stages(rf_grid_batch* B, hipStream_t s) {
         all.insert(all.end(), B->stage[k].begin(), B->stage[k].end());
     }
     for (int k = 0; k < 3; k++)
-        if (B->stripTiles[k] > 0x7fffffffLL || B->fp32Tiles[k] > 0x7fffffffLL) return hipErrorInvalidValue;
+        if (B->stripTiles[k] > rf_max_blocks(256) || B->fp32Tiles[k] > rf_max_blocks(256)) return hipErrorInvalidValue;
     hipError_t e = hipMemcpyAsync(B->d_desc[0], all.data(), all.size() * sizeof(rf_gemm_desc), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     return e;

@@ -470,7 +470,7 @@ hipError_t launch_any(int kind, int mt, const rf_gemm_desc* g, const rf_gemm_des
                       hipStream_t s) {
     if (nTiles <= 0) return hipSuccess;
     const int64_t nb = xcd_blocks(nTiles);
-    if (nb > 0x7fffffffLL || mt < 0 || (mt & ~kStripShort) > kStripMaxMT) return hipErrorInvalidValue;
+    if (nb > rf_max_blocks(256) || mt < 0 || (mt & ~kStripShort) > kStripMaxMT) return hipErrorInvalidValue;
     const unsigned blocks = (unsigned)nb;
     if (kind == RF_GEMM_ISO) return rf_strip_launch_iso(mt, g, d_gs, nG, nTiles, blocks, s);
     if (mt > 0 && g && g->real) {
@@ -713,7 +713,7 @@ void rf_fold_item_init(rf_fold_item* it, const rf_fold_desc& f, int Nmc, uint64_
 hipError_t rf_launch_refold_draw(const rf_fold_item* d_items, int n, int64_t blocks, const int64_t* d_draw,
                                  hipStream_t s) {
     if (n <= 0 || blocks <= 0) return hipSuccess;
-    if (!d_items || !d_draw || xcd_blocks(blocks) > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (!d_items || !d_draw || xcd_blocks(blocks) > rf_max_blocks(256)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_coeffs_fold_draw, dim3((unsigned)xcd_blocks(blocks)), dim3(256), 0, s, d_items, n, d_draw,
                        blocks);
     return hipGetLastError();
@@ -784,7 +784,7 @@ hipError_t rf_launch_iso_grid(const rf_iso_grid_args& a, hipStream_t s) {
         p += a.Nmc * kP * t.w[d];
     }
     const int64_t cnt = a.Nmc * kP * ((int64_t)t.w[0] + t.w[1] + t.w[2]);
-    if ((cnt + 255) / 256 > 0x7fffffffLL) return hipErrorInvalidValue;
+    if ((cnt + 255) / 256 > rf_max_blocks(256)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_iso_tables, dim3(blocks_for(cnt)), dim3(256), 0, s, t);
     rf_gemm_desc g{};
     g.kind = RF_GEMM_ISO;

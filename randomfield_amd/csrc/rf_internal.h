@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/rf_capi.h"
+#include "rf_ranges.h"
 
 // constants_RF.f90:5 -- the reference's pi literal (phases, spectra, tapers).
 #define RF_PI_REF 3.1415926535898

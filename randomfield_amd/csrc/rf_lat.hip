@@ -296,15 +296,15 @@ void k_lat(rf_sum_args a, rf_lat_dev L, int mtTotal, const u32x4* __restrict__ p
 }
 
 // A batch of independent fields on one lattice (requests of a serving batch,
-// all of one shape): block b runs one tile = (field, 32 W points, up to kLatMT
+// all of one shape): block b of a launch from tile0 runs tile tile0 + b = (field, 32 W points, up to kLatMT
 // M-tiles); the per-point operation order is that of k_lat.
 template <typename V, int W, int KG>
 __global__ __launch_bounds__(64 * W * KG) __attribute__((amdgpu_waves_per_eu(4)))
-void k_group_lat(const rf_group_req* __restrict__ reqs, int nReq, rf_lat_dev L) {
+void k_group_lat(const rf_group_req* __restrict__ reqs, int nReq, rf_lat_dev L, int64_t tile0) {
     __shared__ u32x4 panA[lat_units(KG)];
     __shared__ u32x4 panB[lat_units(KG)];
     extern __shared__ float2 lat_tab[];
-    const int64_t b = blockIdx.x;
+    const int64_t b = tile0 + blockIdx.x;
     const rf_group_req& q = reqs[group_find(reqs, nReq, b)];
     const int nSub = (q.mtTotal + kLatMT - 1) / kLatMT;
     const int64_t local = b - q.tile0;
@@ -419,10 +419,13 @@ hipError_t launch(const rf_sum_args& a, const rf_lat_dev& L, int mtTotal, const 
     static const hipError_t ok = allow_lds(k_lat<V, D, MT, W, KG>);
     if (ok != hipSuccess) return ok;
     const int64_t blocks = (a.i1 - a.i0 + 32 * W - 1) / (32 * W);
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_lat<V, D, MT, W, KG>), dim3((unsigned)blocks, (unsigned)((mtTotal + kLatMT - 1) / kLatMT)),
-                       dim3(64 * W * KG), table_bytes(L, W), s, a, L, mtTotal, static_cast<const u32x4*>(B), sc);
-    return hipGetLastError();
+    return rf_block_ranges(blocks, 64 * W * KG, [&](int64_t first, unsigned n) {
+        rf_sum_args q = a;
+        q.i0 += first * (32 * W);
+        hipLaunchKernelGGL((k_lat<V, D, MT, W, KG>), dim3(n, (unsigned)((mtTotal + kLatMT - 1) / kLatMT)),
+                           dim3(64 * W * KG), table_bytes(L, W), s, q, L, mtTotal, static_cast<const u32x4*>(B), sc);
+        return hipGetLastError();
+    });
 }
 
 template <typename V, int D>
@@ -437,9 +440,10 @@ template <typename V, int W, int KG>
 hipError_t launch_group(const rf_lat_dev& L, const rf_group_req* d_reqs, int nReq, int64_t nTiles, hipStream_t s) {
     static const hipError_t ok = allow_lds(k_group_lat<V, W, KG>);
     if (ok != hipSuccess) return ok;
-    hipLaunchKernelGGL((k_group_lat<V, W, KG>), dim3((unsigned)nTiles), dim3(64 * W * KG), table_bytes(L, W), s, d_reqs,
-                       nReq, L);
-    return hipGetLastError();
+    return rf_block_ranges(nTiles, 64 * W * KG, [&](int64_t first, unsigned n) {
+        hipLaunchKernelGGL((k_group_lat<V, W, KG>), dim3(n), dim3(64 * W * KG), table_bytes(L, W), s, d_reqs, nReq, L, first);
+        return hipGetLastError();
+    });
 }
 
 }  // namespace
@@ -471,7 +475,7 @@ hipError_t rf_launch_lat_prep(int form, int nDim, const rf_lat_dev& L, int Nmc, 
                               hipStream_t s) {
     const int mtTotal = Npad / 32;
     const int64_t grid = (L.nSteps * mtTotal * 64 + 255) / 256;
-    if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (grid > rf_max_blocks(256)) return hipErrorInvalidValue;
     if (form == RF_FORM_MFMA_BF16)
         hipLaunchKernelGGL(k_lat_prep<__bf16>, dim3((unsigned)grid), dim3(256), 0, s, nDim, L, Nmc, mtTotal, d_phase, seed,
                            d_amp, ampStrideR, scale, static_cast<__bf16*>(d_B));
@@ -496,7 +500,6 @@ hipError_t rf_launch_sum_lat(int form, const rf_sum_args& a, const rf_lat_dev& L
 hipError_t rf_launch_group_lat(int form, int small, const rf_lat_dev& L, const rf_group_req* d_reqs, int nReq,
                                int64_t nTiles, hipStream_t s) {
     if (nTiles <= 0 || nReq <= 0) return hipSuccess;
-    if (nTiles > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool bf = form == RF_FORM_MFMA_BF16;
     if (small)
         return bf ? launch_group<b8, 4, 4>(L, d_reqs, nReq, nTiles, s) : launch_group<h8, 4, 4>(L, d_reqs, nReq, nTiles, s);

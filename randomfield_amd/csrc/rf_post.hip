@@ -1074,7 +1074,7 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
     const bool g64 = gridDtype == RF_DTYPE_F64, o64 = outDtype == RF_DTYPE_F64;
     const int NT = !wide ? 256 : g64 ? 512 : 1024;
     const int64_t nBlocks = (nNodes + NT - 1) / NT;
-    if (nBlocks > 0x7ffffff8LL) return hipErrorInvalidValue;
+    if ((nBlocks + 7) / 8 * 8 > rf_max_blocks(NT)) return hipErrorInvalidValue;
     const dim3 grid2((unsigned)((nBlocks + 7) / 8 * 8), (unsigned)((Nmc + RC - 1) / RC));
     if (grid2.y > 65535) return hipErrorInvalidValue;
     auto run = [&](auto dim, auto* g, auto* o) {

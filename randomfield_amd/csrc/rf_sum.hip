@@ -12,6 +12,8 @@
 //    FMA.  Wavevector, phase and amplitude operands are wave-uniform and come
 //    through scalar loads, so the inner loop is pure VALU/transcendental work.
 //    With per-realization directions the arguments come from the FP64 matrix cores.
+#include <algorithm>
+
 #include "rf_internal.h"
 
 namespace {
@@ -173,19 +175,19 @@ __global__ __launch_bounds__(64 * kF64Waves) void k_sum_fp64(rf_sum_args a, cons
 __global__ __launch_bounds__(kBlock) void k_prep_fp64(int64_t kN, int Nmc, int Rpad, int iso,
                                                       const double* __restrict__ phase,
                                                       const double* __restrict__ amp, double2* __restrict__ CS) {
-    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (e >= kN * Rpad) return;
-    const int64_t j = iso ? e % kN : e / Rpad;
-    const int r = (int)(iso ? e / kN : e - j * Rpad);
-    double2 v = {0.0, 0.0};
-    if (r < Nmc) {
-        const double A = amp[(int64_t)r * kN + j];
-        double sn, cs;
-        sincos(phase[(int64_t)r * kN + j], &sn, &cs);
-        v.x = A * cs;
-        v.y = -A * sn;
+    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < kN * Rpad; e += (int64_t)gridDim.x * kBlock) {
+        const int64_t j = iso ? e % kN : e / Rpad;
+        const int r = (int)(iso ? e / kN : e - j * Rpad);
+        double2 v = {0.0, 0.0};
+        if (r < Nmc) {
+            const double A = amp[(int64_t)r * kN + j];
+            double sn, cs;
+            sincos(phase[(int64_t)r * kN + j], &sn, &cs);
+            v.x = A * cs;
+            v.y = -A * sn;
+        }
+        CS[e] = v;
     }
-    CS[e] = v;
 }
 
 // ---------------------------------------------------------------- FP32 form
@@ -324,12 +326,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(Q > 2 ? 
                  red);
 }
 
-// Grouped form: block b runs one tile = (field, kGroupIsoPts points, chunk of
+// Grouped form: block b of a launch from tile0 runs tile tile0 + b = (field, kGroupIsoPts points, chunk of
 // 16 realizations), found by binary search over the fields' first tiles; same
 // per-point operation order as k_sum_fp32_iso.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_group_iso(const rf_group_req* __restrict__ reqs, int nReq) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_group_iso(
+    const rf_group_req* __restrict__ reqs, int nReq, int64_t tile0) {
     __shared__ float red[kBlock / 64 * 16][16 * kIsoQ];
-    const int64_t b = blockIdx.x;
+    const int64_t b = tile0 + blockIdx.x;
     int lo = 0, hi = nReq - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -346,11 +349,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 template <int D, int R, bool ISO>
 hipError_t launch_fp64_r(const rf_sum_args& a, const double* k, double bound, const uint8_t* calc,
                          const double2* CS, int Rpad, hipStream_t s) {
+    // 32 work-items per point: fields of 2^27 points and more in several launches
     const int64_t blocks = (a.i1 - a.i0 + kF64Points - 1) / kF64Points;
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_sum_fp64<D, R, ISO>), dim3((unsigned)blocks, (unsigned)(Rpad / R)), dim3(64 * kF64Waves), 0, s,
-                       a, k, bound, calc, CS, Rpad);
-    return hipGetLastError();
+    return rf_block_ranges(blocks, 64 * kF64Waves, [&](int64_t first, unsigned n) {
+        rf_sum_args q = a;
+        q.i0 += first * kF64Points;
+        hipLaunchKernelGGL((k_sum_fp64<D, R, ISO>), dim3(n, (unsigned)(Rpad / R)), dim3(64 * kF64Waves), 0, s, q, k, bound,
+                           calc, CS, Rpad);
+        return hipGetLastError();
+    });
 }
 
 template <int D>
@@ -388,8 +395,8 @@ hipError_t rf_launch_prep_fp64(int64_t kN, int Nmc, int Rpad, int iso, const dou
                                double2* d_CS, hipStream_t s) {
     const int64_t n = kN * Rpad;
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_prep_fp64, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, kN, Nmc, Rpad,
-                       iso, d_phase, d_amp, d_CS);
+    const int64_t blocks = std::min((n + kBlock - 1) / kBlock, rf_max_blocks(kBlock));
+    hipLaunchKernelGGL(k_prep_fp64, dim3((unsigned)blocks), dim3(kBlock), 0, s, kN, Nmc, Rpad, iso, d_phase, d_amp, d_CS);
     return hipGetLastError();
 }
 
@@ -431,18 +438,23 @@ hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kA, co
     const bool wide = (a.i1 - a.i0) / 64 * sh.nChunk >= 16384;
     const int pts = kBlock / 4 * (wide ? 4 : kIsoQ);
     const int64_t blocks = (a.i1 - a.i0 + pts - 1) / pts;
-    if (blocks > 0x7fffffffLL || sh.nChunk > 65535) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)blocks, (unsigned)sh.nChunk);
-    if (wide) hipLaunchKernelGGL(k_sum_fp32_iso<4>, grid, dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
-    else hipLaunchKernelGGL(k_sum_fp32_iso<kIsoQ>, grid, dim3(kBlock), 0, s, a, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
-    return hipGetLastError();
+    if (sh.nChunk > 65535) return hipErrorInvalidValue;
+    return rf_block_ranges(blocks, kBlock, [&](int64_t first, unsigned n) {
+        rf_sum_args q = a;
+        q.i0 += first * pts;
+        const dim3 grid(n, (unsigned)sh.nChunk);
+        if (wide) hipLaunchKernelGGL(k_sum_fp32_iso<4>, grid, dim3(kBlock), 0, s, q, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
+        else hipLaunchKernelGGL(k_sum_fp32_iso<kIsoQ>, grid, dim3(kBlock), 0, s, q, d_kA, d_aA, sh.nJ, sh.Rp, kMax);
+        return hipGetLastError();
+    });
 }
 
 int rf_fp32_rchunk() { return kRChunk; }
 
 hipError_t rf_launch_group_iso(const rf_group_req* d_reqs, int nReq, int64_t nTiles, hipStream_t s) {
     if (nTiles <= 0 || nReq <= 0) return hipSuccess;
-    if (nTiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_group_iso, dim3((unsigned)nTiles), dim3(kBlock), 0, s, d_reqs, nReq);
-    return hipGetLastError();
+    return rf_block_ranges(nTiles, kBlock, [&](int64_t first, unsigned n) {
+        hipLaunchKernelGGL(k_group_iso, dim3(n), dim3(kBlock), 0, s, d_reqs, nReq, first);
+        return hipGetLastError();
+    });
 }
