@@ -4,7 +4,8 @@
 // Two precision forms:
 //  * FP64: one sine and cosine per (point, wavevector), shared by all
 //    realizations of a chunk, cos(t + phi) = cos t cos phi - sin t sin phi; the
-//    wavevectors of a point are split over its block.
+//    wavevectors of a point are split over its block or, few wavevectors or many
+//    points, taken by one lane.
 //  * FP32: one thread per point holding R realization accumulators.  The
 //    argument k.x is formed in FP64, reduced to revolutions in [-1/2, 1/2)
 //    once per (point, k) and reused for all R realizations; each term is then
@@ -167,6 +168,72 @@ __global__ __launch_bounds__(64 * kF64Waves) void k_sum_fp64(rf_sum_args a, cons
         // a realization the caller masks is zero at every point
         const double u = epilogue64(calc[r0 + r] ? a.ampMult * s : 0.0, a.epi);   // :330
         store_out(a.out, (int64_t)(r0 + r) * a.N + ip, u, a.outDtype);
+    }
+}
+
+// The same sum with one point per lane, every wavevector in order, the operands
+// wave-uniform (scalar loads): no reduction and no idle share, so it is the
+// faster one where the wavevectors are few (a block above spends 3 .. 56 ns of the
+// chip on its set-up and reduction, R = 1 .. 16) or the points many, and with
+// per-realization directions, whose chunks hold one realization.  Bound by the
+// latency of its loads and sine up to two waves per SIMD, then by the FP64 VALU.
+// One term and realization at a time with the library cosine / shares / lane:
+// 1M points x 13 wavevectors x 1: 29 / 296 / 17 us; 1M x 392 x 4: 2947 / 1083 /
+// 461; isotropic 100,000 x 61 x 17: 207 / 727 / 106; 20,000 x 2,048 x 4: 765 / 73 /
+// 445.  The accumulators go to running sums every kF64Flush terms, so that the
+// rounding does not grow over that of the shares.
+constexpr int kF64LaneBlock = 256;
+constexpr int kF64Flush = 32;
+template <int D, int R, bool ISO>
+__global__ __launch_bounds__(kF64LaneBlock) void k_sum_fp64_lane(rf_sum_args a, const double* __restrict__ k,
+                                                                 double bound, const uint8_t* __restrict__ calc,
+                                                                 const double2* __restrict__ CS, int Rpad) {
+    const int64_t i = a.i0 + (int64_t)blockIdx.x * kF64LaneBlock + threadIdx.x;
+    if (i >= a.i1) return;
+    const int r0 = blockIdx.y * R;
+    double xn[D], reach = 0.0;
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        xn[d] = a.x[i * D + d] / a.corrL[d];   // :59
+        reach += fabs(xn[d]);
+    }
+    double acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.0;
+    const double* kr = k + (ISO ? (int64_t)r0 * a.kN * D : 0);
+    const double2* C = CS + (ISO ? (int64_t)r0 * a.kN : (int64_t)r0);
+    const int64_t cStep = ISO ? 1 : Rpad;
+    auto sweep = [&](auto sc) {
+        for (int64_t j0 = 0; j0 < a.kN; j0 += kF64Flush) {
+            const int64_t j1 = j0 + kF64Flush < a.kN ? j0 + kF64Flush : a.kN;
+            double part[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) part[r] = 0.0;
+            for (int64_t j = j0; j < j1; j++) {
+                double t = kr[j * D] * xn[0];
+#pragma unroll
+                for (int d = 1; d < D; d++) t = fma(kr[j * D + d], xn[d], t);
+                double sn, cs;
+                sc(t, &sn, &cs);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const double2 c = C[j * cStep + r];
+                    part[r] = fma(c.x, cs, fma(c.y, sn, part[r]));
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) acc[r] += part[r];
+        }
+    };
+    // per wave: arguments past the fast sine's range, infinities, NaN
+    if (!__any(!(reach * bound < 1073741824.0))) sweep([](double t, double* s, double* c) { sincos_fast(t, s, c); });
+    else sweep([](double t, double* s, double* c) { sincos(t, s, c); });
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (r0 + r >= a.Nmc) break;
+        // a realization the caller masks is zero at every point
+        const double u = epilogue64(calc[r0 + r] ? a.ampMult * acc[r] : 0.0, a.epi);   // :330
+        store_out(a.out, (int64_t)(r0 + r) * a.N + i, u, a.outDtype);
     }
 }
 
@@ -346,9 +413,37 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
               (local / sh.nChunk) * kGroupIsoPts, red);
 }
 
+// Shares or one point per lane: the smaller of what the two were measured to
+// take (us) over 1 .. 1M points, 13 .. 6,912 wavevectors, 1 .. 64 realizations.
+// Shares: start-up + per turn of 128 wavevectors, per block, chip-wide, and not below
+// 9 us for 16 realizations (one block's reduction).  Lane: per wavevector, a
+// latency up to about two waves per SIMD, then a rate per wave of a SIMD.
+bool f64_lane(int64_t points, int64_t kN, int chunks, int R) {
+    constexpr double kStart[5] = {2.6e-3, 4.2e-3, 9e-3, 26e-3, 51e-3}, kTurn[5] = {2.17e-3, 2.3e-3, 2.5e-3, 4.8e-3, 5.5e-3};
+    constexpr double kLatency[5] = {0.18, 0.195, 0.225, 0.24, 0.267}, kRate[5] = {0.07, 0.072, 0.085, 0.105, 0.135};
+    constexpr double kLeast[5] = {0.0, 0.0, 0.0, 0.0, 9.0};
+    int i = 0;
+    while ((1 << i) < R) i++;
+    const double blocks = (double)((points + kF64Points - 1) / kF64Points) * chunks;
+    const double turns = (double)((kN + kF64Shares - 1) / kF64Shares);
+    const double perSimd = (double)(((points + 63) / 64 * chunks + 1023) / 1024);
+    const double shares = std::max(kLeast[i], blocks * (kStart[i] + kTurn[i] * turns));
+    return (double)kN * std::max(kLatency[i], perSimd * kRate[i]) < shares;
+}
+
 template <int D, int R, bool ISO>
 hipError_t launch_fp64_r(const rf_sum_args& a, const double* k, double bound, const uint8_t* calc,
                          const double2* CS, int Rpad, hipStream_t s) {
+    if (f64_lane(a.i1 - a.i0, a.kN, Rpad / R, R)) {
+        const int64_t all = (a.i1 - a.i0 + kF64LaneBlock - 1) / kF64LaneBlock;
+        return rf_block_ranges(all, kF64LaneBlock, [&](int64_t first, unsigned n) {
+            rf_sum_args q = a;
+            q.i0 += first * kF64LaneBlock;
+            hipLaunchKernelGGL((k_sum_fp64_lane<D, R, ISO>), dim3(n, (unsigned)(Rpad / R)), dim3(kF64LaneBlock), 0, s, q, k,
+                               bound, calc, CS, Rpad);
+            return hipGetLastError();
+        });
+    }
     // 32 work-items per point: fields of 2^27 points and more in several launches
     const int64_t blocks = (a.i1 - a.i0 + kF64Points - 1) / kF64Points;
     return rf_block_ranges(blocks, 64 * kF64Waves, [&](int64_t first, unsigned n) {
