@@ -21,6 +21,7 @@
 // e = 4 f1 + 2 f2 + f3 (f = 0 cosine, 1 sine); 2-D: j1 = 4 t + 2 h + u,
 // e = 4 u + 2 f1 + f2.  Steps run t fastest, then j2, then j3.
 #include "rf_mfma.h"
+#include "rf_per_device.h"
 #include "rf_philox.h"
 
 namespace {
@@ -407,17 +408,24 @@ __global__ __launch_bounds__(256) void k_lat_prep(int D, rf_lat_dev L, int Nmc, 
 
 size_t table_bytes(const rf_lat_dev& L, int W) { return (size_t)(L.P1 + L.n2) * 32 * W * sizeof(float2); }
 
-// Kernels whose tables pass the default dynamic LDS limit ask for theirs.
+// Kernels whose tables pass the default dynamic LDS limit ask for theirs, on
+// each device that runs them (the limit belongs to the function on a device).
 template <typename K>
-hipError_t allow_lds(K* f) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kLatTableMax);
+hipError_t allow_lds(K* f, rf_per_device* asked) {
+    int device = 0;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    return asked->once(device, [&]() {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   kLatTableMax);
+    });
 }
 
 template <typename V, int D, int MT, int W, int KG>
 hipError_t launch(const rf_sum_args& a, const rf_lat_dev& L, int mtTotal, const void* B, float sc, hipStream_t s) {
-    static const hipError_t ok = allow_lds(k_lat<V, D, MT, W, KG>);
-    if (ok != hipSuccess) return ok;
+    static rf_per_device asked;
+    const hipError_t e = allow_lds(k_lat<V, D, MT, W, KG>, &asked);
+    if (e != hipSuccess) return e;
     const int64_t blocks = (a.i1 - a.i0 + 32 * W - 1) / (32 * W);
     return rf_block_ranges(blocks, 64 * W * KG, [&](int64_t first, unsigned n) {
         rf_sum_args q = a;
@@ -438,8 +446,9 @@ hipError_t launch_d(const rf_sum_args& a, const rf_lat_dev& L, int mtTotal, cons
 
 template <typename V, int W, int KG>
 hipError_t launch_group(const rf_lat_dev& L, const rf_group_req* d_reqs, int nReq, int64_t nTiles, hipStream_t s) {
-    static const hipError_t ok = allow_lds(k_group_lat<V, W, KG>);
-    if (ok != hipSuccess) return ok;
+    static rf_per_device asked;
+    const hipError_t e = allow_lds(k_group_lat<V, W, KG>, &asked);
+    if (e != hipSuccess) return e;
     return rf_block_ranges(nTiles, 64 * W * KG, [&](int64_t first, unsigned n) {
         hipLaunchKernelGGL((k_group_lat<V, W, KG>), dim3(n), dim3(64 * W * KG), table_bytes(L, W), s, d_reqs, nReq, L, first);
         return hipGetLastError();
