@@ -35,6 +35,20 @@ def test_corr_edges_match_oracle(ctx, dtype, nstep):
         assert np.allclose(got[a], ref[a], rtol=0.0, atol=1e-12), (a, np.abs(got[a] - ref[a]).max())
 
 
+@pytest.mark.parametrize("nstep", [(1100, 16, 4), (5, 700, 40), (3, 65, 1500)])
+def test_corr_axes_of_unequal_length(ctx, nstep):
+    """A long axis of many tile pairs beside short ones of many lines, whose
+    lines are dealt to more blocks than an even share per pair."""
+    import torch
+    f = np.random.default_rng(7).normal(0.4, 2.0, int(np.prod(nstep)))
+    avg, sd = float(f.mean()), float(f.std())
+    got, _ = R.corr(ctx, torch.from_numpy(f[None]).cuda(), R.DTYPE_F64, nstep, [0.5] * 3, avg, sd, 0)
+    ref = O.corr(f, nstep, avg, sd)
+    for a in range(3):
+        assert len(got[a]) == nstep[a] // 2
+        assert np.allclose(got[a], ref[a], rtol=0.0, atol=1e-12), (a, np.abs(got[a] - ref[a]).max())
+
+
 def test_corr_not_finite(ctx):
     """A value that is not finite reaches every lag of its lines and only
     those sums: no lag of the field stays finite, as in the plain sum."""
