@@ -20,6 +20,8 @@
 // K-step (16 entries), 3-D: lane half h takes j1 = 2 t + h and its 8 products
 // e = 4 f1 + 2 f2 + f3 (f = 0 cosine, 1 sine); 2-D: j1 = 4 t + 2 h + u,
 // e = 4 u + 2 f1 + f2.  Steps run t fastest, then j2, then j3.
+#include <type_traits>
+
 #include "rf_mfma.h"
 #include "rf_per_device.h"
 #include "rf_philox.h"
@@ -65,10 +67,23 @@ __device__ __forceinline__ void prod_pair<b8>(float x0, float x1, float y, unsig
 // K-steps per stage and K-group (8 KB of panels)
 constexpr int lat_steps(int MT) { return MT == 1 ? 4 : 2; }
 constexpr int lat_units(int KG) { return 512 * KG; }   // 16-byte units of a stage
-// The accumulators of kLatFlush K-steps are added to the running sums: a
-// serial FP32 accumulation over all ~1,400 steps of a 10-correlation-length
-// lattice is off by 5e-6, so by 4e-7.
-constexpr int kLatFlush = 64;
+// The accumulators of every 32 K-steps (16 of a group of up to 64, where they
+// cost nothing) are added to the running sums.  FP16 error of 33,000 points in 2-D
+// boxes of 7 and 10 correlation lengths, one serial sum of the 28 and 56 steps:
+// 2.8e-7 and 3.8e-7, more than the general form's 2.7e-7 and 3.6e-7; so 1.9e-7 and
+// 2.0e-7.  3-D, 10 correlation lengths (1,400 steps): 5e-6 in one sum, 3.9e-7 by 64,
+// 3.1e-7 by 32, 2.9e-7 by 16, which costs 1.5-3 % (32: 0.5 %).
+constexpr int lat_flush(int64_t nG) { return nG <= 64 ? 16 : 32; }
+// BF16 halves carry eight bits each, and the dropped product of the low halves is
+// a third of the form's error variance.  Products of sines and cosines lie less
+// near 1, where a rounding weighs least, than the general form's single sines do:
+// without it errors are 5-8 % above that form's (3-D box of 6 correlation lengths, 32
+// realizations: 4.25e-6 against 3.94e-6).  So the first kLatLowPart-th of the K-steps --
+// the slow axis' long waves, most of the field -- takes it too: 3.66e-6 for 5-8 % of
+// the time (on every step 3.38e-6 for up to 20 %).  Where the K-steps are split over
+// groups of waves every step does: a line inside a group's steps spills (39 % against
+// 8-17 %).
+constexpr int kLatLowPart = 3;
 
 // One block: points pt0 .. pt0 + 32 W - 1 (clipped to a.i1), M-tiles mt0 ..
 // mt0 + MT - 1.  W waves side by side take 32 points each; KG such groups take
@@ -103,6 +118,7 @@ __device__ __forceinline__ void lat_block(const rf_sum_args& a, const rf_lat_dev
     const int64_t stepUnits = (int64_t)mtTotal * 128;
     const int64_t nG = L.nSteps / KG;               // K-steps of a group, a multiple of 4
     const int64_t nStages = nG / S;
+    const int flush = lat_flush(nG) / S;                // stages
 
     u32x4 pre[kCopy];
     const u32x4* src[kCopy];                            // this thread's units of the stage to fetch
@@ -219,7 +235,9 @@ __device__ __forceinline__ void lat_block(const rf_sum_args& a, const rf_lat_dev
             acc[m][r] = 0.0f;
             tot[m][r] = 0.0f;
         }
-    auto stage = [&](int64_t u, const u32x4* cur, u32x4* nxt) {
+    int left = flush;
+    // one stage; lowToo: with the product of the low halves
+    auto stage = [&](int64_t u, const u32x4* cur, u32x4* nxt, auto lowToo) {
         if (u + 1 < nStages) fetch();
 #pragma unroll
         for (int s = 0; s < S; s++) {
@@ -239,10 +257,15 @@ __device__ __forceinline__ void lat_block(const rf_sum_args& a, const rf_lat_dev
             for (int m = 0; m < MT; m++) acc[m] = mfma(ah[m], bl, acc[m]);
 #pragma unroll
             for (int m = 0; m < MT; m++) acc[m] = mfma(al[m], bh, acc[m]);
+            if constexpr (decltype(lowToo)::value) {
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[m] = mfma(al[m], bl, acc[m]);
+            }
             bh = nh;
             bl = nl;
         }
-        if ((u + 1) % (kLatFlush / S) == 0) {
+        if (--left == 0) {                              // uniform
+            left = flush;
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
@@ -255,10 +278,19 @@ __device__ __forceinline__ void lat_block(const rf_sum_args& a, const rf_lat_dev
         if (u + 1 < nStages) stash(nxt);
         __syncthreads();
     };
-    for (int64_t u = 0; u < nStages; u += 2) {
-        stage(u, panA, panB);
-        if (u + 1 < nStages) stage(u + 1, panB, panA);
+    auto stages = [&](int64_t u0, int64_t u1, auto lowToo) {                      // u0 even
+        for (int64_t u = u0; u < u1; u += 2) {
+            stage(u, panA, panB, lowToo);
+            if (u + 1 < nStages) stage(u + 1, panB, panA, lowToo);
+        }
+    };
+    int64_t low = 0;                                    // the same in every wave of the block
+    if constexpr (std::is_same<V, b8>::value) {
+        low = KG == 1 ? (nStages + 2 * kLatLowPart - 1) / (2 * kLatLowPart) * 2 : nStages;
+        if (low > nStages) low = nStages;
+        stages(0, low, std::true_type());
     }
+    if constexpr (!std::is_same<V, b8>::value || KG == 1) stages(low, nStages, std::false_type());
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
