@@ -43,7 +43,15 @@ int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // F16: 1364 against 3190; 5,000 x 256: 225 against 991, its K-steps split over the
 // waves).  In 2-D, where the per-axis sines weigh against few wavevectors, from 65
 // realizations: 300,000 x 100 176 against 141, 500,000 x 64 151 against 165.
-bool use_lat(const rf_field_plan* P, int64_t N) { return P->lat && !(P->d_Bw && N > kLatSmallN); }
+// BF16 stays with it for two rounds of its blocks (128 points x 64 realizations) only:
+// 256 realizations, kN 2,048, three and four rounds 1.0-1.2 times the general form's
+// time.  The FP16 general form would be the faster one there too on small lattices
+// (32,768 x 129: 2-D kN 392 44 us against 73), but with 1.7 times the error.
+bool use_lat(const rf_field_plan* P, int64_t N) {
+    if (!P->lat || !P->d_Bw) return P->lat;
+    const bool many = P->p.form == RF_FORM_MFMA_BF16 && (N + 127) / 128 * (P->Rpad / 64) > 512;
+    return N <= kLatSmallN && !many;
+}
 
 // Form-specific operand build from d_phase / d_amp (Nmc x kN, FP64).
 int build_form_operands(rf_field_plan* P, hipStream_t s) {
