@@ -61,8 +61,7 @@ __global__ __launch_bounds__(kBlock) void k_marginal_vec(int margi, double scale
     }
 }
 
-// Per-realization partial sums of u and u^2 in FP64; grid (nPart, Nmc).
-// Sums of u and u^2 of each realization (grid y); grid (nPart, Nmc).  Bound by
+// Partial sums of u and u^2 of each realization in FP64; grid (nPart, Nmc).  Bound by
 // the read: two independent 16-byte loads per thread and turn where every
 // realization starts on a 16-byte boundary (VEC), one element otherwise
 // (128^3 x 16 FP32: 27 -> 22 us, 6.0 TB/s).
@@ -428,16 +427,15 @@ typedef __attribute__((address_space(3))) void interp_lds;
 // bound is the address rate of the vector memory path: ~33 cycles per wave
 // load and cell corner, whatever the cache does.  Nodes in mesh order are close
 // to each other, so a block finds the box of cells its nodes lie in and, where
-// it fits the LDS (kInterpK elements per thread), copies it there realization
-// by realization -- coalesced, the next realization's values in registers
-// meanwhile -- and gathers from LDS.  Other blocks read the corners directly,
+// it fits the LDS (interp_k elements per thread), copies it there realization
+// by realization, coalesced and straight to LDS, and gathers from LDS.  Other blocks read the corners directly,
 // 2^(D-1) pairs per node.  Blocks of an XCD take one contiguous run of nodes.
 // 4M nodes in mesh order from a 256 x 256 x 128 grid, 16 realizations, FP32:
 // direct single loads 530 us, direct pairs 480-500 us at any block size and
 // chunk, from LDS 345 us (1.2 GB of HBM traffic, 3.5 TB/s; the grid is read
 // 1.2 times).  Two blocks of 1024 per CU (64 VGPRs) share more of the planes
-// in their XCD's L2 than one: 500 us with the next realization held in
-// registers; chunks of realizations repeat the set-up: 8 +20 %, 4 +60 %.
+// in their XCD's L2 than one with the next realization held in registers
+// (500 us); chunks of realizations repeat the set-up: 8 +20 %, 4 +60 %.
 constexpr int interp_k(int NT, int size) { return NT == 256 && size == 4 ? 24 : 12; }
 
 template <typename TG, typename TO, int D, int NT>
@@ -1074,15 +1072,21 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
         q.Ng *= q.nstep[a];
     }
     q.nNodes = nNodes;
-    // blocks of 1024 nodes and all realizations (the most compact boxes, cells
-    // and weights formed once) where that still gives every CU two; else 256
-    // nodes and 4 realizations
-    const bool wide = nNodes >= 512 * 1024;
-    // (FP64 grids: 512, whose box leaves room for two blocks per CU; 136 x 35 x 101,
-    // 3.6M nodes, 8 realizations: 253 us in blocks of 1024, 215 in 512)
+    // Many nodes, at most six grid points to a node: all realizations in a block
+    // (cells and weights formed once); else four, so that small calls fill the
+    // chip and a block's scattered corners stay in L2 (256 x 256 x 128, 600,000 nodes, 16
+    // realizations FP32: 281 us all together in blocks of 1024, 195 in blocks of 256, 181
+    // in fours).  FP32 grids in blocks of 1024 nodes (the most compact boxes) down to
+    // four grid points to a node, a few realizations down to six (4M nodes 345 us;
+    // 2M nodes, 4.2 points to a node, 16 realizations 395 us against 287 in blocks of
+    // 256, one realization 52 against 71).  FP64 grids in blocks of 256: five waves per
+    // SIMD whose set-ups cover each other, 251 x 151 x 32, 3.3M nodes, 1 / 4 / 16
+    // realizations 99 / 127 / 348 us against 118 / 154 / 365 in blocks of 512.
+    const bool wide = nNodes >= 512 * 1024 && q.Ng <= 6 * nNodes;
     const int RC = wide ? Nmc : 4;
     const bool g64 = gridDtype == RF_DTYPE_F64, o64 = outDtype == RF_DTYPE_F64;
-    const int NT = !wide ? 256 : g64 ? 512 : 1024;
+    const bool large = wide && !g64 && (Nmc <= 4 || q.Ng <= 4 * nNodes);
+    const int NT = large ? 1024 : 256;
     const int64_t nBlocks = (nNodes + NT - 1) / NT;
     if ((nBlocks + 7) / 8 * 8 > rf_max_blocks(NT)) return hipErrorInvalidValue;
     const dim3 grid2((unsigned)((nBlocks + 7) / 8 * 8), (unsigned)((Nmc + RC - 1) / RC));
@@ -1090,9 +1094,14 @@ hipError_t rf_launch_interp(int nDim, const int32_t* nstep, const int32_t* lo, c
     auto run = [&](auto dim, auto* g, auto* o) {
         typedef std::remove_const_t<std::remove_pointer_t<decltype(g)>> TG;
         typedef std::remove_pointer_t<decltype(o)> TO;
-        constexpr int D = decltype(dim)::value, NW = sizeof(TG) == 8 ? 512 : 1024;
-        if (wide) hipLaunchKernelGGL((k_interp<TG, TO, D, NW>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
-        else hipLaunchKernelGGL((k_interp<TG, TO, D, 256>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
+        constexpr int D = decltype(dim)::value;
+        if constexpr (sizeof(TG) == 4) {
+            if (large) {
+                hipLaunchKernelGGL((k_interp<TG, TO, D, 1024>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_interp<TG, TO, D, 256>), grid2, dim3(NT), 0, s, q, g, x, o, d_flag, nBlocks, RC);
     };
     auto go = [&](auto* g, auto* o) {
         if (nDim == 3) run(std::integral_constant<int, 3>(), g, o);

@@ -57,3 +57,21 @@ def test_blocks_of_1024(ctx, order, dt):
     s = np.flatnonzero(~outside)[::37]
     ref, bad = O.interp(grid.astype(np.float64), nstep, [0.0] * 3, [1.0] * 3, np.ascontiguousarray(x[s]))
     assert bad == 0 and np.array_equal(got[:, s], ref.astype(dt))
+
+
+@pytest.mark.parametrize("nstep,Nmc", [((120, 110, 160), 5), ((170, 130, 150), 2), ((170, 130, 150), 7), ((160, 160, 160), 6)])
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_many_nodes_of_sparse_grids(ctx, nstep, Nmc, dt):
+    """Half a million nodes with four, between four and six, and more grid points
+    to a node: blocks of 1024 and 256 nodes, all realizations or four a block."""
+    import torch
+    rng = np.random.default_rng(Nmc)
+    m = 512 * 1024 + 129
+    grid = rng.standard_normal((Nmc, int(np.prod(nstep)))).astype(dt)
+    x = _nodes(3, nstep, m, "mesh", rng)
+    out = torch.full((Nmc, m), 7.0, dtype=getattr(torch, dt), device="cuda")
+    assert not R.interpolate(ctx, nstep, [0.0] * 3, [1.0] * 3, Nmc, torch.from_numpy(grid).cuda(),
+                             torch.from_numpy(x).cuda(), out)
+    s = np.r_[np.arange(0, m, 41), m - 1]
+    ref, bad = O.interp(grid.astype(np.float64), nstep, [0.0] * 3, [1.0] * 3, np.ascontiguousarray(x[s]))
+    assert bad == 0 and np.array_equal(out.cpu().numpy()[:, s], ref.astype(dt))
