@@ -305,8 +305,8 @@ __global__ __launch_bounds__(kBlock) void k_sum_fp32(rf_sum_args a, const double
 // an MFMA of 64 cycles, which the VALU does not overlap; k.x by FMAs, v_fract_f64 and
 // the phase cost eight (36 cycles either way), so what is gained is the
 // packing of few realizations and waves of 32 points where a field is small:
-// 200,000 points x 16 realizations, 286 shells 375 -> 284 us (error 1.9e-7 -> 1.8e-7),
-// 128^3 x 64 9.25 -> 9.27 ms.  One instruction less -- v_alignbit of the word to a
+// 200,000 points x 16 realizations, 286 shells 375 -> 284 us (error 1.9e-7 -> 1.8e-7);
+// large fields of full rows take k_sum_fp32_iso_fma.  One instruction less -- v_alignbit of the word to a
 // float 1 + argument of 23 bits -- gave 254 us and 8.66 ms with an error of 2.1e-7.
 // Arguments that may reach 2^19 revolutions (or are not finite) take a zero
 // accumulator and v_fract_f64; the choice is per wave.
@@ -320,6 +320,11 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 typedef const f4v __attribute__((address_space(1))) gf4;
 constexpr int kIsoQ = 2;                               // 16-point groups of a wave, small fields and batches
 static_assert(kGroupIsoPts == kBlock / 64 * 16 * kIsoQ, "points of a block");
+
+constexpr double kIsoBias = 1572864.0;                 // 1.5 2^20
+__device__ __forceinline__ float iso_turn(double t) {
+    return (float)(int)(unsigned)__builtin_bit_cast(uint64_t, t) * 0x1p-32f;
+}
 
 template <int Q>
 __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict__ kA, gf4* __restrict__ aA, int64_t nJ,
@@ -367,7 +372,7 @@ __device__ __forceinline__ void iso_block(const rf_sum_args& a, gdbl* __restrict
         }
     };
     if (!__any(far))
-        sweep(1572864.0, [](double t) { return (float)(int)(unsigned)__builtin_bit_cast(uint64_t, t) * 0x1p-32f; });
+        sweep(kIsoBias, [](double t) { return iso_turn(t); });
     else
         sweep(0.0, [](double t) { return (float)__builtin_amdgcn_fract(t); });
     // D: column c, rows 4 e + g; the wavevectors of a block added in row order
@@ -391,6 +396,53 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(Q > 2 ? 
     __shared__ float red[kBlock / 64 * 16][16 * Q];
     iso_block<Q>(a, (gdbl*)kA, (gf4*)aA, nJ, gridDim.y, blockIdx.y, Rp, kMax, a.i0 + (int64_t)blockIdx.x * (kBlock / 4 * Q),
                  red);
+}
+
+// The same sum by FMAs, one point per lane and 16 realizations of a chunk (Rp 16: one
+// wavevector per operand block): large fields, whose waves of 64 points fill the chip
+// and whose rows the matrix cores' packing has nothing to gain on.  The argument is
+// formed on the same bias in the same order and read the same way: the same bits.
+// Operands wave-uniform; the phase is added on its own because a VALU instruction
+// reads one scalar operand (as the addend of an FMA it took two moves more, 10 %).
+// 16 realizations: 2-D, 1M points, 116 shells 383 us (MFMA form 488), 3-D, 300,000 points,
+// 146 shells 195 (207), 1M 545 (612).
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_sum_fp32_iso_fma(rf_sum_args a, const double* __restrict__ kA,
+                                                             const float* __restrict__ aA, int64_t nJ, double kMax) {
+    const int64_t i = a.i0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= a.i1) return;
+    double x[D];
+    bool far = false;
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        x[d] = a.x[i * D + d] / a.corrL[d];
+        far |= !(3.0 * kMax * fabs(x[d]) + 1.0 < 524288.0);
+    }
+    const int chunk = blockIdx.y, nChunk = gridDim.y;
+    float acc[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    auto sweep = [&](double c0, auto turn) {
+        for (int64_t j = 0; j < nJ; j++) {
+            const double* k = kA + (j * nChunk + chunk) * 64;
+            const float* am = aA + (j * nChunk + chunk) * 16;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                double t = c0;
+#pragma unroll
+                for (int d = 0; d < D; d++) t = fma(k[16 * d + r], x[d], t);
+                t += k[48 + r];
+                acc[r] = fmaf(am[(r & 3) * 4 + (r >> 2)], __builtin_amdgcn_cosf(turn(t)), acc[r]);
+            }
+        }
+    };
+    if (!__any(far)) sweep(kIsoBias, [](double t) { return iso_turn(t); });
+    else sweep(0.0, [](double t) { return (float)__builtin_amdgcn_fract(t); });
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int R = chunk * 16 + r;
+        if (R < a.Nmc) store_out(a.out, (int64_t)R * a.N + i, epilogue32(acc[r], a.epi), a.outDtype);
+    }
 }
 
 // Grouped form: block b of a launch from tile0 runs tile tile0 + b = (field, kGroupIsoPts points, chunk of
@@ -528,12 +580,30 @@ hipError_t rf_launch_sum_fp32_iso_t(const rf_sum_args& a, const double* d_kA, co
                                     hipStream_t s) {
     if (a.i1 <= a.i0) return hipSuccess;
     const rf_iso_shape sh = rf_iso_rows(a.kN, a.Nmc);
+    if (sh.nChunk > 65535) return hipErrorInvalidValue;
+    // FMA form, full rows: by (point, chunk) pairs in units of one wave per SIMD, 65,536.
+    // Time against the MFMA form, whose waves hold 32 points: 3-D 1.3-1.4 at 80,000, 1.11
+    // at 200,000, 0.90-0.96 at 300,000, 0.88 at 2M; 2-D, a quarter of whose MFMA multiplies
+    // zeros, 0.83-0.93 at 100,000 and 131,000, 1.06 at 140,000 (a third round), 0.99 at
+    // 200,000, 0.77 at 2M.
+    const int64_t pairs = (a.i1 - a.i0) * sh.nChunk;
+    const bool fma2 = pairs >= 3 * 65536 || (2 * pairs >= 3 * 65536 && pairs <= 2 * 65536), fma3 = 2 * pairs >= 9 * 65536;
+    if (sh.Rp == 16 && (a.nDim == 2 ? fma2 : fma3)) {
+        const int64_t all = (a.i1 - a.i0 + kBlock - 1) / kBlock;
+        return rf_block_ranges(all, kBlock, [&](int64_t first, unsigned n) {
+            rf_sum_args q = a;
+            q.i0 += first * kBlock;
+            const dim3 grid(n, (unsigned)sh.nChunk);
+            if (a.nDim == 2) hipLaunchKernelGGL(k_sum_fp32_iso_fma<2>, grid, dim3(kBlock), 0, s, q, d_kA, d_aA, sh.nJ, kMax);
+            else hipLaunchKernelGGL(k_sum_fp32_iso_fma<3>, grid, dim3(kBlock), 0, s, q, d_kA, d_aA, sh.nJ, kMax);
+            return hipGetLastError();
+        });
+    }
     // 64 points per wave where that still gives every SIMD about sixteen waves
     // (the operand loads and the loop weigh half), else 32
     const bool wide = (a.i1 - a.i0) / 64 * sh.nChunk >= 16384;
     const int pts = kBlock / 4 * (wide ? 4 : kIsoQ);
     const int64_t blocks = (a.i1 - a.i0 + pts - 1) / pts;
-    if (sh.nChunk > 65535) return hipErrorInvalidValue;
     return rf_block_ranges(blocks, kBlock, [&](int64_t first, unsigned n) {
         rf_sum_args q = a;
         q.i0 += first * pts;
