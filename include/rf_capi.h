@@ -353,7 +353,9 @@ int rf_grid_batch_execute(rf_grid_batch* batch, void* stream);
 #define RF_DRAW_NEXT (-1)
 /* Times each contraction stage of the batch with its phase-table axis held
  * whole by a wave (up to five 32-entry tiles) or split over several, keeps the
- * fastest (chosen[3]: tiles per wave now used per stage, 1..5) and
+ * fastest (chosen[3]: tiles per wave now used per stage, 1..5; for the first
+ * stage of a batch whose redraws form the coefficients in it -- first axes of
+ * up to 160 points -- those of that launch, always the whole axis) and
  * leaves one execute's result in the outputs.  The field values do not depend
  * on the split (the same K order per element).  Synchronous; no
  * counterpart in the reference.  This and rf_grid_batch_fuse_blend rewrite

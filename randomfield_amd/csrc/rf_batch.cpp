@@ -39,6 +39,11 @@ struct rf_grid_batch {
     bool redrawable = true;
     int64_t* d_draw = nullptr;          // draw state: [0] next, [1] current, [2] coefficient mode
     bool genActive = false;             // the last redraw left the first contraction forming the coefficients
+    // the first contraction that forms them: whole axes (formMt tiles per wave, 0 where
+    // an axis does not fit a wave), whatever mt[0] the stored ones are read with
+    rf_gemm_desc* d_form = nullptr;
+    int formMt = 0;
+    int64_t formTiles = 0;
     rf_fold_item* d_items = nullptr;    // the folds as one grouped launch
     int64_t foldBlocks = 0;
     // host copies of the stage descriptors
@@ -74,8 +79,26 @@ hipError_t upload_stages(rf_grid_batch* B, hipStream_t s) {
         B->fp32Tiles[k] = t[1];
         all.insert(all.end(), B->stage[k].begin(), B->stage[k].end());
     }
+    // the first contraction once more, for the launch that forms the coefficients
+    B->formMt = 0;
+    B->formTiles = 0;
+    for (const auto& g : B->stage[0]) {
+        const int tiles = (g.M + 31) / 32;
+        if (g.mt == 0 || !g.genState || tiles > kStripMaxMT) {
+            B->formMt = 0;
+            break;
+        }
+        B->formMt = std::max(B->formMt, tiles);
+    }
+    if (B->formMt > 0)
+        for (rf_gemm_desc g : B->stage[0]) {
+            g.tile0 = B->formTiles;
+            B->formTiles += rf_gemm_tiles(g, B->formMt);
+            all.push_back(g);
+        }
     for (int k = 0; k < 3; k++)
         if (B->stripTiles[k] > rf_max_blocks(256) || B->fp32Tiles[k] > rf_max_blocks(256)) return hipErrorInvalidValue;
+    if (B->formTiles > rf_max_blocks(256)) return hipErrorInvalidValue;
     hipError_t e = hipMemcpyAsync(B->d_desc[0], all.data(), all.size() * sizeof(rf_gemm_desc), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     return e;
@@ -89,12 +112,11 @@ hipError_t run_stage(const rf_grid_batch* B, int k, hipStream_t s) {
     return rf_launch_gemm_group(k, 0, B->d_desc[k] + n, B->nDesc[k] - n, B->fp32Tiles[k], s);
 }
 
-// every field's coefficients are formed by the first contraction itself:
-// strips that hold the whole first axis (each coefficient formed once)
-bool first_forms_coefficients(const rf_grid_batch* B) {
-    bool gen = !B->stage[0].empty();
-    for (const auto& g : B->stage[0]) gen = gen && g.mt > 0 && g.genState && (g.M + 31) / 32 <= B->mt[0];
-    return gen;
+// The first contraction of a batch whose coefficients it forms itself: strips that
+// hold the whole first axis, each coefficient formed once.
+hipError_t run_first(const rf_grid_batch* B, hipStream_t s) {
+    if (!B->genActive) return run_stage(B, 0, s);
+    return rf_launch_gemm_group(RF_GEMM_FIRST, B->formMt, B->d_form, (int)B->stage[0].size(), B->formTiles, s);
 }
 }  // namespace
 
@@ -137,7 +159,7 @@ int rf_grid_batch_create(rf_context* ctx, int32_t n, rf_field_plan* const* plans
         total += align256(rf_grid_scratch_elems(p.nDim, in.kNStep, in.nSignBlocks, p.Nmc, ns) * sizeof(float2));
     }
     const size_t descOff = total;
-    total += align256(sizeof(rf_gemm_desc) * 3 * (size_t)n);
+    total += align256(sizeof(rf_gemm_desc) * 4 * (size_t)n);
     const size_t drawOff = total;
     total += 256;
     const size_t itemOff = total;
@@ -210,6 +232,7 @@ int rf_grid_batch_create(rf_context* ctx, int32_t n, rf_field_plan* const* plans
         B->d_desc[k] = reinterpret_cast<rf_gemm_desc*>(B->d_mem + descOff) + dOff;
         dOff += stage[k].size();
     }
+    B->d_form = reinterpret_cast<rf_gemm_desc*>(B->d_mem + descOff) + dOff;
     hipError_t e = upload_stages(B.get(), s);
     if (e == hipErrorInvalidValue) {
         (void)hipFree(B->d_mem);
@@ -241,7 +264,8 @@ int rf_grid_batch_execute(rf_grid_batch* B, void* stream) {
     if (!B) return rf_set_error(nullptr, RF_E_ARG, "batch is NULL");
     rf_context* ctx = B->ctx;
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    for (int k = 0; k < 3; k++) RF_HIP_TRY(ctx, run_stage(B, k, s));
+    RF_HIP_TRY(ctx, run_first(B, s));
+    for (int k = 1; k < 3; k++) RF_HIP_TRY(ctx, run_stage(B, k, s));
     return RF_OK;
 }
 
@@ -304,7 +328,7 @@ int rf_grid_batch_autotune(rf_grid_batch* B, void* stream, int32_t* chosen) {
     (void)hipEventDestroy(e1);
     if (e != hipSuccess) return rf_set_error(ctx, RF_E_HIP, std::string("batch autotune: ") + hipGetErrorString(e));
     if (chosen)
-        for (int k = 0; k < 3; k++) chosen[k] = B->mt[k];
+        for (int k = 0; k < 3; k++) chosen[k] = k == 0 && B->formMt > 0 ? B->formMt : B->mt[k];
     return RF_OK;
 }
 
@@ -314,10 +338,12 @@ int rf_grid_batch_redraw(rf_grid_batch* B, int64_t drawIndex, void* stream) {
     if (!B->redrawable)
         return rf_set_error(ctx, RF_E_UNSUPPORTED, "rf_grid_batch_redraw: method 4 fields have no phases to redraw");
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
-    // when the first contraction's strips hold the whole first axis, they form
-    // the coefficients of the current draw themselves (no fold, no coefficient
-    // round trip through HBM); otherwise the grouped fold stores them
-    const bool gen = first_forms_coefficients(B);
+    // where a wave holds the whole first axis, the first contraction forms the
+    // coefficients of the current draw itself (no fold, no coefficient round trip
+    // through HBM: 32 fields of ~131^3 x 16 1.44 ms; fold and split contraction 0.73 +
+    // 1.13); otherwise the grouped fold stores them.  Not the autotuner's choice: that
+    // times the contraction of stored coefficients.
+    const bool gen = B->formMt > 0;
     RF_HIP_TRY(ctx, rf_launch_draw_counter(B->d_draw, drawIndex >= 0 ? drawIndex : -1, gen ? 1 : 0, s));
     if (!gen)
         RF_HIP_TRY(ctx, rf_launch_refold_draw(B->d_items, (int)B->folds.size(), B->foldBlocks, B->d_draw + 1, s));
