@@ -1,5 +1,5 @@
-"""The FP64 point-wise sum at the sizes where it can go wrong: blocks of 64
-points, chunks of 1 .. 16 realizations, eight shares of the wavevectors, the
+"""The FP64 point-wise sum at the sizes where it can go wrong: blocks of 16
+points, chunks of 1 .. 16 realizations, 128 shares of the wavevectors, the
 sine's range, masks; against the oracle.
 
 Tolerance 1e-12 of the field's rms: the argument's rounding (|t| 2^-53 ~ 2e-14
@@ -38,6 +38,18 @@ def test_shared_table(ctx, nDim, N, Nmc, mode):
     k = O.kpoints(po)
     ref = O.shinozuka(po, x, k, O.skvec(po, k), phU)
     assert _rel(got, ref) <= 1e-12
+
+
+@pytest.mark.parametrize("N", [15, 16, 17, 31, 33])
+@pytest.mark.parametrize("Nmc", [1, 4, 16])
+def test_block_edges(ctx, N, Nmc):
+    xr = (4.0, 3.0, 2.5)
+    x = np.random.default_rng(N).random((N, 3)) * np.array(xr)
+    p, phU = _field(3, R.SHINOZUKA, R.FIXED, Nmc, x, xr)
+    got = R.generate(ctx, p, x, None, phU, dtype=np.float64)
+    po = O.make_plan(3, O.SHINOZUKA, O.FIXED, list(xr))
+    k = O.kpoints(po)
+    assert _rel(got, O.shinozuka(po, x, k, O.skvec(po, k), phU)) <= 1e-12
 
 
 @pytest.mark.parametrize("big", [1e3, 1e6, 3e8, 1e10, 1e13])

@@ -110,3 +110,12 @@ def test_both_forms_give_the_same_bits(ctx, nDim):
     ctx.sync()
     plan.close()
     assert torch.equal(big[:, :64], small[:, :64]) and torch.equal(big[:, 192:n], small[:, 192:])
+
+
+@pytest.mark.parametrize("N", [2 ** 20 - 1, 2 ** 20 + 77])
+@pytest.mark.parametrize("nDim,Nmc", [(3, 1), (3, 5), (2, 3), (3, 8)])
+def test_waves_of_64_points(ctx, nDim, N, Nmc):
+    """From 1,048,576 points a wave of the matrix-core form takes 64 points: a
+    ragged end, rows of 2 .. 16 wavevectors, far points in one wave and in the last;
+    the first case is just below."""
+    assert _sampled(ctx, nDim, N, Nmc, far=(64, 65, 66, 130, N - 1), bad=(3, N - 70)) <= 3e-6
