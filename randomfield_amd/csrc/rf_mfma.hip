@@ -264,12 +264,12 @@ void k_sum_mfma(rf_sum_args a, int64_t nSteps, int mtTotal, const u32x4* __restr
 // does not depend on what it is batched with.
 template <typename V, int W, int S>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_group_mfma(const rf_group_req* __restrict__ reqs, int nReq) {
+void k_group_mfma(const rf_group_req* __restrict__ reqs, int nReq, int64_t tile0) {
     __shared__ u32x4 ldsA[S * kGroupMT * 128];
     __shared__ u32x4 ldsB[S * kGroupMT * 128];
     __shared__ u32x4 kqA[W * 12 * S];
     __shared__ u32x4 kqB[W * 12 * S];
-    const int64_t b = blockIdx.x;
+    const int64_t b = tile0 + blockIdx.x;
     const rf_group_req& q = reqs[group_find(reqs, nReq, b)];
     const int nSub = (q.mtTotal + kGroupMT - 1) / kGroupMT;
     const int64_t local = b - q.tile0;
@@ -455,12 +455,13 @@ hipError_t rf_launch_mfma_prep(int form, int nDim, int64_t kN, int64_t kNpad, in
 hipError_t rf_launch_group_mfma(int form, const rf_group_req* d_reqs, int nReq, int64_t nTiles,
                                 hipStream_t s) {
     if (nTiles <= 0 || nReq <= 0) return hipSuccess;
-    if (nTiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (form == RF_FORM_MFMA_BF16)
-        hipLaunchKernelGGL((k_group_mfma<b8, kGroupW, 4>), dim3((unsigned)nTiles), dim3(64 * kGroupW), 0, s, d_reqs, nReq);
-    else
-        hipLaunchKernelGGL((k_group_mfma<h8, kGroupW, 4>), dim3((unsigned)nTiles), dim3(64 * kGroupW), 0, s, d_reqs, nReq);
-    return hipGetLastError();
+    return rf_block_ranges(nTiles, 64 * kGroupW, [&](int64_t first, unsigned n) {
+        if (form == RF_FORM_MFMA_BF16)
+            hipLaunchKernelGGL((k_group_mfma<b8, kGroupW, 4>), dim3(n), dim3(64 * kGroupW), 0, s, d_reqs, nReq, first);
+        else
+            hipLaunchKernelGGL((k_group_mfma<h8, kGroupW, 4>), dim3(n), dim3(64 * kGroupW), 0, s, d_reqs, nReq, first);
+        return hipGetLastError();
+    });
 }
 
 hipError_t rf_launch_sum_mfma(int form, int variant, const rf_sum_args& a, int64_t kNpad, int Npad,
