@@ -76,7 +76,9 @@ extern "C" {
 #define RF_REF_COMPAT     0   /* reference behaviour wherever it is defined */
 #define RF_FIXED          1   /* intended mathematics                        */
 /* precision forms of the spectral sum */
-#define RF_FORM_FP64        0 /* FP64 direct sum, reference operation order  */
+#define RF_FORM_FP64        0 /* FP64 direct sum, a fixed order of its own
+                               * (not the reference's): a few 1e-15 relative
+                               * RMS, 1e-12 at arguments of ~1e4              */
 #define RF_FORM_FP32        1 /* FP64 k.x mod 2pi, FP32 cos, FP32 accumulate */
 #define RF_FORM_MFMA_F16    2 /* [cos Kx|sin Kx].[A cos;-A sin] FP16 hi/lo   */
 #define RF_FORM_MFMA_BF16   3 /* same with BF16 hi/lo                         */

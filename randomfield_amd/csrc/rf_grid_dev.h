@@ -28,14 +28,11 @@ typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
 typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
 
 // Fused blend: the group-grid column offset of plane column n, or -1 where
-// another field also covers it; the group row offset of row m, or -1.
+// another field also covers it.
 __device__ __forceinline__ int64_t grp_col(const rf_gemm_desc& g, int n) {
     const int x = n % g.grpNx, y = n / g.grpNx;
     return (x >= g.grpXlo && x < g.grpXhi && y >= g.grpYlo && y < g.grpYhi)
                ? g.grpCol0 + x + g.grpG0 * (int64_t)y : (int64_t)-1;
-}
-__device__ __forceinline__ int64_t grp_row(const rf_gemm_desc& g, int m) {
-    return (m >= g.grpZlo && m < g.grpZhi) ? g.grpRow0 + g.grpPlaneG * (int64_t)m : (int64_t)-1;
 }
 // Fused blend: plane column n inside a first-axis overlap band sits in the
 // band array of its side (*side 0 low, 1 high) at element offset (return) +

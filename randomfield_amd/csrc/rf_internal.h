@@ -197,14 +197,14 @@ struct rf_field_plan {
     double* d_kRad = nullptr;    // isotropic: radii kN
     double* d_kRev = nullptr;    // shared k / (2 pi)
     double* d_kIso = nullptr;    // per-realization k: Nmc x kN x nDim
-    double* d_kIsoT = nullptr;   // FP32 isotropic form: kN x Rpad x nDim, revolutions
+    double* d_kIsoT = nullptr;   // FP32 isotropic form: kA [block][kx, ky, kz, phase][16 rows], revolutions (rf_iso_rows)
     double* d_Sk = nullptr;      // isotropic spectral density
     uint8_t* d_calc = nullptr;   // Nmc flags
     double* d_phase = nullptr;   // Nmc x kN radians (2*pi_ref*U or psi)
     double* d_amp = nullptr;     // Nmc x kN amplitudes (before ampMult)
     double* d_uni = nullptr;     // device copy of the phase uniforms
     float* d_phT = nullptr;      // kN x Rpad   FP32 phase in revolutions
-    float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult
+    float* d_aT = nullptr;       // kN x Rpad   FP32 amplitude * ampMult; isotropic: aA [block][row % 4][row / 4]
     void* d_B = nullptr;         // MFMA coefficient panels (hi, lo)
     void* d_Bw = nullptr;        // the general form's panels beside the product form's (many realizations)
     bool lat = false;            // MFMA forms: product form of the lattice (rf_lat.hip)
