@@ -43,14 +43,20 @@ int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // F16: 1364 against 3190; 5,000 x 256: 225 against 991, its K-steps split over the
 // waves).  In 2-D, where the per-axis sines weigh against few wavevectors, from 65
 // realizations: 300,000 x 100 176 against 141, 500,000 x 64 151 against 165.
-// BF16 stays with it for two rounds of its blocks (128 points x 64 realizations) only:
-// 256 realizations, kN 2,048, three and four rounds 1.0-1.2 times the general form's
-// time.  The FP16 general form would be the faster one there too on small lattices
-// (32,768 x 129: 2-D kN 392 44 us against 73), but with 1.7 times the error.
+// BF16 returns to the general form where the product form's one-per-CU blocks (128
+// points x 64 realizations) take more rounds than measured to be the faster.  Time against
+// the general form's at two, three and four rounds, 256 realizations: 3-D, 10,976
+// wavevectors 0.5, 0.8 and 0.9-1.0; 1,372 to 5,324 0.5-0.75, 0.7-1.0 and 1.0-1.2; 256 and 500
+// below 0.9, 1.1-1.2 and 1.3; 2-D, 200 to 882, 0.8-1.0 and 1.1-1.3, 128 realizations at two
+// rounds 1.0-1.2.  The FP16 general form would be the faster one there too on small
+// lattices (32,768 x 129: 2-D kN 392 44 us against 73), but with 1.7 times the error.
 bool use_lat(const rf_field_plan* P, int64_t N) {
     if (!P->lat || !P->d_Bw) return P->lat;
-    const bool many = P->p.form == RF_FORM_MFMA_BF16 && (N + 127) / 128 * (P->Rpad / 64) > 512;
-    return N <= kLatSmallN && !many;
+    if (N > kLatSmallN) return false;
+    if (P->p.form != RF_FORM_MFMA_BF16) return true;
+    const int64_t kN = P->spec.info.kNTotal;
+    const int rounds = P->p.nDim == 3 ? (kN >= 8000 ? 4 : kN >= 1300 ? 3 : 2) : P->Rpad > 128 ? 2 : 1;
+    return (N + 127) / 128 * (P->Rpad / 64) <= 256 * rounds;
 }
 
 // Form-specific operand build from d_phase / d_amp (Nmc x kN, FP64).

@@ -67,13 +67,14 @@ __device__ __forceinline__ void prod_pair<b8>(float x0, float x1, float y, unsig
 // K-steps per stage and K-group (8 KB of panels)
 constexpr int lat_steps(int MT) { return MT == 1 ? 4 : 2; }
 constexpr int lat_units(int KG) { return 512 * KG; }   // 16-byte units of a stage
-// The accumulators of every 32 K-steps (16 of a group of up to 64, where they
-// cost nothing) are added to the running sums.  FP16 error of 33,000 points in 2-D
-// boxes of 7 and 10 correlation lengths, one serial sum of the 28 and 56 steps:
-// 2.8e-7 and 3.8e-7, more than the general form's 2.7e-7 and 3.6e-7; so 1.9e-7 and
-// 2.0e-7.  3-D, 10 correlation lengths (1,400 steps): 5e-6 in one sum, 3.9e-7 by 64,
-// 3.1e-7 by 32, 2.9e-7 by 16, which costs 1.5-3 % (32: 0.5 %).
-constexpr int lat_flush(int64_t nG) { return nG <= 64 ? 16 : 32; }
+// The accumulators of 64 K-steps, of 16 where a group has up to 128, are added to the
+// running sums: a serial FP32 accumulation over all ~1,400 steps of a 10-correlation-
+// length lattice is off by 5e-6, so by 4e-7 (general form 1.9e-6).  On short groups 64
+// are nearly one sum: FP16 errors of 33,000 points in 2-D boxes of 7 and 10 correlation
+// lengths (28 and 56 steps) were 2.8e-7 and 3.8e-7, in a 3-D box of 3 (75) 4.0e-7, more
+// than the general form's 2.7e-7, 3.6e-7 and 3.8e-7; so 1.9e-7, 2.0e-7 and 2.1e-7.  (16
+// everywhere: 1.5-3 % of the time.)
+constexpr int lat_flush(int64_t nG) { return nG <= 128 ? 16 : 64; }
 // BF16 halves carry eight bits each, and the dropped product of the low halves is
 // a third of the form's error variance.  Products of sines and cosines lie less
 // near 1, where a rounding weighs least, than the general form's single sines do:
@@ -81,8 +82,8 @@ constexpr int lat_flush(int64_t nG) { return nG <= 64 ? 16 : 32; }
 // realizations: 4.25e-6 against 3.94e-6).  So the first kLatLowPart-th of the K-steps --
 // the slow axis' long waves, most of the field -- takes it too: 3.66e-6 for 5-8 % of
 // the time (on every step 3.38e-6 for up to 20 %).  Where the K-steps are split over
-// groups of waves every step does: a line inside a group's steps spills (39 % against
-// 8-17 %).
+// groups of waves every other stage does (3.84e-6 for 3-9 %): two loops spill there
+// (39 %), and a choice per step does in both shapes.
 constexpr int kLatLowPart = 3;
 
 // One block: points pt0 .. pt0 + 32 W - 1 (clipped to a.i1), M-tiles mt0 ..
@@ -278,19 +279,24 @@ __device__ __forceinline__ void lat_block(const rf_sum_args& a, const rf_lat_dev
         if (u + 1 < nStages) stash(nxt);
         __syncthreads();
     };
-    auto stages = [&](int64_t u0, int64_t u1, auto lowToo) {                      // u0 even
+    auto stages = [&](int64_t u0, int64_t u1, auto even, auto odd) {              // u0 even
         for (int64_t u = u0; u < u1; u += 2) {
-            stage(u, panA, panB, lowToo);
-            if (u + 1 < nStages) stage(u + 1, panB, panA, lowToo);
+            stage(u, panA, panB, even);
+            if (u + 1 < nStages) stage(u + 1, panB, panA, odd);
         }
     };
-    int64_t low = 0;                                    // the same in every wave of the block
-    if constexpr (std::is_same<V, b8>::value) {
-        low = KG == 1 ? (nStages + 2 * kLatLowPart - 1) / (2 * kLatLowPart) * 2 : nStages;
+    const std::true_type with{};
+    const std::false_type without{};
+    if constexpr (!std::is_same<V, b8>::value) {
+        stages(0, nStages, without, without);
+    } else if constexpr (KG == 1) {
+        int64_t low = (nStages + 2 * kLatLowPart - 1) / (2 * kLatLowPart) * 2;
         if (low > nStages) low = nStages;
-        stages(0, low, std::true_type());
+        stages(0, low, with, with);
+        stages(low, nStages, without, without);
+    } else {
+        stages(0, nStages, with, without);
     }
-    if constexpr (!std::is_same<V, b8>::value || KG == 1) stages(low, nStages, std::false_type());
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
