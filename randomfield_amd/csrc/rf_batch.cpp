@@ -340,8 +340,8 @@ int rf_grid_batch_redraw(rf_grid_batch* B, int64_t drawIndex, void* stream) {
     const hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
     // where a wave holds the whole first axis, the first contraction forms the
     // coefficients of the current draw itself (no fold, no coefficient round trip
-    // through HBM: 32 fields of ~131^3 x 16 1.44 ms; fold and split contraction 0.73 +
-    // 1.13); otherwise the grouped fold stores them.  Not the autotuner's choice: that
+    // through HBM: 32 fields of ~131^3 x 16 1.44 ms; fold and contraction of the stored 0.73 +
+    // 0.89); otherwise the grouped fold stores them.  Not the autotuner's choice: that
     // times the contraction of stored coefficients.
     const bool gen = B->formMt > 0;
     RF_HIP_TRY(ctx, rf_launch_draw_counter(B->d_draw, drawIndex >= 0 ? drawIndex : -1, gen ? 1 : 0, s));
